@@ -5,11 +5,14 @@
 
 namespace sfno {
 
-// both answer SFNO_EUNSUPPORTED for a length the part does not hold
+// all answer SFNO_EUNSUPPORTED for a length the part does not hold
 #define SFNO_FFT_PART_DECL(P)                                                                                                 \
     int fft_part_lon_##P(bool inverse, const FftPlan& p, const void* in, void* out, int64_t rows, int nlat, int mmax, int ld, int grid_dtype, \
                          hipStream_t s, float2* lat_stats);                                                                   \
-    int fft_part_lat_##P(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s)
+    int fft_part_lat_##P(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);   \
+    int fft_part_rows_##P(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s); \
+    int fft_part_cols_##P(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, \
+                          const float* mscale, hipStream_t s)
 SFNO_FFT_PART_DECL(A);
 SFNO_FFT_PART_DECL(B);
 SFNO_FFT_PART_DECL(C);
@@ -27,6 +30,12 @@ SFNO_FFT_PART_DECL(F);
     case N_:                                                                                                                  \
         if constexpr (N_ <= kLatMax) return go_lat<N_, A_, B_, C_>(inverse, p, in, out, mmax, lmax, ld, mscale, s);           \
         break;
+#define SFNO_FFT_ROWS_CASE(N_, A_, B_, C_) \
+    case N_: return go_rows<N_, A_, B_, C_>(inverse, p, in, out, rows, nlat, mmax, cs, s);
+#define SFNO_FFT_COLS_CASE(N_, A_, B_, C_)                                                                                    \
+    case N_:                                                                                                                  \
+        if constexpr (N_ <= kLatMax) return go_cols<N_, A_, B_, C_>(inverse, p, in, out, rows, mmax, lmax, mscale, s); \
+        break;
 // the definition of one part: instantiates every kernel of its lengths
 #define SFNO_FFT_PART(P, LENGTHS)                                                                                             \
     namespace sfno {                                                                                                          \
@@ -37,6 +46,15 @@ SFNO_FFT_PART_DECL(F);
     }                                                                                                                         \
     int fft_part_lat_##P(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s) { \
         switch (p.n) { LENGTHS(SFNO_FFT_LAT_CASE) }                                                                           \
+        return SFNO_EUNSUPPORTED;                                                                                             \
+    }                                                                                                                         \
+    int fft_part_rows_##P(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s) { \
+        switch (p.n) { LENGTHS(SFNO_FFT_ROWS_CASE) }                                                                          \
+        return SFNO_EUNSUPPORTED;                                                                                             \
+    }                                                                                                                         \
+    int fft_part_cols_##P(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, \
+                          const float* mscale, hipStream_t s) {                                                               \
+        switch (p.n) { LENGTHS(SFNO_FFT_COLS_CASE) }                                                                          \
         return SFNO_EUNSUPPORTED;                                                                                             \
     }                                                                                                                         \
     }

@@ -117,6 +117,26 @@ int latfft_fast_launch(bool inverse, const FftPlan& p, const float* in, float* o
     return SFNO_EUNSUPPORTED;
 }
 
+int fft_col_shift(int n) { return n <= kLatMax && find_fast(n) ? col_shift(n) : 0; }
+
+int fft_rows_launch(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s) {
+    for (auto part : {fft_part_rows_A, fft_part_rows_B, fft_part_rows_C, fft_part_rows_D, fft_part_rows_E, fft_part_rows_F}) {
+        const int rc = part(inverse, p, in, out, rows, nlat, mmax, cs, s);
+        if (rc != SFNO_EUNSUPPORTED) return rc;
+    }
+    return SFNO_EUNSUPPORTED;
+}
+
+int fft_cols_launch(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, const float* mscale,
+                    hipStream_t s) {
+    if (lmax < 1 || lmax > p.n || mmax < 1 || !mscale) return SFNO_EINVAL;
+    for (auto part : {fft_part_cols_A, fft_part_cols_B, fft_part_cols_C, fft_part_cols_D, fft_part_cols_E, fft_part_cols_F}) {
+        const int rc = part(inverse, p, in, out, rows, mmax, lmax, mscale, s);
+        if (rc != SFNO_EUNSUPPORTED) return rc;
+    }
+    return SFNO_EUNSUPPORTED;
+}
+
 int fft_fast_plan_init(FftPlan& p) {
     const FastEntry* f = find_fast(p.n);
     return f ? upload_pass_twiddles(*f, p) : SFNO_OK;

@@ -797,6 +797,227 @@ __global__ __launch_bounds__(FT) void latfft_fast_kernel(const float2* __restric
     }
 }
 
+// ---- planar pair on the reference layout ----------------------------------------------------------------------
+// RealFFT2 / InverseRealFFT2 have no Legendre stage that wants the channels side by side, so between the grid and the reference
+// coefficients [row][lmax][mmax] they go through an intermediate buffer y[row][group][nlat][C] of groups of C neighbouring orders (C = 8 or 16,
+// by the latitude length): real FFTs along the grid rows, then complex FFTs along latitude, a group at a time (one contiguous
+// block of y), that leave in the reference layout -- four kernels and passes over memory for the pair where the order-major
+// buffers and their layout passes take six.  The two latitudes of a row pair fill whole 128-byte lines of y. 720 x 1440, 73 channels:
+// 878 -> 599 us per pair (rows 131 + 133 us, columns 176 + 178).
+//
+// Rows.  Two neighbouring latitudes of a channel share one complex sequence; a tile is S such pairs, persistent workgroups as in
+// the order-major kernels above (next tile requested into registers before the passes, unconditional requests and stores: a pair
+// slot past the end repeats the last pair, a last latitude without a partner is its own partner).
+struct RowPair {
+    int64_t a, b;            // grid rows of the pair
+    int r, lat;              // its channel and first latitude
+    __device__ __forceinline__ RowPair(int pair, int npairs, int npl, int nlat) {
+        const int q = pair < npairs ? pair : npairs - 1;
+        r = q / npl;
+        lat = 2 * (q - r * npl);
+        a = (int64_t)r * nlat + lat;
+        b = lat + 1 < nlat ? a + 1 : a;
+    }
+    // element of y that holds order m of the first row; order m + u TP (TP a multiple of C) lies u TP nlat further on, the second
+    // row's value (b - a) C further on
+    __device__ __forceinline__ int64_t y_index(int m, int ng, int cs, int nlat) const {
+        return ((((int64_t)r * ng + (m >> cs)) * nlat + lat) << cs) + (m & ((1 << cs) - 1));
+    }
+};
+
+template <int N, int R0, int R1, int R2, int S, int FT>
+__global__ __launch_bounds__(FT, 4) void rows_fwd_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
+                                                         const float* __restrict__ x, float2* __restrict__ y, int npairs, int npl, int nlat, int mmax, int ng, int cs,
+                                                         float scale) {
+    using G = Geo<N, R0, R1, R2>;
+    __shared__ __align__(16) float2 z[S * G::PITCH];
+    __shared__ LdsTables<N, R0, R1, R2> tab;
+    const int tid = threadIdx.x;
+    constexpr int TP = FT / S, Q = N / 4, IT = (Q + TP - 1) / TP;
+    constexpr int NSW = (N / 2 + 1 + TP - 1) / TP;
+    const int pl = tid / TP, q0 = tid - pl * TP;
+    const int ntiles = (npairs + S - 1) / S;
+    int t = blockIdx.x;
+    if (t >= ntiles) return;
+    lds_tables<N, R0, R1, R2, FT>(tab, tw0, tw1, post, tid);
+    float4 a[IT], b[IT];
+    auto request = [&](int tile) {
+        const RowPair rp(tile * S + pl, npairs, npl, nlat);
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const bool in = (it + 1) * TP <= Q || q0 + it * TP < Q;
+            const int off = in ? 4 * (q0 + it * TP) : 0;
+            a[it] = *reinterpret_cast<const float4*>(x + rp.a * N + off);
+            b[it] = *reinterpret_cast<const float4*>(x + rp.b * N + off);
+        }
+    };
+    const float h = 0.5f * scale;
+    const float2* zz = z + pl * G::PITCH;
+    request(t);
+    for (;;) {
+        const int tn = t + gridDim.x;
+        const RowPair rp(t * S + pl, npairs, npl, nlat);
+        {
+            float4* dst = reinterpret_cast<float4*>(z + pl * G::PITCH) + 2 * q0;
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                use_here(a[it]);
+                use_here(b[it]);
+            }
+#pragma unroll
+            for (int it = 0; it < IT; ++it)
+                if ((it + 1) * TP <= Q || q0 + it * TP < Q) {
+                    dst[2 * it * TP] = make_float4(a[it].x, b[it].x, a[it].y, b[it].y);
+                    dst[2 * it * TP + 1] = make_float4(a[it].z, b[it].z, a[it].w, b[it].w);
+                }
+        }
+        request(tn < ntiles ? tn : t);
+        __syncthreads();
+        passes_dif<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+        float2* ya = y + rp.y_index(q0, ng, cs, nlat);
+        float2* yb = ya + ((rp.b - rp.a) << cs);
+        const int64_t ystep = (int64_t)TP * nlat;
+#pragma unroll
+        for (int u = 0; u < NSW; ++u)
+            if (q0 + u * TP < mmax) {
+                const unsigned pp = tab.post[q0 + u * TP];
+                const float2 zp = zz[pp & 0xffffu], zq = zz[pp >> 16];
+                ya[u * ystep] = make_float2(h * (zp.x + zq.x), h * (zp.y - zq.y));
+                yb[u * ystep] = make_float2(h * (zp.y + zq.y), h * (zq.x - zp.x));
+            }
+        if (tn >= ntiles) break;
+        __syncthreads();
+        t = tn;
+    }
+}
+
+template <int N, int R0, int R1, int R2, int S, int FT>
+__global__ __launch_bounds__(FT, 4) void rows_inv_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
+                                                         const float2* __restrict__ y, float* __restrict__ x, int npairs, int npl, int nlat, int mmax, int ng, int cs) {
+    using G = Geo<N, R0, R1, R2>;
+    __shared__ __align__(16) float2 z[S * G::PITCH];
+    __shared__ LdsTables<N, R0, R1, R2> tab;
+    const int tid = threadIdx.x;
+    constexpr int HALF = N / 2, TP = FT / S, NSW = (HALF + 1 + TP - 1) / TP;
+    const int pl = tid / TP, q0 = tid - pl * TP;
+    const int ntiles = (npairs + S - 1) / S;
+    int t = blockIdx.x;
+    if (t >= ntiles) return;
+    lds_tables<N, R0, R1, R2, FT>(tab, tw0, tw1, post, tid);
+    float2 va[NSW], vb[NSW];
+    // (an order the plan does not keep reads one of the kept groups instead and is zeroed when it is used)
+    auto request = [&](int tile) {
+        const RowPair rp(tile * S + pl, npairs, npl, nlat);
+        const float2* ya = y + rp.y_index(q0, ng, cs, nlat);
+        const float2* yb = ya + ((rp.b - rp.a) << cs);
+        const int64_t ystep = (int64_t)TP * nlat;
+#pragma unroll
+        for (int u = 0; u < NSW; ++u) {
+            const int64_t off = q0 + u * TP < mmax ? u * ystep : q0 < mmax ? 0 : -((int64_t)(q0 >> cs) * nlat << cs);
+            va[u] = ya[off];
+            vb[u] = yb[off];
+        }
+    };
+    float2* zz = z + pl * G::PITCH;
+    request(t);
+    __syncthreads();                                      // tables
+    for (;;) {
+        const int tn = t + gridDim.x;
+        const RowPair rp(t * S + pl, npairs, npl, nlat);
+#pragma unroll
+        for (int u = 0; u < NSW; ++u) asm volatile("" : "+v"(va[u].x), "+v"(va[u].y), "+v"(vb[u].x), "+v"(vb[u].y));
+#pragma unroll
+        for (int u = 0; u < NSW; ++u) {
+            const int m = q0 + u * TP;
+            if (m <= HALF) {
+                const unsigned pp = tab.post[m];
+                float2 fa = va[u], fb = vb[u];
+                if (m >= mmax) fa = fb = make_float2(0.f, 0.f);
+                if (m == 0 || m == HALF) {
+                    zz[pp & 0xffffu] = make_float2(fa.x, fb.x);                  // C2R: Im of mean and Nyquist bins dropped
+                } else {
+                    zz[pp & 0xffffu] = make_float2(fa.x - fb.y, fa.y + fb.x);
+                    zz[pp >> 16] = make_float2(fa.x + fb.y, fb.x - fa.y);
+                }
+            }
+        }
+        __syncthreads();
+        request(tn < ntiles ? tn : t);
+        passes_dit<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+        {
+            constexpr int Q = N / 4, ITS = (Q + TP - 1) / TP;
+            const float4* src = reinterpret_cast<const float4*>(z + pl * G::PITCH);
+#pragma unroll
+            for (int it = 0; it < ITS; ++it) {
+                int i4 = q0 + it * TP;
+                if ((it + 1) * TP > Q) i4 = i4 < Q ? i4 : Q - 1;
+                const float4 u0 = src[2 * i4], u1 = src[2 * i4 + 1];
+                *reinterpret_cast<float4*>(x + rp.a * N + 4 * i4) = make_float4(u0.x, u0.z, u1.x, u1.z);
+                *reinterpret_cast<float4*>(x + rp.b * N + 4 * i4) = make_float4(u0.y, u0.w, u1.y, u1.w);
+            }
+        }
+        if (tn >= ntiles) break;
+        __syncthreads();
+        t = tn;
+    }
+}
+
+// Columns.  A workgroup transforms C neighbouring orders of one row along latitude: between a group's
+// block of y and pieces of 8 C bytes of the reference layout.  The pieces of one line meet in one XCD's L2: groups are dealt to the
+// XCDs in units of eight.
+constexpr int kColUnit = 8;
+constexpr int col_shift(int n) { return n > 400 ? 3 : 4; }      // log2 of the orders per group
+
+template <int N, int R0, int R1, int R2, int C, int FT, int INV>
+__global__ __launch_bounds__(FT) void cols_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const float2* __restrict__ in,
+                                                  float2* __restrict__ out, int rows, int mmax, int lmax, int ngroups,
+                                                  const float* __restrict__ mscale) {
+    using G = Geo<N, R0, R1, R2>;
+    __shared__ __align__(16) float2 z[C * G::PITCH];
+    const int tid = threadIdx.x;
+    const int q = blockIdx.x >> 3, nu = (ngroups + kColUnit - 1) / kColUnit;
+    const int unit = (q / kColUnit) * 8 + (blockIdx.x & 7);
+    const int row = unit / nu, group = (unit - row * nu) * kColUnit + q % kColUnit;
+    if (row >= rows || group >= ngroups) return;
+    const int lhigh = (lmax + 1) / 2, gap = N - lmax;
+    const int nin = INV ? lmax : N, nout = INV ? N : lmax;
+    const int c = tid & (C - 1), m = group * C + c;
+    const bool live = m < mmax;
+    const int pin = INV ? mmax : C, pout = INV ? C : mmax;
+    const int64_t block = ((int64_t)row * ngroups + group) * N * C + c;
+    const float2* src = in + (INV ? (int64_t)row * nin * mmax + m : block);
+    {
+        // all global loads of the workgroup are issued before the first LDS store
+        constexpr int TOT = C * N, IT = (TOT + FT - 1) / FT;
+        float2 v[IT];
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int i = (tid + it * FT) / C;
+            const int k = !INV ? i : i < lhigh ? i : i >= lhigh + gap ? i - gap : -1;      // (-1: a dropped frequency)
+            v[it] = make_float2(0.f, 0.f);
+            if (i < N && k >= 0 && live) v[it] = src[(int64_t)k * pin];
+        }
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int i = (tid + it * FT) / C;
+            if (i < N) z[c * G::PITCH + (INV ? G::pos(i) : i)] = v[it];
+        }
+    }
+    __syncthreads();
+    if (INV)
+        passes_dit<N, R0, R1, R2, C, FT>(z, tw0, tw1, tid);
+    else
+        passes_dif<N, R0, R1, R2, C, FT>(z, tw0, tw1, tid);
+    if (!live) return;
+    const float sc = mscale[m];
+    float2* dst = out + (INV ? block : (int64_t)row * nout * mmax + m);
+    for (int j = tid / C; j < nout; j += FT / C) {
+        const int i = INV ? j : G::pos(j < lhigh ? j : j + gap);
+        const float2 v = z[c * G::PITCH + i];
+        dst[(int64_t)j * pout] = make_float2(sc * v.x, sc * v.y);
+    }
+}
+
 // Latitude FFT of a length n with a large prime factor (721 = 7 * 103, the 0.25 degree grid with both poles), as a
 // circular convolution of length M >= 2n - 1 on the specialised passes (Bluestein):
 //     X[j] = c[j] sum_k (x[k] c[k]) conj(c)[j - k],   c[k] = exp(-i pi k^2 / n)          (forward; conjugate c for the inverse)
@@ -888,6 +1109,42 @@ int go_lat(bool inverse, const FftPlan& p, const float* in, float* out, int mmax
         hipLaunchKernelGGL((latfft_fast_kernel<N, R0, R1, R2, FT, 1>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, in, out, mmax, lmax, ld, ngroups, mscale);
     else
         hipLaunchKernelGGL((latfft_fast_kernel<N, R0, R1, R2, FT, 0>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, in, out, mmax, lmax, ld, ngroups, mscale);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+template <int N, int R0, int R1, int R2>
+int go_rows(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s) {
+    constexpr int S = (N >= 1024) ? 4 : 8;
+    constexpr int FT = (S * N >= 4096) ? 512 : 256;
+    constexpr int WG_PER_CU = 1024 / FT;
+    static_assert(FT / S % 16 == 0, "a sweep covers whole groups");
+    const int npl = (nlat + 1) / 2, ng = (mmax + (1 << cs) - 1) >> cs;
+    const int64_t npairs = rows * npl;
+    if (npairs > 0x7fffffffLL - S) return SFNO_EUNSUPPORTED;
+    const dim3 grid((unsigned)std::min<int64_t>((npairs + S - 1) / S, std::max(1, WG_PER_CU * p.n_cu)));
+    if (inverse)
+        hipLaunchKernelGGL((rows_inv_kernel<N, R0, R1, R2, S, FT>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, reinterpret_cast<const float2*>(in), out,
+                           (int)npairs, npl, nlat, mmax, ng, cs);
+    else
+        hipLaunchKernelGGL((rows_fwd_kernel<N, R0, R1, R2, S, FT>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, reinterpret_cast<float2*>(out),
+                           (int)npairs, npl, nlat, mmax, ng, cs, (float)(kTwoPi / (double)N));
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+template <int N, int R0, int R1, int R2>
+int go_cols(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, const float* mscale, hipStream_t s) {
+    constexpr int C = 1 << col_shift(N);                // orders per workgroup: 46 KB of LDS at 720 points, 51 KB at 400
+    constexpr int FT = (C * N >= 4096) ? 512 : 256;
+    const int ngroups = (mmax + C - 1) / C, nu = (ngroups + kColUnit - 1) / kColUnit;
+    const int64_t blocks = (rows * nu + 7) / 8 * 8 * kColUnit;
+    if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
+    const dim3 grid((unsigned)blocks);
+    if (inverse)
+        hipLaunchKernelGGL((cols_kernel<N, R0, R1, R2, C, FT, 1>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, in, out, (int)rows, mmax, lmax, ngroups,
+                           mscale);
+    else
+        hipLaunchKernelGGL((cols_kernel<N, R0, R1, R2, C, FT, 0>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, in, out, (int)rows, mmax, lmax, ngroups,
+                           mscale);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

@@ -156,11 +156,11 @@ int legendre_f16_launch(bool analysis, const PgemmArgs& a, int n_work, hipStream
 // ---- FFT (fft.hip) -----------------------------------------------------------------------
 struct FftPlan {
     int n = 0;                     // transform length (nlon)
-    int n_cu = 256;                // compute units of the plan's device (sizes the persistent grids of fft_fast.hip)
+    int n_cu = 256;                // compute units of the plan's device (sizes the persistent grids of the specialised kernels)
     int npass = 0;
     int radix[24];
     float2* d_tw = nullptr;        // [n] exp(-2 pi i j / n)
-    float2* d_tw0 = nullptr;       // inter-pass twiddles of the specialised kernels (fft_fast.hip)
+    float2* d_tw0 = nullptr;       // inter-pass twiddles of the specialised kernels (fft_kernels.h)
     float2* d_tw1 = nullptr;
     unsigned* d_post = nullptr;    // [n/2+1] LDS slot of bin m (low half) and of bin n - m (high half) around the specialised passes
     // latitude plans of lengths with a large prime factor (fft_chirp_plan_init): the DFT as a circular convolution of
@@ -177,6 +177,13 @@ int fft_fast_launch(bool inverse, const FftPlan& p, const void* in, void* out, i
                     hipStream_t s, float2* lat_stats = nullptr);
 // latitude FFT on the specialised passes; SFNO_EUNSUPPORTED for a length without them
 int latfft_fast_launch(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
+// planar pair on the reference layout: real FFTs along the grid rows, x [rows][nlat][n] <-> y [rows][group][nlat][2^cs] complex (groups
+// of 2^cs orders; forward scaled by 2 pi / n), and complex FFTs along latitude, y <-> coefficients [rows][lmax][mmax] (outputs times
+// mscale[m]); lengths with specialised kernels only.  cs is fft_col_shift of the latitude length, 0 if it has none
+int fft_col_shift(int n);
+int fft_rows_launch(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s);
+int fft_cols_launch(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, const float* mscale,
+                    hipStream_t s);
 int fft_plan_init(FftPlan& p, int n);
 // adds the chirp tables to a latitude plan whose length has no specialised passes and a prime factor above 7 (no-op otherwise)
 int fft_chirp_plan_init(FftPlan& p);
