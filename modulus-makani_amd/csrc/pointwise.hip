@@ -12,9 +12,9 @@
 // per pixel of its pair; MFMA column q of N-tile t then stands for pixel 2q + t, so every lane ends up
 // with 2 consecutive pixels of each output row and stores them as one 4-byte piece.
 // Two kernels.  Convolutions with at most 96 output channels (pw_gemm_kernel): a wavefront owns 96 rows x 64
-// pixels, eight wavefronts side by side along the pixels; weights come from global memory (L2 resident) as A
+// pixels, eight (or, for few pixels, two) wavefronts side by side along the pixels; weights come from global memory (L2 resident) as A
 // fragments, packed so that a fragment is 1 KiB of consecutive memory, activations through a triple-buffered LDS
-// stage, both prefetched in registers.  All others (pw_gemm_dma_kernel, further down): 384 rows x 256 pixels per
+// stage, both prefetched in registers.  All others (pw_gemm_dma_kernel, further down): 128, 256 or 384 rows x 256 pixels per
 // workgroup with both operand streams loaded straight into LDS.
 #include "sfno_internal.h"
 #include <type_traits>
@@ -31,7 +31,7 @@ constexpr int PW_MT = 3;          // 32-row tiles per wavefront
 constexpr int PW_ROWS = 32 * PW_MT;
 constexpr int PW_KC = 16;         // k rows per MFMA K step
 constexpr int PW_KS = 2;          // MFMA K steps per chunk (one LDS stage, one barrier)
-constexpr int PW_KALIGN = 128;    // K is padded to whole unrolled loop bodies (PW_KC * prefetch distance)
+constexpr int PW_KALIGN = 64;     // K is padded to whole unrolled loop bodies (PW_KC * prefetch distance)
 
 __device__ __forceinline__ float bf16_to_f(unsigned short h) { return __uint_as_float((unsigned int)h << 16); }
 __device__ __forceinline__ unsigned short f_to_bf16(float f) { return __builtin_bit_cast(unsigned short, (__bf16)f); }
@@ -68,21 +68,17 @@ __device__ __forceinline__ float gelu(float x) {
     return fmaf(-fabsf(x), __builtin_amdgcn_exp2f(q), __builtin_amdgcn_fmed3f(x, 0.f, __builtin_inff()));
 }
 
-// WM = wavefronts along the output rows: 4 (x 2 along pixels: 384 rows x 128 pixels per workgroup) or
-// 1 (x 8 along pixels: 96 rows x 512 pixels, for convolutions with few output channels)
-// NT = pixels per lane = N tiles per wavefront: 2 (eight wavefronts of 96 x 64, two per SIMD) or 4 (four wavefronts of
-// 96 x 128, one per SIMD, half the weight-fragment traffic per MFMA)
-template <int WM, int NT>
-__global__ __launch_bounds__(NT == 2 ? 512 : 256) void pw_gemm_kernel(PointwiseArgs a) {
-    constexpr int NW = (NT == 2) ? 8 : 4;         // wavefronts per workgroup
+// NW = wavefronts per workgroup, side by side along the pixels, 64 pixels each: 8, or 2 where that leaves CUs idle
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
+    constexpr int NT = 2;                         // pixels per lane = N tiles per wavefront
     constexpr int PW_THREADS = 64 * NW;
     constexpr int PW_PX = 32 * NT;                // pixels per wavefront
-    constexpr int WN = NW / WM;
-    constexpr int WPX = WN * PW_PX;               // pixels per workgroup
+    constexpr int WPX = NW * PW_PX;               // pixels per workgroup
     constexpr int PITCH = WPX * 2 + 16;           // bytes per LDS row
     constexpr int CK = PW_KC * PW_KS;             // k rows per chunk = per loop step
     constexpr int STAGE = CK * PITCH;
-    constexpr int D = (WM == 4) ? 4 : 2;          // prefetch distance in chunks
+    constexpr int D = 2;                          // prefetch distance in chunks
     constexpr int XW = CK * WPX * 2 / (16 * PW_THREADS);   // 16-byte pieces of the activation chunk per thread
     static_assert(PW_KALIGN % (CK * D) == 0, "loop body divides the padded K");
     static_assert(CK * WPX * 2 == XW * 16 * PW_THREADS, "chunk split evenly over the threads");
@@ -98,8 +94,8 @@ __global__ __launch_bounds__(NT == 2 ? 512 : 256) void pw_gemm_kernel(PointwiseA
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane & 31, ko = lane >> 5;
-    const int o0 = ob * (PW_ROWS * WM) + (wave / WN) * PW_ROWS;
-    const int pxw = (wave % WN) * PW_PX;                                  // wavefront's pixel offset inside the stage
+    const int o0 = ob * PW_ROWS;
+    const int pxw = wave * PW_PX;                                         // wavefront's pixel offset inside the stage
 
     // input channels k < K1 come from X, the others (if any) from X2: a convolution over the concatenation of two tensors
     const int K1 = a.X2 ? a.K1 : a.K;
@@ -215,13 +211,16 @@ __global__ __launch_bounds__(NT == 2 ? 512 : 256) void pw_gemm_kernel(PointwiseA
         }
     }
 
-    // epilogue: lane holds rows 8 (v / 4) + 4 ko + v % 4 of each 32-row tile and pixels NT q .. NT q + NT - 1
+    // epilogue: lane holds rows 8 (v / 4) + 4 ko + v % 4 of each 32-row tile and pixels 2 q, 2 q + 1.  Bias, scale and shift come
+    // through the scalar unit, the rows of both lane halves: a vector load between the stores would make every store wait for the
+    // one before it (the counter retires in order).
     const int64_t px = pw0 + pxw + NT * q;
     if (px >= a.P) return;
     unsigned short* __restrict__ Y = a.Y + (int64_t)b * a.O * a.P;
     const unsigned short* __restrict__ R = a.addend ? a.addend + (int64_t)b * a.O * a.P : nullptr;
 #pragma unroll
     for (int mt = 0; mt < PW_MT; ++mt) {
+        if (o0 + 32 * mt >= a.O) break;
         rw_t rv[16];
         if (R) {
             // all addend loads of the tile first
@@ -232,38 +231,43 @@ __global__ __launch_bounds__(NT == 2 ? 512 : 256) void pw_gemm_kernel(PointwiseA
             }
         }
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int o = o0 + 32 * mt + 8 * (v >> 2) + 4 * ko + (v & 3);
-            if (o >= a.O) continue;
-            const float bs = a.bias ? a.bias[o] : 0.f;
-            float y[NT];
+        for (int g = 0; g < 4; ++g) {
+            const int og = o0 + 32 * mt + 8 * g;                        // rows og .. og + 7 (ko = 0: the first four)
+            float ub[8], usc[8], ush[8];
 #pragma unroll
-            for (int t = 0; t < NT; ++t) y[t] = acc[mt][t][v] + bs;
-            if (a.act == SFNO_ACT_GELU) {
-#pragma unroll
-                for (int t = 0; t < NT; ++t) y[t] = gelu(y[t]);
+            for (int i = 0; i < 8; ++i) {
+                const int64_t u = min(og + i, a.O - 1);
+                ub[i] = a.bias ? uniform_load(a.bias, u) : 0.f;
+                usc[i] = R && a.add_scale ? uniform_load(a.add_scale, (int64_t)b * a.O + u) : 1.f;
+                ush[i] = R && a.add_shift ? uniform_load(a.add_shift, (int64_t)b * a.O + u) : 0.f;
             }
-            if (R) {
-                const float sc = a.add_scale ? a.add_scale[(int64_t)b * a.O + o] : 1.f;
-                const float sh = a.add_shift ? a.add_shift[(int64_t)b * a.O + o] : 0.f;
 #pragma unroll
-                for (int pp = 0; pp < NT / 2; ++pp) {
-                    y[2 * pp] += fmaf(sc, __uint_as_float(rv[v][pp] << 16), sh);
-                    y[2 * pp + 1] += fmaf(sc, __uint_as_float(rv[v][pp] & 0xffff0000u), sh);
+            for (int j = 0; j < 4; ++j) {
+                const int v = 4 * g + j, o = og + 4 * ko + j;
+                if (o >= a.O) continue;
+                const float bs = ko ? ub[4 + j] : ub[j];
+                float y0 = acc[mt][0][v] + bs, y1 = acc[mt][1][v] + bs;
+                if (a.act == SFNO_ACT_GELU) {
+                    y0 = gelu(y0);
+                    y1 = gelu(y1);
                 }
+                if (R) {
+                    const float sc = ko ? usc[4 + j] : usc[j], sh = ko ? ush[4 + j] : ush[j];
+                    y0 += fmaf(sc, __uint_as_float(rv[v][0] << 16), sh);
+                    y1 += fmaf(sc, __uint_as_float(rv[v][0] & 0xffff0000u), sh);
+                }
+                rw_t out;
+                out[0] = bf16_pair(y0, y1);
+                *reinterpret_cast<rw_t*>(Y + (int64_t)o * a.P + px) = out;
             }
-            rw_t out;
-#pragma unroll
-            for (int pp = 0; pp < NT / 2; ++pp) out[pp] = bf16_pair(y[2 * pp], y[2 * pp + 1]);
-            *reinterpret_cast<rw_t*>(Y + (int64_t)o * a.P + px) = out;
         }
     }
 }
 
 // ---- tall variant with direct-to-LDS loads ----------------------------------------------------------
 // For O > 96 the kernel above is bound by the weight fragments every wavefront pulls through L1 for only 6 MFMAs
-// each.  This variant gives a wavefront 96 rows x 128 pixels (3 x 4 tiles, 192 accumulator registers), eight
-// wavefronts per workgroup (384 rows x 256 pixels, half the weight traffic per pixel), and moves both operand
+// each.  This variant gives a wavefront up to 96 rows x 128 pixels (3 x 4 tiles, 192 accumulator registers), eight
+// wavefronts per workgroup (up to 384 rows x 256 pixels, half the weight traffic per pixel), and moves both operand
 // streams with global_load_lds_dwordx4: lane i's 16 bytes land at LDS base + 16 i, no staging registers.
 //
 // One persistent workgroup per CU walks its tiles as one unbroken stream of 32-row K chunks, so the operands of the
@@ -277,17 +281,28 @@ __global__ __launch_bounds__(NT == 2 ? 512 : 256) void pw_gemm_kernel(PointwiseA
 // and the waits are written out by hand.  Other memory operations of a wavefront (the epilogue's stores and addend
 // loads) are older than the loads a wait is meant for or younger than all of them; either way the wait covers
 // at least the loads it is meant for.
-constexpr int DM_MT = 3, DM_NT = 4;
-constexpr int DM_ROWS = 4 * 32 * DM_MT;          // 384 rows per workgroup
+//
+// MT = 32-row tiles per wavefront: 128 MT rows per workgroup.  Rows past the matrix are multiplied all the same, so MT follows the
+// number of output channels (pointwise_mt); with MT = 1 a workgroup needs half of the registers and, with three activation
+// stages, half of the LDS, and two of them share a CU.
+constexpr int DM_NT = 4;
 constexpr int DM_PX = 2 * 32 * DM_NT;            // 256 pixels per workgroup
 constexpr int DM_CK = 32;                        // k rows per chunk
-constexpr int DM_ABYTES = 2 * (DM_ROWS / 32) * 1024;   // weight stage: 24 fragment blocks of 1 KiB
 constexpr int DM_XBLK = 1024 + 16;               // two pixel rows of the chunk (2 x 512 bytes) + padding
 constexpr int DM_XBYTES = (DM_CK / 2) * DM_XBLK; // activation stage
-constexpr int DM_WSTAGES = 3, DM_XSTAGES = 5;    // chunks in LDS or on their way, per stream
-constexpr int DM_XBASE = DM_WSTAGES * DM_ABYTES;
-constexpr int DM_LDS = DM_XBASE + DM_XSTAGES * DM_XBYTES;
-static_assert(DM_LDS <= 160 * 1024, "one workgroup per CU");
+constexpr int DM_WSTAGES = 3;                    // weight chunks in LDS or on their way
+template <int MT>
+struct DmGeo {
+    static constexpr int ROWS = 4 * 32 * MT;         // rows per workgroup
+    static constexpr int ABYTES = 2 * (ROWS / 32) * 1024;   // weight stage: 8 MT fragment blocks of 1 KiB
+    static constexpr int XSTAGES = MT == 1 ? 3 : 5;  // activation chunks in LDS or on their way
+    static constexpr int XBASE = DM_WSTAGES * ABYTES;
+    static constexpr int LDS = XBASE + XSTAGES * DM_XBYTES;
+    static constexpr int WG_PER_CU = MT == 1 ? 2 : 1;
+    static_assert(WG_PER_CU * LDS <= 160 * 1024, "resident workgroups");
+};
+// s_waitcnt immediate: at most n vector memory operations in flight, no LDS operation
+constexpr int dm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | 0x70; }
 
 // M0 carries the LDS destination.  The compiler refuses "m0" in a clobber list (a reserved register), so nothing may
 // keep a value in M0 across this call: the kernels that use it index no register array dynamically and use no
@@ -307,9 +322,10 @@ __device__ __forceinline__ void dm_barrier() {
 }
 
 // GELU: exact GELU on the output; ADD: "+ scale * addend + shift"
-template <bool GELU, bool ADD>
-__global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
-    __shared__ __align__(16) unsigned char lds[DM_LDS];
+template <int MT, bool GELU, bool ADD>
+__global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_kernel(PointwiseArgs a) {
+    using DM = DmGeo<MT>;
+    __shared__ __align__(16) unsigned char lds[DM::LDS];
     // tiles of this XCD, row block fastest: q -> (row block q % n_oblk, strip (q / n_oblk) * 8 + xcd); the workgroups of the
     // XCD deal them out round robin, so the row blocks of one strip run at the same time on one L2
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, nslot = gridDim.x >> 3;
@@ -340,7 +356,7 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
         pw0 = (int64_t)(sl - (unsigned)b * n_strips) * DM_PX;
     };
 
-    // load stream of this wavefront: weight blocks (row blocks 3 lw .. 3 lw + 2 of both 16-row k steps), or activation blocks
+    // load stream of this wavefront: weight blocks (row blocks MT lw .. MT lw + MT - 1 of both 16-row k steps), or activation blocks
     // 4 lw .. 4 lw + 3 (block xb = rows 2 xb, 2 xb + 1 of the chunk; lane = row (lane >> 5), 8 pixels (lane & 31))
     int iq = slot, ic = 0, isg = 0;                             // next chunk to ask for: tile, chunk, stage
     const unsigned short *sp0 = nullptr, *sp1 = nullptr;        // wavefront-uniform bases of the stream's tile
@@ -352,7 +368,7 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
             int64_t pw0;
             tile_of(iq, ob, b, pw0);
             if (wload) {
-                sp0 = a.W + ((int64_t)(ob * (DM_ROWS / 32) + 3 * lw) * nc16) * 512;
+                sp0 = a.W + ((int64_t)(ob * (DM::ROWS / 32) + MT * lw) * nc16) * 512;
             } else {
                 sp0 = a.X + (int64_t)b * K1 * a.P;
                 sp1 = a.X2 ? a.X2 + (int64_t)b * (a.K - K1) * a.P : sp0;
@@ -360,15 +376,15 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
             }
         }
         if (wload) {
-            const unsigned sb = lds0 + isg * DM_ABYTES + 3 * lw * 1024;
+            const unsigned sb = lds0 + isg * DM::ABYTES + MT * lw * 1024;
             const unsigned short* src = sp0 + (int64_t)ic * 1024 + voff;
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-                for (int i = 0; i < 3; ++i) dma16(src + ks * 512 + i * wrb, sb + (ks * 12 + i) * 1024);
+                for (int i = 0; i < MT; ++i) dma16(src + ks * 512 + i * wrb, sb + (ks * 4 * MT + i) * 1024);
             isg = (isg == DM_WSTAGES - 1) ? 0 : isg + 1;
         } else {
-            const unsigned sb = lds0 + DM_XBASE + isg * DM_XBYTES + 4 * lw * DM_XBLK;
+            const unsigned sb = lds0 + DM::XBASE + isg * DM_XBYTES + 4 * lw * DM_XBLK;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 // rows k0 and k0 + 1 for the two halves of the wavefront; rows past K meet zero weights
@@ -377,7 +393,7 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
                 const unsigned short* r1 = k1 < K1 ? sp0 + (int64_t)k1 * a.P : sp1 + (int64_t)(k1 - K1) * a.P;
                 dma16((lane >> 5 ? r1 : r0) + voff, sb + i * DM_XBLK);
             }
-            isg = (isg == DM_XSTAGES - 1) ? 0 : isg + 1;
+            isg = (isg == DM::XSTAGES - 1) ? 0 : isg + 1;
         }
         if (++ic == nchunks) {
             ic = 0;
@@ -386,30 +402,32 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
         return true;
     };
 
-    f32x16 acc[DM_MT][DM_NT];
+    f32x16 acc[MT][DM_NT];
 
-    // fill the pipeline: three weight chunks or five activation chunks, then chunk 0 must have landed
+    // fill the pipeline: three weight chunks or the activation stages, then chunk 0 must have landed
     bool full = true;
-    for (int i = 0; i < (wload ? DM_WSTAGES : DM_XSTAGES); ++i) full = issue() && full;
-    if (full)
-        __builtin_amdgcn_s_waitcnt(0x007C);        // vmcnt(12) lgkmcnt(0): two chunks of weights, three of the four later activation chunks
+    for (int i = 0; i < (wload ? DM_WSTAGES : DM::XSTAGES); ++i) full = issue() && full;
+    if (!full)
+        __builtin_amdgcn_s_waitcnt(dm_wait(0));
+    else if (wload)
+        __builtin_amdgcn_s_waitcnt(dm_wait(2 * 2 * MT));               // the two later weight chunks
     else
-        __builtin_amdgcn_s_waitcnt(0x0070);        // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(dm_wait(4 * (DM::XSTAGES - 1)));    // the later activation chunks
     dm_barrier();
 
-    const unsigned char* abase = lds + (DM_MT * wo) * 1024 + lane * 16;
-    const unsigned char* xbase = lds + DM_XBASE + (4 * ko) * DM_XBLK + wp * 256 + 8 * q;
+    const unsigned char* abase = lds + (MT * wo) * 1024 + lane * 16;
+    const unsigned char* xbase = lds + DM::XBASE + (4 * ko) * DM_XBLK + wp * 256 + 8 * q;
     int sw = 0, sx = 0;
     // Operands of a 16-row k step: eight raw words of activations (rw), regrouped by byte permutes into the four B fragments
     // (bf), and three A fragments (af).  The LDS reads of the next k step are issued into rw and af as soon as the current
     // step has consumed them (rw after the permutes, af[mt] after the MFMAs of row tile mt), so they run under the MFMAs.
     u32x2 rw[8];
-    u32x4 af[DM_MT], bf[DM_NT];
+    u32x4 af[MT], bf[DM_NT];
     auto load_rw = [&](const unsigned char* sxp, int ks) {
 #pragma unroll
         for (int r = 0; r < 8; ++r) rw[r] = *reinterpret_cast<const u32x2*>(sxp + (8 * ks + (r >> 1)) * DM_XBLK + (r & 1) * 512);
     };
-    auto load_af = [&](const unsigned char* sa, int ks, int mt) { af[mt] = *reinterpret_cast<const u32x4*>(sa + (ks * 12 + mt) * 1024); };
+    auto load_af = [&](const unsigned char* sa, int ks, int mt) { af[mt] = *reinterpret_cast<const u32x4*>(sa + (ks * 4 * MT + mt) * 1024); };
     auto regroup = [&]() {
 #pragma unroll
         for (int pp = 0; pp < 2; ++pp)
@@ -470,10 +488,10 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
         load_addend(0);
         load_scalars(0);
 #pragma unroll
-        for (int mh = 0; mh < 2 * DM_MT; ++mh) {
+        for (int mh = 0; mh < 2 * MT; ++mh) {
             const int mt = mh >> 1;
             if (!WHOLE && o0 + 32 * mt >= a.O) break;
-            if (mh + 1 < 2 * DM_MT && (WHOLE || o0 + 32 * ((mh + 1) >> 1) < a.O)) load_addend(mh + 1);
+            if (mh + 1 < 2 * MT && (WHOLE || o0 + 32 * ((mh + 1) >> 1) < a.O)) load_addend(mh + 1);
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
                 const int qq = 2 * mh + g;
@@ -481,7 +499,7 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
                 const int oq = o0 + row_of(mt, v0);
                 asm volatile("" ::"s"(ub[qq & 1][0]), "s"(ub[qq & 1][7]));       // the wait for this quarter's scalars goes here
                 __builtin_amdgcn_sched_barrier(0);
-                if (qq + 1 < 4 * DM_MT) load_scalars(qq + 1);
+                if (qq + 1 < 4 * MT) load_scalars(qq + 1);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int jj = 0; jj < 4; ++jj) {
@@ -514,18 +532,18 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
     };
 
     for (int tl = 0; tl < ntl; ++tl) {
-        const unsigned char* sa = abase + sw * DM_ABYTES;
+        const unsigned char* sa = abase + sw * DM::ABYTES;
         const unsigned char* sxp = xbase + sx * DM_XBYTES;
         load_rw(sxp, 0);
 #pragma unroll
-        for (int mt = 0; mt < DM_MT; ++mt) load_af(sa, 0, mt);
+        for (int mt = 0; mt < MT; ++mt) load_af(sa, 0, mt);
         for (int c = 0; c < nchunks; ++c) {
             // first k step of the chunk; the second one's operands follow it into the registers
             regroup();
             __builtin_amdgcn_sched_barrier(0);
             load_rw(sxp, 1);
 #pragma unroll
-            for (int mt = 0; mt < DM_MT; ++mt) {
+            for (int mt = 0; mt < MT; ++mt) {
                 mfma_row(mt, c == 0);
                 __builtin_amdgcn_sched_barrier(0);
                 load_af(sa, 1, mt);
@@ -533,26 +551,26 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
             }
             regroup();
             // Every wavefront has read all of this chunk.  The next chunk must have landed for every wavefront before it is
-            // read; in flight may stay the loads of one weight chunk (6) or of three activation chunks (12), everything once
-            // the stream has run dry.  Then this chunk's stages take the chunk three (five) further on.
+            // read; in flight may stay the loads of one weight chunk (2 MT) or of all but two of the activation chunks (4 each),
+            // nothing once the stream has run dry.  Then this chunk's stages take the chunk that many stages further on.
             if (!full)
-                __builtin_amdgcn_s_waitcnt(0x0070);    // vmcnt(0) lgkmcnt(0)
+                __builtin_amdgcn_s_waitcnt(dm_wait(0));
             else if (wload)
-                __builtin_amdgcn_s_waitcnt(0x0076);    // vmcnt(6) lgkmcnt(0)
+                __builtin_amdgcn_s_waitcnt(dm_wait(2 * MT));
             else
-                __builtin_amdgcn_s_waitcnt(0x007C);    // vmcnt(12) lgkmcnt(0)
+                __builtin_amdgcn_s_waitcnt(dm_wait(4 * (DM::XSTAGES - 2)));
             dm_barrier();
             full = issue();
             sw = (sw == DM_WSTAGES - 1) ? 0 : sw + 1;
-            sx = (sx == DM_XSTAGES - 1) ? 0 : sx + 1;
-            sa = abase + sw * DM_ABYTES;
+            sx = (sx == DM::XSTAGES - 1) ? 0 : sx + 1;
+            sa = abase + sw * DM::ABYTES;
             sxp = xbase + sx * DM_XBYTES;
             // second k step; the first one of the next chunk follows (after the last chunk of a tile these reads are
             // repeated behind the epilogue, which needs the registers)
             __builtin_amdgcn_sched_barrier(0);
             load_rw(sxp, 0);
 #pragma unroll
-            for (int mt = 0; mt < DM_MT; ++mt) {
+            for (int mt = 0; mt < MT; ++mt) {
                 mfma_row(mt, false);
                 __builtin_amdgcn_sched_barrier(0);
                 load_af(sa, 0, mt);
@@ -569,12 +587,12 @@ __global__ __launch_bounds__(512) void pw_gemm_dma_kernel(PointwiseArgs a) {
         int lane_ = lane;
         asm volatile("" : "+v"(lane_));
         const int ko4 = (lane_ >> 5) * 4;
-        const int o0 = ob * DM_ROWS + wo * 32 * DM_MT;          // first row of the wavefront
+        const int o0 = ob * DM::ROWS + wo * 32 * MT;          // first row of the wavefront
         const int64_t px = pw0 + wp * 128 + 4 * (lane_ & 31);
         if (px < a.P && o0 < a.O) {
             const int64_t lane_off = ((int64_t)b * a.O + o0 + ko4) * a.P + px;      // lane's first row
             // whole wavefront tile inside the matrix: no row needs a check or a clamp
-            if (o0 + 32 * DM_MT <= a.O)
+            if (o0 + 32 * MT <= a.O)
                 epilogue(std::true_type{}, o0, ko4, b, lane_off);
             else
                 epilogue(std::false_type{}, o0, ko4, b, lane_off);
@@ -733,9 +751,19 @@ int pointwise_kpad(int K, int O) {
     const int align = O > PW_ROWS ? DM_CK : PW_KALIGN;
     return (K + align - 1) / align * align;
 }
+// 32-row tiles per wavefront of the direct-to-LDS kernel: the fewest multiplied rows, a block of rows counted 96 rows more for
+// streaming the activations once more (O = 128: one block of 128, 256: of 256, 384 and 768: of 384, 512: two of 256, 640: two of 384)
+static int pointwise_mt(int O) {
+    int best = 3, cost = 1 << 30;
+    for (int mt = 3; mt >= 1; --mt) {
+        const int blocks = (O + 128 * mt - 1) / (128 * mt), c = blocks * (128 * mt + 96);
+        if (c < cost) { cost = c; best = mt; }
+    }
+    return best;
+}
 // rows are padded to whole workgroup tiles so that no fragment load needs a bound check
 int pointwise_opad(int O) {
-    const int tile = O > PW_ROWS ? 4 * PW_ROWS : PW_ROWS;
+    const int tile = O > PW_ROWS ? 128 * pointwise_mt(O) : PW_ROWS;
     return (O + tile - 1) / tile * tile;
 }
 
@@ -748,30 +776,47 @@ int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, 
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
+template <int MT>
+static void dma_go(const PointwiseArgs& a, int64_t blocks, hipStream_t s) {
+    const dim3 grid((unsigned)std::min<int64_t>(blocks, std::max(8, DmGeo<MT>::WG_PER_CU * (device_cus() / 8 * 8))));
+    const bool g = a.act == SFNO_ACT_GELU, r = a.addend != nullptr;
+    if (g && r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, true, true>), grid, dim3(512), 0, s, a);
+    else if (g) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, true, false>), grid, dim3(512), 0, s, a);
+    else if (r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, false, true>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, false, false>), grid, dim3(512), 0, s, a);
+}
+
 int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s) {
     a.Kpad = pointwise_kpad(a.K, a.O);
     if (a.P % 8 != 0 || a.K < 1 || a.O < 1 || a.B < 1 || a.P < 8) return SFNO_EUNSUPPORTED;
-    const bool tall = a.O > PW_ROWS;              // several wavefronts share a pixel strip
-    const int wm = tall ? 4 : 1;
-    const bool dma = tall;                        // direct-to-LDS kernel for O > 96
+    const bool dma = a.O > PW_ROWS;               // several wavefronts share a pixel strip: direct-to-LDS kernel
     if (a.X2 && (a.K1 < 1 || a.K1 >= a.K)) return SFNO_EINVAL;
-    const int wpx = dma ? DM_PX : 512;            // pixels per workgroup
-    a.n_oblk = (a.O + PW_ROWS * wm - 1) / (PW_ROWS * wm);
+    int mt = pointwise_mt(a.O), nw = 8;
+    const int64_t cus = device_cus();
+    const int64_t px_strips = (a.P + (dma ? DM_PX : 512) - 1) / (dma ? DM_PX : 512) * a.B;
+    // Smaller tiles where the CUs outnumber the large ones: 50 tiles of 256 x 256 (464 -> 232 channels, 80 x 160 pixels) 22.5 -> 17.3 us
+    // with MT = 1, 128 of 384 x 256 (192 -> 384, 2 x 90 x 180, GELU) 23.0 -> 18.5, but 226 of 256 x 256 (512 -> 512, 120 x 240) 26.1 ->
+    // 29.4: three blocks of rows each stream the activations.  Two wavefronts per workgroup read no more than eight, only the
+    // weights four times as often (64 -> 64, 128 x 256 pixels: 15.2 -> below 10.7).
+    if (dma && 3 * px_strips * ((a.O + 128 * mt - 1) / (128 * mt)) < 2 * cus) mt = 1;
+    if (!dma && px_strips < cus) nw = 2;
+    const int wpx = dma ? DM_PX : 64 * nw;        // pixels per workgroup
+    const int rows = dma ? 128 * mt : PW_ROWS;    // output channels per workgroup
+    a.n_oblk = (a.O + rows - 1) / rows;
     a.n_strips = (a.P + wpx - 1) / wpx;
     const int64_t strips = a.n_strips * a.B;
     const int64_t blocks = (strips + 7) / 8 * 8 * a.n_oblk;
     if (blocks > 0x7fffffffLL || (dma && a.P > 0x7fffffffLL)) return SFNO_EUNSUPPORTED;
-    if (dma)       // persistent: one workgroup per CU (its LDS admits no second one), the same number on every XCD
-    {
-        const dim3 grid((unsigned)std::min<int64_t>(blocks, std::max(8, device_cus() / 8 * 8)));
-        const bool g = a.act == SFNO_ACT_GELU, r = a.addend != nullptr;
-        if (g && r) hipLaunchKernelGGL((pw_gemm_dma_kernel<true, true>), grid, dim3(512), 0, s, a);
-        else if (g) hipLaunchKernelGGL((pw_gemm_dma_kernel<true, false>), grid, dim3(512), 0, s, a);
-        else if (r) hipLaunchKernelGGL((pw_gemm_dma_kernel<false, true>), grid, dim3(512), 0, s, a);
-        else hipLaunchKernelGGL((pw_gemm_dma_kernel<false, false>), grid, dim3(512), 0, s, a);
-    }
+    if (dma) {     // persistent: as many workgroups as stay resident, the same number on every XCD
+        switch (mt) {
+            case 1: dma_go<1>(a, blocks, s); break;
+            case 2: dma_go<2>(a, blocks, s); break;
+            default: dma_go<3>(a, blocks, s); break;
+        }
+    } else if (nw == 2)
+        hipLaunchKernelGGL(pw_gemm_kernel<2>, dim3((unsigned)blocks), dim3(128), 0, s, a);
     else
-        hipLaunchKernelGGL((pw_gemm_kernel<1, 2>), dim3((unsigned)blocks), dim3(512), 0, s, a);
+        hipLaunchKernelGGL(pw_gemm_kernel<8>, dim3((unsigned)blocks), dim3(512), 0, s, a);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
