@@ -315,10 +315,21 @@ size_t sfno_pointwise_weight_grad_workspace_bytes(int batch, int K, int O, int64
 int sfno_pointwise_weight_grad(const void* gy, const void* x, float* gweight, float* gbias, int batch, int K, int O,
                                int64_t P, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The two convolutions a GELU needs in training: forward with the pre-activation kept,
+ *   z = sum_k w[o][k] x[b][k][p] + bias[o],   y = gelu(z)     (z rounded to bf16 first, both bf16 [B][O][P])
+ * and the input gradient of the convolution behind the GELU, times the GELU's derivative,
+ *   gz = gelu'(z) * sum_k wt[o][k] gy[b][k][p]                (wt: the transposed weight of that convolution, packed). */
+int sfno_pointwise_conv_gelu(const void* x, const void* w, const float* bias, void* y, void* z, int batch, int K, int O,
+                             int64_t P, void* stream);
+int sfno_pointwise_conv_gelu_grad(const void* gy, const void* wt, const void* z, void* gz, int batch, int K, int O,
+                                  int64_t P, void* stream);
+
 /* Packs a 1x1 convolution weight (float32 [O][K], the nn.Conv2d parameter viewed as a matrix) into the bf16
  * MFMA operand stream sfno_pointwise_conv reads; `packed` holds sfno_pointwise_weight_elems(O, K) bf16 values. */
 int64_t sfno_pointwise_weight_elems(int O, int K);
 int sfno_pointwise_pack_weight(const float* w, void* packed, int O, int K, void* stream);
+/* the same stream from the transposed matrix: w is float32 [K][O] (the weight of an input gradient) */
+int sfno_pointwise_pack_weight_transposed(const float* w, void* packed, int O, int K, void* stream);
 
 /* Instance norm as a per-(b, c) affine: scale = gamma[c] / sqrt(var + eps), shift = beta[c] - mean * scale over
  * the P pixels of each of the `rows` = B*C rows of x (bf16), statistics in fp32 with the biased variance
@@ -336,6 +347,53 @@ int sfno_instance_norm_coeffs_lat(const float* lat_stats, const float* gamma, co
  * sfnonet.py:246-251 once the coefficients above are known. */
 int sfno_scale_shift_act(const void* x, const float* scale, const float* shift, void* y, int64_t rows, int64_t P,
                          int act, void* stream);
+
+/* ---- one block of the network (bf16 activations) ----------------------------------------- */
+
+/* makani/models/networks/sfnonet.py:239-267 with a linear dhconv filter, instance norms, a two-layer GELU MLP and a
+ * linear outer skip, as one call per direction:
+ *   (x', r) = filter(x),   h0 = gelu(norm0(x')),   y2 = W2 gelu(W1 h0 + b1) + b2,   out = norm1(y2) + Wskip r
+ * where r is x, or x taken through the transforms where the grids of the two plans differ.  Every longitude length of the
+ * plans has to have bf16 input and output (sfno_sht_io_dtype_supported), H*W of the output grid is a multiple of 8.
+ * All pointers of the structure stay the caller's; the calls enqueue kernels only. */
+typedef struct {
+    const sfno_sht_plan *fwd, *inv;                 /* filter transforms (equal lmax, mmax) */
+    const sfno_sht_plan *fwd_adj, *inv_adj;         /* plans with their adjoint directions (backward only) */
+    const sfno_dhconv_weights *weights, *weights_adj;   /* packed filter weight c_in x embed, and its adjoint (backward only) */
+    const void *w1, *w2, *wskip;                    /* packed [hidden][embed], [embed][hidden], [embed][c_in] */
+    const void *w1t, *w2t, *wskipt;                 /* packed transposed (backward only) */
+    const float *b1, *b2;                           /* null: no bias */
+    const float *gamma0, *beta0, *gamma1, *beta1;   /* null: ones / zeros */
+    float eps0, eps1;
+    int batch, c_in, embed, hidden;
+} sfno_block;
+
+/* tensors of a forward call inside one buffer `kept` (byte offsets; -1: not there) */
+#define SFNO_BLOCK_SPEC 0     /* spectral-layout coefficients of x (training) */
+#define SFNO_BLOCK_X 1        /* bf16 [B][embed][P] filter output (training) */
+#define SFNO_BLOCK_COEF0 2    /* float32 [4][B*embed]: scale, shift of norm0, then its (mean, 1/std) pairs */
+#define SFNO_BLOCK_H0 3       /* bf16 [B][embed][P] */
+#define SFNO_BLOCK_Z1 4       /* bf16 [B][hidden][P] W1 h0 + b1 (training) */
+#define SFNO_BLOCK_A1 5       /* bf16 [B][hidden][P] its GELU */
+#define SFNO_BLOCK_Y2 6       /* bf16 [B][embed][P] */
+#define SFNO_BLOCK_COEF1 7    /* float32 [4][B*embed]: as COEF0, of norm1 */
+#define SFNO_BLOCK_RES 8      /* bf16 [B][c_in][P] the residual, where it passes through the transforms */
+#define SFNO_BLOCK_TENSORS 9
+/* fills offsets; returns the bytes of `kept` (0: invalid).  training = 0: only what the forward itself needs, some of it shared */
+size_t sfno_block_layout(const sfno_block* b, int training, int64_t offsets[SFNO_BLOCK_TENSORS]);
+/* bytes of scratch of a forward (backward = 0) or backward call */
+size_t sfno_block_workspace_bytes(const sfno_block* b, int backward);
+/* out null: stops in front of the last sum; y2, the residual and norm1's scale and shift are then in `kept`. */
+int sfno_block_forward(const sfno_block* b, int training, const void* x, void* out, void* kept, size_t kept_bytes, void* workspace,
+                       size_t workspace_bytes, void* stream);
+/* gradients of a training forward: g = d/d out -> gx (bf16, as x), gfilter complex64 [c_in][embed][lmax], float32 gradients of the
+ * MLP's and the skip's matrices, the biases and the norms' parameters; any of them may be null. */
+typedef struct {
+    void *gx, *gfilter;
+    float *gw1, *gb1, *gw2, *gb2, *gwskip, *ggamma0, *gbeta0, *ggamma1, *gbeta1;
+} sfno_block_grads;
+int sfno_block_backward(const sfno_block* b, const void* g, const void* x, const void* kept, const sfno_block_grads* grads, void* workspace,
+                        size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -398,36 +398,44 @@ extern "C" int sfno_sht_inverse(const sfno_sht_plan* p, const void* coeffs, floa
 
 // ---- adjoints (vector-Jacobian products of the transforms) -----------------------------------------
 
+// spectral layout -> grid / grid -> spectral layout with the Fourier buffer passed in
+int sfno::analysis_adjoint_launch(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, float* xm, int64_t rows, hipStream_t s) {
+    if (!(p->directions & SFNO_DIR_FORWARD_ADJOINT)) return SFNO_EINVAL;
+    int rc;
+    if (planar(p)) {
+        rc = planar_stage(p, MS_FWD_ADJ, true, gspec, xm, rows, s);
+    } else {
+        PgemmArgs a = legendre_args(p, p->fwd_adj, gspec, xm, sfno_spectral_ld(rows));
+        rc = legendre_fold_launch(false, p->format, a, p->fwd_adj.n_work, s);
+    }
+    return rc != SFNO_OK ? rc : sfno_irfft(p, xm, gx, x_dtype, rows, s);
+}
+
+int sfno::synthesis_adjoint_launch(const sfno_sht_plan* p, const void* gx, int x_dtype, float* xm, float* gspec, int64_t rows, hipStream_t s) {
+    if (!(p->directions & SFNO_DIR_INVERSE_ADJOINT)) return SFNO_EINVAL;
+    const int rc = sfno_rfft(p, gx, x_dtype, xm, rows, s);
+    if (rc != SFNO_OK) return rc;
+    if (planar(p)) return planar_stage(p, MS_INV_ADJ, false, xm, gspec, rows, s);
+    PgemmArgs a = legendre_args(p, p->inv_adj, xm, gspec, sfno_spectral_ld(rows));
+    return legendre_fold_launch(true, p->format, a, p->inv_adj.n_work, s);
+}
+
 extern "C" int sfno_sht_analysis_adjoint(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, int64_t rows, void* workspace,
                                          size_t workspace_bytes, void* stream) {
     if (!p || !gspec || !gx || !rows_ok(rows)) return SFNO_EINVAL;
     if (!(p->directions & SFNO_DIR_FORWARD_ADJOINT)) return SFNO_EINVAL;
     Ws w = carve(p, rows, workspace);
     if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
-    const int64_t ld = sfno_spectral_ld(rows);
-    int rc;
-    if (planar(p)) {
-        rc = planar_stage(p, MS_FWD_ADJ, true, gspec, w.xm, rows, stream);
-    } else {
-        PgemmArgs a = legendre_args(p, p->fwd_adj, gspec, w.xm, ld);
-        rc = legendre_fold_launch(false, p->format, a, p->fwd_adj.n_work, (hipStream_t)stream);
-    }
-    if (rc != SFNO_OK) return rc;
-    return sfno_irfft(p, w.xm, gx, x_dtype, rows, stream);
+    return analysis_adjoint_launch(p, gspec, gx, x_dtype, w.xm, rows, (hipStream_t)stream);
 }
 
 extern "C" int sfno_sht_synthesis_adjoint(const sfno_sht_plan* p, const void* gx, int x_dtype, float* gspec, int64_t rows, void* workspace,
                                           size_t workspace_bytes, void* stream) {
-    if (!p || !gspec || !gx || !rows_ok(rows)) return SFNO_EINVAL;
+    if (!p || !gx || !gspec || !rows_ok(rows)) return SFNO_EINVAL;
     if (!(p->directions & SFNO_DIR_INVERSE_ADJOINT)) return SFNO_EINVAL;
     Ws w = carve(p, rows, workspace);
     if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
-    int rc = sfno_rfft(p, gx, x_dtype, w.xm, rows, stream);
-    if (rc != SFNO_OK) return rc;
-    if (planar(p)) return planar_stage(p, MS_INV_ADJ, false, w.xm, gspec, rows, stream);
-    const int64_t ld = sfno_spectral_ld(rows);
-    PgemmArgs a = legendre_args(p, p->inv_adj, w.xm, gspec, ld);
-    return legendre_fold_launch(true, p->format, a, p->inv_adj.n_work, (hipStream_t)stream);
+    return synthesis_adjoint_launch(p, gx, x_dtype, w.xm, gspec, rows, (hipStream_t)stream);
 }
 
 extern "C" int sfno_sht_forward_adjoint(const sfno_sht_plan* p, const void* gcoeffs, float* gx, int64_t rows, void* workspace,
@@ -644,7 +652,39 @@ extern "C" int64_t sfno_pointwise_weight_elems(int O, int K) {
 
 extern "C" int sfno_pointwise_pack_weight(const float* w, void* packed, int O, int K, void* stream) {
     if (!w || !packed || O < 1 || K < 1) return SFNO_EINVAL;
-    return pointwise_pack_launch(w, reinterpret_cast<unsigned short*>(packed), O, K, (hipStream_t)stream);
+    return pointwise_pack_launch(w, reinterpret_cast<unsigned short*>(packed), O, K, 0, (hipStream_t)stream);
+}
+
+extern "C" int sfno_pointwise_pack_weight_transposed(const float* w, void* packed, int O, int K, void* stream) {
+    if (!w || !packed || O < 1 || K < 1) return SFNO_EINVAL;
+    return pointwise_pack_launch(w, reinterpret_cast<unsigned short*>(packed), O, K, 1, (hipStream_t)stream);
+}
+
+extern "C" int sfno_pointwise_conv_gelu(const void* x, const void* w, const float* bias, void* y, void* z, int batch, int K, int O, int64_t P,
+                                        void* stream) {
+    if (!x || !w || !y || !z || batch < 1 || K < 1 || O < 1 || P < 1) return SFNO_EINVAL;
+    PointwiseArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.X = reinterpret_cast<const unsigned short*>(x);
+    a.W = reinterpret_cast<const unsigned short*>(w);
+    a.bias = bias;
+    a.Y = reinterpret_cast<unsigned short*>(y);
+    a.Z = reinterpret_cast<unsigned short*>(z);
+    a.K = K; a.O = O; a.B = batch; a.act = SFNO_ACT_GELU; a.P = P;
+    return pointwise_gemm_launch(a, (hipStream_t)stream);
+}
+
+extern "C" int sfno_pointwise_conv_gelu_grad(const void* gy, const void* wt, const void* z, void* gz, int batch, int K, int O, int64_t P, void* stream) {
+    if (!gy || !wt || !z || !gz || batch < 1 || K < 1 || O < 1 || P < 1) return SFNO_EINVAL;
+    PointwiseArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.X = reinterpret_cast<const unsigned short*>(gy);
+    a.W = reinterpret_cast<const unsigned short*>(wt);
+    a.Y = reinterpret_cast<unsigned short*>(gz);
+    a.addend = reinterpret_cast<const unsigned short*>(z);
+    a.grad = 1;
+    a.K = K; a.O = O; a.B = batch; a.act = SFNO_ACT_NONE; a.P = P;
+    return pointwise_gemm_launch(a, (hipStream_t)stream);
 }
 
 extern "C" int sfno_pointwise_conv(const void* x, const void* w, const float* bias, void* y, int batch, int K, int O, int64_t P,

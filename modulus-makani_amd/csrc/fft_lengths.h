@@ -16,6 +16,6 @@
     X(256, 16, 16, 1) X(240, 16, 15, 1) X(200, 5, 8, 5) X(192, 16, 12, 1) X(180, 12, 15, 1) X(160, 4, 8, 5) X(144, 16, 9, 1) X(128, 8, 16, 1)
 #define SFNO_FFT_LENGTHS_F(X) \
     X(120, 8, 15, 1) X(100, 10, 10, 1) X(96, 8, 12, 1) X(80, 16, 5, 1) X(72, 8, 9, 1) X(64, 8, 8, 1) X(60, 4, 15, 1) X(48, 16, 3, 1) X(40, 8, 5, 1) \
-        X(36, 4, 9, 1) X(32, 4, 8, 1)
+        X(36, 4, 9, 1) X(32, 4, 8, 1) X(24, 8, 3, 1) X(20, 4, 5, 1) X(16, 4, 4, 1) X(12, 4, 3, 1) X(8, 4, 2, 1)
 #define SFNO_FFT_LENGTHS(X) \
     SFNO_FFT_LENGTHS_A(X) SFNO_FFT_LENGTHS_B(X) SFNO_FFT_LENGTHS_C(X) SFNO_FFT_LENGTHS_D(X) SFNO_FFT_LENGTHS_E(X) SFNO_FFT_LENGTHS_F(X)

@@ -4,6 +4,8 @@
 // "spectral" layout float [mmax][lmax][ld] the contraction kernels work on.
 #include "sfno_internal.h"
 
+#include <algorithm>
+
 namespace sfno {
 
 // A tile is 64 orders x 80 complex rows of one degree: on the order-major side 64 pieces of up to 640 contiguous bytes
@@ -141,6 +143,40 @@ int spectral_to_coeffs_launch(const float* spec, float2* coeffs, int64_t rows, i
     const unsigned blocks = tile_blocks(lmax, mmax, (rows + LT_R - 1) / LT_R);
     if (!blocks) return SFNO_EINVAL;
     hipLaunchKernelGGL(spectral_to_coeffs_kernel, dim3(blocks), dim3(LT_T), 0, s, spec, coeffs, rows, lmax, mmax, ld, tri, (mmax + LT_M - 1) / LT_M);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+// grid (x, mmax): the rows l >= m of an order are contiguous
+__global__ __launch_bounds__(256) void spectral_add_kernel(float* __restrict__ a, const float* __restrict__ b, int lmax, int ld, int tri) {
+    const int m = blockIdx.y, l0 = tri ? min(m, lmax) : 0;
+    const int64_t base = ((int64_t)m * lmax + l0) * ld / 4, n = (int64_t)(lmax - l0) * ld / 4;        // ld is a multiple of 16
+    float4* pa = reinterpret_cast<float4*>(a) + base;
+    const float4* pb = reinterpret_cast<const float4*>(b) + base;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const float4 u = pa[i], v = pb[i];
+        pa[i] = make_float4(u.x + v.x, u.y + v.y, u.z + v.z, u.w + v.w);
+    }
+}
+
+int spectral_add_launch(float* a, const float* b, int lmax, int mmax, int ld, int tri, hipStream_t s) {
+    if (mmax > 65535) return SFNO_EUNSUPPORTED;
+    const int64_t n = (int64_t)lmax * ld / 4;
+    const dim3 grid((unsigned)std::min<int64_t>(std::max<int64_t>((n + 1023) / 1024, 1), 64), (unsigned)mmax);
+    hipLaunchKernelGGL(spectral_add_kernel, grid, dim3(256), 0, s, a, b, lmax, ld, tri);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+__global__ __launch_bounds__(256) void spectral_zero_padding_kernel(float* __restrict__ spec, int first, int64_t n, int ld) {
+    const int pad = ld - first;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n * pad) spec[i / pad * ld + first + i % pad] = 0.f;
+}
+
+int spectral_zero_padding_launch(float* spec, int64_t rows, int64_t n, int ld, hipStream_t s) {
+    const int64_t blocks = (n * (ld - 2 * rows) + 255) / 256;
+    if (blocks < 1) return SFNO_OK;
+    if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
+    hipLaunchKernelGGL(spectral_zero_padding_kernel, dim3((unsigned)blocks), dim3(256), 0, s, spec, (int)(2 * rows), n, ld);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

@@ -68,6 +68,21 @@ __device__ __forceinline__ float gelu(float x) {
     return fmaf(-fabsf(x), __builtin_amdgcn_exp2f(q), __builtin_amdgcn_fmed3f(x, 0.f, __builtin_inff()));
 }
 
+// derivative of the exact GELU: Phi(x) + x phi(x), with Phi from the erfc fit of gelu() (absolute error below 2e-5, an eighth of
+// the half ulp of a bf16 result of 0.1) and phi(x) = 2^(-x^2 log2(e) / 2) / sqrt(2 pi)
+__device__ __forceinline__ float gelu_grad(float x) {
+    const float t = __builtin_amdgcn_fmed3f(fabsf(x), 0.f, 6.5f);
+    float q = fmaf(t, 2.008575651e-05f, -5.615057212e-04f);
+    q = fmaf(t, q, 6.880626770e-03f);
+    q = fmaf(t, q, -5.027262948e-02f);
+    q = fmaf(t, q, -4.624537704e-01f);
+    q = fmaf(t, q, -1.149621597e+00f);
+    q = fmaf(t, q, -1.000106287211f);
+    const float e = __builtin_amdgcn_exp2f(q);                                     // Phi(-|x|)
+    const float phi = 0.39894228040143267794f * __builtin_amdgcn_exp2f(-0.72134752044448170368f * x * x);
+    return fmaf(x, phi, x > 0.f ? 1.f - e : e);
+}
+
 // NW = wavefronts per workgroup, side by side along the pixels, 64 pixels each: 8, or 2 where that leaves CUs idle
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
@@ -247,11 +262,21 @@ __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
                 if (o >= a.O) continue;
                 const float bs = ko ? ub[4 + j] : ub[j];
                 float y0 = acc[mt][0][v] + bs, y1 = acc[mt][1][v] + bs;
+                if (a.Z) {                       // training: the pre-activation is stored as well, and activated as stored
+                    rw_t zz;
+                    zz[0] = bf16_pair(y0, y1);
+                    *reinterpret_cast<rw_t*>(a.Z + (int64_t)b * a.O * a.P + (int64_t)o * a.P + px) = zz;
+                    y0 = __uint_as_float(zz[0] << 16);
+                    y1 = __uint_as_float(zz[0] & 0xffff0000u);
+                }
                 if (a.act == SFNO_ACT_GELU) {
                     y0 = gelu(y0);
                     y1 = gelu(y1);
                 }
-                if (R) {
+                if (a.grad) {
+                    y0 *= gelu_grad(__uint_as_float(rv[v][0] << 16));
+                    y1 *= gelu_grad(__uint_as_float(rv[v][0] & 0xffff0000u));
+                } else if (R) {
                     const float sc = ko ? usc[4 + j] : usc[j], sh = ko ? ush[4 + j] : ush[j];
                     y0 += fmaf(sc, __uint_as_float(rv[v][0] << 16), sh);
                     y1 += fmaf(sc, __uint_as_float(rv[v][0] & 0xffff0000u), sh);
@@ -321,10 +346,13 @@ __device__ __forceinline__ void dm_barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// GELU: exact GELU on the output; ADD: "+ scale * addend + shift"
-template <int MT, bool GELU, bool ADD>
+// Epilogue: exact GELU on the output and / or "+ scale * addend + shift"; for training GELU_PRE (the output before the GELU is stored as
+// well, to a.Z, and activated as stored) and GELU_BWD (the output times the GELU's derivative at `addend`)
+enum { DM_PLAIN = 0, DM_GELU = 1, DM_ADD = 2, DM_GELU_PRE = 4, DM_GELU_BWD = 8 };
+template <int MT, int EPI>
 __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_kernel(PointwiseArgs a) {
     using DM = DmGeo<MT>;
+    constexpr bool GELU = EPI & (DM_GELU | DM_GELU_PRE), AFF = EPI & DM_ADD, ADD = EPI & (DM_ADD | DM_GELU_BWD);
     __shared__ __align__(16) unsigned char lds[DM::LDS];
     // tiles of this XCD, row block fastest: q -> (row block q % n_oblk, strip (q / n_oblk) * 8 + xcd); the workgroups of the
     // XCD deal them out round robin, so the row blocks of one strip run at the same time on one L2
@@ -481,8 +509,8 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
             for (int i = 0; i < 8; ++i) {
                 const int64_t u = WHOLE ? oq + i : min(oq + i, a.O - 1);
                 ub[qq & 1][i] = a.bias ? uniform_load(a.bias, u) : 0.f;
-                usc[qq & 1][i] = (ADD && a.add_scale) ? uniform_load(a.add_scale, (int64_t)b * a.O + u) : 1.f;
-                ush[qq & 1][i] = (ADD && a.add_shift) ? uniform_load(a.add_shift, (int64_t)b * a.O + u) : 0.f;
+                usc[qq & 1][i] = (AFF && a.add_scale) ? uniform_load(a.add_scale, (int64_t)b * a.O + u) : 1.f;
+                ush[qq & 1][i] = (AFF && a.add_shift) ? uniform_load(a.add_shift, (int64_t)b * a.O + u) : 0.f;
             }
         };
         load_addend(0);
@@ -509,11 +537,29 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
                     float y[4];
 #pragma unroll
                     for (int t = 0; t < 4; ++t) y[t] = acc[mt][t][v] + bs;
+                    if constexpr (EPI & DM_GELU_PRE) {
+                        u32x2 z;
+#pragma unroll
+                        for (int pp = 0; pp < 2; ++pp) {
+                            z[pp] = bf16_pair(y[2 * pp], y[2 * pp + 1]);
+                            y[2 * pp] = __uint_as_float(z[pp] << 16);
+                            y[2 * pp + 1] = __uint_as_float(z[pp] & 0xffff0000u);
+                        }
+                        *reinterpret_cast<u32x2*>(a.Z + lane_off + (int64_t)row_of(mt, v) * a.P) = z;
+                    }
                     if constexpr (GELU) {
 #pragma unroll
                         for (int t = 0; t < 4; ++t) y[t] = gelu(y[t]);
                     }
-                    if constexpr (ADD) {
+                    if constexpr (EPI & DM_GELU_BWD) {
+                        const u32x2 r = rv[mh & 1][4 * g + jj];
+#pragma unroll
+                        for (int pp = 0; pp < 2; ++pp) {
+                            y[2 * pp] *= gelu_grad(__uint_as_float(r[pp] << 16));
+                            y[2 * pp + 1] *= gelu_grad(__uint_as_float(r[pp] & 0xffff0000u));
+                        }
+                    }
+                    if constexpr (AFF) {
                         const float sc = ko4 ? usc[qq & 1][4 + jj] : usc[qq & 1][jj], sh = ko4 ? ush[qq & 1][4 + jj] : ush[qq & 1][jj];
                         const u32x2 r = rv[mh & 1][4 * g + jj];
 #pragma unroll
@@ -601,16 +647,16 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
 }
 
 // packed[rb][c][lane][e] = bf16(w[32 rb + (lane & 31)][16 c + 8 (lane >> 5) + e]), zero outside the O x K weight:
-// the A fragment of one wavefront for row block rb and chunk c is 1 KiB of consecutive memory
+// the A fragment of one wavefront for row block rb and chunk c is 1 KiB of consecutive memory (transposed: w is [K][O])
 __global__ __launch_bounds__(256) void pointwise_pack_kernel(const float* __restrict__ w, unsigned short* __restrict__ packed, int O, int K, int nc,
-                                                             int64_t total) {
+                                                             int64_t total, int transposed) {
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= total) return;
     const int e = (int)(idx & 7), lane = (int)((idx >> 3) & 63);
     const int64_t blk = idx >> 9;
     const int c = (int)(blk % nc), rb = (int)(blk / nc);
     const int o = 32 * rb + (lane & 31), k = 16 * c + 8 * (lane >> 5) + e;
-    packed[idx] = (o < O && k < K) ? f_to_bf16(w[(int64_t)o * K + k]) : (unsigned short)0;
+    packed[idx] = (o < O && k < K) ? f_to_bf16(w[transposed ? (int64_t)k * O + o : (int64_t)o * K + k]) : (unsigned short)0;
 }
 
 // ---- instance-norm statistics ------------------------------------------------------------------
@@ -660,8 +706,8 @@ __global__ __launch_bounds__(ST_THREADS) void row_stats_partial_kernel(const uns
 
 // scale = gamma * rstd, shift = beta - mean * scale  (biased variance, as torch.nn.functional.instance_norm)
 __global__ void row_stats_finalize_kernel(const unsigned short* __restrict__ x, const float2* __restrict__ partial, const float* __restrict__ gamma,
-                                          const float* __restrict__ beta, float* __restrict__ scale, float* __restrict__ shift, int64_t rows,
-                                          int channels, int64_t P, int nseg, float eps) {
+                                          const float* __restrict__ beta, float* __restrict__ scale, float* __restrict__ shift,
+                                          float2* __restrict__ moments, int64_t rows, int channels, int64_t P, int nseg, float eps) {
     const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (row >= rows) return;
     double s = 0.0, s2 = 0.0;
@@ -678,6 +724,7 @@ __global__ void row_stats_finalize_kernel(const unsigned short* __restrict__ x, 
     const float sc = (gamma ? gamma[c] : 1.f) * rstd;
     scale[row] = sc;
     shift[row] = (beta ? beta[c] : 0.f) - mean * sc;
+    if (moments) moments[row] = make_float2(mean, rstd);
 }
 
 // The same coefficients from per-latitude moments of the field (the inverse longitude kernel's by-product):
@@ -685,7 +732,7 @@ __global__ void row_stats_finalize_kernel(const unsigned short* __restrict__ x, 
 // mean = avg_k a_k, variance = avg_k ((a_k - mean)^2 + d_k); one wavefront per row, sums in double.
 __global__ __launch_bounds__(64) void lat_stats_finalize_kernel(const float2* __restrict__ stats, const float* __restrict__ gamma,
                                                                 const float* __restrict__ beta, float* __restrict__ scale, float* __restrict__ shift,
-                                                                int channels, int nlat, float eps) {
+                                                                float2* __restrict__ moments, int channels, int nlat, float eps) {
     const int64_t row = blockIdx.x;
     const float2* __restrict__ sr = stats + row * nlat;
     double s = 0.0;
@@ -707,6 +754,7 @@ __global__ __launch_bounds__(64) void lat_stats_finalize_kernel(const float2* __
         const float sc = (gamma ? gamma[c] : 1.f) * rstd;
         scale[row] = sc;
         shift[row] = (beta ? beta[c] : 0.f) - (float)mean * sc;
+        if (moments) moments[row] = make_float2((float)mean, rstd);
     }
 }
 
@@ -731,6 +779,119 @@ __global__ __launch_bounds__(256) void scale_shift_act_kernel(const unsigned sho
         o[i] = bf16_pair(lo, hi);
     }
     *reinterpret_cast<u32x4*>(y + i0) = o;
+}
+
+// ---- backward of y = act(scale * x + shift), scale and shift from the row's own statistics (instance norm) ------
+// With d = g act'(scale x + shift) and xh = (x - mean) rstd:   dx = scale (d - avg d - xh avg(d xh)),   dgamma = sum d xh,   dbeta = sum d.
+// Two passes over (g, x), 8 pixels per thread and step: the first leaves partial[row][seg] = (sum d, sum d xh), the second adds them up per
+// row and writes dx; norm_param_grad_kernel adds them up per channel.  Bound by memory: five tensor passes in all (two of them writes
+// and reads of nothing else), with the activation's derivative computed twice instead of a tensor written between the passes.
+__device__ __forceinline__ void norm_terms(unsigned gw, unsigned xw, bool act, float sc, float sh, float mean, float rstd, float (&d)[2], float (&xh)[2]) {
+    const float x[2] = {__uint_as_float(xw << 16), __uint_as_float(xw & 0xffff0000u)};
+    d[0] = __uint_as_float(gw << 16);
+    d[1] = __uint_as_float(gw & 0xffff0000u);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        xh[i] = (x[i] - mean) * rstd;
+        if (act) d[i] *= gelu_grad(fmaf(sc, x[i], sh));
+    }
+}
+
+template <bool ACT>
+__global__ __launch_bounds__(ST_THREADS) void norm_grad_reduce_kernel(const unsigned short* __restrict__ g, const unsigned short* __restrict__ x,
+                                                                      const float* __restrict__ scale, const float* __restrict__ shift,
+                                                                      const float2* __restrict__ moments, float2* __restrict__ partial, int64_t P, int nseg) {
+    const int64_t row = blockIdx.x;
+    const int seg = blockIdx.y;
+    const float sc = scale[row], sh = shift[row];
+    const float2 mo = moments[row];
+    const int64_t ngroups = P / 8;
+    const int64_t g0 = ngroups * seg / nseg, g1 = ngroups * (seg + 1) / nseg;
+    float s = 0.f, s2 = 0.f;
+    for (int64_t i = g0 + threadIdx.x; i < g1; i += ST_THREADS) {
+        const u32x4 gv = *reinterpret_cast<const u32x4*>(g + row * P + 8 * i), xv = *reinterpret_cast<const u32x4*>(x + row * P + 8 * i);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            float d[2], xh[2];
+            norm_terms(gv[w], xv[w], ACT, sc, sh, mo.x, mo.y, d, xh);
+            s += d[0] + d[1];
+            s2 = fmaf(d[0], xh[0], fmaf(d[1], xh[1], s2));
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        s += __shfl_down(s, off, 64);
+        s2 += __shfl_down(s2, off, 64);
+    }
+    __shared__ float2 red[ST_THREADS / 64];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_float2(s, s2);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        float2 t = red[0];
+        for (int w = 1; w < ST_THREADS / 64; ++w) {
+            t.x += red[w].x;
+            t.y += red[w].y;
+        }
+        partial[row * nseg + seg] = t;
+    }
+}
+
+template <bool ACT>
+__global__ __launch_bounds__(ST_THREADS) void norm_grad_apply_kernel(const unsigned short* __restrict__ g, const unsigned short* __restrict__ x,
+                                                                     const float* __restrict__ scale, const float* __restrict__ shift,
+                                                                     const float2* __restrict__ moments, const float2* __restrict__ partial,
+                                                                     unsigned short* __restrict__ dx, int64_t P, int nseg) {
+    const int64_t row = blockIdx.x;
+    const int seg = blockIdx.y;
+    __shared__ float2 total;
+    if (threadIdx.x < 64) {                      // nseg <= 64
+        float2 t = make_float2(0.f, 0.f);
+        if ((int)threadIdx.x < nseg) t = partial[row * nseg + threadIdx.x];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            t.x += __shfl_xor(t.x, off, 64);
+            t.y += __shfl_xor(t.y, off, 64);
+        }
+        if (threadIdx.x == 0) total = t;
+    }
+    __syncthreads();
+    const float sc = scale[row], sh = shift[row];
+    const float2 mo = moments[row];
+    const float m1 = total.x / (float)P, m2 = total.y / (float)P;
+    const int64_t ngroups = P / 8;
+    const int64_t g0 = ngroups * seg / nseg, g1 = ngroups * (seg + 1) / nseg;
+    for (int64_t i = g0 + threadIdx.x; i < g1; i += ST_THREADS) {
+        const u32x4 gv = *reinterpret_cast<const u32x4*>(g + row * P + 8 * i), xv = *reinterpret_cast<const u32x4*>(x + row * P + 8 * i);
+        u32x4 o;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            float d[2], xh[2];
+            norm_terms(gv[w], xv[w], ACT, sc, sh, mo.x, mo.y, d, xh);
+            o[w] = bf16_pair(sc * (d[0] - fmaf(xh[0], m2, m1)), sc * (d[1] - fmaf(xh[1], m2, m1)));
+        }
+        *reinterpret_cast<u32x4*>(dx + row * P + 8 * i) = o;
+    }
+}
+
+// one wavefront per channel: dgamma and dbeta from the partial sums of its rows
+__global__ __launch_bounds__(64) void norm_param_grad_kernel(const float2* __restrict__ partial, float* __restrict__ dgamma, float* __restrict__ dbeta, int batch,
+                                                             int channels, int nseg) {
+    const int c = blockIdx.x;
+    double s = 0.0, s2 = 0.0;
+    for (int i = threadIdx.x; i < batch * nseg; i += 64) {
+        const float2 t = partial[((int64_t)(i / nseg) * channels + c) * nseg + i % nseg];
+        s += t.x;
+        s2 += t.y;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        s += __shfl_down(s, off, 64);
+        s2 += __shfl_down(s2, off, 64);
+    }
+    if (threadIdx.x == 0) {
+        if (dgamma) dgamma[c] = (float)s2;
+        if (dbeta) dbeta[c] = (float)s;
+    }
 }
 
 }  // namespace
@@ -767,12 +928,12 @@ int pointwise_opad(int O) {
     return (O + tile - 1) / tile * tile;
 }
 
-int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, hipStream_t s) {
+int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, int transposed, hipStream_t s) {
     const int nc = pointwise_kpad(K, O) / PW_KC;
     const int64_t total = (int64_t)(pointwise_opad(O) / 32) * nc * 512;
     const int64_t blocks = (total + 255) / 256;
     if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
-    hipLaunchKernelGGL(pointwise_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w, packed, O, K, nc, total);
+    hipLaunchKernelGGL(pointwise_pack_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w, packed, O, K, nc, total, transposed);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
@@ -780,10 +941,12 @@ template <int MT>
 static void dma_go(const PointwiseArgs& a, int64_t blocks, hipStream_t s) {
     const dim3 grid((unsigned)std::min<int64_t>(blocks, std::max(8, DmGeo<MT>::WG_PER_CU * (device_cus() / 8 * 8))));
     const bool g = a.act == SFNO_ACT_GELU, r = a.addend != nullptr;
-    if (g && r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, true, true>), grid, dim3(512), 0, s, a);
-    else if (g) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, true, false>), grid, dim3(512), 0, s, a);
-    else if (r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, false, true>), grid, dim3(512), 0, s, a);
-    else hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, false, false>), grid, dim3(512), 0, s, a);
+    if (a.Z) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU_PRE>), grid, dim3(512), 0, s, a);
+    else if (a.grad) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU_BWD>), grid, dim3(512), 0, s, a);
+    else if (g && r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU | DM_ADD>), grid, dim3(512), 0, s, a);
+    else if (g) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU>), grid, dim3(512), 0, s, a);
+    else if (r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_ADD>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_PLAIN>), grid, dim3(512), 0, s, a);
 }
 
 int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s) {
@@ -791,6 +954,7 @@ int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s) {
     if (a.P % 8 != 0 || a.K < 1 || a.O < 1 || a.B < 1 || a.P < 8) return SFNO_EUNSUPPORTED;
     const bool dma = a.O > PW_ROWS;               // several wavefronts share a pixel strip: direct-to-LDS kernel
     if (a.X2 && (a.K1 < 1 || a.K1 >= a.K)) return SFNO_EINVAL;
+    if ((a.Z && (a.act != SFNO_ACT_GELU || a.addend || a.grad)) || (a.grad && (!a.addend || a.act != SFNO_ACT_NONE))) return SFNO_EINVAL;
     int mt = pointwise_mt(a.O), nw = 8;
     const int64_t cus = device_cus();
     const int64_t px_strips = (a.P + (dma ? DM_PX : 512) - 1) / (dma ? DM_PX : 512) * a.B;
@@ -828,20 +992,21 @@ int row_stats_segments(int64_t rows, int64_t P) {
 }
 
 int instance_norm_coeffs_launch(const unsigned short* x, const float* gamma, const float* beta, float* scale, float* shift, float2* partial,
-                                int64_t rows, int channels, int64_t P, float eps, hipStream_t s) {
+                                int64_t rows, int channels, int64_t P, float eps, hipStream_t s, float2* moments) {
     if (rows < 1 || P < 1 || channels < 1 || rows > 0x7fffffffLL / 64) return SFNO_EUNSUPPORTED;
     if (P % 8 != 0) return SFNO_EUNSUPPORTED;     // 16-byte loads from every row start
     const int nseg = row_stats_segments(rows, P);
     hipLaunchKernelGGL(row_stats_partial_kernel, dim3((unsigned)rows, (unsigned)nseg), dim3(ST_THREADS), 0, s, x, partial, P, nseg);
-    hipLaunchKernelGGL(row_stats_finalize_kernel, dim3((unsigned)((rows + 127) / 128)), dim3(128), 0, s, x, partial, gamma, beta, scale, shift, rows,
-                       channels, P, nseg, eps);
+    hipLaunchKernelGGL(row_stats_finalize_kernel, dim3((unsigned)((rows + 127) / 128)), dim3(128), 0, s, x, partial, gamma, beta, scale, shift, moments,
+                       rows, channels, P, nseg, eps);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
 int instance_norm_coeffs_lat_launch(const float2* stats, const float* gamma, const float* beta, float* scale, float* shift, int64_t rows, int channels,
-                                    int nlat, float eps, hipStream_t s) {
+                                    int nlat, float eps, hipStream_t s, float2* moments) {
     if (rows < 1 || rows > 0x7fffffffLL || channels < 1 || nlat < 1) return SFNO_EINVAL;
-    hipLaunchKernelGGL(lat_stats_finalize_kernel, dim3((unsigned)rows), dim3(64), 0, s, stats, gamma, beta, scale, shift, channels, nlat, eps);
+    hipLaunchKernelGGL(lat_stats_finalize_kernel, dim3((unsigned)rows), dim3(64), 0, s, stats, gamma, beta, scale, shift, moments, channels, nlat,
+                       eps);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
@@ -852,6 +1017,24 @@ int scale_shift_act_launch(const unsigned short* x, const float* scale, const fl
     const int64_t blocks = (total + 255) / 256;
     if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
     hipLaunchKernelGGL(scale_shift_act_kernel, dim3((unsigned)blocks), dim3(256), 0, s, x, scale, shift, y, P, gpr, total, act);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+int norm_grad_launch(const unsigned short* g, const unsigned short* x, const float* scale, const float* shift, const float2* moments, float2* partial,
+                     unsigned short* dx, float* dgamma, float* dbeta, int batch, int channels, int64_t P, int act, hipStream_t s) {
+    const int64_t rows = (int64_t)batch * channels;
+    if (rows < 1 || P < 8 || P % 8 != 0 || rows > 0x7fffffffLL / 64) return SFNO_EUNSUPPORTED;
+    const int nseg = row_stats_segments(rows, P);
+    const dim3 grid((unsigned)rows, (unsigned)nseg);
+    if (act == SFNO_ACT_GELU) {
+        hipLaunchKernelGGL(norm_grad_reduce_kernel<true>, grid, dim3(ST_THREADS), 0, s, g, x, scale, shift, moments, partial, P, nseg);
+        hipLaunchKernelGGL(norm_grad_apply_kernel<true>, grid, dim3(ST_THREADS), 0, s, g, x, scale, shift, moments, partial, dx, P, nseg);
+    } else {
+        hipLaunchKernelGGL(norm_grad_reduce_kernel<false>, grid, dim3(ST_THREADS), 0, s, g, x, scale, shift, moments, partial, P, nseg);
+        hipLaunchKernelGGL(norm_grad_apply_kernel<false>, grid, dim3(ST_THREADS), 0, s, g, x, scale, shift, moments, partial, dx, P, nseg);
+    }
+    if (dgamma || dbeta)
+        hipLaunchKernelGGL(norm_param_grad_kernel, dim3((unsigned)channels), dim3(64), 0, s, partial, dgamma, dbeta, batch, channels, nseg);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

@@ -99,6 +99,8 @@ struct PointwiseArgs {
     const unsigned short* addend;  // bf16 [B][O][P] or null: y += add_scale[b][o] * addend + add_shift[b][o]
     const float* add_scale;        // [B][O] or null (1)
     const float* add_shift;        // [B][O] or null (0)
+    unsigned short* Z;             // null, or bf16 [B][O][P]: the output before its GELU goes there as well (training)
+    int grad;                      // the output is multiplied by the GELU's derivative at `addend` (backward of a GELU)
     int K, Kpad, O, B, act;
     int64_t P;
     int n_oblk;                    // filled by the launcher
@@ -107,16 +109,20 @@ struct PointwiseArgs {
 int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s);
 int pointwise_kpad(int K, int O);
 int pointwise_opad(int O);
-int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, hipStream_t s);
+int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, int transposed, hipStream_t s);
 // weight and bias gradient of the 1x1 convolution (pointwise_wgrad.hip); db null: no bias column
 size_t pointwise_wgrad_workspace_bytes(int O, int K, int has_bias, int B, int64_t P);
 int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, float* dW, float* db, int B, int K, int O, int64_t P, float* ws,
                            size_t ws_bytes, hipStream_t s);
 int row_stats_segments(int64_t rows, int64_t P);
 int instance_norm_coeffs_launch(const unsigned short* x, const float* gamma, const float* beta, float* scale, float* shift, float2* partial,
-                                int64_t rows, int channels, int64_t P, float eps, hipStream_t s);
+                                int64_t rows, int channels, int64_t P, float eps, hipStream_t s, float2* moments = nullptr);
 int instance_norm_coeffs_lat_launch(const float2* stats, const float* gamma, const float* beta, float* scale, float* shift, int64_t rows, int channels,
-                                    int nlat, float eps, hipStream_t s);
+                                    int nlat, float eps, hipStream_t s, float2* moments = nullptr);
+// backward of act(scale x + shift) with the instance norm's scale and shift; moments [rows] = (mean, 1 / standard deviation), partial holds
+// rows * row_stats_segments float2; dgamma, dbeta [channels] may be null
+int norm_grad_launch(const unsigned short* g, const unsigned short* x, const float* scale, const float* shift, const float2* moments, float2* partial,
+                     unsigned short* dx, float* dgamma, float* dbeta, int batch, int channels, int64_t P, int act, hipStream_t s);
 int scale_shift_act_launch(const unsigned short* x, const float* scale, const float* shift, unsigned short* y, int64_t rows, int64_t P, int act,
                            hipStream_t s);
 
@@ -204,11 +210,19 @@ int degree_power_grad_launch(const float* spec, const float* gpower, float* gspe
 // looks up, once per device, the device address of the array on the current device; called at plan creation
 int static_scratch_prepare();
 
+// ---- adjoint transforms with the Fourier buffer passed in (capi.cpp) ----------------------------
+int analysis_adjoint_launch(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, float* xm, int64_t rows, hipStream_t s);
+int synthesis_adjoint_launch(const sfno_sht_plan* p, const void* gx, int x_dtype, float* xm, float* gspec, int64_t rows, hipStream_t s);
+
 // ---- layout passes (layout.hip) ----------------------------------------------------------
 int coeffs_to_spectral_launch(const float2* coeffs, float* spec, int64_t rows, int lmax, int mmax, int ld, int tri,
                               hipStream_t s);
 int spectral_to_coeffs_launch(const float* spec, float2* coeffs, int64_t rows, int lmax, int mmax, int ld, int tri,
                               hipStream_t s);
+// a += b on the spectral layout (orders above the degree left alone in triangular mode)
+int spectral_add_launch(float* a, const float* b, int lmax, int mmax, int ld, int tri, hipStream_t s);
+// zeroes the floats between 2 rows and ld of n rows of ld floats
+int spectral_zero_padding_launch(float* spec, int64_t rows, int64_t n, int ld, hipStream_t s);
 int dhconv_pack_launch(const float2* w, float* packed, int I, int O, int L, int adjoint, hipStream_t s);
 
 }  // namespace sfno

@@ -18,6 +18,23 @@ DTYPE_F32, DTYPE_BF16 = 0, 1
 ACT_NONE, ACT_GELU = 0, 1
 
 
+BLOCK_COEF1, BLOCK_Y2, BLOCK_RES, BLOCK_TENSORS = 7, 6, 8, 9      # SFNO_BLOCK_*
+
+
+class Block(ctypes.Structure):
+    """sfno_block"""
+
+    _fields_ = [(n, ctypes.c_void_p) for n in ("fwd", "inv", "fwd_adj", "inv_adj", "weights", "weights_adj", "w1", "w2", "wskip", "w1t", "w2t", "wskipt",
+                                               "b1", "b2", "gamma0", "beta0", "gamma1", "beta1")]
+    _fields_ += [("eps0", ctypes.c_float), ("eps1", ctypes.c_float)] + [(n, ctypes.c_int) for n in ("batch", "c_in", "embed", "hidden")]
+
+
+class BlockGrads(ctypes.Structure):
+    """sfno_block_grads"""
+
+    _fields_ = [(n, ctypes.c_void_p) for n in ("gx", "gfilter", "gw1", "gb1", "gw2", "gb2", "gwskip", "ggamma0", "gbeta0", "ggamma1", "gbeta1")]
+
+
 class SfnoError(RuntimeError):
     pass
 
@@ -77,6 +94,13 @@ def _load():
         "sfno_pointwise_weight_elems": (i64, [i32, i32]),
         "sfno_pointwise_pack_weight": (i32, [vp, vp, i32, i32, vp]),
         "sfno_pointwise_conv": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, i32, vp, vp, vp, vp]),
+        "sfno_pointwise_conv_gelu": (i32, [vp, vp, vp, vp, vp, i32, i32, i32, i64, vp]),
+        "sfno_pointwise_conv_gelu_grad": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, vp]),
+        "sfno_pointwise_pack_weight_transposed": (i32, [vp, vp, i32, i32, vp]),
+        "sfno_block_layout": (sz, [vp, i32, vp]),
+        "sfno_block_workspace_bytes": (sz, [vp, i32]),
+        "sfno_block_forward": (i32, [vp, i32, vp, vp, vp, sz, vp, sz, vp]),
+        "sfno_block_backward": (i32, [vp, vp, vp, vp, vp, vp, sz, vp]),
         "sfno_pointwise_conv_cat": (i32, [vp, i32, vp, i32, vp, vp, vp, i32, i32, i64, i32, vp]),
         "sfno_pointwise_weight_grad_workspace_bytes": (sz, [i32, i32, i32, i64, i32]),
         "sfno_pointwise_weight_grad": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, vp, sz, vp]),

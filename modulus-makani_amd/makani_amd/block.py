@@ -1,0 +1,153 @@
+"""One SFNO block per native call: filter -> norm0 -> GELU -> MLP -> norm1 -> + outer skip (makani/models/networks/sfnonet.py:239-267)
+with every kernel enqueued by sfno_block_forward / sfno_block_backward, for bfloat16 activations.
+
+Inference runs it on buffers that the call needs anyway; training keeps the tensors the backward reads in one buffer.  The
+parameters stay those of the PyTorch modules; packed copies come from the caches of contractions.py and pointwise.py.
+"""
+import ctypes
+
+import torch
+import torch.nn as nn
+from torch.autograd.function import once_differentiable
+
+from . import _lib
+from ._lib import lib, check
+from . import pointwise as pw
+from .contractions import packed_for
+from .sht import _stream_ptr
+
+
+def _f32(t):
+    return t.detach().float().contiguous() if t is not None else None
+
+
+def _ptr(t):
+    return t.data_ptr() if t is not None else None
+
+
+def _no_hooks(*mods):
+    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in mods)
+
+
+def mlp_convs(blk):
+    """(fc1, fc2) of a conv -> GELU -> conv MLP, or None."""
+    m = [f for f in blk.mlp.fwd if not isinstance(f, nn.Identity)]
+    ok = len(m) == 3 and isinstance(m[0], nn.Conv2d) and isinstance(m[2], nn.Conv2d) and isinstance(m[1], nn.GELU) and m[1].approximate == "none"
+    return (m[0], m[2]) if ok else None
+
+
+def supported(blk, x):
+    """Whether the native block serves this block (whose fusable() the caller has checked) and input."""
+    conv, fwd, inv = blk.filter.filter, blk.filter.filter.forward_transform, blk.filter.filter.inverse_transform
+    if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or mlp_convs(blk) is None:
+        return False
+    if not (isinstance(blk.norm0, nn.InstanceNorm2d) and isinstance(blk.norm1, nn.InstanceNorm2d)) or inv.mmax > inv.nlon // 2 + 1:
+        return False
+    if tuple(x.shape[2:]) != (fwd.nlat, fwd.nlon) or (inv.nlat * inv.nlon) % 8 != 0:
+        return False
+    if not lib.sfno_sht_io_dtype_supported(fwd.plan(x.device).handle, _lib.DTYPE_BF16) or not lib.sfno_sht_io_dtype_supported(inv.plan(x.device).handle, _lib.DTYPE_BF16):
+        return False
+    fc1, fc2 = mlp_convs(blk)
+    params = [p for m in (blk.norm0, blk.norm1, fc1, fc2, blk.outer_skip) for p in (m.weight, m.bias) if p is not None]
+    return all(p.dtype == torch.float32 and p.is_cuda for p in params) and _no_hooks(
+        blk.filter, conv, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.mlp.fwd, *blk.mlp.fwd, blk.outer_skip)
+
+
+class _Call:
+    """The sfno_block structure of one call, and what has to stay alive while it is used."""
+
+    def __init__(self, blk, x, filter_weight, skip_weight, backward=False):
+        conv = blk.filter.filter
+        fwd, inv = conv.forward_transform, conv.inverse_transform
+        fc1, fc2 = mlp_convs(blk)
+        n0, n1, dev = blk.norm0, blk.norm1, x.device
+        b = _lib.Block()
+        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(filter_weight, conv.compute), pw.packed_weight(fc1.weight), pw.packed_weight(fc2.weight),
+                            pw.packed_weight(skip_weight)]
+        b.fwd, b.inv, b.weights = keep[0].handle, keep[1].handle, keep[2].handle
+        b.w1, b.w2, b.wskip = (t.data_ptr() for t in keep[3:6])
+        if backward:
+            adj = [fwd.plan(dev, adjoint=True), inv.plan(dev, adjoint=True), packed_for(filter_weight, conv.compute, adjoint=True),
+                   pw.packed_weight(fc1.weight, transposed=True), pw.packed_weight(fc2.weight, transposed=True), pw.packed_weight(skip_weight, transposed=True)]
+            b.fwd_adj, b.inv_adj, b.weights_adj = adj[0].handle, adj[1].handle, adj[2].handle
+            b.w1t, b.w2t, b.wskipt = (t.data_ptr() for t in adj[3:6])
+            keep += adj
+        b.b1, b.b2 = _ptr(fc1.bias), _ptr(fc2.bias)
+        b.gamma0, b.beta0, b.gamma1, b.beta1 = _ptr(n0.weight), _ptr(n0.bias), _ptr(n1.weight), _ptr(n1.bias)
+        b.eps0, b.eps1 = n0.eps, n1.eps
+        b.batch, b.c_in, b.embed, b.hidden = x.shape[0], x.shape[1], conv.out_channels, fc1.out_channels
+        self.b = b
+        self.P = (inv.nlat, inv.nlon)
+        self.stream = _stream_ptr(dev)
+        self.offsets = (ctypes.c_int64 * _lib.BLOCK_TENSORS)()
+
+    def forward(self, x, training, out):
+        ref = ctypes.byref(self.b)
+        nkept, nws = lib.sfno_block_layout(ref, training, self.offsets), lib.sfno_block_workspace_bytes(ref, 0)
+        kept = torch.empty(nkept, dtype=torch.uint8, device=x.device)
+        ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
+        check(lib.sfno_block_forward(ref, training, x.data_ptr(), _ptr(out), kept.data_ptr(), nkept, ws.data_ptr(), nws, self.stream), "sfno_block_forward")
+        return kept
+
+
+def forward(blk, x, filter_weight=None, skip_weight=None, defer_skip=False):
+    """The block without autograd.  filter_weight, skip_weight: in place of the block's own.  defer_skip: returns (y2, residual, scale,
+    shift) of the last sum scale * y2 + shift + skip(residual) instead of running it."""
+    x = x.contiguous()
+    c = _Call(blk, x, blk.filter.filter.weight if filter_weight is None else filter_weight, blk.outer_skip.weight if skip_weight is None else skip_weight)
+    B, E = x.shape[0], c.b.embed
+    if not defer_skip:
+        out = torch.empty((B, E, *c.P), dtype=torch.bfloat16, device=x.device)
+        c.forward(x, 0, out)
+        return out
+    kept = c.forward(x, 0, None)
+
+    def view(i, shape, dtype):
+        n = dtype.itemsize
+        for d in shape:
+            n *= d
+        return kept[c.offsets[i]:c.offsets[i] + n].view(dtype).view(shape)
+
+    coef = view(_lib.BLOCK_COEF1, (2, B, E), torch.float32)
+    res = x if c.offsets[_lib.BLOCK_RES] < 0 else view(_lib.BLOCK_RES, (B, x.shape[1], *c.P), torch.bfloat16)
+    return view(_lib.BLOCK_Y2, (B, E, *c.P), torch.bfloat16), res, coef[0], coef[1]
+
+
+class _BlockFn(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, blk, *params):
+        x = x.detach().contiguous()
+        c = _Call(blk, x, blk.filter.filter.weight, blk.outer_skip.weight)
+        out = torch.empty((x.shape[0], c.b.embed, *c.P), dtype=torch.bfloat16, device=x.device)
+        kept = c.forward(x, 1, out)
+        ctx.blk = blk
+        ctx.save_for_backward(x, kept, *params)
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g):
+        x, kept, *params = ctx.saved_tensors
+        g = g.to(torch.bfloat16).contiguous()
+        blk, need = ctx.blk, ctx.needs_input_grad
+        c = _Call(blk, x, blk.filter.filter.weight, blk.outer_skip.weight, backward=True)
+        # in the order of trainable_params: filter, skip, W1, b1, W2, b2, gamma0, beta0, gamma1, beta1
+        want = [p is not None and n for p, n in zip(params, need[2:])]
+        want[2], want[4] = want[2] or want[3], want[4] or want[5]          # a bias gradient is a column of its matrix's kernel
+        grads = [torch.empty_like(p) if w else None for p, w in zip(params, want)]
+        gx = torch.empty_like(x) if need[0] else None
+        s = _lib.BlockGrads()
+        s.gx, s.gfilter = _ptr(gx), _ptr(grads[0])
+        s.gwskip, s.gw1, s.gb1, s.gw2, s.gb2, s.ggamma0, s.gbeta0, s.ggamma1, s.gbeta1 = (_ptr(t) for t in grads[1:])
+        ref = ctypes.byref(c.b)
+        nws = lib.sfno_block_workspace_bytes(ref, 1)
+        ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
+        check(lib.sfno_block_backward(ref, g.data_ptr(), x.data_ptr(), kept.data_ptr(), ctypes.byref(s), ws.data_ptr(), nws, c.stream), "sfno_block_backward")
+        return (gx, None, *(t if n else None for t, n in zip(grads, need[2:])))
+
+
+def train(blk, x):
+    """The block with autograd (supported() holds and a gradient is being recorded)."""
+    fc1, fc2 = mlp_convs(blk)
+    n0, n1 = blk.norm0, blk.norm1
+    return _BlockFn.apply(x, blk, blk.filter.filter.weight, blk.outer_skip.weight, fc1.weight, fc1.bias, fc2.weight, fc2.bias, n0.weight, n0.bias, n1.weight, n1.bias)

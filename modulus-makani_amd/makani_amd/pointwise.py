@@ -18,7 +18,7 @@ from ._lib import lib, check
 
 ACT = {None: _lib.ACT_NONE, "none": _lib.ACT_NONE, "gelu": _lib.ACT_GELU}
 
-# id(parameter) -> (weakref, stamp, packed bf16 [O, Kpad])
+# (id(parameter), transposed) -> (weakref, stamp, packed bf16 [O, Kpad])
 _wcache = {}
 
 
@@ -30,19 +30,20 @@ def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-def packed_weight(weight):
-    """MFMA operand stream of a 1x1 convolution weight ([O, K, 1, 1] or [O, K]); cached per parameter and
-    rebuilt when the parameter changes."""
-    key = id(weight)
+def packed_weight(weight, transposed=False):
+    """MFMA operand stream of a 1x1 convolution weight ([O, K, 1, 1] or [O, K]), or of its transpose (the weight of the
+    convolution's input gradient); cached per parameter and rebuilt when the parameter changes."""
+    key = (id(weight), transposed)
     # (tensors made under inference_mode carry no version counter: they are packed once per tensor object)
     stamp = (weight.data_ptr(), -1 if weight.is_inference() else weight._version, weight.device)
     hit = _wcache.get(key)
     if hit is not None and hit[0]() is weight and hit[1] == stamp:
         return hit[2]
     w = weight.detach().reshape(weight.shape[0], -1).float().contiguous()
-    O, K = w.shape
+    O, K = (w.shape[1], w.shape[0]) if transposed else w.shape
     p = torch.empty(lib.sfno_pointwise_weight_elems(O, K), dtype=torch.bfloat16, device=w.device)
-    check(lib.sfno_pointwise_pack_weight(_ptr(w), _ptr(p), O, K, _stream(w.device)), "sfno_pointwise_pack_weight")
+    pack = lib.sfno_pointwise_pack_weight_transposed if transposed else lib.sfno_pointwise_pack_weight
+    check(pack(_ptr(w), _ptr(p), O, K, _stream(w.device)), "sfno_pointwise_pack_weight")
     _wcache[key] = (weakref.ref(weight, lambda _, k=key: _wcache.pop(k, None)), stamp, p)
     return p
 
@@ -53,7 +54,8 @@ def clear_cache(weight=None):
     if weight is None:
         _wcache.clear()
     else:
-        _wcache.pop(id(weight), None)
+        _wcache.pop((id(weight), False), None)
+        _wcache.pop((id(weight), True), None)
 
 
 def supported(x):
@@ -63,14 +65,16 @@ def supported(x):
 
 def conv1x1(x, weight, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
     """act(conv1x1(x, weight) + bias) + add_scale * addend + add_shift  ->  bf16 [B, O, H, W]."""
+    return _conv1x1(x, packed_weight(weight), weight.shape[0], weight.shape[1], bias, act, addend, add_scale, add_shift)
+
+
+def _conv1x1(x, pw, O, K_weight, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
     if not supported(x):
         raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
     x = x.contiguous()
     B, K, H, W = x.shape
-    pw = packed_weight(weight)
-    O = weight.shape[0]
-    if weight.shape[1] != K:
-        raise RuntimeError(f"conv1x1: input has {K} channels, weight expects {weight.shape[1]}")
+    if K_weight != K:
+        raise RuntimeError(f"conv1x1: input has {K} channels, weight expects {K_weight}")
     y = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
     if bias is not None:
         bias = bias.detach().float().contiguous()
@@ -197,14 +201,64 @@ class _Conv1x1(torch.autograd.Function):
         gy = gy.to(torch.bfloat16).contiguous()
         gx = gw = gb = None
         if ctx.needs_input_grad[0]:
-            wt = weight.detach().reshape(weight.shape[0], -1).t().contiguous()       # [K, O]: packed afresh, it is no parameter
-            gx = conv1x1(gy, wt).to(ctx.x_dtype)
+            gx = _conv1x1(gy, packed_weight(weight, transposed=True), weight.shape[1], weight.shape[0]).to(ctx.x_dtype)
         if ctx.needs_input_grad[1] or (ctx.has_bias and ctx.needs_input_grad[2]):
             gw, gb = conv1x1_weight_grad(gy, xb, ctx.has_bias)
             gw = gw.reshape(weight.shape).to(weight.dtype)
             if gb is not None:
                 gb = gb.to(ctx.b_dtype)
         return gx, gw, gb
+
+
+class _ConvGeluConv(torch.autograd.Function):
+    """y = W2 gelu(W1 x + b1) + b2 (makani/models/common/layers.py:95-116: the encoder's and the decoder's two convolutions): the first
+    convolution stores its output before and after the GELU, the input gradient of the second one is multiplied by the GELU's derivative
+    where it is stored."""
+
+    @staticmethod
+    def forward(ctx, x, w1, b1, w2, b2):
+        xb = x.detach().to(torch.bfloat16).contiguous()
+        B, K, H, W = xb.shape
+        O = w1.shape[0]
+        z = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
+        a = torch.empty_like(z)
+        bias = b1.detach().float().contiguous() if b1 is not None else None
+        check(lib.sfno_pointwise_conv_gelu(_ptr(xb), _ptr(packed_weight(w1)), _ptr(bias), _ptr(a), _ptr(z), B, K, O, H * W, _stream(x.device)),
+              "sfno_pointwise_conv_gelu")
+        ctx.save_for_backward(xb, z, a, w1, w2)
+        ctx.biases = (b1 is not None, b2 is not None)
+        ctx.x_dtype = x.dtype
+        return conv1x1(a, w2, b2)
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, gy):
+        xb, z, a, w1, w2 = ctx.saved_tensors
+        gy = gy.to(torch.bfloat16).contiguous()
+        need = ctx.needs_input_grad
+        gx = gw1 = gb1 = gw2 = gb2 = None
+        if need[3] or need[4]:
+            gw2, gb2 = conv1x1_weight_grad(gy, a, ctx.biases[1])
+            gw2 = gw2.reshape(w2.shape)
+        if need[0] or need[1] or need[2]:
+            B, O, H, W = gy.shape
+            gz = torch.empty_like(z)
+            check(lib.sfno_pointwise_conv_gelu_grad(_ptr(gy), _ptr(packed_weight(w2, transposed=True)), _ptr(z), _ptr(gz), B, O, z.shape[1], H * W,
+                                                    _stream(gy.device)), "sfno_pointwise_conv_gelu_grad")
+            if need[1] or need[2]:
+                gw1, gb1 = conv1x1_weight_grad(gz, xb, ctx.biases[0])
+                gw1 = gw1.reshape(w1.shape)
+            if need[0]:
+                gx = _conv1x1(gz, packed_weight(w1, transposed=True), w1.shape[1], w1.shape[0]).to(ctx.x_dtype)
+        return gx, gw1, gb1, gw2, gb2
+
+
+def conv_gelu_conv_trainable(x, conv1, conv2):
+    """conv2(gelu(conv1(x))) -> bf16, differentiable; None where the kernels do not serve the parameters (float32 on the device)."""
+    params = [p for p in (conv1.weight, conv1.bias, conv2.weight, conv2.bias) if p is not None]
+    if not all(p.dtype == torch.float32 and p.is_cuda for p in params):
+        return None
+    return _ConvGeluConv.apply(x, conv1.weight, conv1.bias, conv2.weight, conv2.bias)
 
 
 def trainable_active(x):

@@ -15,6 +15,7 @@ from functools import partial
 import torch
 import torch.nn as nn
 
+from . import block as native_block
 from . import pointwise as pw
 from .sht import RealSHT, InverseRealSHT
 from .layers import RealFFT2, InverseRealFFT2
@@ -103,6 +104,12 @@ class EncoderDecoder(nn.Module):
         self.fwd = nn.Sequential(*mods)
 
     def forward(self, x):
+        # training under bf16: convolution, GELU and convolution with the GELU in the convolutions' epilogues, both ways
+        if len(self.fwd) == 3 and pw.trainable_active(x) and _is_conv1x1(self.fwd[0]) and _is_gelu(self.fwd[1]) and _is_conv1x1(self.fwd[2]) \
+                and native_block._no_hooks(self.fwd, *self.fwd):
+            y = pw.conv_gelu_conv_trainable(x, self.fwd[0], self.fwd[2])
+            if y is not None:
+                return y
         return self.fwd(x)
 
 
@@ -220,6 +227,13 @@ class FourierNeuralOperatorBlock(nn.Module):
         return pw.conv1x1(residual, self.outer_skip.weight if skip_weight is None else skip_weight, None, None, x, sc, sh)
 
     def forward(self, x, defer_skip=False):
+        if getattr(self, "fused_pointwise", True) and x.is_cuda and x.dtype == torch.bfloat16:
+            # the whole block as one native call, with its gradients while they are recorded
+            if torch.is_grad_enabled():
+                if pw.trainable_active(x) and self._fusable() and native_block.supported(self, x):
+                    return native_block.train(self, x)
+            elif not self.training and fused_pointwise_active(x) and self._fusable() and native_block.supported(self, x):
+                return native_block.forward(self, x, defer_skip=defer_skip)
         # on the fused inference path the inverse transform hands over the moments norm0 needs together with its output
         want_stats = getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x) and x.dtype == torch.bfloat16 and self._fusable()
         if want_stats:
@@ -413,6 +427,8 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         blk = self.blocks[0]
         conv = blk.filter.filter
         B = h.shape[0]
+        if native_block.supported(blk, h):
+            return native_block.forward(blk, h, wf, wsk)
         spec = conv.forward_transform.analysis(h)
         residual = conv.inverse_transform.synthesis(spec, (B, h.shape[1]), dtype=torch.bfloat16)
         spec = dhconv_spectral(spec, wf, B, conv.modes_lon, triangular=conv._triangular, compute=conv.compute)

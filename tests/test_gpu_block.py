@@ -1,0 +1,135 @@
+"""The native block (makani_amd/block.py, csrc/block.cpp) and the convolution -> GELU -> convolution pair of encoder and decoder in
+training: output and every gradient against the same modules in float32, next to the layer-by-layer modules under bf16 autocast.
+
+Bound: both bf16 evaluations round the output of a layer to 8 bits (2^-8 / sqrt 3 / 1.4 = 1.7e-3 relative L2 each).  About a dozen such
+roundings lie between an input and a gradient, sqrt(12) 1.7e-3 = 6e-3, up to twice that where a norm or a cancelling sum amplifies
+them: 1.5e-2 asserted.  The native block rounds less often than the modules, so its error may exceed theirs by sampling only (a
+quarter, plus 1e-3)."""
+import contextlib
+
+import pytest
+import torch
+import torch.nn as nn
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    a, b = (torch.view_as_real(t) if t.is_complex() else t for t in (a.detach(), b.detach()))
+    return float((a.double() - b.double()).norm() / b.double().norm().clamp_min(1e-300))
+
+
+def make_block(fwd, inv, embed, ratio, affine=True):
+    from functools import partial
+
+    from makani_amd.sfnonet import FourierNeuralOperatorBlock
+
+    norm = partial(nn.InstanceNorm2d, num_features=embed, eps=1e-6, affine=affine, track_running_stats=False)
+    blk = FourierNeuralOperatorBlock(fwd, inv, embed, operator_type="dhconv", mlp_ratio=ratio, norm_layer=(norm, norm), inner_skip="none", outer_skip="linear",
+                                     use_mlp=True)
+    with torch.no_grad():
+        for p in blk.parameters():
+            if not p.is_complex() and p.dim() == 1:
+                p.add_(0.2 * torch.randn(p.shape))
+    return blk.cuda()
+
+
+def passes(blk, x, gy, autocast, leaf=None):
+    for p in blk.parameters():
+        p.grad = None
+    xi = x.clone().requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16) if autocast else contextlib.nullcontext():
+        y = blk(xi)
+    y.backward(gy.to(y.dtype))
+    return {"y": y, "x": xi.grad, **{n: p.grad.clone() for n, p in blk.named_parameters()}}
+
+
+CASES = [
+    # forward grid, inverse grid, batch, embed, MLP ratio
+    ((32, 64, "legendre-gauss"), (32, 64, "legendre-gauss"), 2, 24, 2.0),       # equal grids: the residual is the input
+    ((33, 64, "equiangular"), (16, 32, "legendre-gauss"), 3, 36, 1.5),          # down: the residual goes through the transforms, padded channel slots
+    ((16, 32, "legendre-gauss"), (33, 64, "equiangular"), 1, 104, 2.0),         # up
+    ((24, 48, "planar"), (24, 48, "planar"), 2, 17, 3.0),                       # planar pair, odd channels
+]
+
+
+@pytest.mark.parametrize("f,i,B,E,ratio", CASES)
+def test_block_gradients(lib_built, f, i, B, E, ratio):
+    import makani_amd as ma
+    from makani_amd import block as nb
+
+    print(f"case block {f} -> {i} B={B} E={E}", flush=True)
+    torch.manual_seed(4)
+    lmax, mmax = min(f[0], i[0]) - (i[2] == "planar") * 3, min(f[1], i[1]) // 2 + 1
+    if f[2] == "planar":
+        fwd, inv = ma.RealFFT2(*f[:2], lmax, mmax), ma.InverseRealFFT2(*i[:2], lmax, mmax)
+    else:
+        fwd, inv = ma.RealSHT(*f[:2], lmax=lmax, mmax=mmax, grid=f[2]), ma.InverseRealSHT(*i[:2], lmax=lmax, mmax=mmax, grid=i[2])
+    blk = make_block(fwd, inv, E, ratio, affine=B != 3)
+    x = torch.randn(B, E, *f[:2], device="cuda").to(torch.bfloat16)
+    gy = torch.randn(B, E, *i[:2], device="cuda").to(torch.bfloat16)
+    calls = []
+    keep = nb._BlockFn.apply
+    nb._BlockFn.apply = lambda *a: calls.append(1) or keep(*a)
+    try:
+        got = passes(blk, x, gy, True)
+    finally:
+        nb._BlockFn.apply = keep
+    assert calls
+    again = passes(blk, x, gy, True)
+    blk.fused_pointwise = False
+    mod = passes(blk, x, gy, True)
+    ref = passes(blk, x.float(), gy.float(), False)
+    for n, r in ref.items():
+        if n == "mlp.fwd.3.bias":
+            continue                      # in front of an instance norm: its gradient is zero but for rounding
+        assert torch.equal(got[n], again[n]), n
+        e, em = rel(got[n], r), rel(mod[n], r)
+        assert e < 1.5e-2 and e < 1.25 * em + 1e-3, (n, e, em)
+    # inference: the same block without a gradient
+    blk.fused_pointwise = True
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert rel(blk.eval()(x), ref["y"]) < 1.5e-2
+
+
+def test_frozen_parameters_and_input(lib_built):
+    """Only what asks for a gradient gets one."""
+    import makani_amd as ma
+
+    torch.manual_seed(5)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    names = [n for n, _ in blk.named_parameters()]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = blk(x)
+        full = dict(zip(names, torch.autograd.grad(y.float().square().sum(), list(blk.parameters()))))
+    for only in names:
+        if only == "mlp.fwd.3.bias":
+            continue
+        for n, p in blk.named_parameters():
+            p.requires_grad_(n == only)
+            p.grad = None
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            blk(x).float().square().sum().backward()
+        for n, p in blk.named_parameters():
+            assert (p.grad is not None) == (n == only), n
+            if n == only:
+                assert torch.equal(p.grad, full[n]), n
+
+
+@pytest.mark.parametrize("cin,hid,cout,H,W", [(5, 33, 7, 12, 16), (73, 128, 100, 24, 32), (16, 200, 130, 40, 64)])
+def test_conv_gelu_conv(lib_built, cin, hid, cout, H, W):
+    from makani_amd.sfnonet import EncoderDecoder
+
+    print(f"case chain {cin} {hid} {cout}", flush=True)
+    torch.manual_seed(6)
+    enc = EncoderDecoder(1, cin, cout, hid, nn.GELU).cuda()
+    with torch.no_grad():
+        enc.fwd[0].bias.normal_()
+    x = torch.randn(2, cin, H, W, device="cuda")
+    gy = torch.randn(2, cout, H, W, device="cuda")
+    got = passes(enc, x, gy, True)
+    ref = passes(enc, x, gy, False)
+    for n, r in ref.items():
+        assert rel(got[n], r) < 1e-2, n
