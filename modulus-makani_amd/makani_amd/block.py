@@ -15,10 +15,7 @@ from ._lib import lib, check
 from . import pointwise as pw
 from .contractions import packed_for
 from .sht import _stream_ptr
-
-
-def _f32(t):
-    return t.detach().float().contiguous() if t is not None else None
+from .spectral_convolution import SpectralConv
 
 
 def _ptr(t):
@@ -26,13 +23,20 @@ def _ptr(t):
 
 
 def _no_hooks(*mods):
+    if torch.nn.modules.module._has_any_global_hook():
+        return False
     return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in mods)
+
+
+def plain_conv(m):
+    """A convolution whose forward is known: subclasses (quantisation, adapters) bring their own."""
+    return type(m) in (nn.Conv2d, pw.PointwiseConv2d)
 
 
 def mlp_convs(blk):
     """(fc1, fc2) of a conv -> GELU -> conv MLP, or None."""
     m = [f for f in blk.mlp.fwd if not isinstance(f, nn.Identity)]
-    ok = len(m) == 3 and isinstance(m[0], nn.Conv2d) and isinstance(m[2], nn.Conv2d) and isinstance(m[1], nn.GELU) and m[1].approximate == "none"
+    ok = len(m) == 3 and plain_conv(m[0]) and plain_conv(m[2]) and type(m[1]) is nn.GELU and m[1].approximate == "none"
     return (m[0], m[2]) if ok else None
 
 
@@ -41,41 +45,50 @@ def supported(blk, x):
     conv, fwd, inv = blk.filter.filter, blk.filter.filter.forward_transform, blk.filter.filter.inverse_transform
     if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or mlp_convs(blk) is None:
         return False
-    if not (isinstance(blk.norm0, nn.InstanceNorm2d) and isinstance(blk.norm1, nn.InstanceNorm2d)) or inv.mmax > inv.nlon // 2 + 1:
+    if type(blk.norm0) is not nn.InstanceNorm2d or type(blk.norm1) is not nn.InstanceNorm2d or inv.mmax > inv.nlon // 2 + 1:
+        return False
+    if type(blk.act_layer0) is not nn.GELU or type(conv) is not SpectralConv or not plain_conv(blk.outer_skip):
         return False
     if tuple(x.shape[2:]) != (fwd.nlat, fwd.nlon) or (inv.nlat * inv.nlon) % 8 != 0:
         return False
     if not lib.sfno_sht_io_dtype_supported(fwd.plan(x.device).handle, _lib.DTYPE_BF16) or not lib.sfno_sht_io_dtype_supported(inv.plan(x.device).handle, _lib.DTYPE_BF16):
         return False
-    fc1, fc2 = mlp_convs(blk)
-    params = [p for m in (blk.norm0, blk.norm1, fc1, fc2, blk.outer_skip) for p in (m.weight, m.bias) if p is not None]
-    return all(p.dtype == torch.float32 and p.is_cuda for p in params) and _no_hooks(
+    wf, *params = [p for p in block_params(blk) if p is not None]
+    return wf.dtype == torch.complex64 and wf.is_cuda and all(p.dtype == torch.float32 and p.is_cuda for p in params) and _no_hooks(
         blk.filter, conv, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.mlp.fwd, *blk.mlp.fwd, blk.outer_skip)
 
 
-class _Call:
-    """The sfno_block structure of one call, and what has to stay alive while it is used."""
+def block_params(blk):
+    """The block's parameters in the order of _Call: filter, skip, W1, b1, W2, b2, gamma0, beta0, gamma1, beta1 (None where there is none)."""
+    fc1, fc2 = mlp_convs(blk)
+    n0, n1 = blk.norm0, blk.norm1
+    return [blk.filter.filter.weight, blk.outer_skip.weight, fc1.weight, fc1.bias, fc2.weight, fc2.bias, n0.weight, n0.bias, n1.weight, n1.bias]
 
-    def __init__(self, blk, x, filter_weight, skip_weight, backward=False):
+
+class _Call:
+    """The sfno_block structure of one call, and what has to stay alive while it is used.  The values come from `params` alone: the
+    modules may hold others by the time of the backward (functional calls, parametrisations)."""
+
+    def __init__(self, blk, x, params, backward=False):
         conv = blk.filter.filter
         fwd, inv = conv.forward_transform, conv.inverse_transform
-        fc1, fc2 = mlp_convs(blk)
-        n0, n1, dev = blk.norm0, blk.norm1, x.device
+        wf, wskip, w1, b1, w2, b2, g0, be0, g1, be1 = params
+        dev = x.device
         b = _lib.Block()
-        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(filter_weight, conv.compute), pw.packed_weight(fc1.weight), pw.packed_weight(fc2.weight),
-                            pw.packed_weight(skip_weight)]
+        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(wf, conv.compute), pw.packed_weight(w1), pw.packed_weight(w2), pw.packed_weight(wskip)]
         b.fwd, b.inv, b.weights = keep[0].handle, keep[1].handle, keep[2].handle
         b.w1, b.w2, b.wskip = (t.data_ptr() for t in keep[3:6])
         if backward:
-            adj = [fwd.plan(dev, adjoint=True), inv.plan(dev, adjoint=True), packed_for(filter_weight, conv.compute, adjoint=True),
-                   pw.packed_weight(fc1.weight, transposed=True), pw.packed_weight(fc2.weight, transposed=True), pw.packed_weight(skip_weight, transposed=True)]
+            adj = [fwd.plan(dev, adjoint=True), inv.plan(dev, adjoint=True), packed_for(wf, conv.compute, adjoint=True),
+                   pw.packed_weight(w1, transposed=True), pw.packed_weight(w2, transposed=True), pw.packed_weight(wskip, transposed=True)]
             b.fwd_adj, b.inv_adj, b.weights_adj = adj[0].handle, adj[1].handle, adj[2].handle
             b.w1t, b.w2t, b.wskipt = (t.data_ptr() for t in adj[3:6])
             keep += adj
-        b.b1, b.b2 = _ptr(fc1.bias), _ptr(fc2.bias)
-        b.gamma0, b.beta0, b.gamma1, b.beta1 = _ptr(n0.weight), _ptr(n0.bias), _ptr(n1.weight), _ptr(n1.bias)
-        b.eps0, b.eps1 = n0.eps, n1.eps
-        b.batch, b.c_in, b.embed, b.hidden = x.shape[0], x.shape[1], conv.out_channels, fc1.out_channels
+        vectors = [t.detach().contiguous() if t is not None else None for t in (b1, b2, g0, be0, g1, be1)]
+        keep += vectors
+        b.b1, b.b2, b.gamma0, b.beta0, b.gamma1, b.beta1 = (_ptr(t) for t in vectors)
+        b.eps0, b.eps1 = blk.norm0.eps, blk.norm1.eps
+        b.batch, b.c_in, b.embed, b.hidden = x.shape[0], x.shape[1], conv.out_channels, w1.shape[0]
         self.b = b
         self.P = (inv.nlat, inv.nlon)
         self.stream = _stream_ptr(dev)
@@ -94,7 +107,12 @@ def forward(blk, x, filter_weight=None, skip_weight=None, defer_skip=False):
     """The block without autograd.  filter_weight, skip_weight: in place of the block's own.  defer_skip: returns (y2, residual, scale,
     shift) of the last sum scale * y2 + shift + skip(residual) instead of running it."""
     x = x.contiguous()
-    c = _Call(blk, x, blk.filter.filter.weight if filter_weight is None else filter_weight, blk.outer_skip.weight if skip_weight is None else skip_weight)
+    params = block_params(blk)
+    if filter_weight is not None:
+        params[0] = filter_weight
+    if skip_weight is not None:
+        params[1] = skip_weight
+    c = _Call(blk, x, params)
     B, E = x.shape[0], c.b.embed
     if not defer_skip:
         out = torch.empty((B, E, *c.P), dtype=torch.bfloat16, device=x.device)
@@ -117,7 +135,7 @@ class _BlockFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, blk, *params):
         x = x.detach().contiguous()
-        c = _Call(blk, x, blk.filter.filter.weight, blk.outer_skip.weight)
+        c = _Call(blk, x, params)
         out = torch.empty((x.shape[0], c.b.embed, *c.P), dtype=torch.bfloat16, device=x.device)
         kept = c.forward(x, 1, out)
         ctx.blk = blk
@@ -130,11 +148,10 @@ class _BlockFn(torch.autograd.Function):
         x, kept, *params = ctx.saved_tensors
         g = g.to(torch.bfloat16).contiguous()
         blk, need = ctx.blk, ctx.needs_input_grad
-        c = _Call(blk, x, blk.filter.filter.weight, blk.outer_skip.weight, backward=True)
-        # in the order of trainable_params: filter, skip, W1, b1, W2, b2, gamma0, beta0, gamma1, beta1
+        c = _Call(blk, x, params, backward=True)
         want = [p is not None and n for p, n in zip(params, need[2:])]
         want[2], want[4] = want[2] or want[3], want[4] or want[5]          # a bias gradient is a column of its matrix's kernel
-        grads = [torch.empty_like(p) if w else None for p, w in zip(params, want)]
+        grads = [torch.empty(p.shape, dtype=p.dtype, device=p.device) if w else None for p, w in zip(params, want)]
         gx = torch.empty_like(x) if need[0] else None
         s = _lib.BlockGrads()
         s.gx, s.gfilter = _ptr(gx), _ptr(grads[0])
@@ -148,6 +165,4 @@ class _BlockFn(torch.autograd.Function):
 
 def train(blk, x):
     """The block with autograd (supported() holds and a gradient is being recorded)."""
-    fc1, fc2 = mlp_convs(blk)
-    n0, n1 = blk.norm0, blk.norm1
-    return _BlockFn.apply(x, blk, blk.filter.filter.weight, blk.outer_skip.weight, fc1.weight, fc1.bias, fc2.weight, fc2.bias, n0.weight, n0.bias, n1.weight, n1.bias)
+    return _BlockFn.apply(x, blk, *block_params(blk))

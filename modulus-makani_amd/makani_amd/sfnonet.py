@@ -106,7 +106,7 @@ class EncoderDecoder(nn.Module):
     def forward(self, x):
         # training under bf16: convolution, GELU and convolution with the GELU in the convolutions' epilogues, both ways
         if len(self.fwd) == 3 and pw.trainable_active(x) and _is_conv1x1(self.fwd[0]) and _is_gelu(self.fwd[1]) and _is_conv1x1(self.fwd[2]) \
-                and native_block._no_hooks(self.fwd, *self.fwd):
+                and native_block.plain_conv(self.fwd[0]) and native_block.plain_conv(self.fwd[2]) and native_block._no_hooks(self.fwd, *self.fwd):
             y = pw.conv_gelu_conv_trainable(x, self.fwd[0], self.fwd[2])
             if y is not None:
                 return y

@@ -118,6 +118,54 @@ def test_frozen_parameters_and_input(lib_built):
                 assert torch.equal(p.grad, full[n]), n
 
 
+def test_backward_uses_the_values_of_the_forward(lib_built):
+    """A functional call swaps other values in for the forward only; a strided parameter is read as its values, not as its memory."""
+    import makani_amd as ma
+
+    torch.manual_seed(6)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    a, b = make_block(sht, isht, 16, 2.0), make_block(sht, isht, 16, 2.0)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    want = passes(b, x, torch.ones_like(x), True)
+    values = {}
+    for n, p in b.named_parameters():
+        store = torch.empty(*p.shape, 2, dtype=p.dtype, device=p.device)
+        store[..., 0] = p.detach()
+        values[n] = store[..., 0].requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = torch.func.functional_call(a, values, (x,))
+    grads = torch.autograd.grad(y, list(values.values()), torch.ones_like(y))
+    assert torch.equal(y, want["y"])
+    for n, g in zip(values, grads):
+        assert torch.equal(g, want[n]), n
+
+
+def test_subclassed_convolutions_and_global_hooks_keep_the_modules(lib_built):
+    import makani_amd as ma
+
+    class Doubled(nn.Conv2d):
+        def forward(self, x):
+            return 2.0 * super().forward(x)
+
+    torch.manual_seed(7)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    gy = torch.randn_like(x)
+    seen = []
+    handle = nn.modules.module.register_module_forward_hook(lambda m, a, y: seen.append(m))
+    try:
+        passes(blk, x, gy, True)
+    finally:
+        handle.remove()
+    assert blk.mlp.fwd[0] in seen and blk.norm1 in seen
+    fc1 = Doubled(16, 32, 1).cuda()
+    fc1.load_state_dict(blk.mlp.fwd[0].state_dict())
+    blk.mlp.fwd[0] = fc1
+    ref = passes(blk, x.float(), gy.float(), False)
+    assert rel(passes(blk, x, gy, True)["y"], ref["y"]) < 1.5e-2
+
+
 @pytest.mark.parametrize("cin,hid,cout,H,W", [(5, 33, 7, 12, 16), (73, 128, 100, 24, 32), (16, 200, 130, 40, 64)])
 def test_conv_gelu_conv(lib_built, cin, hid, cout, H, W):
     from makani_amd.sfnonet import EncoderDecoder
