@@ -65,16 +65,18 @@ def supported(x):
 
 def conv1x1(x, weight, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
     """act(conv1x1(x, weight) + bias) + add_scale * addend + add_shift  ->  bf16 [B, O, H, W]."""
-    return _conv1x1(x, packed_weight(weight), weight.shape[0], weight.shape[1], bias, act, addend, add_scale, add_shift)
+    return _conv1x1(x, weight, False, bias, act, addend, add_scale, add_shift)
 
 
-def _conv1x1(x, pw, O, K_weight, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
+def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
+    O, K_weight = (weight.shape[1], weight.shape[0]) if transposed else weight.shape[:2]
     if not supported(x):
         raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
     x = x.contiguous()
     B, K, H, W = x.shape
     if K_weight != K:
         raise RuntimeError(f"conv1x1: input has {K} channels, weight expects {K_weight}")
+    pw = packed_weight(weight, transposed)
     y = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
     if bias is not None:
         bias = bias.detach().float().contiguous()
@@ -201,7 +203,7 @@ class _Conv1x1(torch.autograd.Function):
         gy = gy.to(torch.bfloat16).contiguous()
         gx = gw = gb = None
         if ctx.needs_input_grad[0]:
-            gx = _conv1x1(gy, packed_weight(weight, transposed=True), weight.shape[1], weight.shape[0]).to(ctx.x_dtype)
+            gx = _conv1x1(gy, weight, True).to(ctx.x_dtype)
         if ctx.needs_input_grad[1] or (ctx.has_bias and ctx.needs_input_grad[2]):
             gw, gb = conv1x1_weight_grad(gy, xb, ctx.has_bias)
             gw = gw.reshape(weight.shape).to(weight.dtype)
@@ -249,7 +251,7 @@ class _ConvGeluConv(torch.autograd.Function):
                 gw1, gb1 = conv1x1_weight_grad(gz, xb, ctx.biases[0])
                 gw1 = gw1.reshape(w1.shape)
             if need[0]:
-                gx = _conv1x1(gz, packed_weight(w1, transposed=True), w1.shape[1], w1.shape[0]).to(ctx.x_dtype)
+                gx = _conv1x1(gz, w1, True).to(ctx.x_dtype)
         return gx, gw1, gb1, gw2, gb2
 
 
