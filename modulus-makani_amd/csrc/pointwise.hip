@@ -83,9 +83,14 @@ __device__ __forceinline__ float gelu_grad(float x) {
     return fmaf(x, phi, x > 0.f ? 1.f - e : e);
 }
 
+// Epilogues: exact GELU on the output and / or "+ scale * addend + shift"; for training GELU_PRE (the output before the GELU is stored as
+// well, to a.Z, and activated as stored) and GELU_BWD (the output times the GELU's derivative at `addend`)
+enum { PW_PLAIN = 0, PW_GELU = 1, PW_ADD = 2, PW_GELU_PRE = 4, PW_GELU_BWD = 8 };
+
 // NW = wavefronts per workgroup, side by side along the pixels, 64 pixels each: 8, or 2 where that leaves CUs idle
-template <int NW>
+template <int NW, int EPI>
 __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
+    constexpr bool GELU = EPI & (PW_GELU | PW_GELU_PRE), AFF = EPI & PW_ADD, ADD = EPI & (PW_ADD | PW_GELU_BWD);
     constexpr int NT = 2;                         // pixels per lane = N tiles per wavefront
     constexpr int PW_THREADS = 64 * NW;
     constexpr int PW_PX = 32 * NT;                // pixels per wavefront
@@ -167,6 +172,20 @@ __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[mt][t][v] = 0.f;
 
+    // Bias, and the addend's scale and shift, of the wavefront's rows: row r of a 32-row tile in lanes r and r + 32, asked for here, where
+    // the wait for the operands covers them.  In the epilogue a vector load between the stores would make every store wait for the one
+    // before it (the counter retires in order), and scalar loads, a batch of eight rows at a time, were a chain of twelve round trips.
+    // At 721 x 1440, vector loads between the stores / scalar loads / this: 457 -> 73 channels 272 / 300 / 265 us; 64 -> 64 with GELU and
+    // addend 198 -> 136, 64 -> 32 83 -> 61.
+    float bias[PW_MT], scale[PW_MT], shift[PW_MT];
+#pragma unroll
+    for (int mt = 0; mt < PW_MT; ++mt) {
+        const int r = min(o0 + 32 * mt + q, a.O - 1);
+        bias[mt] = a.bias ? a.bias[r] : 0.f;
+        scale[mt] = AFF && a.add_scale ? a.add_scale[(int64_t)b * a.O + r] : 1.f;
+        shift[mt] = AFF && a.add_shift ? a.add_shift[(int64_t)b * a.O + r] : 0.f;
+    }
+
     // prologue: chunks 0 and 1 into LDS, chunks 2..D+1 of the activations and 0..D-1 of the weights in flight
     {
         u32x4 x0[XW], x1[XW];
@@ -226,65 +245,60 @@ __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
         }
     }
 
-    // epilogue: lane holds rows 8 (v / 4) + 4 ko + v % 4 of each 32-row tile and pixels 2 q, 2 q + 1.  Bias, scale and shift come
-    // through the scalar unit, the rows of both lane halves: a vector load between the stores would make every store wait for the
-    // one before it (the counter retires in order).
+    // epilogue: lane holds rows 8 (v / 4) + 4 ko + v % 4 of each 32-row tile and pixels 2 q, 2 q + 1.  (Only whole wavefronts leave here:
+    // row_value reads every lane.)
+    if (pw0 + pxw >= a.P) return;
     const int64_t px = pw0 + pxw + NT * q;
-    if (px >= a.P) return;
+    const bool inside = px < a.P;
+    const int64_t pxc = inside ? px : a.P - NT;
     unsigned short* __restrict__ Y = a.Y + (int64_t)b * a.O * a.P;
-    const unsigned short* __restrict__ R = a.addend ? a.addend + (int64_t)b * a.O * a.P : nullptr;
+    const unsigned short* __restrict__ R = ADD ? a.addend + (int64_t)b * a.O * a.P : nullptr;
+    // value of row 8 g + 4 ko + j of a 32-row tile whose lane r holds that of row r
+    auto row_value = [&](float v, int g, int j) {
+        const int lo = __builtin_amdgcn_readlane(__float_as_int(v), 8 * g + j), hi = __builtin_amdgcn_readlane(__float_as_int(v), 8 * g + 4 + j);
+        return __int_as_float(ko ? hi : lo);
+    };
 #pragma unroll
     for (int mt = 0; mt < PW_MT; ++mt) {
         if (o0 + 32 * mt >= a.O) break;
         rw_t rv[16];
-        if (R) {
+        if constexpr (ADD) {
             // all addend loads of the tile first
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int o = min(o0 + 32 * mt + 8 * (v >> 2) + 4 * ko + (v & 3), a.O - 1);
-                rv[v] = *reinterpret_cast<const rw_t*>(R + (int64_t)o * a.P + px);
+                rv[v] = *reinterpret_cast<const rw_t*>(R + (int64_t)o * a.P + pxc);
             }
         }
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int og = o0 + 32 * mt + 8 * g;                        // rows og .. og + 7 (ko = 0: the first four)
-            float ub[8], usc[8], ush[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int64_t u = min(og + i, a.O - 1);
-                ub[i] = a.bias ? uniform_load(a.bias, u) : 0.f;
-                usc[i] = R && a.add_scale ? uniform_load(a.add_scale, (int64_t)b * a.O + u) : 1.f;
-                ush[i] = R && a.add_shift ? uniform_load(a.add_shift, (int64_t)b * a.O + u) : 0.f;
+        for (int v = 0; v < 16; ++v) {
+            const int o = o0 + 32 * mt + 8 * (v >> 2) + 4 * ko + (v & 3);
+            const float bs = row_value(bias[mt], v >> 2, v & 3);
+            const float sc = AFF ? row_value(scale[mt], v >> 2, v & 3) : 1.f, sh = AFF ? row_value(shift[mt], v >> 2, v & 3) : 0.f;
+            if (o >= a.O || !inside) continue;
+            float y0 = acc[mt][0][v] + bs, y1 = acc[mt][1][v] + bs;
+            if constexpr (EPI & PW_GELU_PRE) {   // training: the pre-activation is stored as well, and activated as stored
+                rw_t zz;
+                zz[0] = bf16_pair(y0, y1);
+                *reinterpret_cast<rw_t*>(a.Z + (int64_t)b * a.O * a.P + (int64_t)o * a.P + px) = zz;
+                y0 = __uint_as_float(zz[0] << 16);
+                y1 = __uint_as_float(zz[0] & 0xffff0000u);
             }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int v = 4 * g + j, o = og + 4 * ko + j;
-                if (o >= a.O) continue;
-                const float bs = ko ? ub[4 + j] : ub[j];
-                float y0 = acc[mt][0][v] + bs, y1 = acc[mt][1][v] + bs;
-                if (a.Z) {                       // training: the pre-activation is stored as well, and activated as stored
-                    rw_t zz;
-                    zz[0] = bf16_pair(y0, y1);
-                    *reinterpret_cast<rw_t*>(a.Z + (int64_t)b * a.O * a.P + (int64_t)o * a.P + px) = zz;
-                    y0 = __uint_as_float(zz[0] << 16);
-                    y1 = __uint_as_float(zz[0] & 0xffff0000u);
-                }
-                if (a.act == SFNO_ACT_GELU) {
-                    y0 = gelu(y0);
-                    y1 = gelu(y1);
-                }
-                if (a.grad) {
-                    y0 *= gelu_grad(__uint_as_float(rv[v][0] << 16));
-                    y1 *= gelu_grad(__uint_as_float(rv[v][0] & 0xffff0000u));
-                } else if (R) {
-                    const float sc = ko ? usc[4 + j] : usc[j], sh = ko ? ush[4 + j] : ush[j];
-                    y0 += fmaf(sc, __uint_as_float(rv[v][0] << 16), sh);
-                    y1 += fmaf(sc, __uint_as_float(rv[v][0] & 0xffff0000u), sh);
-                }
-                rw_t out;
-                out[0] = bf16_pair(y0, y1);
-                *reinterpret_cast<rw_t*>(Y + (int64_t)o * a.P + px) = out;
+            if constexpr (GELU) {
+                y0 = gelu(y0);
+                y1 = gelu(y1);
             }
+            if constexpr (EPI & PW_GELU_BWD) {
+                y0 *= gelu_grad(__uint_as_float(rv[v][0] << 16));
+                y1 *= gelu_grad(__uint_as_float(rv[v][0] & 0xffff0000u));
+            }
+            if constexpr (AFF) {
+                y0 += fmaf(sc, __uint_as_float(rv[v][0] << 16), sh);
+                y1 += fmaf(sc, __uint_as_float(rv[v][0] & 0xffff0000u), sh);
+            }
+            rw_t out;
+            out[0] = bf16_pair(y0, y1);
+            *reinterpret_cast<rw_t*>(Y + (int64_t)o * a.P + px) = out;
         }
     }
 }
@@ -346,13 +360,10 @@ __device__ __forceinline__ void dm_barrier() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// Epilogue: exact GELU on the output and / or "+ scale * addend + shift"; for training GELU_PRE (the output before the GELU is stored as
-// well, to a.Z, and activated as stored) and GELU_BWD (the output times the GELU's derivative at `addend`)
-enum { DM_PLAIN = 0, DM_GELU = 1, DM_ADD = 2, DM_GELU_PRE = 4, DM_GELU_BWD = 8 };
 template <int MT, int EPI>
 __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_kernel(PointwiseArgs a) {
     using DM = DmGeo<MT>;
-    constexpr bool GELU = EPI & (DM_GELU | DM_GELU_PRE), AFF = EPI & DM_ADD, ADD = EPI & (DM_ADD | DM_GELU_BWD);
+    constexpr bool GELU = EPI & (PW_GELU | PW_GELU_PRE), AFF = EPI & PW_ADD, ADD = EPI & (PW_ADD | PW_GELU_BWD);
     __shared__ __align__(16) unsigned char lds[DM::LDS];
     // tiles of this XCD, row block fastest: q -> (row block q % n_oblk, strip (q / n_oblk) * 8 + xcd); the workgroups of the
     // XCD deal them out round robin, so the row blocks of one strip run at the same time on one L2
@@ -537,7 +548,7 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
                     float y[4];
 #pragma unroll
                     for (int t = 0; t < 4; ++t) y[t] = acc[mt][t][v] + bs;
-                    if constexpr (EPI & DM_GELU_PRE) {
+                    if constexpr (EPI & PW_GELU_PRE) {
                         u32x2 z;
 #pragma unroll
                         for (int pp = 0; pp < 2; ++pp) {
@@ -551,7 +562,7 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
 #pragma unroll
                         for (int t = 0; t < 4; ++t) y[t] = gelu(y[t]);
                     }
-                    if constexpr (EPI & DM_GELU_BWD) {
+                    if constexpr (EPI & PW_GELU_BWD) {
                         const u32x2 r = rv[mh & 1][4 * g + jj];
 #pragma unroll
                         for (int pp = 0; pp < 2; ++pp) {
@@ -938,15 +949,29 @@ int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, 
 }
 
 template <int MT>
-static void dma_go(const PointwiseArgs& a, int64_t blocks, hipStream_t s) {
+static void dma_go(const PointwiseArgs& a, int64_t blocks, int epi, hipStream_t s) {
     const dim3 grid((unsigned)std::min<int64_t>(blocks, std::max(8, DmGeo<MT>::WG_PER_CU * (device_cus() / 8 * 8))));
-    const bool g = a.act == SFNO_ACT_GELU, r = a.addend != nullptr;
-    if (a.Z) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU_PRE>), grid, dim3(512), 0, s, a);
-    else if (a.grad) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU_BWD>), grid, dim3(512), 0, s, a);
-    else if (g && r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU | DM_ADD>), grid, dim3(512), 0, s, a);
-    else if (g) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_GELU>), grid, dim3(512), 0, s, a);
-    else if (r) hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_ADD>), grid, dim3(512), 0, s, a);
-    else hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, DM_PLAIN>), grid, dim3(512), 0, s, a);
+    switch (epi) {
+        case PW_GELU_PRE: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU_PRE>), grid, dim3(512), 0, s, a); break;
+        case PW_GELU_BWD: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU_BWD>), grid, dim3(512), 0, s, a); break;
+        case PW_GELU | PW_ADD: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU | PW_ADD>), grid, dim3(512), 0, s, a); break;
+        case PW_GELU: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU>), grid, dim3(512), 0, s, a); break;
+        case PW_ADD: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_ADD>), grid, dim3(512), 0, s, a); break;
+        default: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_PLAIN>), grid, dim3(512), 0, s, a);
+    }
+}
+
+template <int NW>
+static void gemm_go(const PointwiseArgs& a, int64_t blocks, int epi, hipStream_t s) {
+    const dim3 grid((unsigned)blocks), block(64 * NW);
+    switch (epi) {
+        case PW_GELU_PRE: hipLaunchKernelGGL((pw_gemm_kernel<NW, PW_GELU_PRE>), grid, block, 0, s, a); break;
+        case PW_GELU_BWD: hipLaunchKernelGGL((pw_gemm_kernel<NW, PW_GELU_BWD>), grid, block, 0, s, a); break;
+        case PW_GELU | PW_ADD: hipLaunchKernelGGL((pw_gemm_kernel<NW, PW_GELU | PW_ADD>), grid, block, 0, s, a); break;
+        case PW_GELU: hipLaunchKernelGGL((pw_gemm_kernel<NW, PW_GELU>), grid, block, 0, s, a); break;
+        case PW_ADD: hipLaunchKernelGGL((pw_gemm_kernel<NW, PW_ADD>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((pw_gemm_kernel<NW, PW_PLAIN>), grid, block, 0, s, a);
+    }
 }
 
 int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s) {
@@ -971,16 +996,17 @@ int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s) {
     const int64_t strips = a.n_strips * a.B;
     const int64_t blocks = (strips + 7) / 8 * 8 * a.n_oblk;
     if (blocks > 0x7fffffffLL || (dma && a.P > 0x7fffffffLL)) return SFNO_EUNSUPPORTED;
+    const int epi = a.Z ? PW_GELU_PRE : a.grad ? PW_GELU_BWD : (a.act == SFNO_ACT_GELU ? PW_GELU : 0) | (a.addend ? PW_ADD : 0);
     if (dma) {     // persistent: as many workgroups as stay resident, the same number on every XCD
         switch (mt) {
-            case 1: dma_go<1>(a, blocks, s); break;
-            case 2: dma_go<2>(a, blocks, s); break;
-            default: dma_go<3>(a, blocks, s); break;
+            case 1: dma_go<1>(a, blocks, epi, s); break;
+            case 2: dma_go<2>(a, blocks, epi, s); break;
+            default: dma_go<3>(a, blocks, epi, s); break;
         }
     } else if (nw == 2)
-        hipLaunchKernelGGL(pw_gemm_kernel<2>, dim3((unsigned)blocks), dim3(128), 0, s, a);
+        gemm_go<2>(a, blocks, epi, s);
     else
-        hipLaunchKernelGGL(pw_gemm_kernel<8>, dim3((unsigned)blocks), dim3(512), 0, s, a);
+        gemm_go<8>(a, blocks, epi, s);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
