@@ -5,16 +5,18 @@
 // (what autograd derives for nn.Conv2d(kernel_size=1), makani/models/common/layers.py:95-116,160-216).  Both operands are
 // pixel-contiguous and the sum runs over the pixels, so a row of g is an A operand and a row of x a B operand of
 // v_mfma_f32_32x32x16_bf16 as they lie in memory: 8 consecutive pixels per lane, no transposition.  The bias gradient
-// rides along as one more column: row K of x is taken to be all ones.
+// is one more column against a B operand of ones, in registers, of the wavefronts that hold the first columns: as column K of the
+// tiles it took a column of tiles to itself where K is a multiple of 256 (eight instead of six for 768 -> 384 channels with bias:
+// 1249 -> 997 us at 721 x 1440).
 //
 // A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile of dW and a contiguous share of the (sample, 32-pixel chunk)
 // sequence.  Per chunk 256 rows of g and 256 rows of x (64 bytes each) go straight from memory into a ring of four LDS
 // stages with global_load_lds_dwordx4, three chunks ahead of the matrix instructions (issued from inline assembly with a
 // counted wait, as in the forward kernel); a lane fetches the 16-byte piece whose LDS slot it owns, and the pieces of a row
 // are permuted by (row >> 1) & 3 so that the 16-byte fragment reads of eight consecutive rows cover all banks.  Pieces
-// past the end of a sample come from a block of zeros, the bias column from a block of ones.  Each wavefront multiplies
+// past the end of a sample come from a block of zeros.  Each wavefront multiplies
 // 64 x 128 (two A and four B fragments per 16 pixels for eight matrix instructions).  The shares' partial tiles go to a
-// workspace [share][O][K + 1] and a second kernel adds them up in a fixed order: results do not depend on scheduling.
+// workspace [share][O][K (+ 1 with bias)] and a second kernel adds them up in a fixed order: results do not depend on scheduling.
 // All tiles of one share run on one XCD (workgroups are dealt to the XCDs round robin by linear id), where they meet
 // the share's rows of g and x in L2.
 #include "sfno_internal.h"
@@ -27,7 +29,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int WG_THREADS = 512;
 constexpr int WG_TO = 256;            // rows of dW (output channels) per workgroup
-constexpr int WG_TK = 256;            // columns of dW (input channels, + the bias column) per workgroup
+constexpr int WG_TK = 256;            // columns of dW (input channels) per workgroup
 constexpr int WG_PX = 32;             // pixels per chunk: four 16-byte pieces per row
 constexpr int WG_ROWS = WG_TO + WG_TK;
 constexpr int WG_STAGE = WG_ROWS * 2 * WG_PX;                 // bytes per LDS stage
@@ -40,9 +42,8 @@ static_assert(WG_TO * (WG_PX / 8) % WG_THREADS == 0, "a thread's piece j is a ro
 static_assert(WG_RSTEP % 8 == 0, "a thread's pieces share the permutation of their rows");
 static_assert(WG_STAGES * WG_STAGE <= 160 * 1024, "one workgroup per CU");
 
-// sources of the pieces that are not read from the tensors
+// source of the pieces that are not read from the tensors
 __device__ __align__(16) const unsigned int wg_zero16[4] = {0u, 0u, 0u, 0u};
-__device__ __align__(16) const unsigned int wg_ones16[4] = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
 
 // 16 bytes per lane from global memory to LDS base + 16 lane (M0 carries the base; the compiler reserves M0 and does not
 // accept it on a clobber list: nothing else in this file may depend on M0)
@@ -57,10 +58,10 @@ struct WgradShape {
 
 // how the launcher and the workspace query divide the work: shares of at least eight chunks, one workgroup per CU (all
 // workgroups resident at once, the tiles of a share side by side on one XCD)
-static WgradShape wgrad_shape(int O, int Kext, int B, int64_t P) {
+static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
     WgradShape s;
     s.n_ot = (O + WG_TO - 1) / WG_TO;
-    s.n_kt = (Kext + WG_TK - 1) / WG_TK;
+    s.n_kt = (K + WG_TK - 1) / WG_TK;
     s.cps = (P + WG_PX - 1) / WG_PX;
     s.chunks = s.cps * B;
     const int tiles = s.n_ot * s.n_kt;
@@ -104,21 +105,12 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     constexpr int JG = WG_TO * (WG_PX / 8) / WG_THREADS;
     const int part = (tid & 3) ^ ((tid >> 3) & 3);
     const unsigned short* rowp[WG_PIECES];     // first pixel of the row in sample 0 (rows past the matrix: its last row, whose products are never stored)
-    bool ones[WG_PIECES];                      // the bias column: all ones
 #pragma unroll
     for (int j = 0; j < WG_PIECES; ++j) {
         const int row = (tid >> 2) + WG_RSTEP * j;
-        if (j < JG) {
-            rowp[j] = a.G + (int64_t)min(o0 + row, a.O - 1) * a.P;
-            ones[j] = false;
-        } else {
-            const int k = k0 + row - WG_TO;
-            rowp[j] = a.X + (int64_t)min(k, a.K - 1) * a.P;
-            ones[j] = k == a.K && a.Kext > a.K;
-        }
+        rowp[j] = j < JG ? a.G + (int64_t)min(o0 + row, a.O - 1) * a.P : a.X + (int64_t)min(k0 + row - WG_TO, a.K - 1) * a.P;
     }
     const unsigned short* zero16 = reinterpret_cast<const unsigned short*>(wg_zero16);
-    const unsigned short* ones16 = reinterpret_cast<const unsigned short*>(wg_ones16);
     // next chunk to ask for: sample ib, chunk ic of the sample, and where its pieces lie (counted along: a chunk inside a
     // sample costs one addition per piece; the addresses are worked out afresh once per sample)
     int64_t ib = c_begin / a.cps;
@@ -128,7 +120,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
         const int64_t p = ic * WG_PX + 8 * part;
         const int64_t og = ib * a.O * a.P + p, ox = ib * a.K * a.P + p;
 #pragma unroll
-        for (int j = 0; j < WG_PIECES; ++j) cur[j] = ones[j] ? ones16 : rowp[j] + (j < JG ? og : ox);
+        for (int j = 0; j < WG_PIECES; ++j) cur[j] = rowp[j] + (j < JG ? og : ox);
     };
     locate();
     auto issue = [&](int stage) {
@@ -148,11 +140,15 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
             locate();
         } else {
 #pragma unroll
-            for (int j = 0; j < WG_PIECES; ++j) cur[j] += (j >= JG && ones[j]) ? 0 : WG_PX;
+            for (int j = 0; j < WG_PIECES; ++j) cur[j] += WG_PX;
         }
     };
 
-    f32x16 acc[2][4];
+    f32x16 acc[2][4], accb[2];
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) accb[mt][v] = 0.f;
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -166,7 +162,9 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     const unsigned fa = (wo * 64 + (lane & 31)) * 64, fb = (WG_TO + wk * 128 + (lane & 31)) * 64;
     const unsigned pk[2] = {(unsigned)((kg ^ sw) * 16), (unsigned)(((2 + kg) ^ sw) * 16)};
 
-    const bool live = o0 + wo * 64 < a.O && k0 + wk * 128 < a.Kext;
+    const bool live = o0 + wo * 64 < a.O && k0 + wk * 128 < a.K;
+    const bool bias = a.Kext > a.K && k0 + wk * 128 == 0;
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
     // Ring of four stages: chunk i is multiplied while chunks i + 1 .. i + 3 are on their way.  The only vector memory
     // operations of the loop are the four loads per wavefront and chunk, so "at most eight outstanding" means chunk i has
     // landed while two later ones may still be under way.
@@ -200,6 +198,10 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
             for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
                 for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mt], bf[nt], acc[mt][nt], 0, 0, 0);
+            if (bias) {
+#pragma unroll
+                for (int mt = 0; mt < 2; ++mt) accb[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mt], ones, accb[mt], 0, 0, 0);
+            }
         }
         stage = stage == WG_STAGES - 1 ? 0 : stage + 1;
     }
@@ -214,46 +216,55 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int o = o0 + wo * 64 + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (o < a.O && kk < a.Kext) out[(int64_t)o * a.Kext + kk] = acc[mt][nt][v];
+                if (o < a.O && kk < a.K) out[(int64_t)o * a.Kext + kk] = acc[mt][nt][v];
             }
         }
+    if (bias && (lane & 31) == 0) {           // all columns of accb are the same
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int o = o0 + wo * 64 + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                if (o < a.O) out[(int64_t)o * a.Kext + a.K] = accb[mt][v];
+            }
+    }
 }
 
-// dW[o][k] = sum over the shares, in order; column K goes to db.  A thread sums four consecutive entries of the
-// [O][Kext] matrices (16-byte loads, eight shares in flight) and stores them one by one: they may straddle a row.
-__global__ __launch_bounds__(256) void pw_wgrad_reduce_kernel(const float* __restrict__ ws, float* __restrict__ dW, float* __restrict__ db, int O, int K,
-                                                              int Kext, int splits) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const int64_t n = (int64_t)O * Kext;
-    const int64_t idx = 4 * ((int64_t)blockIdx.x * blockDim.x + threadIdx.x);
-    if (idx >= n) return;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    if (idx + 4 <= n && n % 4 == 0) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-        for (int i = 0; i < splits; ++i) acc += *reinterpret_cast<const f32x4*>(ws + (int64_t)i * n + idx);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[e] = acc[e];
-    } else {
-        for (int i = 0; i < splits; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (idx + e < n) s[e] += ws[(int64_t)i * n + idx + e];
+// dW[o][k] = sum over the shares, in a fixed order; column K goes to db.  A workgroup's 16 wavefronts take every 16th share each of
+// the same 64 V entries and meet in LDS: latency is what bounds small matrices (up to 256 shares of 73 x 73 entries; one thread per
+// four entries walked all shares in turn: both kernels 145 us for 73 -> 73 channels at 2 x 181 x 360, now 20; 128 -> 256 with bias 45 -> 35).  V = 4 entries per lane (16-byte loads; a share must then start on
+// 16 bytes) where that still makes 256 workgroups, else one.
+constexpr int WR_WAVES = 16;
+template <int V>
+__global__ __launch_bounds__(64 * WR_WAVES) void pw_wgrad_reduce_kernel(const float* __restrict__ ws, float* __restrict__ dW, float* __restrict__ db, int K,
+                                                                        int Kext, int64_t n, int splits) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    __shared__ __align__(16) float part[WR_WAVES][64 * V];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t base = (int64_t)blockIdx.x * (64 * V), idx = base + V * lane;
+    vec acc = (vec)(0.f);
+    if (idx < n) {
+#pragma unroll 4
+        for (int i = wave; i < splits; i += WR_WAVES) acc += *reinterpret_cast<const vec*>(ws + (int64_t)i * n + idx);
     }
+    *reinterpret_cast<vec*>(&part[wave][V * lane]) = acc;
+    __syncthreads();
+    const int64_t e = base + threadIdx.x;
+    if (threadIdx.x >= 64 * V || e >= n) return;
+    float s = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        if (idx + e >= n) break;
-        const int o = (int)((idx + e) / Kext), k = (int)(idx + e - (int64_t)o * Kext);
-        if (k < K)
-            dW[(int64_t)o * K + k] = s[e];
-        else if (db)
-            db[o] = s[e];
-    }
+    for (int w = 0; w < WR_WAVES; ++w) s += part[w][threadIdx.x];
+    const int64_t o = e / Kext;
+    const int k = (int)(e - o * Kext);
+    if (k < K)
+        dW[o * K + k] = s;
+    else if (db)
+        db[o] = s;
 }
 
 size_t pointwise_wgrad_workspace_bytes(int O, int K, int has_bias, int B, int64_t P) {
     const int Kext = K + (has_bias ? 1 : 0);
-    const WgradShape s = wgrad_shape(O, Kext, B, P);
+    const WgradShape s = wgrad_shape(O, K, B, P);
     return sizeof(float) * (size_t)s.splits * (size_t)O * (size_t)Kext;
 }
 
@@ -261,7 +272,7 @@ int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, flo
                            size_t ws_bytes, hipStream_t s) {
     if (P < 8 || P % 8) return SFNO_EINVAL;
     const int Kext = K + (db ? 1 : 0);
-    const WgradShape sh = wgrad_shape(O, Kext, B, P);
+    const WgradShape sh = wgrad_shape(O, K, B, P);
     if (ws_bytes < sizeof(float) * (size_t)sh.splits * (size_t)O * (size_t)Kext) return SFNO_EINVAL;
     WgradArgs a;
     a.G = g; a.X = x; a.ws = ws;
@@ -272,7 +283,10 @@ int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, flo
     hipLaunchKernelGGL(pw_wgrad_kernel, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
     if (hipGetLastError() != hipSuccess) return SFNO_EHIP;
     const int64_t n = (int64_t)O * Kext;
-    hipLaunchKernelGGL(pw_wgrad_reduce_kernel, dim3((unsigned)((n + 1023) / 1024)), dim3(256), 0, s, ws, dW, db, O, K, Kext, sh.splits);
+    if (n % 4 == 0 && n >= 256 * 256)
+        hipLaunchKernelGGL(pw_wgrad_reduce_kernel<4>, dim3((unsigned)((n + 255) / 256)), dim3(64 * WR_WAVES), 0, s, ws, dW, db, K, Kext, n, sh.splits);
+    else
+        hipLaunchKernelGGL(pw_wgrad_reduce_kernel<1>, dim3((unsigned)((n + 63) / 64)), dim3(64 * WR_WAVES), 0, s, ws, dW, db, K, Kext, n, sh.splits);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

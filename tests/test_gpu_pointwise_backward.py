@@ -27,6 +27,9 @@ WGRAD_CASES = [
     (1, 1, 1, 1, 8, True),             # smallest shape
     (1, 384, 768, 120, 240, True),     # MLP fc1 at a quarter of the model's grid: many shares
     (2, 768, 384, 60, 124, False),     # MLP fc2, two samples, 232.5 chunks per sample
+    (1, 257, 70, 24, 16, True),        # one column in the second column tile: the bias belongs to the first only
+    (2, 73, 73, 64, 96, False),        # an odd number of entries, 48 shares: the reduction's single loads
+    (1, 256, 256, 16, 40, True),       # 65792 entries: its 16-byte loads, few shares (fewer than its wavefronts)
 ]
 
 
