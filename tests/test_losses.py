@@ -115,3 +115,31 @@ def test_h1_loss_gradient(lib_built, absolute, squared):
     (v if absolute else v / norms(tar.double())).sum().backward()
     g, gr = x.grad.cpu().double(), xr.grad
     assert float(torch.linalg.norm(g - gr) / torch.linalg.norm(gr)) < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,lmax,mmax", [(1, 5, 4), (2, 1, 1), (3, 40, 70), (73, 91, 50), (128, 33, 33), (129, 20, 9), (333, 12, 12)])
+def test_degree_power_kernels_on_coefficients(lib_built, rows, lmax, mmax):
+    """Odd and even row counts, one and several workgroups of 64 row pairs, more and fewer orders than run in parallel; what stands in
+    the padding columns and above the diagonal is never used.  fp32 sums of positive terms: 1e-6 relative bounds them for <= 100 terms."""
+    from makani_amd._lib import lib
+    from makani_amd.losses import _DegreePowerFn
+
+    print(f"case power rows={rows} l={lmax} m={mmax}", flush=True)
+    ld = int(lib.sfno_spectral_ld(rows))
+    g = torch.Generator().manual_seed(rows)
+    spec = torch.full((mmax, lmax, ld), float("nan"))
+    keep = torch.arange(mmax)[:, None] <= torch.arange(lmax)[None, :]
+    spec[..., :2 * rows] = torch.where(keep[..., None], torch.randn(mmax, lmax, 2 * rows, generator=g), torch.nan)
+    w = torch.where(torch.arange(mmax) == 0, 1.0, 2.0).double()
+    c = torch.where(keep[..., None], spec[..., :2 * rows], 0.0).double().reshape(mmax, lmax, rows, 2)
+    want = torch.einsum("m,mlrc->rl", w, c ** 2)
+    gp = torch.randn(rows, lmax, generator=g)
+    want_g = 2 * w[:, None, None, None] * gp.double().t()[None, :, :, None] * c
+    x = spec.cuda().requires_grad_()
+    power = _DegreePowerFn.apply(x, rows, lmax, mmax)
+    got_g = torch.autograd.grad(power, x, gp.cuda())[0].cpu()
+    assert (torch.linalg.norm(power.detach().cpu().double() - want) / torch.linalg.norm(want)) < 1e-6
+    inside = got_g[keep]
+    assert (inside[:, 2 * rows:] == 0).all()
+    assert (torch.linalg.norm(inside[:, :2 * rows].double() - want_g.reshape(mmax, lmax, -1)[keep]) / torch.linalg.norm(want_g)) < 1e-6
