@@ -5,16 +5,19 @@
 // (what autograd derives for nn.Conv2d(kernel_size=1), makani/models/common/layers.py:95-116,160-216).  Both operands are
 // pixel-contiguous and the sum runs over the pixels, so a row of g is an A operand and a row of x a B operand of
 // v_mfma_f32_32x32x16_bf16 as they lie in memory: 8 consecutive pixels per lane, no transposition.  The bias gradient
-// is one more column against a B operand of ones, in registers, of the wavefronts that hold the first columns: as column K of the
+// is summed from the A fragments by the wavefronts that hold the first columns: as column K of the
 // tiles it took a column of tiles to itself where K is a multiple of 256 (eight instead of six for 768 -> 384 channels with bias:
 // 1249 -> 997 us at 721 x 1440).
 //
-// A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile of dW and a contiguous share of the (sample, 32-pixel chunk)
-// sequence.  Per chunk 256 rows of g and 256 rows of x (64 bytes each) go straight from memory into a ring of four LDS
-// stages with global_load_lds_dwordx4, three chunks ahead of the matrix instructions (issued from inline assembly with a
+// A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile of dW and a contiguous share of the (sample, 64-pixel chunk)
+// sequence.  Per chunk 256 rows of g and 256 rows of x, a whole 128-byte line each (with 64-byte pieces of 32-pixel chunks the
+// same bytes were 1.4 times as long on their way, 989 against 704 us without the products for 384 -> 768 channels at 721 x 1440, and
+// the kernel took as long as its loads: 1029 -> 902 us in all, 768 -> 384 with bias 997 -> 858),
+// go straight from memory into LDS with global_load_lds_dwordx4 (issued from inline assembly with a
 // counted wait, as in the forward kernel); a lane fetches the 16-byte piece whose LDS slot it owns, and the pieces of a row
-// are permuted by (row >> 1) & 3 so that the 16-byte fragment reads of eight consecutive rows cover all banks.  Pieces
-// past the end of a sample come from a block of zeros.  Each wavefront multiplies
+// are permuted by (row >> 1) & 7 so that the 16-byte fragment reads of sixteen consecutive rows cover all banks.  A chunk is two
+// halves, its rows of g and its rows of x, and LDS a ring of five of them: three are on their way while two are read.
+// Pieces past the end of a sample come from a block of zeros.  Each wavefront multiplies
 // 64 x 128 (two A and four B fragments per 16 pixels for eight matrix instructions).  The shares' partial tiles go to a
 // workspace [share][O][K (+ 1 with bias)] and a second kernel adds them up in a fixed order: results do not depend on scheduling.
 // All tiles of one share run on one XCD (workgroups are dealt to the XCDs round robin by linear id), where they meet
@@ -30,17 +33,15 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 constexpr int WG_THREADS = 512;
 constexpr int WG_TO = 256;            // rows of dW (output channels) per workgroup
 constexpr int WG_TK = 256;            // columns of dW (input channels) per workgroup
-constexpr int WG_PX = 32;             // pixels per chunk: four 16-byte pieces per row
-constexpr int WG_ROWS = WG_TO + WG_TK;
-constexpr int WG_STAGE = WG_ROWS * 2 * WG_PX;                 // bytes per LDS stage
-constexpr int WG_STAGES = 4;
-constexpr int WG_PIECES = WG_ROWS * (WG_PX / 8) / WG_THREADS; // 16-byte pieces per thread and chunk
+constexpr int WG_PX = 64;             // pixels per chunk: eight 16-byte pieces per row
+constexpr int WG_HALF = WG_TO * 2 * WG_PX;                    // bytes of the rows of g, or of x, of a chunk
+constexpr int WG_HALVES = 5;                                  // ring of halves
+constexpr int WG_PIECES = WG_HALF / (16 * WG_THREADS);        // 16-byte pieces per thread and half
 constexpr int WG_RSTEP = WG_THREADS / (WG_PX / 8);            // rows between a thread's pieces
-static_assert(WG_PX == 32, "four pieces per row: the permutation and the slot arithmetic below");
-static_assert(WG_ROWS * (WG_PX / 8) % WG_THREADS == 0, "the chunk divides evenly among the threads");
-static_assert(WG_TO * (WG_PX / 8) % WG_THREADS == 0, "a thread's piece j is a row of g for all threads or a row of x for all threads");
-static_assert(WG_RSTEP % 8 == 0, "a thread's pieces share the permutation of their rows");
-static_assert(WG_STAGES * WG_STAGE <= 160 * 1024, "one workgroup per CU");
+static_assert(WG_PX == 64, "eight pieces per row: the permutation and the slot arithmetic below");
+static_assert(WG_TO == WG_TK, "halves of one size");
+static_assert(WG_RSTEP % 16 == 0, "a thread's pieces share the permutation of their rows");
+static_assert(WG_HALVES * WG_HALF <= 160 * 1024, "one workgroup per CU");
 
 // source of the pieces that are not read from the tensors
 __device__ __align__(16) const unsigned int wg_zero16[4] = {0u, 0u, 0u, 0u};
@@ -51,12 +52,28 @@ __device__ __forceinline__ void wg_dma16(const void* g, unsigned lds_byte_addr) 
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_byte_addr) : "memory");
 }
 
+// s_waitcnt immediate: at most n vector memory operations in flight, no LDS operation
+constexpr int wg_wait(int n) { return (n & 15) | ((n >> 4) << 14) | 0x70; }
+// workgroup barrier behind such a wait; no LDS access moves across it
+__device__ __forceinline__ void wg_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+}
+
+// the same with a wavefront-uniform base and a 32-bit offset per lane
+__device__ __forceinline__ void wg_dma16(const void* base, unsigned offset, unsigned lds_byte_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_byte_addr) : "memory");
+}
+
 struct WgradShape {
     int n_ot, n_kt, splits;
     int64_t cps, chunks;               // chunks per sample, chunks in all
 };
 
-// how the launcher and the workspace query divide the work: shares of at least eight chunks, one workgroup per CU (all
+// how the launcher and the workspace query divide the work: shares of at least four chunks, one workgroup per CU (all
 // workgroups resident at once, the tiles of a share side by side on one XCD)
 static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
     WgradShape s;
@@ -67,7 +84,7 @@ static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
     const int tiles = s.n_ot * s.n_kt;
     int64_t want = 256 / tiles / 8 * 8;
     if (want < 8) want = 8;
-    const int64_t most = (s.chunks + 7) / 8;       // at least eight chunks per share
+    const int64_t most = (s.chunks + 3) / 4;       // at least four chunks per share
     if (want > most) want = most;
     if (want < 1) want = 1;
     s.splits = (int)want;
@@ -86,7 +103,7 @@ struct WgradArgs {
 
 // grid = 8 * ceil(splits / 8) * n_ot * n_kt workgroups of 512 threads
 __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
-    __shared__ __align__(16) unsigned char lds[WG_STAGES * WG_STAGE];
+    __shared__ __align__(16) unsigned char lds[WG_HALVES * WG_HALF];
     const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
     const int tiles = a.n_ot * a.n_kt;
     const int split = (q / tiles) * 8 + xcd, tile = q % tiles;
@@ -100,55 +117,55 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     const int wo = wave & 3, wk = wave >> 2;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)lds);
 
-    // ---- loads: LDS slot s = 512 j + tid of a stage (16 bytes) holds row s >> 2, piece (s & 3) ^ ((row >> 1) & 3); rows below
-    // WG_TO are rows of g, the others rows of x.  A thread's four slots lie 128 rows apart: same piece, same permutation.
-    constexpr int JG = WG_TO * (WG_PX / 8) / WG_THREADS;
-    const int part = (tid & 3) ^ ((tid >> 3) & 3);
-    const unsigned short* rowp[WG_PIECES];     // first pixel of the row in sample 0 (rows past the matrix: its last row, whose products are never stored)
-#pragma unroll
-    for (int j = 0; j < WG_PIECES; ++j) {
-        const int row = (tid >> 2) + WG_RSTEP * j;
-        rowp[j] = j < JG ? a.G + (int64_t)min(o0 + row, a.O - 1) * a.P : a.X + (int64_t)min(k0 + row - WG_TO, a.K - 1) * a.P;
-    }
+    // ---- loads: LDS slot s = 512 j + tid of a half (16 bytes) holds row s >> 3, piece (s & 7) ^ ((row >> 1) & 7).  A thread's four
+    // slots lie 64 rows apart: same piece, same permutation.  Rows past the matrix are its last row, whose products are never stored.
+    const int part = (tid & 7) ^ ((tid >> 4) & 7), row0 = tid >> 3;
     const unsigned short* zero16 = reinterpret_cast<const unsigned short*>(wg_zero16);
-    // next chunk to ask for: sample ib, chunk ic of the sample, and where its pieces lie (counted along: a chunk inside a
-    // sample costs one addition per piece; the addresses are worked out afresh once per sample)
-    int64_t ib = c_begin / a.cps;
-    int64_t ic = c_begin - ib * a.cps;
-    const unsigned short* cur[WG_PIECES];
-    auto locate = [&]() {
-        const int64_t p = ic * WG_PX + 8 * part;
-        const int64_t og = ib * a.O * a.P + p, ox = ib * a.K * a.P + p;
-#pragma unroll
-        for (int j = 0; j < WG_PIECES; ++j) cur[j] = rowp[j] + (j < JG ? og : ox);
+    // One stream per operand: the next chunk to ask for lies in sample ib at chunk ic of the sample.  Inside a sample the addresses are
+    // a scalar base and the lane's 32-bit offsets from the tile's first row; they are worked out in 64 bits for the last chunk of a
+    // sample, whose pieces may lie outside, and where the rows of a tile lie further apart than 32 bits reach.
+    struct Stream {
+        const unsigned short* base;
+        int r0, last;                  // first row of the tile, last row of the tensor
+        int64_t ib, ic;
+        unsigned off[WG_PIECES];
     };
-    locate();
-    auto issue = [&](int stage) {
-        const unsigned dst = lds0 + stage * WG_STAGE + wave * 1024;
-        if ((ic + 1) * WG_PX <= a.P) {         // (uniform) every piece of the chunk lies inside the sample
+    const unsigned row_bytes = (unsigned)(2 * a.P);
+    const bool near = a.P < (1 << 23);
+    auto stream = [&](const unsigned short* base, int r0, int rows) {
+        Stream t{base, r0, rows - 1, c_begin / a.cps, 0, {}};
+        t.ic = c_begin - t.ib * a.cps;
 #pragma unroll
-            for (int j = 0; j < WG_PIECES; ++j) wg_dma16(cur[j], dst + j * (WG_THREADS * 16));
+        for (int j = 0; j < WG_PIECES; ++j) t.off[j] = (unsigned)min(row0 + WG_RSTEP * j, t.last - r0) * row_bytes + 16 * part;
+        return t;
+    };
+    Stream sg = stream(a.G, o0, a.O), sx = stream(a.X, k0, a.K);
+    auto issue = [&](Stream& t, int slot) {
+        const unsigned dst = lds0 + slot * WG_HALF + wave * 1024;
+        const unsigned short* base = t.base + ((t.ib * (t.last + 1) + t.r0) * a.P + t.ic * WG_PX);
+        if (near && (t.ic + 1) * WG_PX <= a.P) {
+            // (uniform, but the division by the chunks per sample left it in vector registers)
+            const uint64_t bits = reinterpret_cast<uint64_t>(base);
+            const void* ubase = reinterpret_cast<const void*>((uint64_t)__builtin_amdgcn_readfirstlane((int)(bits >> 32)) << 32 |
+                                                              (unsigned)__builtin_amdgcn_readfirstlane((int)bits));
+#pragma unroll
+            for (int j = 0; j < WG_PIECES; ++j) wg_dma16(ubase, t.off[j], dst + j * (WG_THREADS * 16));
         } else {
-            // the last chunk of a sample: P is a multiple of 8, so a piece lies inside the row or outside
-            const bool in = ic * WG_PX + 8 * part < a.P;
+            const bool in = t.ic * WG_PX + 8 * part < a.P;         // P is a multiple of 8: a piece lies inside the row or outside
 #pragma unroll
-            for (int j = 0; j < WG_PIECES; ++j) wg_dma16(in ? cur[j] : zero16, dst + j * (WG_THREADS * 16));
+            for (int j = 0; j < WG_PIECES; ++j) {
+                const unsigned short* p = base + (int64_t)min(row0 + WG_RSTEP * j, t.last - t.r0) * a.P + 8 * part;
+                wg_dma16(in ? p : zero16, dst + j * (WG_THREADS * 16));
+            }
         }
-        if (++ic == a.cps) {
-            ic = 0;
-            ++ib;
-            locate();
-        } else {
-#pragma unroll
-            for (int j = 0; j < WG_PIECES; ++j) cur[j] += WG_PX;
+        if (++t.ic == a.cps) {
+            t.ic = 0;
+            ++t.ib;
         }
     };
 
-    f32x16 acc[2][4], accb[2];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) accb[mt][v] = 0.f;
+    f32x16 acc[2][4];
+    float accb[2] = {0.f, 0.f}, chunkb[2] = {0.f, 0.f};       // sums of the lane's pixels of its two rows: all chunks, this chunk
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
@@ -156,54 +173,93 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.f;
 
-    // fragments of this lane: row (lane & 31) of a 32-row block, pieces (lane >> 5) and 2 + (lane >> 5) of the row (pixels
-    // 8 (lane >> 5) .. + 7 of the first and of the second 16-pixel step), at their permuted places
-    const int sw = (lane >> 1) & 3, kg = lane >> 5;
-    const unsigned fa = (wo * 64 + (lane & 31)) * 64, fb = (WG_TO + wk * 128 + (lane & 31)) * 64;
-    const unsigned pk[2] = {(unsigned)((kg ^ sw) * 16), (unsigned)(((2 + kg) ^ sw) * 16)};
+    // fragments of this lane: row (lane & 31) of a 32-row block, pieces 2 ks + (lane >> 5) of the row (pixels 8 (lane >> 5) .. + 7 of
+    // the 16-pixel step ks), at their permuted places
+    const int sw = (lane >> 1) & 7, kg = lane >> 5;
+    const unsigned fa = (wo * 64 + (lane & 31)) * 128, fb = (wk * 128 + (lane & 31)) * 128;
 
     const bool live = o0 + wo * 64 < a.O && k0 + wk * 128 < a.K;
     const bool bias = a.Kext > a.K && k0 + wk * 128 == 0;
-    const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
-    // Ring of four stages: chunk i is multiplied while chunks i + 1 .. i + 3 are on their way.  The only vector memory
-    // operations of the loop are the four loads per wavefront and chunk, so "at most eight outstanding" means chunk i has
-    // landed while two later ones may still be under way.
-    static_assert(WG_STAGES == 4 && WG_PIECES == 4, "the wait counts below");
-    for (int i = 0; i < WG_STAGES - 1; ++i)
-        if (i < nch) issue(i);
-    int stage = 0;
-    for (int i = 0; i < nch; ++i) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (i + 2 < nch)
-            asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-        else if (i + 1 < nch)
-            asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        // (every wavefront has read chunk i - 1: its stage takes chunk i + 3)
-        if (i + 3 < nch) issue(stage == 0 ? WG_STAGES - 1 : stage - 1);
-        const unsigned char* sb = lds + stage * WG_STAGE;
-        // (a wavefront whose 64 x 128 part of the tile lies outside the matrix only moves data)
-        if (live)
+    // Half h (chunk h / 2; g, then x) lives in slot h % 5.  Fragments are read one 16-pixel step ahead of the matrix instructions, those of
+    // a chunk's first step under the products of the last step of the chunk before.  In front of that, once a wavefront holds all it
+    // needs of chunk i, it waits for its pieces of chunk i + 1 and meets the others: chunk i's slots take halves 2 i + 5 (x of chunk
+    // i + 2) and 2 i + 6 (g of chunk i + 3), chunk i + 1 may be read.  The only vector memory operations of the loop are the four loads per
+    // wavefront and half, so "at most four outstanding" leaves half 2 i + 4 under way.
+    static_assert(WG_HALVES == 5 && WG_PIECES == 4, "the wait counts below");
+    bf16x8 af[2][2], bf[2][4];                // [step & 1][32-row block]
+    auto fragments = [&](int slot_g, int slot_x, int ks) {
+        const unsigned pk = (unsigned)(((2 * ks + kg) ^ sw) * 16);
+        const unsigned char *pa = lds + slot_g * WG_HALF + fa + pk, *pb = lds + slot_x * WG_HALF + fb + pk;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            bf16x8 af[2], bf[4];
+        for (int mt = 0; mt < 2; ++mt) af[ks & 1][mt] = *reinterpret_cast<const bf16x8*>(pa + mt * 32 * 128);
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt) af[mt] = *reinterpret_cast<const bf16x8*>(sb + fa + mt * 32 * 64 + pk[ks]);
+        for (int nt = 0; nt < 4; ++nt) bf[ks & 1][nt] = *reinterpret_cast<const bf16x8*>(pb + nt * 32 * 128);
+    };
+    auto products = [&](int ks) {
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) bf[nt] = *reinterpret_cast<const bf16x8*>(sb + fb + nt * 32 * 64 + pk[ks]);
+        for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt)
+            for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][mt], bf[ks & 1][nt], acc[mt][nt], 0, 0, 0);
+        if (bias) {
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mt], bf[nt], acc[mt][nt], 0, 0, 0);
-            if (bias) {
+            for (int mt = 0; mt < 2; ++mt) {
+                const u32x4 p = __builtin_bit_cast(u32x4, af[ks & 1][mt]);
+                float lo = 0.f, hi = 0.f;
 #pragma unroll
-                for (int mt = 0; mt < 2; ++mt) accb[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mt], ones, accb[mt], 0, 0, 0);
+                for (int i = 0; i < 4; ++i) {
+                    lo += __uint_as_float(p[i] << 16);
+                    hi += __uint_as_float(p[i] & 0xffff0000u);
+                }
+                chunkb[mt] += lo + hi;
+                if (ks == 3) {
+                    accb[mt] += chunkb[mt];
+                    chunkb[mt] = 0.f;
+                }
             }
         }
-        stage = stage == WG_STAGES - 1 ? 0 : stage + 1;
+    };
+    issue(sg, 0);
+    issue(sx, 1);
+    if (nch > 1) {
+        issue(sg, 2);
+        issue(sx, 3);
+    }
+    if (nch > 2) issue(sg, 4);
+    __builtin_amdgcn_sched_barrier(0);
+    if (nch > 2)
+        __builtin_amdgcn_s_waitcnt(wg_wait(12));
+    else
+        __builtin_amdgcn_s_waitcnt(wg_wait(0));
+    wg_barrier();
+    int cg = 0, cx = 1;                       // slots of chunk i
+    // (a wavefront whose 64 x 128 part of the tile lies outside the matrix only moves data)
+    if (live) fragments(cg, cx, 0);
+    for (int i = 0; i < nch; ++i) {
+        if (live) {
+#pragma unroll
+            for (int ks = 0; ks < 3; ++ks) {
+                fragments(cg, cx, ks + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                products(ks);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // (the builtin and not inline assembly: the compiler then knows that the fragments have arrived)
+        if (i + 3 <= nch)
+            __builtin_amdgcn_s_waitcnt(wg_wait(4));
+        else
+            __builtin_amdgcn_s_waitcnt(wg_wait(0));
+        wg_barrier();
+        if (i + 2 < nch) issue(sx, cg);
+        if (i + 3 < nch) issue(sg, cx);
+        cg = cg >= 3 ? cg - 3 : cg + 2;
+        cx = cx >= 3 ? cx - 3 : cx + 2;
+        if (live) {
+            fragments(cg, cx, 0);             // (past the last chunk: whatever those slots hold, and not used)
+            __builtin_amdgcn_sched_barrier(0);
+            products(3);
+        }
     }
 
     // D layout of the 32x32 MFMA: register v of lane j holds D[8 (v / 4) + 4 (j / 32) + v % 4][j % 32]
@@ -219,14 +275,13 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
                 if (o < a.O && kk < a.K) out[(int64_t)o * a.Kext + kk] = acc[mt][nt][v];
             }
         }
-    if (bias && (lane & 31) == 0) {           // all columns of accb are the same
+    if (bias) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int o = o0 + wo * 64 + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (o < a.O) out[(int64_t)o * a.Kext + a.K] = accb[mt][v];
-            }
+        for (int mt = 0; mt < 2; ++mt) {
+            const int o = o0 + wo * 64 + mt * 32 + (lane & 31);
+            const float b = accb[mt] + __shfl_xor(accb[mt], 32, 64);
+            if (lane < 32 && o < a.O) out[(int64_t)o * a.Kext + a.K] = b;
+        }
     }
 }
 
