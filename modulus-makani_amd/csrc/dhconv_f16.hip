@@ -276,7 +276,7 @@ __global__ __launch_bounds__(256, 2) void dhconv_f16_kernel(DhconvArgs a) {
     }
 }
 
-// cmax[l][o] = largest |Re|, |Im| of w[.][o][l] over the input channels (adjoint: of w[o][.][l], w being [O][I][L]).  A thread
+// cmax[o][l] = largest |Re|, |Im| of w[.][o][l] over the input channels (adjoint: of w[o][.][l], w being [O][I][L]).  A thread
 // takes DHF_CMAX_I input channels of one (o, l) and joins the others with an integer atomic maximum on the bit pattern (the
 // values are magnitudes: their order as unsigned integers is their order as floats, a NaN ranks above all and stays); cmax is
 // cleared by the kernel in front.  grid (ceil(O L / 256), ceil(I / DHF_CMAX_I))
@@ -291,31 +291,33 @@ __global__ __launch_bounds__(256) void dhconv_colmax_kernel(const float2* __rest
     const int o = (int)(idx / L), l = (int)(idx - (int64_t)o * L);
     const int i0 = blockIdx.y * DHF_CMAX_I, i1 = min(i0 + DHF_CMAX_I, I);
     float mx = 0.f;
-#pragma unroll 4
+#pragma unroll 8
     for (int i = i0; i < i1; ++i) {
         const float2 z = adjoint ? w[((int64_t)o * I + i) * L + l] : w[((int64_t)i * O + o) * L + l];
         mx = fmaxf(mx, fmaxf(fabsf(z.x), fabsf(z.y)));
     }
-    atomicMax(reinterpret_cast<unsigned int*>(cmax) + ((int64_t)l * O + o), __float_as_uint(mx));
+    atomicMax(reinterpret_cast<unsigned int*>(cmax) + idx, __float_as_uint(mx));
 }
 
 // Writes the stage images.  packed[l][ob][c] = [part (Re, Im)][plane][o (CO)][two 16-byte halves, see dhf_piece]: the half kg
 // of channel o holds plane `plane` of part `part` of w[16c + 8kg + e][CO ob + o][l] * 2^s[l][o], e = 0..7, as fp16; plane 0 is
 // the value rounded to fp16, plane 1 the rounded remainder; zero outside the weight (adjoint: the weight is conj(w[o][i][l]),
 // w being [O][I][L]).  cinv[l][CO ob + o] = 2^-s.  The parameter has l fastest, the stream has it slowest: a workgroup moves
-// the 16 x 32 channel pairs of one (c, ob, quarter of the channel block) for 8 degrees through LDS, reading 64 contiguous
-// bytes per pair.  grid (nc * nob * (CO / 32), ceil(L / 8)), block 256
+// the 16 x 32 channel pairs of one (c, ob, quarter of the channel block) for 16 degrees through LDS, reading 128 contiguous
+// bytes per pair, whole lines where L is a multiple of 16 (8 degrees and half lines: column
+// maxima and packing of 384 x 384 x 240 264 us, now 236; 128 x 128 x 90 21.6 -> 16.0).  grid (nc * nob * (CO / 32), ceil(L / 16)), block 512
+constexpr int DHF_PL = 16;
 template <int NTC>
-__global__ __launch_bounds__(256) void dhconv_pack_f16_kernel(const float2* __restrict__ w, const float* __restrict__ cmax, unsigned char* __restrict__ packed,
+__global__ __launch_bounds__(512) void dhconv_pack_f16_kernel(const float2* __restrict__ w, const float* __restrict__ cmax, unsigned char* __restrict__ packed,
                                                               float* __restrict__ cinv, int I, int O, int L, int nob, int nc, int adjoint) {
     constexpr int CO = 32 * NTC, STAGE = 4 * CO * 32;
-    __shared__ float2 tile[512][9];                  // [pair = ii * 32 + o][degree], padded
+    __shared__ float2 tile[512][DHF_PL + 1];         // [pair = ii * 32 + o][degree], padded
     const int q = blockIdx.x % NTC, c = (blockIdx.x / NTC) % nc, ob = blockIdx.x / (NTC * nc);
-    const int l0 = blockIdx.y * 8;
-    const int tid = threadIdx.x, dl = tid & 7;
-#pragma unroll 4
-    for (int pass = 0; pass < 16; ++pass) {
-        const int pr = pass * 32 + (tid >> 3);       // eight lanes per pair: one 64-byte segment
+    const int l0 = blockIdx.y * DHF_PL;
+    const int tid = threadIdx.x, dl = tid & (DHF_PL - 1);
+#pragma unroll
+    for (int pass = 0; pass < DHF_PL; ++pass) {
+        const int pr = pass * (512 / DHF_PL) + tid / DHF_PL;     // sixteen lanes per pair: one 128-byte segment
         const int ii = pr >> 5, o = pr & 31;
         const int i = DHF_KC * c + ii, oo = CO * ob + 32 * q + o, l = l0 + dl;
         float2 z = make_float2(0.f, 0.f);
@@ -330,19 +332,19 @@ __global__ __launch_bounds__(256) void dhconv_pack_f16_kernel(const float2* __re
         tile[pr][dl] = z;
     }
     __syncthreads();
-    // thread -> one 16-byte piece per degree: (part, plane, half kg, channel o)
-    const int o = tid & 31, kg = (tid >> 5) & 1, plane = (tid >> 6) & 1, part = tid >> 7;
+    // thread -> one 16-byte piece per two degrees: (degree parity, part, plane, half kg, channel o)
+    const int o = tid & 31, kg = (tid >> 5) & 1, plane = (tid >> 6) & 1, part = (tid >> 7) & 1;
     const int oo = CO * ob + 32 * q + o;
-    for (int d = 0; d < 8; ++d) {
+    for (int d = tid >> 8; d < DHF_PL; d += 2) {
         const int l = l0 + d;
         if (l >= L) break;
         // scale: the column's largest magnitude lands in [2^TOP, 2^(TOP+1))
         int sh = 0;
         if (oo < O) {
-            const unsigned int mb = __builtin_bit_cast(unsigned int, cmax[(int64_t)l * O + oo]);
+            const unsigned int mb = __builtin_bit_cast(unsigned int, cmax[(int64_t)oo * L + l]);
             if (mb != 0) sh = DHF_SH - (int)(mb >> 23);
         }
-        if (c == 0 && tid < 32) cinv[(int64_t)l * (nob * CO) + CO * ob + 32 * q + o] = __builtin_ldexpf(1.0f, -sh);
+        if (c == 0 && (tid & 255) < 32) cinv[(int64_t)l * (nob * CO) + CO * ob + 32 * q + o] = __builtin_ldexpf(1.0f, -sh);
         u4 piece;
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2) {
@@ -367,18 +369,18 @@ int dhconv_f16_ntc(int O) { return O > 64 ? 4 : 2; }
 int dhconv_pack_f16_launch(const float2* w, void* packed, float* cinv, float* cmax, int I, int O, int L, int adjoint, hipStream_t s) {
     const int ntc = dhconv_f16_ntc(O);
     const int nob = (O + 32 * ntc - 1) / (32 * ntc), nc = (I + DHF_KC - 1) / DHF_KC;
-    if ((int64_t)nob * nc * ntc > 0x7fffffffLL || (L + 7) / 8 > 65535) return SFNO_EUNSUPPORTED;
+    if ((int64_t)nob * nc * ntc > 0x7fffffffLL || (L + DHF_PL - 1) / DHF_PL > 65535) return SFNO_EUNSUPPORTED;
     const int64_t cols = (int64_t)O * L;
     if ((cols + 255) / 256 > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
     if ((I + DHF_CMAX_I - 1) / DHF_CMAX_I > 65535) return SFNO_EUNSUPPORTED;
     hipLaunchKernelGGL(dhconv_colmax_clear_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, cmax, cols);
     hipLaunchKernelGGL(dhconv_colmax_kernel, dim3((unsigned)((cols + 255) / 256), (unsigned)((I + DHF_CMAX_I - 1) / DHF_CMAX_I)), dim3(256), 0, s, w, cmax, I,
                        O, L, adjoint);
-    const dim3 grid((unsigned)(nob * nc * ntc), (unsigned)((L + 7) / 8));
+    const dim3 grid((unsigned)(nob * nc * ntc), (unsigned)((L + DHF_PL - 1) / DHF_PL));
     if (ntc == 4)
-        hipLaunchKernelGGL((dhconv_pack_f16_kernel<4>), grid, dim3(256), 0, s, w, cmax, reinterpret_cast<unsigned char*>(packed), cinv, I, O, L, nob, nc, adjoint);
+        hipLaunchKernelGGL((dhconv_pack_f16_kernel<4>), grid, dim3(512), 0, s, w, cmax, reinterpret_cast<unsigned char*>(packed), cinv, I, O, L, nob, nc, adjoint);
     else
-        hipLaunchKernelGGL((dhconv_pack_f16_kernel<2>), grid, dim3(256), 0, s, w, cmax, reinterpret_cast<unsigned char*>(packed), cinv, I, O, L, nob, nc, adjoint);
+        hipLaunchKernelGGL((dhconv_pack_f16_kernel<2>), grid, dim3(512), 0, s, w, cmax, reinterpret_cast<unsigned char*>(packed), cinv, I, O, L, nob, nc, adjoint);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

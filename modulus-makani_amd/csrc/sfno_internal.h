@@ -68,7 +68,7 @@ int dhconv_split_launch(const DhconvArgs& a, hipStream_t s);
 int dhconv_pack_split_launch(const float2* w, void* packed, int I, int O, int L, int adjoint, hipStream_t s);
 // fp32 operands on the fp16 matrix pipe (two fp16 planes per operand, power-of-two scales per weight column and per activation
 // row): 32 dhconv_f16_ntc(O) output channels per workgroup (a.nob blocks of them), a.nc chunks of 16 input channels; cinv
-// receives [L][nob * 32 ntc] inverse column scales, cmax is [L][O] scratch
+// receives [L][nob * 32 ntc] inverse column scales, cmax is [O][L] scratch
 int dhconv_f16_ntc(int O);
 int dhconv_f16_launch(const DhconvArgs& a, hipStream_t s);
 int dhconv_pack_f16_launch(const float2* w, void* packed, float* cinv, float* cmax, int I, int O, int L, int adjoint, hipStream_t s);
@@ -245,5 +245,5 @@ struct sfno_dhconv_weights {
     int nob, nc;                   // column blocks (over 2*O) and K chunks (over 2*I) per degree
     float* d_W = nullptr;          // packed complex weights
     float* d_cinv = nullptr;       // f16: [L][nob * channels per block] inverse column scales
-    float* d_cmax = nullptr;       // f16: [L][O] scratch of the pack kernels
+    float* d_cmax = nullptr;       // f16: [O][L] scratch of the pack kernels
 };
