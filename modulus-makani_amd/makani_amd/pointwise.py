@@ -222,6 +222,8 @@ class _ConvGeluConv(torch.autograd.Function):
         xb = x.detach().to(torch.bfloat16).contiguous()
         B, K, H, W = xb.shape
         O = w1.shape[0]
+        if w1.shape[1] != K or w2.shape[1] != O:
+            raise RuntimeError(f"conv1x1: input has {K} channels, weights expect {w1.shape[1]} and {w2.shape[1]} (of {O})")
         z = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
         a = torch.empty_like(z)
         bias = b1.detach().float().contiguous() if b1 is not None else None

@@ -181,3 +181,16 @@ def test_conv_gelu_conv(lib_built, cin, hid, cout, H, W):
     ref = passes(enc, x, gy, False)
     for n, r in ref.items():
         assert rel(got[n], r) < 1e-2, n
+
+
+def test_conv_gelu_conv_refuses_other_channel_counts(lib_built):
+    """The packed weights are addressed by the input's channel count: a wrong one is an error of the host, not a read past them."""
+    from makani_amd.sfnonet import EncoderDecoder
+
+    enc = EncoderDecoder(1, 6, 5, 8, nn.GELU).cuda()
+    for channels in (5, 7):
+        with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
+            enc(torch.randn(1, channels, 8, 16, device="cuda"))
+    enc.fwd[2] = nn.Conv2d(9, 5, 1).cuda()
+    with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
+        enc(torch.randn(1, 6, 8, 16, device="cuda"))
