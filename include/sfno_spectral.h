@@ -355,7 +355,8 @@ int sfno_scale_shift_act(const void* x, const float* scale, const float* shift, 
  *   (x', r) = filter(x),   h0 = gelu(norm0(x')),   y2 = W2 gelu(W1 h0 + b1) + b2,   out = norm1(y2) + Wskip r
  * where r is x, or x taken through the transforms where the grids of the two plans differ.  Every longitude length of the
  * plans has to have bf16 input and output (sfno_sht_io_dtype_supported), H*W of the output grid is a multiple of 8.
- * All pointers of the structure stay the caller's; the calls enqueue kernels only. */
+ * All pointers of the structure stay the caller's; tensors and buffers are 16-byte aligned (SFNO_EINVAL otherwise); the calls
+ * enqueue kernels only. */
 typedef struct {
     const sfno_sht_plan *fwd, *inv;                 /* filter transforms (equal lmax, mmax) */
     const sfno_sht_plan *fwd_adj, *inv_adj;         /* plans with their adjoint directions (backward only) */

@@ -2,6 +2,7 @@
 // makani/models/networks/sfnonet.py:239-267 applies them, enqueued from native code -- a dozen launches per direction without
 // an interpreter between them -- and their backward.
 #include <algorithm>
+#include <cstdint>
 #include <cstring>
 
 #include "sfno_internal.h"
@@ -136,6 +137,12 @@ int mix(const sfno_dhconv_weights* w, const float* in, float* out, const Dims& d
     return sfno_dhconv_spectral(w, in, out, d.B, d.mmax, d.tri, s);
 }
 
+// the kernels load and store 16 bytes at a time
+template <class... T>
+bool aligned(const T*... p) {
+    return ((reinterpret_cast<uintptr_t>(p) | ...) & 15) == 0;
+}
+
 bool bf16_io(const sfno_sht_plan* p) { return sfno_sht_io_dtype_supported(p, SFNO_DTYPE_BF16) && sfno_sht_lat_stats_supported(p); }
 
 }  // namespace
@@ -160,7 +167,7 @@ extern "C" size_t sfno_block_workspace_bytes(const sfno_block* b, int backward) 
 extern "C" int sfno_block_forward(const sfno_block* b, int training, const void* x, void* out, void* kept, size_t kept_bytes, void* workspace,
                                   size_t workspace_bytes, void* stream) {
     const Dims d(b);
-    if (!d.valid || !x || !kept || !workspace) return SFNO_EINVAL;
+    if (!d.valid || !x || !kept || !workspace || !aligned(x, out, kept, workspace)) return SFNO_EINVAL;
     if (!(b->fwd->directions & SFNO_DIR_FORWARD) || !(b->inv->directions & SFNO_DIR_INVERSE)) return SFNO_EINVAL;
     if (!bf16_io(b->fwd) || !bf16_io(b->inv)) return SFNO_EUNSUPPORTED;
     int64_t off[SFNO_BLOCK_TENSORS];
@@ -199,7 +206,7 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
 extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const void* x, const void* kept, const sfno_block_grads* grads, void* workspace,
                                    size_t workspace_bytes, void* stream) {
     const Dims d(b);
-    if (!d.valid || !gv || !x || !kept || !grads || !workspace) return SFNO_EINVAL;
+    if (!d.valid || !gv || !x || !kept || !grads || !workspace || !aligned(gv, x, kept, grads->gx, workspace)) return SFNO_EINVAL;
     if (!b->fwd_adj || !b->inv_adj) return SFNO_EINVAL;
     int64_t off[SFNO_BLOCK_TENSORS];
     (void)layout(d, true, off);

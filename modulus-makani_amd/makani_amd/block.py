@@ -40,8 +40,17 @@ def mlp_convs(blk):
     return (m[0], m[2]) if ok else None
 
 
-def supported(blk, x):
-    """Whether the native block serves this block (whose fusable() the caller has checked) and input."""
+def shapes_fit(params, c_in, embed, lmax):
+    """Whether the parameters (in the order of block_params) belong to one block: the native calls address all of them by c_in, embed,
+    hidden and lmax, so anything else is left to the modules, which raise their own errors."""
+    hidden = params[2].shape[0]
+    want = [(c_in, embed, lmax), (embed, c_in, 1, 1), (hidden, embed, 1, 1), (hidden,), (embed, hidden, 1, 1)] + 5 * [(embed,)]
+    return all(p is None or tuple(p.shape) == w for p, w in zip(params, want))
+
+
+def supported(blk, x, filter_weight=None, skip_weight=None):
+    """Whether the native block serves this block (whose fusable() the caller has checked) and input; filter_weight, skip_weight: as of
+    forward()."""
     conv, fwd, inv = blk.filter.filter, blk.filter.filter.forward_transform, blk.filter.filter.inverse_transform
     if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or mlp_convs(blk) is None:
         return False
@@ -53,7 +62,12 @@ def supported(blk, x):
         return False
     if not lib.sfno_sht_io_dtype_supported(fwd.plan(x.device).handle, _lib.DTYPE_BF16) or not lib.sfno_sht_io_dtype_supported(inv.plan(x.device).handle, _lib.DTYPE_BF16):
         return False
-    wf, *params = [p for p in block_params(blk) if p is not None]
+    if x.is_contiguous() and x.data_ptr() % 16 != 0:      # a view into the middle of a buffer: the kernels load 16 bytes at a time
+        return False
+    params = _with(block_params(blk), filter_weight, skip_weight)
+    if not shapes_fit(params, x.shape[1], conv.out_channels, inv.lmax):
+        return False
+    wf, *params = [p for p in params if p is not None]
     return wf.dtype == torch.complex64 and wf.is_cuda and all(p.dtype == torch.float32 and p.is_cuda for p in params) and _no_hooks(
         blk.filter, conv, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.mlp.fwd, *blk.mlp.fwd, blk.outer_skip)
 
@@ -63,6 +77,11 @@ def block_params(blk):
     fc1, fc2 = mlp_convs(blk)
     n0, n1 = blk.norm0, blk.norm1
     return [blk.filter.filter.weight, blk.outer_skip.weight, fc1.weight, fc1.bias, fc2.weight, fc2.bias, n0.weight, n0.bias, n1.weight, n1.bias]
+
+
+def _with(params, filter_weight, skip_weight):
+    """params with other filter and skip weights in place of the block's own, where there are any."""
+    return [params[0] if filter_weight is None else filter_weight, params[1] if skip_weight is None else skip_weight, *params[2:]]
 
 
 class _Call:
@@ -107,12 +126,7 @@ def forward(blk, x, filter_weight=None, skip_weight=None, defer_skip=False):
     """The block without autograd.  filter_weight, skip_weight: in place of the block's own.  defer_skip: returns (y2, residual, scale,
     shift) of the last sum scale * y2 + shift + skip(residual) instead of running it."""
     x = x.contiguous()
-    params = block_params(blk)
-    if filter_weight is not None:
-        params[0] = filter_weight
-    if skip_weight is not None:
-        params[1] = skip_weight
-    c = _Call(blk, x, params)
+    c = _Call(blk, x, _with(block_params(blk), filter_weight, skip_weight))
     B, E = x.shape[0], c.b.embed
     if not defer_skip:
         out = torch.empty((B, E, *c.P), dtype=torch.bfloat16, device=x.device)
@@ -147,6 +161,8 @@ class _BlockFn(torch.autograd.Function):
     def backward(ctx, g):
         x, kept, *params = ctx.saved_tensors
         g = g.to(torch.bfloat16).contiguous()
+        if g.data_ptr() % 16 != 0:
+            g = g.clone()
         blk, need = ctx.blk, ctx.needs_input_grad
         c = _Call(blk, x, params, backward=True)
         want = [p is not None and n for p, n in zip(params, need[2:])]

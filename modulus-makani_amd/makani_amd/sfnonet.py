@@ -427,7 +427,7 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         blk = self.blocks[0]
         conv = blk.filter.filter
         B = h.shape[0]
-        if native_block.supported(blk, h):
+        if native_block.supported(blk, h, wf, wsk):
             return native_block.forward(blk, h, wf, wsk)
         spec = conv.forward_transform.analysis(h)
         residual = conv.inverse_transform.synthesis(spec, (B, h.shape[1]), dtype=torch.bfloat16)

@@ -194,3 +194,29 @@ def test_conv_gelu_conv_refuses_other_channel_counts(lib_built):
     enc.fwd[2] = nn.Conv2d(9, 5, 1).cuda()
     with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
         enc(torch.randn(1, 6, 8, 16, device="cuda"))
+
+
+def test_offset_tensors_and_foreign_shapes(lib_built):
+    """Views that start between 16-byte boundaries give the results of their copies; inputs and parameters of another size raise."""
+    import makani_amd as ma
+
+    torch.manual_seed(8)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x, gy = (torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16) for _ in range(2))
+
+    def offset(t):
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+
+    want = passes(blk, x, gy, True)
+    got = passes(blk, x, offset(gy), True)
+    for n, w in want.items():
+        assert torch.equal(got[n], w), n
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert rel(blk.eval()(offset(x)), want["y"].float()) < 1.5e-2
+    for mode in (torch.enable_grad, torch.no_grad):
+        with mode(), torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
+            blk(x[:, :15].contiguous())
+    blk.mlp.fwd[0] = nn.Conv2d(15, 32, 1).cuda()
+    with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
+        blk.train()(x)
