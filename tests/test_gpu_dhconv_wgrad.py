@@ -51,3 +51,24 @@ def test_weight_grad_edges(lib_built, B, I, O, L, M, triangular):
     err = (got - ref).norm(dim=0) / ref.norm(dim=0).clamp_min(1e-300)      # per output channel and degree: each has its own scale
     assert torch.isfinite(torch.view_as_real(got)).all()
     assert float(err.max()) < 1.5e-6
+
+
+@pytest.mark.parametrize("I,O,L", [(256, 200, 333), (600, 610, 49)])
+def test_weights_packed_in_slabs_of_degrees(lib_built, I, O, L):
+    """Weights above 96 MB are packed a slab of degrees at a time (here two slabs, the last one shorter and no multiple of 16): output and
+    input gradient of two rows per degree against complex128, with the bound above (K <= 610)."""
+    from makani_amd.contractions import _contract_dhconv
+
+    print(f"case slabs {I} {O} {L}", flush=True)
+    gen = torch.Generator().manual_seed(3)
+    w = torch.randn(I, O, L, dtype=torch.complex64, generator=gen) * torch.logspace(-3, 3, L)
+    x = torch.randn(1, I, L, 2, dtype=torch.complex64, generator=gen)
+    g = torch.randn(1, O, L, 2, dtype=torch.complex64, generator=gen)
+    xd = x.cuda().requires_grad_()
+    y = _contract_dhconv(xd, w.cuda())
+    y.backward(g.cuda())
+    # per degree, so that every slab counts alike
+    wl, xl, gl = (t.to(torch.complex128) for t in (w.permute(2, 0, 1), x[0].permute(1, 2, 0), g[0].permute(1, 2, 0)))
+    for got, ref in ((y.detach(), torch.matmul(xl, wl)), (xd.grad, torch.matmul(gl, wl.conj().transpose(1, 2)))):
+        d = got[0].cpu().permute(1, 2, 0).to(torch.complex128) - ref
+        assert float((d.abs().square().sum((1, 2)) / ref.abs().square().sum((1, 2))).max()) ** 0.5 < 1.5e-6
