@@ -3,25 +3,27 @@
 // (the backward of einsum("bixy,iox->boxy") at makani/models/common/contractions.py:130-136 with
 // respect to `bc`).  Per degree l this is four real GEMMs whose K dimension is the rows of the spectral layout,
 //     Re gw = Xr^T Gr + Xi^T Gi,      Im gw = Xr^T Gi - Xi^T Gr,
-// with fp32 accuracy from the fp16 matrix pipe: every value, scaled by a power of two below 2^15, is the sum of two fp16
-// numbers (both rounded to nearest: the value to 2^-24 on average), and x g = x0 g0 + x0 g1 + x1 g0, each product exact,
-// into the fp32 accumulator (see dhconv_f16.hip, which computes the forward and the input gradient this way).
+// with fp32 accuracy from the bf16 matrix pipe: every value is cut exactly into three bf16 numbers, each the rounded remainder
+// of those before it (8 + 8 + 8 significant bits), and x g is the six partial products x0 g0 + x0 g1 + x1 g0 + x0 g2 + x1 g1 +
+// x2 g0, each exact, into the fp32 accumulator.  What is left out is below 2^-23 |x g| for every single product: the cut has
+// no scale, so rows whose magnitudes differ by any power of two keep their bits.  (Two fp16 numbers per value under a scale
+// per channel and 16 rows need half the matrix instructions, but keep a product only as far as its operands lie
+// near the largest of their rows: with x rising and g falling by 2^22 within 16 rows, so that all products count alike, the error
+// against float64 is 1e-5.)  The parts of an infinite value are no sum of it: a row that holds one gives NaN.
 //
-// Operands.  v_mfma_f32_32x32x16_f16 wants, per lane, 8 consecutive k of one channel.  Rows are K here, so a lane that loads the
+// Operands.  v_mfma_f32_32x32x16_bf16 wants, per lane, 8 consecutive k of one channel.  Rows are K here, so a lane that loads the
 // (re, im) pair of its channel from 8 rows holds its fragment without any transpose: lanes 0-31 take rows 0-7 of a chunk
-// of 16, lanes 32-63 rows 8-15, each load is 256 contiguous bytes per half.  Scales are per channel and chunk, a bound on the exponent
-// that follows the rows as they stream by and rescales the partial sums when it moves (the first chunks only, in practice): a
-// value keeps 22 bits or more down to 2^-14 of the largest of its channel within the 16 rows, and down to 2^-38 of the
-// largest of all its rows.
+// of 16, lanes 32-63 rows 8-15, each load is 256 contiguous bytes per half.
 //
 // A workgroup is 8 wavefronts = the 8 degrees that share 64-byte lines of gw ([i][o][l], l fastest),
 // all on the same tile of (i, o).  The results meet in LDS and leave as whole lines.
 //
-// What bounds it: per chunk and 64 x 64 tile a wavefront issues 48 matrix instructions (1536 cycles) and about 330 vector
-// instructions, most of them cutting the 64 values it loaded, on a SIMD shared by two wavefronts; they overlap little (leaving out
-// the cut or every load takes a tenth off each), and the store of gw (283 MB for 384 x 384 x 240) follows the sums.  384 x 384 channels,
-// 240 degrees: 182 / 334 / 566 us for 1 / 2 / 4 samples (on v_mfma_f32_32x32x2_f32, 512 matrix cycles per 16 rows instead of 96: 433 /
-// 710 / 1324), error against float64 2.1e-7 (3.2e-7 there: the sums are shorter).
+// What bounds it: per chunk and 64 x 64 tile a wavefront issues 96 matrix instructions (3072 cycles) and about 400 vector
+// instructions, most of them cutting the 64 values it loaded, on a SIMD shared by two wavefronts; the store of gw (283 MB for
+// 384 x 384 x 240) follows the sums.  384 x 384 channels, 240 degrees: 223 / 425 / 763 us for 1 / 2 / 4 samples (on
+// v_mfma_f32_32x32x2_f32, 512 matrix cycles per 16 rows and product instead of 192: 387 / 689 / 1322; two fp16 numbers, 96 cycles:
+// 191 / 338 / 578), 241 degrees, whose lines of gw are partial, 385 for one sample (416; 354).  Error against float64 of operands of
+// one magnitude, 1080 rows: 7.2e-7 (fp32 instruction 8.3e-7), and the same where they differ.
 #include "sfno_internal.h"
 
 namespace sfno {
@@ -29,24 +31,20 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
-constexpr int WG_TI = 64;            // i per workgroup
 constexpr int WG_DEG = 8;            // degrees (wavefronts) per workgroup
 constexpr int WG_KC = 16;            // rows per chunk: one matrix K step
 constexpr int WG_PITCH = WG_DEG + 1; // float2 per staged line of gw; odd so that the 32 lanes of a store hit 32 banks pairs
-constexpr int WG_SH = 14 + 127;      // scaled = x * 2^(SH - E), E = biased exponent bound of the channel: magnitudes below 2^15
-constexpr int WG_HEAD = 3;           // bits of headroom left when a bound is set
-constexpr int WG_SLACK = 7;          // a bound this far above a chunk's magnitudes (and the headroom) comes down
-constexpr int WG_DOWN = 24;
 
-// (value, remainder) of two numbers as packed fp16, both rounded to nearest
-__device__ __forceinline__ void cut_pair(float a, float b, unsigned& hi, unsigned& lo) {
-    const f16x2 h = __builtin_convertvector(f2{a, b}, f16x2);
-    hi = __builtin_bit_cast(unsigned, h);
-    lo = __builtin_bit_cast(unsigned, __builtin_convertvector(f2{__builtin_fmaf((float)h[0], -1.0f, a), __builtin_fmaf((float)h[1], -1.0f, b)}, f16x2));
+// rounds a pair of numbers to bf16 (packed) and leaves what that lost
+__device__ __forceinline__ unsigned take_bf16(float& a, float& b) {
+    const unsigned h = __builtin_bit_cast(unsigned, __builtin_convertvector(f2{a, b}, bf16x2));
+    a -= __uint_as_float(h << 16);
+    b -= __uint_as_float(h & 0xffff0000u);
+    return h;
 }
 
 // gw is written once and read by another kernel: past the caches, which the rows of X and G need
@@ -54,15 +52,15 @@ __device__ __forceinline__ void store_line(float2* p, float2 z) {
     __builtin_nontemporal_store(__builtin_bit_cast(double, z), reinterpret_cast<double*>(p));
 }
 
-struct Planes {                      // a channel's 8 rows: real and imaginary part, value and remainder
-    u4 r0, r1, i0, i1;
+struct Planes {                      // a channel's 8 rows: real and imaginary part, in three bf16 numbers each
+    u4 r[3], i[3];
 };
 
-// IB, OB: 32-channel blocks of i and o per workgroup (1 for up to 32 channels, and OB = 1 where larger tiles would leave CUs idle)
+// IB, OB: 32-channel blocks of i and o per workgroup: 2 x 2, or 1 x 1 (half of the registers and LDS) where those leave CUs idle
 // OFF: type of a lane's byte offset within a row chunk (64 bits only where 16 row strides do not fit 32)
 template <int IB, int OB, typename OFF>
 __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) void dhconv_wgrad_kernel(DhconvWgradArgs p, int ni, int no) {
-    constexpr int WG_TO = 32 * OB;   // o per workgroup
+    constexpr int WG_TI = 32 * IB, WG_TO = 32 * OB;      // channels per workgroup
     __shared__ float2 stage[32 * WG_TO * WG_PITCH];
 
     // Workgroups are dealt to the 8 XCDs round-robin by linear id.  All tiles of one group of 8 degrees run
@@ -104,12 +102,6 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
         for (int ob = 0; ob < OB; ++ob)
 #pragma unroll
             for (int v = 0; v < 16; ++v) re[ib][ob][v] = im[ib][ob][v] = 0.f;
-    int ex[IB], eg[OB], tx[IB], tg[OB];   // biased exponent bounds of my channels (lanes jj and jj + 32 agree), and their highest values
-#pragma unroll
-    for (int ib = 0; ib < IB; ++ib) ex[ib] = tx[ib] = 0;
-#pragma unroll
-    for (int ob = 0; ob < OB; ++ob) eg[ob] = tg[ob] = 0;
-
     // 8 rows of one channel, each from a wavefront-uniform row address plus a lane offset
     auto load = [&](const char* base, int64_t ms, OFF off, int m0, float2 (&r)[8]) {
         const char* row = base + max(min(m0, p.M - WG_KC), 0) * ms;
@@ -130,40 +122,15 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
         for (int j = 0; j < 8; ++j)
             if (first + j < lo || first + j >= nm) r[j] = make_float2(0.f, 0.f);
     };
-    // moves the channel's bound to the chunk's largest magnitude where that exceeds it, or lies far below it; returns the change
-    // the partial sums have to follow.  The bound comes down by at most WG_DOWN from its highest value top (the sums would
-    // overflow; what a chunk so far below loses is 2^-60 of the largest product).
-    auto bound = [&](const float2 (&r)[8], int& e, int& top) {
-        float mx = 0.f;
+    auto cut = [&](float2 (&r)[8], Planes& f) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(r[j].x), "v"(r[j].y));
-        const unsigned mb = __builtin_bit_cast(unsigned, mx);
-        const auto sw = __builtin_amdgcn_permlane32_swap(mb, mb, false, false);      // the other 8 rows sit 32 lanes away
-        const int eb = (int)(max(sw[0], sw[1]) >> 23);
-        int en = e;
-        if (eb > e || eb < e - WG_HEAD - WG_SLACK) en = max(eb + WG_HEAD, top - WG_DOWN);
-        top = max(top, en);
-        const int d = e - en;
-        e = en;
-        return d;
-    };
-    auto cut = [&](const float2 (&r)[8], int e, Planes& f) {
-        const int sh = WG_SH - e;
+        for (int w = 0; w < 4; ++w)
 #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            unsigned h, s;
-            cut_pair(__builtin_ldexpf(r[2 * w].x, sh), __builtin_ldexpf(r[2 * w + 1].x, sh), h, s);
-            f.r0[w] = h;
-            f.r1[w] = s;
-            cut_pair(__builtin_ldexpf(r[2 * w].y, sh), __builtin_ldexpf(r[2 * w + 1].y, sh), h, s);
-            f.i0[w] = h;
-            f.i1[w] = s;
-        }
+            for (int k = 0; k < 3; ++k) {
+                f.r[k][w] = take_bf16(r[2 * w].x, r[2 * w + 1].x);
+                f.i[k][w] = take_bf16(r[2 * w].y, r[2 * w + 1].y);
+            }
     };
-    // D row of accumulator element v, as the lane that holds that i: 4 x (4 kg) (made opaque where it is used, so that the
-    // sixteen addresses are not kept in registers) plus a constant
-    auto row_lane = [](int base, int v) { return base + 4 * (8 * (v >> 2) + (v & 3)); };
-
     const int64_t nchunks = (int64_t)nch * p.B;
     if (nchunks > 0) {
         float2 rx[IB][8], rg[OB][8];
@@ -187,8 +154,7 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
 #pragma unroll
                 for (int ob = 0; ob < OB; ++ob) mask(mc, rg[ob]);
             }
-            // the next chunk (the last one again after it) is requested into the registers of this one once they are cut and a
-            // batch of matrix instructions is issued
+            // the next chunk (the last one again after it) is requested into the registers of this one as they come free
             if (c + 1 < nchunks) {
                 m0 += WG_KC;
                 if (m0 >= nm) {
@@ -200,61 +166,46 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
             Planes fx[IB];
 #pragma unroll
             for (int ib = 0; ib < IB; ++ib) {
-                const int d = bound(rx[ib], ex[ib], tx[ib]);
-                cut(rx[ib], ex[ib], fx[ib]);
+                cut(rx[ib], fx[ib]);
                 __builtin_amdgcn_sched_barrier(0);
-                if (__builtin_amdgcn_ballot_w64(d != 0) != 0) {
-                    int rl = 16 * kg;
-                    asm volatile("" : "+v"(rl));
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int dv = __builtin_amdgcn_ds_bpermute(row_lane(rl, v), d);
-#pragma unroll
-                        for (int ob = 0; ob < OB; ++ob) {
-                            re[ib][ob][v] = __builtin_ldexpf(re[ib][ob][v], dv);
-                            im[ib][ob][v] = __builtin_ldexpf(im[ib][ob][v], dv);
-                        }
-                    }
-                }
             }
 #pragma unroll
             for (int ob = 0; ob < OB; ++ob) {
                 Planes fg;
-                const int d = bound(rg[ob], eg[ob], tg[ob]);
-                cut(rg[ob], eg[ob], fg);
-                if (__builtin_amdgcn_ballot_w64(d != 0) != 0) {
-#pragma unroll
-                    for (int ib = 0; ib < IB; ++ib)
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) {
-                            re[ib][ob][v] = __builtin_ldexpf(re[ib][ob][v], d);
-                            im[ib][ob][v] = __builtin_ldexpf(im[ib][ob][v], d);
-                        }
-                }
+                cut(rg[ob], fg);
                 __builtin_amdgcn_sched_barrier(0);
-                const f16x8 gr0 = __builtin_bit_cast(f16x8, fg.r0), gr1 = __builtin_bit_cast(f16x8, fg.r1);
-                const f16x8 gi0 = __builtin_bit_cast(f16x8, fg.i0), gi1 = __builtin_bit_cast(f16x8, fg.i1);
-                const f16x8 ng0 = __builtin_bit_cast(f16x8, fg.r0 ^ 0x80008000u), ng1 = __builtin_bit_cast(f16x8, fg.r1 ^ 0x80008000u);     // -Gr
-                // smallest terms first; consecutive instructions go to different accumulators
-#define WG_STEP(A, B, C, D)                                                                                                     \
-    _Pragma("unroll") for (int ib = 0; ib < IB; ++ib) {                                                                        \
-        re[ib][ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fx[ib].A), B, re[ib][ob], 0, 0, 0);       \
-        im[ib][ob] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fx[ib].C), D, im[ib][ob], 0, 0, 0);       \
-    }
-                WG_STEP(r1, gr0, r1, gi0)
-                WG_STEP(i1, gi0, i1, ng0)
-                WG_STEP(r0, gr1, r0, gi1)
-                WG_STEP(i0, gi1, i0, ng1)
-                WG_STEP(r0, gr0, r0, gi0)
-                WG_STEP(i0, gi0, i0, ng0)
-#undef WG_STEP
-                __builtin_amdgcn_sched_barrier(0);
-                if (ob == 0) {
+                // part A of x times part B of g; consecutive instructions go to different accumulators
+                auto step = [&](int A, int B) {
+                    const bf16x8 gr = __builtin_bit_cast(bf16x8, fg.r[B]), gi = __builtin_bit_cast(bf16x8, fg.i[B]);
+                    const bf16x8 ng = __builtin_bit_cast(bf16x8, fg.r[B] ^ 0x80008000u);     // -Gr
+#pragma unroll
+                    for (int ib = 0; ib < IB; ++ib) {
+                        const bf16x8 xr = __builtin_bit_cast(bf16x8, fx[ib].r[A]);
+                        re[ib][ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xr, gr, re[ib][ob], 0, 0, 0);
+                        im[ib][ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xr, gi, im[ib][ob], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int ib = 0; ib < IB; ++ib) {
+                        const bf16x8 xi = __builtin_bit_cast(bf16x8, fx[ib].i[A]);
+                        re[ib][ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xi, gi, re[ib][ob], 0, 0, 0);
+                        im[ib][ob] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xi, ng, im[ib][ob], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                // smallest terms first
+                step(2, 0);
+                step(1, 1);
+                step(0, 2);
+                step(1, 0);
+                // (only now, with parts 1 and 2 of x spent, are there registers for its next rows)
+                if (ob == OB - 1) {
 #pragma unroll
                     for (int ib = 0; ib < IB; ++ib) load(Xb, ms_x, offx[ib], m0, rx[ib]);
                 }
                 load(Gb, ms_g, offg[ob], m0, rg[ob]);
                 __builtin_amdgcn_sched_barrier(0);
+                step(0, 1);
+                step(0, 0);
             }
         }
     }
@@ -267,12 +218,10 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
         if (ib) __syncthreads();
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const int er = __builtin_amdgcn_ds_bpermute(row_lane(16 * kg, v), ex[ib]) - 2 * WG_SH;
             const int il = 8 * (v >> 2) + 4 * kg + (v & 3);
 #pragma unroll
             for (int ob = 0; ob < OB; ++ob)
-                stage[(il * WG_TO + 32 * ob + jj) * WG_PITCH + wave] =
-                    make_float2(__builtin_ldexpf(re[ib][ob][v], er + eg[ob]), __builtin_ldexpf(im[ib][ob][v], er + eg[ob]));
+                stage[(il * WG_TO + 32 * ob + jj) * WG_PITCH + wave] = make_float2(re[ib][ob][v], im[ib][ob][v]);
         }
         __syncthreads();
         // eight lanes per line, 64 lines per pass
@@ -300,24 +249,22 @@ int dhconv_wgrad_launch(const DhconvWgradArgs& a, hipStream_t s) {
     const int64_t ld = a.ld_in > a.ld_out ? a.ld_in : a.ld_out;
     const bool wide = 64 * (int64_t)a.L * ld + 4 * ld > 0xffffffffLL;
     const int64_t groups = 8 * (((a.L + WG_DEG - 1) / WG_DEG + 7) / 8);
-    const int ni = (a.I + WG_TI - 1) / WG_TI;
-    // 64 x 64 tiles cut and load a third less per product, 64 x 32 tiles need half the registers and LDS (two workgroups per CU,
-    // twice as many): 182 against 273 us for 384 x 384 channels and 240 degrees (1080 tiles of 64 x 64), 43 against 32 us for
-    // 128 x 128 and 90 (48 tiles).  The line: two tiles per CU.
-    const int no2 = (a.O + 63) / 64;
-    const bool narrow = a.O <= 32 || (!wide && groups * ni * no2 < 512);
-    const int no = narrow ? (a.O + 31) / 32 : no2;
+    // 64 x 64 tiles cut and load half as much per product, 32 x 32 tiles need half the registers and LDS (two workgroups per CU, four
+    // times as many): 31 against 15 us for 128 x 128 channels and 90 degrees (64 tiles of 64 x 64), 84 against 72 for 384 x 384 and
+    // 120 (576 tiles), but 214 against 240 for 384 x 384 and 240 (1152 tiles).  The line: three tiles per CU.
+    const int64_t n2 = (int64_t)((a.I + 63) / 64) * ((a.O + 63) / 64);
+    const bool narrow = !wide && ((a.I <= 32 && a.O <= 32) || groups * n2 < 768);
+    const int tile = narrow ? 32 : 64;
+    const int ni = (a.I + tile - 1) / tile, no = (a.O + tile - 1) / tile;
     const int64_t blocks = groups * ni * no;
     if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
     const dim3 grid((unsigned)blocks), block(64 * WG_DEG);
     if (wide)
         hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, uint64_t>), grid, block, 0, s, a, ni, no);
-    else if (!narrow)
-        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, unsigned>), grid, block, 0, s, a, ni, no);
-    else if (a.I > 32)
-        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 1, unsigned>), grid, block, 0, s, a, ni, no);
-    else
+    else if (narrow)
         hipLaunchKernelGGL((dhconv_wgrad_kernel<1, 1, unsigned>), grid, block, 0, s, a, ni, no);
+    else
+        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, unsigned>), grid, block, 0, s, a, ni, no);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

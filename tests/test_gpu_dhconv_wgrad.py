@@ -1,11 +1,10 @@
-"""Weight gradient of dhconv (csrc/dhconv_wgrad.hip) at the sizes where its tiles, row chunks and scales can go wrong, against
+"""Weight gradient of dhconv (csrc/dhconv_wgrad.hip) at the sizes where its tiles and row chunks can go wrong, against
 the complex128 sum on the same operands.
 
-Bound: both fp16 parts of an operand are rounded to nearest (2^-23 of the value at worst) and one partial product is dropped (2^-22),
-2^-21 per product; the sums add at most sqrt(6 K / 16) roundings of 2^-24 in relative L2 (K / 16 steps of six partial sums): below
-1.2e-6 for the K <= 1100 rows here, 1.5e-6 asserted.  The bound holds for operands that vary by less than 2^14 within a channel's
-16 consecutive orders (fp16 reaches 2^-24 below its 2^15) and by less than 2^38 over all its rows (a channel's scale comes down by
-2^24 at most); they vary by 2^9 and 2^34 here.
+Bound: both operands are cut exactly into three bf16 numbers (each rounded to nearest: 2^-8, 2^-16 of the value at worst) and the
+partial products left out are below 2^-23 of a product, whatever its operands' magnitudes; the sums are 12 K / 16 fp32 additions,
+each off by 2^-24 at worst, on average by half of that and with either sign: 0.5 sqrt(12 K / 16) 2^-24 = 8.6e-7 in relative L2
+for the K <= 1100 rows here, 1.5e-6 asserted.
 """
 import pytest
 import torch
@@ -23,7 +22,8 @@ pytestmark = pytest.mark.gpu
         (1, 64, 65, 20, 16, True),      # exactly one chunk
         (2, 65, 64, 31, 17, True),      # the last chunk starts early
         (4, 40, 96, 50, 270, False),    # many chunks per sample, rectangle
-        (1, 520, 519, 60, 61, True),    # 64 x 64 tiles (enough of them for every CU)
+        (1, 520, 519, 60, 61, True),    # 32 x 32 tiles, many of them
+        (1, 648, 641, 60, 61, True),    # 64 x 64 tiles (enough of them for every CU)
     ],
 )
 def test_weight_grad_edges(lib_built, B, I, O, L, M, triangular):
@@ -32,8 +32,8 @@ def test_weight_grad_edges(lib_built, B, I, O, L, M, triangular):
     print(f"case wgrad B={B} I={I} O={O} L={L} M={M} tri={triangular}", flush=True)
     gen = torch.Generator().manual_seed(3)
     x, g = (torch.randn(B, c, L, M, dtype=torch.complex64, generator=gen) for c in (I, O))
-    # magnitudes that grow or fall along the orders and jump between samples move every channel's scale while the rows stream by,
-    # in opposite directions for the two operands so that every chunk counts in the sum
+    # magnitudes that grow or fall along the orders and jump between samples, in opposite directions for the two operands so that
+    # every chunk counts in the sum
     slope, jump = min(0.5, 16 / M) * torch.arange(M), 6.0 * torch.arange(B).reshape(B, 1, 1, 1)
     x = (x * 2.0 ** (slope - jump)).cuda()
     g = (g * 2.0 ** (torch.randint(-20, 20, (1, O, 1, 1), generator=gen) - slope + jump)).cuda()
@@ -50,6 +50,30 @@ def test_weight_grad_edges(lib_built, B, I, O, L, M, triangular):
     ref = torch.bmm(xl.conj().resolve_conj(), gl).permute(1, 2, 0)
     err = (got - ref).norm(dim=0) / ref.norm(dim=0).clamp_min(1e-300)      # per output channel and degree: each has its own scale
     assert torch.isfinite(torch.view_as_real(got)).all()
+    assert float(err.max()) < 1.5e-6
+
+
+@pytest.mark.parametrize("bits", [15, 22, 40])
+@pytest.mark.parametrize("B,I,O,L,M,triangular", [(2, 48, 40, 24, 100, False), (1, 648, 641, 60, 61, True)])
+def test_orders_of_any_magnitude_count(lib_built, B, I, O, L, M, triangular, bits):
+    """x rises by 2^bits within 16 consecutive orders where g falls by as much, so that the smallest values of either count as much as the
+    largest; the first 16 orders are another 2^6 off.  The bound is the one above: fp32 arithmetic does not see such a range."""
+    from makani_amd.contractions import _to_spectral, _weight_grad
+
+    print(f"case wgrad range B={B} I={I} O={O} L={L} M={M} tri={triangular} bits={bits}", flush=True)
+    gen = torch.Generator().manual_seed(5)
+    x, g = (torch.randn(B, c, L, M, dtype=torch.complex64, generator=gen) for c in (I, O))
+    m = torch.arange(M)
+    ramp = 2.0 ** (bits * (m % 16) / 15.0 + 6.0 * (m < 16))
+    x, g = (x * ramp).cuda(), (g / ramp).cuda()
+    got = _weight_grad(_to_spectral(x, B * I, L, M, triangular), _to_spectral(g, B * O, L, M, triangular), (I, O, L), B, M, triangular).to(torch.complex128)
+    keep = torch.ones(L, M, dtype=torch.bool, device="cuda")
+    if triangular:
+        keep = torch.arange(M, device="cuda")[None, :] <= torch.arange(L, device="cuda")[:, None]
+    xl = (x.to(torch.complex128) * keep).permute(2, 1, 0, 3).reshape(L, I, B * M).contiguous()
+    gl = (g.to(torch.complex128) * keep).permute(2, 0, 3, 1).reshape(L, B * M, O).contiguous()
+    ref = torch.bmm(xl.conj().resolve_conj(), gl).permute(1, 2, 0)
+    err = (got - ref).norm(dim=0) / ref.norm(dim=0).clamp_min(1e-300)
     assert float(err.max()) < 1.5e-6
 
 
