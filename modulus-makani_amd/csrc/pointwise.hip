@@ -738,6 +738,55 @@ __global__ void row_stats_finalize_kernel(const unsigned short* __restrict__ x, 
     if (moments) moments[row] = make_float2(mean, rstd);
 }
 
+// The same in one kernel for short rows (P <= NORM_SMALL_PIXELS): a wavefront per row, its values in registers, mean first and then the
+// moments of the deviations from it.
+constexpr int SS_GROUPS = 8;                                  // groups of eight pixels per lane
+static_assert(SS_GROUPS * 64 * 8 == NORM_SMALL_PIXELS, "a row fits the registers of a wavefront");
+__global__ __launch_bounds__(64) void row_stats_small_kernel(const unsigned short* __restrict__ x, const float* __restrict__ gamma,
+                                                             const float* __restrict__ beta, float* __restrict__ scale, float* __restrict__ shift,
+                                                             float2* __restrict__ moments, int channels, int P, float eps) {
+    const int64_t row = blockIdx.x;
+    const u32x4* __restrict__ xr = reinterpret_cast<const u32x4*>(x + row * P);
+    const int ngroups = P / 8;
+    u32x4 v[SS_GROUPS];
+#pragma unroll
+    for (int k = 0; k < SS_GROUPS; ++k) {
+        const int g = (int)threadIdx.x + 64 * k;
+        if (g < ngroups) v[k] = xr[g];
+    }
+    auto sums = [&](float about, float& s, float& s2) {
+        s = s2 = 0.f;
+#pragma unroll
+        for (int k = 0; k < SS_GROUPS; ++k) {
+            if ((int)threadIdx.x + 64 * k >= ngroups) break;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float lo = __uint_as_float(v[k][i] << 16) - about, hi = __uint_as_float(v[k][i] & 0xffff0000u) - about;
+                s += lo + hi;
+                s2 = fmaf(lo, lo, fmaf(hi, hi, s2));
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            s += __shfl_xor(s, off, 64);
+            s2 += __shfl_xor(s2, off, 64);
+        }
+    };
+    float s, s2;
+    sums(0.f, s, s2);
+    const float about = s / (float)P;
+    sums(about, s, s2);
+    if (threadIdx.x == 0) {
+        const double md = (double)s / P, var = fmax((double)s2 / P - md * md, 0.0);
+        const float mean = about + (float)md, rstd = (float)(1.0 / sqrt(var + (double)eps));
+        const int c = (int)(row % channels);
+        const float sc = (gamma ? gamma[c] : 1.f) * rstd;
+        scale[row] = sc;
+        shift[row] = (beta ? beta[c] : 0.f) - mean * sc;
+        if (moments) moments[row] = make_float2(mean, rstd);
+    }
+}
+
 // The same coefficients from per-latitude moments of the field (the inverse longitude kernel's by-product):
 // stats[row][k] = (a_k, d_k), the mean over longitude of latitude row k and of its squared deviation from a_k.
 // mean = avg_k a_k, variance = avg_k ((a_k - mean)^2 + d_k); one wavefront per row, sums in double.
@@ -1021,6 +1070,10 @@ int instance_norm_coeffs_launch(const unsigned short* x, const float* gamma, con
                                 int64_t rows, int channels, int64_t P, float eps, hipStream_t s, float2* moments) {
     if (rows < 1 || P < 1 || channels < 1 || rows > 0x7fffffffLL / 64) return SFNO_EUNSUPPORTED;
     if (P % 8 != 0) return SFNO_EUNSUPPORTED;     // 16-byte loads from every row start
+    if (P <= NORM_SMALL_PIXELS) {
+        hipLaunchKernelGGL(row_stats_small_kernel, dim3((unsigned)rows), dim3(64), 0, s, x, gamma, beta, scale, shift, moments, channels, (int)P, eps);
+        return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+    }
     const int nseg = row_stats_segments(rows, P);
     hipLaunchKernelGGL(row_stats_partial_kernel, dim3((unsigned)rows, (unsigned)nseg), dim3(ST_THREADS), 0, s, x, partial, P, nseg);
     hipLaunchKernelGGL(row_stats_finalize_kernel, dim3((unsigned)((rows + 127) / 128)), dim3(128), 0, s, x, partial, gamma, beta, scale, shift, moments,

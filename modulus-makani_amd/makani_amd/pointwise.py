@@ -141,6 +141,10 @@ def instance_norm_coeffs(x, gamma=None, beta=None, eps=1e-5):
     return scale, shift
 
 
+# grids of at most this many pixels are normalised by the moments of the stored field (NORM_SMALL_PIXELS in csrc/sfno_internal.h)
+NORM_SMALL_PIXELS = 4096
+
+
 def instance_norm_coeffs_lat(lat_stats, batch, gamma=None, beta=None, eps=1e-5):
     """(scale, shift) float32 [B, C] from the per-latitude moments [B*C, nlat, 2] that InverseRealSHT.synthesis_with_lat_stats returns."""
     rows, nlat, _ = lat_stats.shape

@@ -204,6 +204,9 @@ class FourierNeuralOperatorBlock(nn.Module):
             return False
         return hasattr(self, "outer_skip") and _is_conv1x1(self.outer_skip) and self.outer_skip.bias is None
 
+    def _norm0_from_transform(self):
+        return self.output_shape_loc[0] * self.output_shape_loc[1] > pw.NORM_SMALL_PIXELS
+
     def _forward_fused(self, x, residual, lat_stats=None, skip_weight=None, defer_skip=False):
         """norm0 -> GELU -> MLP -> norm1 -> + outer_skip(residual) in five kernels: row statistics (or, for norm0, the
         per-latitude moments the inverse transform delivered with x), scale/shift + GELU, two 1x1 convolutions with bias
@@ -235,7 +238,8 @@ class FourierNeuralOperatorBlock(nn.Module):
             elif not self.training and fused_pointwise_active(x) and self._fusable() and native_block.supported(self, x):
                 return native_block.forward(self, x, defer_skip=defer_skip)
         # on the fused inference path the inverse transform hands over the moments norm0 needs together with its output
-        want_stats = getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x) and x.dtype == torch.bfloat16 and self._fusable()
+        want_stats = getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x) and x.dtype == torch.bfloat16 \
+            and self._norm0_from_transform() and self._fusable()
         if want_stats:
             x, residual, lat_stats = self.filter(x, lat_stats=True)
         else:
@@ -433,6 +437,8 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         residual = conv.inverse_transform.synthesis(spec, (B, h.shape[1]), dtype=torch.bfloat16)
         spec = dhconv_spectral(spec, wf, B, conv.modes_lon, triangular=conv._triangular, compute=conv.compute)
         x, stats = conv.inverse_transform.synthesis_with_lat_stats(spec, (B, conv.out_channels), dtype=torch.bfloat16)
+        if not blk._norm0_from_transform():
+            stats = None
         return blk._forward_fused(x.contiguous(), residual.contiguous(), stats, skip_weight=wsk)
 
     # The last block ends in  x = scale * m + shift + W_skip r  (norm1 of the MLP output m as a per-(sample, channel) affine, plus

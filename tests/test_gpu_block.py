@@ -92,6 +92,35 @@ def test_block_gradients(lib_built, f, i, B, E, ratio):
         assert rel(blk.eval()(x), ref["y"]) < 1.5e-2
 
 
+@pytest.mark.parametrize("grid,B,E", [((4, 8), 4, 32), ((16, 32), 1, 5), ((9, 24), 2, 3), ((64, 64), 1, 4)])
+def test_norm_of_a_small_grid_follows_the_stored_field(lib_built, grid, B, E):
+    """Up to 4096 pixels norm0 takes the moments of the field as it is stored: with those of the field before its rounding to bf16 the
+    normalised field keeps the mean of the rounding errors (2^-9 / sqrt(3 P) of the field: 2e-4 at 32 pixels).  Moments in fp32 from
+    exact values: 1e-6 of the standard deviation asserted."""
+    import makani_amd as ma
+    from makani_amd import block as nb
+
+    print(f"case small norm {grid} B={B} E={E}", flush=True)
+    torch.manual_seed(9)
+    fwd, inv = ma.RealSHT(*grid, grid="legendre-gauss"), ma.InverseRealSHT(*grid, grid="legendre-gauss")
+    blk = make_block(fwd, inv, E, 2.0)
+    x = (3.0 + torch.randn(B, E, *grid, device="cuda")).to(torch.bfloat16)
+    c = nb._Call(blk, x, nb.block_params(blk))
+    kept = c.forward(x, 1, torch.empty_like(x))
+    rows, P = B * E, grid[0] * grid[1]
+
+    def part(i, n, dtype):
+        return kept[c.offsets[i]:c.offsets[i] + n * dtype.itemsize].view(dtype)
+
+    xf = part(1, rows * P, torch.bfloat16).view(rows, P).double()
+    mean, rstd = part(2, 4 * rows, torch.float32)[2 * rows:].view(rows, 2).double().unbind(1)
+    want = 1.0 / (xf.var(1, unbiased=False) + blk.norm0.eps).sqrt()
+    assert float(((mean - xf.mean(1)).abs() * want).max()) < 1e-6
+    assert float((rstd / want - 1.0).abs().max()) < 1e-6
+    # the module path on these grids too
+    assert not blk._norm0_from_transform()
+
+
 def test_frozen_parameters_and_input(lib_built):
     """Only what asks for a gradient gets one."""
     import makani_amd as ma
