@@ -200,7 +200,7 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
         TRY(irfft_launch(b->inv->fft, w.xm, xf, SFNO_DTYPE_BF16, d.rows, b->inv->nlat, d.mmax, (int)sfno_spectral_ld(d.rows), s, w.stats));
         TRY(instance_norm_coeffs_lat_launch(w.stats, b->gamma0, b->beta0, c0, c0 + d.rows, d.rows, d.e, b->inv->nlat, b->eps0, s, m0));
     }
-    TRY(scale_shift_act_launch(xf, c0, c0 + d.rows, h0, d.rows, d.P, SFNO_ACT_GELU, s));
+    TRY(scale_shift_act_launch(xf, c0, c0 + d.rows, h0, d.rows, d.P, training ? ACT_GELU_TRAIN : SFNO_ACT_GELU, s));
     TRY(conv(h0, b->w1, b->b1, a1, d.B, d.e, d.h, d.P, SFNO_ACT_GELU, nullptr, nullptr, nullptr, z1, 0, s));
     TRY(conv(a1, b->w2, b->b2, y2, d.B, d.h, d.e, d.P, SFNO_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0, s));
     TRY(instance_norm_coeffs_launch(y2, b->gamma1, b->beta1, c1, c1 + d.rows, w.partial, d.rows, d.e, d.P, b->eps1, s, reinterpret_cast<float2*>(c1 + 2 * d.rows)));

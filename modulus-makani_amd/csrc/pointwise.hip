@@ -68,17 +68,31 @@ __device__ __forceinline__ float gelu(float x) {
     return fmaf(-fabsf(x), __builtin_amdgcn_exp2f(q), __builtin_amdgcn_fmed3f(x, 0.f, __builtin_inff()));
 }
 
-// derivative of the exact GELU: Phi(x) + x phi(x), with Phi from the erfc fit of gelu() (absolute error below 2e-5, an eighth of
-// the half ulp of a bf16 result of 0.1) and phi(x) = 2^(-x^2 log2(e) / 2) / sqrt(2 pi)
-__device__ __forceinline__ float gelu_grad(float x) {
+// The same in training, where the derivative passes through zero and a bf16 result no longer hides the fit above (its error of
+// Phi is 4e-5): degree 11, Phi(-|x|) = 2^Q(|x|) to 7e-8 with every step in fp32, what 1 + erf in fp32 gives.
+__device__ __forceinline__ float phi_neg(float x) {
     const float t = __builtin_amdgcn_fmed3f(fabsf(x), 0.f, 6.5f);
-    float q = fmaf(t, 2.008575651e-05f, -5.615057212e-04f);
-    q = fmaf(t, q, 6.880626770e-03f);
-    q = fmaf(t, q, -5.027262948e-02f);
-    q = fmaf(t, q, -4.624537704e-01f);
-    q = fmaf(t, q, -1.149621597e+00f);
-    q = fmaf(t, q, -1.000106287211f);
-    const float e = __builtin_amdgcn_exp2f(q);                                     // Phi(-|x|)
+    float q = fmaf(t, 1.487025059e-09f, -6.108023598e-08f);
+    q = fmaf(t, q, 1.104927378e-06f);
+    q = fmaf(t, q, -1.145743681e-05f);
+    q = fmaf(t, q, 7.265697059e-05f);
+    q = fmaf(t, q, -2.514593652e-04f);
+    q = fmaf(t, q, -8.251464169e-05f);
+    q = fmaf(t, q, 7.073279005e-03f);
+    q = fmaf(t, q, -5.254369602e-02f);
+    q = fmaf(t, q, -4.591809213e-01f);
+    q = fmaf(t, q, -1.151109934e+00f);
+    q = fmaf(t, q, -9.999998808e-01f);
+    return __builtin_amdgcn_exp2f(q);
+}
+
+__device__ __forceinline__ float gelu_train(float x) {
+    return fmaf(-fabsf(x), phi_neg(x), __builtin_amdgcn_fmed3f(x, 0.f, __builtin_inff()));
+}
+
+// derivative of the GELU: Phi(x) + x phi(x), phi(x) = 2^(-x^2 log2(e) / 2) / sqrt(2 pi)
+__device__ __forceinline__ float gelu_grad(float x) {
+    const float e = phi_neg(x);
     const float phi = 0.39894228040143267794f * __builtin_amdgcn_exp2f(-0.72134752044448170368f * x * x);
     return fmaf(x, phi, x > 0.f ? 1.f - e : e);
 }
@@ -284,7 +298,10 @@ __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
                 y0 = __uint_as_float(zz[0] << 16);
                 y1 = __uint_as_float(zz[0] & 0xffff0000u);
             }
-            if constexpr (GELU) {
+            if constexpr (EPI & PW_GELU_PRE) {
+                y0 = gelu_train(y0);
+                y1 = gelu_train(y1);
+            } else if constexpr (GELU) {
                 y0 = gelu(y0);
                 y1 = gelu(y1);
             }
@@ -560,7 +577,7 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
                     }
                     if constexpr (GELU) {
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) y[t] = gelu(y[t]);
+                        for (int t = 0; t < 4; ++t) y[t] = EPI & PW_GELU_PRE ? gelu_train(y[t]) : gelu(y[t]);
                     }
                     if constexpr (EPI & PW_GELU_BWD) {
                         const u32x2 r = rv[mh & 1][4 * g + jj];
@@ -835,6 +852,9 @@ __global__ __launch_bounds__(256) void scale_shift_act_kernel(const unsigned sho
         if (act == SFNO_ACT_GELU) {
             lo = gelu(lo);
             hi = gelu(hi);
+        } else if (act == ACT_GELU_TRAIN) {
+            lo = gelu_train(lo);
+            hi = gelu_train(hi);
         }
         o[i] = bf16_pair(lo, hi);
     }

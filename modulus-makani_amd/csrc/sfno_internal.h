@@ -128,6 +128,8 @@ int instance_norm_coeffs_lat_launch(const float2* stats, const float* gamma, con
 // rows * row_stats_segments float2; dgamma, dbeta [channels] may be null
 int norm_grad_launch(const unsigned short* g, const unsigned short* x, const float* scale, const float* shift, const float2* moments, float2* partial,
                      unsigned short* dx, float* dgamma, float* dbeta, int batch, int channels, int64_t P, int act, hipStream_t s);
+// act: as in the C interface, or ACT_GELU_TRAIN, the GELU to fp32 accuracy
+constexpr int ACT_GELU_TRAIN = 0x100;
 int scale_shift_act_launch(const unsigned short* x, const float* scale, const float* shift, unsigned short* y, int64_t rows, int64_t P, int act,
                            hipStream_t s);
 

@@ -196,3 +196,40 @@ def test_training_step_through_the_network_matches_the_module_path(lib_built):
     assert worst[0] < 5e-2, worst
     err = sum(float(torch.linalg.norm((g_hip[n] - g_ref[n]).double())) ** 2 for n in g_ref) ** 0.5
     assert err < 3e-2 * sum(v * v for v in norms.values()) ** 0.5
+
+
+@pytest.mark.parametrize("channels", [8, 104])
+def test_training_gelu_and_its_derivative_on_every_bf16_value(lib_built, channels):
+    """conv -> GELU and the GELU's derivative in the convolutions' epilogues, through an identity matrix, at every bf16 value between -6
+    and 8.  fp32 arithmetic (2^-23 of Phi) and one rounding to bf16: half a unit of the result and 3e-7 beside it.  An activation within
+    the fp32 error (1e-6 relative in the tail) of a rounding boundary may fall on its other side: 2e-6 / 2^-8, one of the 2242 values
+    from 2^-6 on."""
+    import ctypes
+
+    from makani_amd import pointwise as pw
+    from makani_amd._lib import check, lib
+
+    print(f"case training gelu {channels}", flush=True)
+    z = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    z = z[torch.isfinite(z) & (z >= -6) & (z <= 8)]
+    P = (z.numel() // channels + 8) // 8 * 8
+    x = torch.zeros(channels * P, dtype=torch.bfloat16)
+    x[:z.numel()] = z
+    x = x.reshape(1, channels, 1, P).cuda()
+    eye, ones = torch.eye(channels, device="cuda"), torch.ones_like(x)
+    y, pre, gx = (torch.empty_like(x) for _ in range(3))
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    check(lib.sfno_pointwise_conv_gelu(ptr(x), ptr(pw.packed_weight(eye)), None, ptr(y), ptr(pre), 1, channels, channels, P, pw._stream(x.device)), "forward")
+    check(lib.sfno_pointwise_conv_gelu_grad(ptr(ones), ptr(pw.packed_weight(eye, transposed=True)), ptr(x), ptr(gx), 1, channels, channels, P,
+                                            pw._stream(x.device)), "backward")
+    torch.cuda.synchronize()
+    xd = x.double().cpu()
+    assert torch.equal(pre.float().cpu(), x.float().cpu())
+    Phi = 0.5 * torch.special.erfc(-xd / 2 ** 0.5)
+    pdf = torch.exp(-0.5 * xd * xd) / (2 * torch.pi) ** 0.5
+    want = xd * Phi
+    got = y.double().cpu()
+    assert bool(((got - want).abs() <= want.abs() * 2 ** -8 + 3e-7).all())
+    assert int(((got != want.to(torch.bfloat16).double()) & (xd.abs() >= 2 ** -6)).sum()) < 5
+    want = Phi + xd * pdf
+    assert bool(((gx.double().cpu() - want).abs() <= want.abs() * 2 ** -8 + 3e-7).all())
