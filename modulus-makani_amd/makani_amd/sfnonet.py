@@ -103,9 +103,10 @@ class EncoderDecoder(nn.Module):
         mods.append(_pointwise(cur, output_dim, False, math.sqrt(gain / cur)))
         self.fwd = nn.Sequential(*mods)
 
-    def forward(self, x):
-        # training under bf16: convolution, GELU and convolution with the GELU in the convolutions' epilogues, both ways
-        if len(self.fwd) == 3 and pw.trainable_active(x) and _is_conv1x1(self.fwd[0]) and _is_gelu(self.fwd[1]) and _is_conv1x1(self.fwd[2]) \
+    def forward(self, x, fused=True):
+        # training under bf16: convolution, GELU and convolution with the GELU in the convolutions' epilogues, both ways (fused = False:
+        # the modules, as the network's fused_pointwise asks for)
+        if fused and len(self.fwd) == 3 and pw.trainable_active(x) and _is_conv1x1(self.fwd[0]) and _is_gelu(self.fwd[1]) and _is_conv1x1(self.fwd[2]) \
                 and native_block.plain_conv(self.fwd[0]) and native_block.plain_conv(self.fwd[2]) and native_block._no_hooks(self.fwd, *self.fwd):
             y = pw.conv_gelu_conv_trainable(x, self.fwd[0], self.fwd[2])
             if y is not None:
@@ -375,6 +376,9 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         self.out_shape_loc = (self.itrans_up.nlat, self.itrans_up.nlon)
         self.h_loc, self.w_loc = self.itrans.nlat, self.itrans.nlon
 
+    def _coder(self, m, x):
+        return m(x) if getattr(self, "fused_pointwise", True) or type(m) is not EncoderDecoder else m(x, fused=False)
+
     def _forward_features(self, x):
         for _ in range(self.repeat_layers):
             for blk in self.blocks:
@@ -565,7 +569,7 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
                 residual = self.itrans_up(self.trans_down(x.to(torch.float32)).contiguous()).to(dtype=xtype)
             else:
                 residual = x
-        x = self.encoder(x)
+        x = self._coder(self.encoder, x)
         if hasattr(self, "pos_embed"):
             if self.pos_embed.type == "frequency":
                 pe = torch.stack([self.pos_embed[0], nn.functional.pad(self.pos_embed[1], (1, 0), "constant", 0)], dim=-1)
@@ -575,7 +579,7 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
             x = x + pe
         x = self.pos_drop(x)
         x = self._forward_features(x)
-        x = self.decoder(x)
+        x = self._coder(self.decoder, x)
         if self.big_skip:
             x = x + self.residual_transform(residual)
         return x

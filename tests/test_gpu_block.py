@@ -249,3 +249,28 @@ def test_offset_tensors_and_foreign_shapes(lib_built):
     blk.mlp.fwd[0] = nn.Conv2d(15, 32, 1).cuda()
     with torch.autocast("cuda", dtype=torch.bfloat16), pytest.raises(RuntimeError):
         blk.train()(x)
+
+
+@pytest.mark.parametrize("at_construction", [True, False])
+def test_switch_reaches_encoder_and_decoder_in_training(lib_built, at_construction, monkeypatch):
+    """fused_pointwise=False keeps the modules of encoder and decoder too while gradients are recorded."""
+    from makani_amd import block as nb, pointwise as pw
+    from makani_amd.sfnonet import SphericalFourierNeuralOperatorNet
+
+    calls = []
+    for fn in (pw._ConvGeluConv, nb._BlockFn):
+        monkeypatch.setattr(fn, "apply", lambda *a, f=fn, keep=fn.apply: calls.append(f) or keep(*a))
+    torch.manual_seed(10)
+    net = SphericalFourierNeuralOperatorNet(inp_shape=(33, 64), out_shape=(33, 64), inp_chans=3, out_chans=3, scale_factor=2, embed_dim=16, num_layers=2,
+                                            fused_pointwise=not at_construction).cuda()
+    x = torch.randn(1, 3, 33, 64, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        if not at_construction:
+            net(x)
+            assert calls.count(pw._ConvGeluConv) == 2 and calls.count(nb._BlockFn) == 2
+            calls.clear()
+            net.fused_pointwise = False
+            for b in net.blocks:
+                b.fused_pointwise = False
+        net(x).float().square().sum().backward()
+    assert not calls and all(p.grad is not None for p in net.parameters())
