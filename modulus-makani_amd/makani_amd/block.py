@@ -33,6 +33,12 @@ def plain_conv(m):
     return type(m) in (nn.Conv2d, pw.PointwiseConv2d)
 
 
+def trainable(x, params, *convs):
+    """Whether a call with gradients enabled may run on the HIP kernels: something asks for a gradient, and every convolution is one that
+    would train on them by itself (nn.Conv2d put in by a user is differentiable twice, the kernels once)."""
+    return pw.trainable_active(x) and all(type(m) is pw.PointwiseConv2d for m in convs) and (x.requires_grad or any(p is not None and p.requires_grad for p in params))
+
+
 def mlp_convs(blk):
     """(fc1, fc2) of a conv -> GELU -> conv MLP, or None."""
     m = [f for f in blk.mlp.fwd if not isinstance(f, nn.Identity)]
@@ -179,6 +185,12 @@ class _BlockFn(torch.autograd.Function):
         return (gx, None, *(t if n else None for t, n in zip(grads, need[2:])))
 
 
+def train_asked(blk, x):
+    """Whether the block (fusable, see supported) may run with its gradients on the kernels: see trainable()."""
+    convs = mlp_convs(blk)
+    return convs is not None and trainable(x, block_params(blk), *convs, blk.outer_skip)
+
+
 def train(blk, x):
-    """The block with autograd (supported() holds and a gradient is being recorded)."""
+    """The block with autograd (supported() and train_asked() hold)."""
     return _BlockFn.apply(x, blk, *block_params(blk))

@@ -106,8 +106,8 @@ class EncoderDecoder(nn.Module):
     def forward(self, x, fused=True):
         # training under bf16: convolution, GELU and convolution with the GELU in the convolutions' epilogues, both ways (fused = False:
         # the modules, as the network's fused_pointwise asks for)
-        if fused and len(self.fwd) == 3 and pw.trainable_active(x) and _is_conv1x1(self.fwd[0]) and _is_gelu(self.fwd[1]) and _is_conv1x1(self.fwd[2]) \
-                and native_block.plain_conv(self.fwd[0]) and native_block.plain_conv(self.fwd[2]) and native_block._no_hooks(self.fwd, *self.fwd):
+        if fused and len(self.fwd) == 3 and _is_conv1x1(self.fwd[0]) and _is_gelu(self.fwd[1]) and _is_conv1x1(self.fwd[2]) \
+                and native_block.trainable(x, self.parameters(), self.fwd[0], self.fwd[2]) and native_block._no_hooks(self.fwd, *self.fwd):
             y = pw.conv_gelu_conv_trainable(x, self.fwd[0], self.fwd[2])
             if y is not None:
                 return y
@@ -234,7 +234,7 @@ class FourierNeuralOperatorBlock(nn.Module):
         if getattr(self, "fused_pointwise", True) and x.is_cuda and x.dtype == torch.bfloat16:
             # the whole block as one native call, with its gradients while they are recorded
             if torch.is_grad_enabled():
-                if pw.trainable_active(x) and self._fusable() and native_block.supported(self, x):
+                if self._fusable() and native_block.train_asked(self, x) and native_block.supported(self, x):
                     return native_block.train(self, x)
             elif not self.training and fused_pointwise_active(x) and self._fusable() and native_block.supported(self, x):
                 return native_block.forward(self, x, defer_skip=defer_skip)

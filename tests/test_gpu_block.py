@@ -274,3 +274,45 @@ def test_switch_reaches_encoder_and_decoder_in_training(lib_built, at_constructi
                 b.fused_pointwise = False
         net(x).float().square().sum().backward()
     assert not calls and all(p.grad is not None for p in net.parameters())
+
+
+def test_kernels_train_only_what_asks_for_a_gradient(lib_built, monkeypatch):
+    """With gradients enabled but asked for by nothing, the modules run (as they do for each convolution by itself)."""
+    import makani_amd as ma
+    from makani_amd import block as nb, pointwise as pw
+    from makani_amd.sfnonet import EncoderDecoder
+
+    calls = []
+    for fn in (pw._ConvGeluConv, nb._BlockFn):
+        monkeypatch.setattr(fn, "apply", lambda *a, f=fn, keep=fn.apply: calls.append(f) or keep(*a))
+    torch.manual_seed(11)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk, enc = make_block(sht, isht, 16, 2.0).requires_grad_(False), EncoderDecoder(1, 16, 16, 16, nn.GELU).cuda().requires_grad_(False)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    for mod in (blk, enc):
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = mod(x)
+            assert not calls and not y.requires_grad
+            mod(x.clone().requires_grad_()).float().sum().backward()
+            assert len(calls) == 1
+            next(mod.parameters()).requires_grad_()
+            mod(x).float().sum().backward()
+            assert len(calls) == 2
+        calls.clear()
+
+
+def test_library_convolutions_keep_their_second_derivative(lib_built):
+    """nn.Conv2d in the place of the package's convolution trains on the library's kernels and can be differentiated twice."""
+    from makani_amd.sfnonet import EncoderDecoder
+
+    torch.manual_seed(12)
+    enc = EncoderDecoder(1, 6, 5, 8, nn.GELU).cuda()
+    for i in (0, 2):
+        conv = nn.Conv2d(*enc.fwd[i].weight.shape[1::-1], 1, bias=enc.fwd[i].bias is not None).cuda()
+        conv.load_state_dict(enc.fwd[i].state_dict())
+        enc.fwd[i] = conv
+    x = torch.randn(1, 6, 8, 16, device="cuda", requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        (g,) = torch.autograd.grad(enc(x).float().square().sum(), x, create_graph=True)
+    g.square().sum().backward()
+    assert all(p.grad is not None and torch.isfinite(p.grad).all() for p in enc.parameters())
