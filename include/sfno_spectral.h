@@ -388,13 +388,15 @@ size_t sfno_block_workspace_bytes(const sfno_block* b, int backward);
 int sfno_block_forward(const sfno_block* b, int training, const void* x, void* out, void* kept, size_t kept_bytes, void* workspace,
                        size_t workspace_bytes, void* stream);
 /* gradients of a training forward: g = d/d out -> gx (bf16, as x), gfilter complex64 [c_in][embed][lmax], float32 gradients of the
- * MLP's and the skip's matrices, the biases and the norms' parameters; any of them may be null. */
+ * MLP's and the skip's matrices, the biases and the norms' parameters; any of them may be null (a matrix whose bias is asked for
+ * may not).  `kept` is the buffer of a call with training = 1: kept_bytes below that layout is SFNO_EWORKSPACE.  Adjoint plans or
+ * weights that are not those of the block's own are SFNO_EINVAL; nothing is enqueued then. */
 typedef struct {
     void *gx, *gfilter;
     float *gw1, *gb1, *gw2, *gb2, *gwskip, *ggamma0, *gbeta0, *ggamma1, *gbeta1;
 } sfno_block_grads;
-int sfno_block_backward(const sfno_block* b, const void* g, const void* x, const void* kept, const sfno_block_grads* grads, void* workspace,
-                        size_t workspace_bytes, void* stream);
+int sfno_block_backward(const sfno_block* b, const void* g, const void* x, const void* kept, size_t kept_bytes, const sfno_block_grads* grads,
+                        void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

@@ -110,7 +110,6 @@ struct BwdWs {
 
 int conv(const bf16* x, const void* w, const float* bias, bf16* y, int B, int K, int O, int64_t P, int act, const bf16* addend, const float* scale,
          const float* shift, bf16* z, int grad, hipStream_t s) {
-    if (!w) return SFNO_EINVAL;
     PointwiseArgs a;
     std::memset(&a, 0, sizeof(a));
     a.X = x;
@@ -128,7 +127,6 @@ int conv(const bf16* x, const void* w, const float* bias, bf16* y, int B, int K,
 
 // channel mix; row slots between the channels and ld are padding and become zeros (the transform reads whole rows)
 int mix(const sfno_dhconv_weights* w, const float* in, float* out, const Dims& d, int64_t rows_out, hipStream_t s) {
-    if (!w) return SFNO_EINVAL;
     const int64_t ld = sfno_spectral_ld(rows_out);
     if (ld != 2 * rows_out) {
         const int rc = spectral_zero_padding_launch(out, rows_out, (int64_t)d.mmax * d.lmax, (int)ld, s);
@@ -141,6 +139,14 @@ int mix(const sfno_dhconv_weights* w, const float* in, float* out, const Dims& d
 template <class... T>
 bool aligned(const T*... p) {
     return ((reinterpret_cast<uintptr_t>(p) | ...) & 15) == 0;
+}
+
+bool weights_fit(const sfno_dhconv_weights* w, int in, int out, int lmax) { return w && w->I == in && w->O == out && w->L == lmax; }
+
+// adj holds the adjoint of p in the given direction
+bool adjoint_of(const sfno_sht_plan* adj, const sfno_sht_plan* p, int direction) {
+    return adj && (adj->directions & direction) && adj->nlat == p->nlat && adj->nlon == p->nlon && adj->lmax == p->lmax && adj->mmax == p->mmax &&
+           adj->grid == p->grid && adj->norm == p->norm && adj->csphase == p->csphase && adj->device == p->device;
 }
 
 bool bf16_io(const sfno_sht_plan* p) { return sfno_sht_io_dtype_supported(p, SFNO_DTYPE_BF16) && sfno_sht_lat_stats_supported(p); }
@@ -169,6 +175,7 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
     const Dims d(b);
     if (!d.valid || !x || !kept || !workspace || !aligned(x, out, kept, workspace)) return SFNO_EINVAL;
     if (!(b->fwd->directions & SFNO_DIR_FORWARD) || !(b->inv->directions & SFNO_DIR_INVERSE)) return SFNO_EINVAL;
+    if (!weights_fit(b->weights, d.ci, d.e, d.lmax) || !b->w1 || !b->w2 || (out && !b->wskip)) return SFNO_EINVAL;
     if (!bf16_io(b->fwd) || !bf16_io(b->inv)) return SFNO_EUNSUPPORTED;
     int64_t off[SFNO_BLOCK_TENSORS];
     if (kept_bytes < layout(d, training != 0, off)) return SFNO_EWORKSPACE;
@@ -208,13 +215,16 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
     return conv(res, b->wskip, nullptr, reinterpret_cast<bf16*>(out), d.B, d.ci, d.e, d.P, SFNO_ACT_NONE, y2, c1, c1 + d.rows, nullptr, 0, s);
 }
 
-extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const void* x, const void* kept, const sfno_block_grads* grads, void* workspace,
-                                   size_t workspace_bytes, void* stream) {
+extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const void* x, const void* kept, size_t kept_bytes, const sfno_block_grads* grads,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
     const Dims d(b);
     if (!d.valid || !gv || !x || !kept || !grads || !workspace || !aligned(gv, x, kept, grads->gx, workspace)) return SFNO_EINVAL;
-    if (!b->fwd_adj || !b->inv_adj) return SFNO_EINVAL;
+    if (!adjoint_of(b->fwd_adj, b->fwd, SFNO_DIR_FORWARD_ADJOINT) || !adjoint_of(b->inv_adj, b->inv, SFNO_DIR_INVERSE_ADJOINT)) return SFNO_EINVAL;
+    const bool need_in = grads->gx || grads->gfilter, need_h0 = need_in || grads->ggamma0 || grads->gbeta0;
+    if (!b->w2t || (need_h0 && !b->w1t) || (grads->gb1 && !grads->gw1) || (grads->gb2 && !grads->gw2)) return SFNO_EINVAL;
+    if (grads->gx && (!b->wskipt || !weights_fit(b->weights_adj, d.e, d.ci, d.lmax))) return SFNO_EINVAL;
     int64_t off[SFNO_BLOCK_TENSORS];
-    (void)layout(d, true, off);
+    if (kept_bytes < layout(d, true, off)) return SFNO_EWORKSPACE;     // (the buffer of an inference call is smaller)
     const BwdWs w(d, workspace);
     if (workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
     hipStream_t s = (hipStream_t)stream;
@@ -225,23 +235,16 @@ extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const vo
     const float *c0 = (const float*)(k + off[SFNO_BLOCK_COEF0]), *c1 = (const float*)(k + off[SFNO_BLOCK_COEF1]);
     const bf16* res = d.scale_residual ? (const bf16*)(k + off[SFNO_BLOCK_RES]) : reinterpret_cast<const bf16*>(x);
     const bf16* g = reinterpret_cast<const bf16*>(gv);
-    const bool need_in = grads->gx || grads->gfilter;
 
     if (grads->gwskip) TRY(pointwise_wgrad_launch(g, res, grads->gwskip, nullptr, d.B, d.ci, d.e, d.P, w.wgrad, w.wgrad_bytes, s));
     // norm1, W2
     TRY(norm_grad_launch(g, y2, c1, c1 + d.rows, reinterpret_cast<const float2*>(c1 + 2 * d.rows), w.partial, w.dy2, grads->ggamma1, grads->gbeta1, d.B, d.e, d.P,
                          SFNO_ACT_NONE, s));
-    if (grads->gw2 || grads->gb2) {
-        if (!grads->gw2) return SFNO_EINVAL;
-        TRY(pointwise_wgrad_launch(w.dy2, a1, grads->gw2, grads->gb2, d.B, d.h, d.e, d.P, w.wgrad, w.wgrad_bytes, s));
-    }
+    if (grads->gw2) TRY(pointwise_wgrad_launch(w.dy2, a1, grads->gw2, grads->gb2, d.B, d.h, d.e, d.P, w.wgrad, w.wgrad_bytes, s));
     // GELU, W1
     TRY(conv(w.dy2, b->w2t, nullptr, w.dz1, d.B, d.e, d.h, d.P, SFNO_ACT_NONE, z1, nullptr, nullptr, nullptr, 1, s));
-    if (grads->gw1 || grads->gb1) {
-        if (!grads->gw1) return SFNO_EINVAL;
-        TRY(pointwise_wgrad_launch(w.dz1, h0, grads->gw1, grads->gb1, d.B, d.e, d.h, d.P, w.wgrad, w.wgrad_bytes, s));
-    }
-    if (!need_in && !grads->ggamma0 && !grads->gbeta0) return SFNO_OK;
+    if (grads->gw1) TRY(pointwise_wgrad_launch(w.dz1, h0, grads->gw1, grads->gb1, d.B, d.e, d.h, d.P, w.wgrad, w.wgrad_bytes, s));
+    if (!need_h0) return SFNO_OK;
     TRY(conv(w.dz1, b->w1t, nullptr, w.dh0, d.B, d.h, d.e, d.P, SFNO_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0, s));
     // GELU, norm0
     TRY(norm_grad_launch(w.dh0, xf, c0, c0 + d.rows, reinterpret_cast<const float2*>(c0 + 2 * d.rows), w.partial, w.dx, grads->ggamma0, grads->gbeta0, d.B, d.e, d.P,

@@ -100,7 +100,7 @@ def _load():
         "sfno_block_layout": (sz, [vp, i32, vp]),
         "sfno_block_workspace_bytes": (sz, [vp, i32]),
         "sfno_block_forward": (i32, [vp, i32, vp, vp, vp, sz, vp, sz, vp]),
-        "sfno_block_backward": (i32, [vp, vp, vp, vp, vp, vp, sz, vp]),
+        "sfno_block_backward": (i32, [vp, vp, vp, vp, sz, vp, vp, sz, vp]),
         "sfno_pointwise_conv_cat": (i32, [vp, i32, vp, i32, vp, vp, vp, i32, i32, i64, i32, vp]),
         "sfno_pointwise_weight_grad_workspace_bytes": (sz, [i32, i32, i32, i64, i32]),
         "sfno_pointwise_weight_grad": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, vp, sz, vp]),

@@ -181,7 +181,7 @@ class _BlockFn(torch.autograd.Function):
         ref = ctypes.byref(c.b)
         nws = lib.sfno_block_workspace_bytes(ref, 1)
         ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
-        check(lib.sfno_block_backward(ref, g.data_ptr(), x.data_ptr(), kept.data_ptr(), ctypes.byref(s), ws.data_ptr(), nws, c.stream), "sfno_block_backward")
+        check(lib.sfno_block_backward(ref, g.data_ptr(), x.data_ptr(), kept.data_ptr(), kept.numel(), ctypes.byref(s), ws.data_ptr(), nws, c.stream), "sfno_block_backward")
         return (gx, None, *(t if n else None for t, n in zip(grads, need[2:])))
 
 

@@ -316,3 +316,50 @@ def test_library_convolutions_keep_their_second_derivative(lib_built):
         (g,) = torch.autograd.grad(enc(x).float().square().sum(), x, create_graph=True)
     g.square().sum().backward()
     assert all(p.grad is not None and torch.isfinite(p.grad).all() for p in enc.parameters())
+
+
+def test_backward_refuses_foreign_buffers_plans_and_weights(lib_built):
+    """The C entry points check what they address by the block's sizes before anything is enqueued."""
+    import ctypes
+
+    import makani_amd as ma
+    from makani_amd import _lib, block as nb
+    from makani_amd._lib import lib
+    from makani_amd.contractions import packed_for
+
+    torch.manual_seed(13)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    out, gx = torch.empty_like(x), torch.empty_like(x)
+    EINVAL, EWORKSPACE = -1, -4
+    c = nb._Call(blk, x, nb.block_params(blk), backward=True)
+    kept = c.forward(x, 1, out)
+    grads = _lib.BlockGrads(gx=gx.data_ptr())
+    ref = ctypes.byref(c.b)
+    nws = lib.sfno_block_workspace_bytes(ref, 1)
+    ws = torch.empty(max(nws, lib.sfno_block_workspace_bytes(ref, 0)), dtype=torch.uint8, device="cuda")
+
+    def backward(kept_bytes):
+        return lib.sfno_block_backward(ref, x.data_ptr(), x.data_ptr(), kept.data_ptr(), kept_bytes, ctypes.byref(grads), ws.data_ptr(), nws, c.stream)
+
+    assert backward(kept.numel()) == 0
+    assert backward(kept.numel() - 1) == EWORKSPACE
+    small = lib.sfno_block_layout(ref, 0, c.offsets)
+    assert small < kept.numel() and backward(small) == EWORKSPACE
+    other = ma.RealSHT(24, 48, grid="legendre-gauss").plan(x.device, adjoint=True), ma.InverseRealSHT(24, 48, grid="legendre-gauss").plan(x.device, adjoint=True)
+    weight = torch.randn(16, 8, 16, dtype=torch.complex64, device="cuda")
+    for field, value in (("fwd_adj", other[0].handle), ("inv_adj", other[1].handle), ("fwd_adj", c.keep[0].handle), ("inv_adj", None),
+                         ("weights_adj", packed_for(weight, adjoint=True).handle), ("weights_adj", None), ("w2t", None), ("wskipt", None)):
+        keep = getattr(c.b, field)
+        setattr(c.b, field, value)
+        assert backward(kept.numel()) == EINVAL, field
+        setattr(c.b, field, keep)
+    bias = torch.empty(32, device="cuda")
+    grads.gb1 = bias.data_ptr()                # a bias without its matrix
+    assert backward(kept.numel()) == EINVAL
+    keep = c.b.weights
+    c.b.weights = packed_for(weight).handle
+    assert lib.sfno_block_forward(ref, 1, x.data_ptr(), out.data_ptr(), kept.data_ptr(), kept.numel(), ws.data_ptr(), ws.numel(), c.stream) == EINVAL
+    c.b.weights = keep
+    torch.cuda.synchronize()
