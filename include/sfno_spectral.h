@@ -318,7 +318,8 @@ int sfno_pointwise_weight_grad(const void* gy, const void* x, float* gweight, fl
 /* The two convolutions a GELU needs in training: forward with the pre-activation kept,
  *   z = sum_k w[o][k] x[b][k][p] + bias[o],   y = gelu(z)     (z rounded to bf16 first, both bf16 [B][O][P])
  * and the input gradient of the convolution behind the GELU, times the GELU's derivative,
- *   gz = gelu'(z) * sum_k wt[o][k] gy[b][k][p]                (wt: the transposed weight of that convolution, packed). */
+ *   gz = gelu'(z) * sum_k wt[o][k] gy[b][k][p]                (wt: the transposed weight of that convolution, packed).
+ * Tensors are 16-byte aligned (SFNO_EINVAL otherwise). */
 int sfno_pointwise_conv_gelu(const void* x, const void* w, const float* bias, void* y, void* z, int batch, int K, int O,
                              int64_t P, void* stream);
 int sfno_pointwise_conv_gelu_grad(const void* gy, const void* wt, const void* z, void* gz, int batch, int K, int O,

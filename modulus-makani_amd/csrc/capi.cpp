@@ -660,9 +660,14 @@ extern "C" int sfno_pointwise_pack_weight_transposed(const float* w, void* packe
     return pointwise_pack_launch(w, reinterpret_cast<unsigned short*>(packed), O, K, 1, (hipStream_t)stream);
 }
 
+// 16-byte loads of eight bf16 values
+static bool on16(const void* a, const void* b, const void* c, const void* d) {
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(d)) & 15) == 0;
+}
+
 extern "C" int sfno_pointwise_conv_gelu(const void* x, const void* w, const float* bias, void* y, void* z, int batch, int K, int O, int64_t P,
                                         void* stream) {
-    if (!x || !w || !y || !z || batch < 1 || K < 1 || O < 1 || P < 1) return SFNO_EINVAL;
+    if (!x || !w || !y || !z || batch < 1 || K < 1 || O < 1 || P < 1 || !on16(x, w, y, z)) return SFNO_EINVAL;
     PointwiseArgs a;
     std::memset(&a, 0, sizeof(a));
     a.X = reinterpret_cast<const unsigned short*>(x);
@@ -675,7 +680,7 @@ extern "C" int sfno_pointwise_conv_gelu(const void* x, const void* w, const floa
 }
 
 extern "C" int sfno_pointwise_conv_gelu_grad(const void* gy, const void* wt, const void* z, void* gz, int batch, int K, int O, int64_t P, void* stream) {
-    if (!gy || !wt || !z || !gz || batch < 1 || K < 1 || O < 1 || P < 1) return SFNO_EINVAL;
+    if (!gy || !wt || !z || !gz || batch < 1 || K < 1 || O < 1 || P < 1 || !on16(gy, wt, z, gz)) return SFNO_EINVAL;
     PointwiseArgs a;
     std::memset(&a, 0, sizeof(a));
     a.X = reinterpret_cast<const unsigned short*>(gy);
@@ -728,8 +733,7 @@ extern "C" size_t sfno_pointwise_weight_grad_workspace_bytes(int batch, int K, i
 extern "C" int sfno_pointwise_weight_grad(const void* gy, const void* x, float* gweight, float* gbias, int batch, int K, int O, int64_t P,
                                           void* workspace, size_t workspace_bytes, void* stream) {
     if (!gy || !x || !gweight || !workspace || batch < 1 || K < 1 || O < 1 || P < 8 || P % 8) return SFNO_EINVAL;
-    // 16-byte loads of eight bf16 values
-    if ((reinterpret_cast<uintptr_t>(gy) | reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(workspace)) & 15) return SFNO_EINVAL;
+    if (!on16(gy, x, workspace, nullptr)) return SFNO_EINVAL;
     return pointwise_wgrad_launch(reinterpret_cast<const unsigned short*>(gy), reinterpret_cast<const unsigned short*>(x), gweight, gbias, batch, K, O, P,
                                   reinterpret_cast<float*>(workspace), workspace_bytes, (hipStream_t)stream);
 }

@@ -166,9 +166,7 @@ class _BlockFn(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, g):
         x, kept, *params = ctx.saved_tensors
-        g = g.to(torch.bfloat16).contiguous()
-        if g.data_ptr() % 16 != 0:
-            g = g.clone()
+        g = pw._dense(g.to(torch.bfloat16))
         blk, need = ctx.blk, ctx.needs_input_grad
         c = _Call(blk, x, params, backward=True)
         want = [p is not None and n for p, n in zip(params, need[2:])]

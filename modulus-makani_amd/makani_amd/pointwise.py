@@ -63,6 +63,12 @@ def supported(x):
     return x.is_cuda and x.dim() == 4 and x.dtype == torch.bfloat16 and (x.shape[2] * x.shape[3]) % 8 == 0 and x.shape[2] * x.shape[3] >= 8
 
 
+def _dense(x):
+    """x contiguous and on a 16-byte boundary, as the kernels load it; a view into the middle of a buffer is copied."""
+    x = x.contiguous()
+    return x if x.data_ptr() % 16 == 0 else x.clone()
+
+
 def conv1x1(x, weight, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
     """act(conv1x1(x, weight) + bias) + add_scale * addend + add_shift  ->  bf16 [B, O, H, W]."""
     return _conv1x1(x, weight, False, bias, act, addend, add_scale, add_shift)
@@ -72,7 +78,7 @@ def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=
     O, K_weight = (weight.shape[1], weight.shape[0]) if transposed else weight.shape[:2]
     if not supported(x):
         raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
-    x = x.contiguous()
+    x = _dense(x)
     B, K, H, W = x.shape
     if K_weight != K:
         raise RuntimeError(f"conv1x1: input has {K} channels, weight expects {K_weight}")
@@ -83,7 +89,7 @@ def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=
     if addend is not None:
         if addend.shape != y.shape or addend.dtype != torch.bfloat16:
             raise RuntimeError("conv1x1: addend must be a bfloat16 tensor of the output's shape")
-        addend = addend.contiguous()
+        addend = _dense(addend)
         if add_scale is not None:
             add_scale = add_scale.float().contiguous()
             add_shift = add_shift.float().contiguous()
@@ -101,7 +107,7 @@ def conv1x1_cat(x1, x2, weight, bias=None, act=None, out=None):
     weight [O, K1 + K2] (or [O, K1 + K2, 1, 1]); out: a contiguous bf16 tensor of the result's shape to write into."""
     if not (supported(x1) and supported(x2)) or x1.shape[0] != x2.shape[0] or x1.shape[2:] != x2.shape[2:]:
         raise RuntimeError("conv1x1_cat takes two contiguous bfloat16 NCHW HIP tensors of one batch and grid size, H*W a multiple of 8")
-    x1, x2 = x1.contiguous(), x2.contiguous()
+    x1, x2 = _dense(x1), _dense(x2)
     B, K1, H, W = x1.shape
     K2 = x2.shape[1]
     O = weight.shape[0]
@@ -125,7 +131,7 @@ def instance_norm_coeffs(x, gamma=None, beta=None, eps=1e-5):
     """(scale, shift) float32 [B, C] such that instance_norm(x) = scale * x + shift."""
     if not supported(x):
         raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
-    x = x.contiguous()
+    x = _dense(x)
     B, C, H, W = x.shape
     rows, P = B * C, H * W
     scale = torch.empty((B, C), dtype=torch.float32, device=x.device)
@@ -162,7 +168,7 @@ def scale_shift_act(x, scale, shift, act=None):
     """act(scale[b, c] * x + shift[b, c]) -> bf16, same shape."""
     if not supported(x):
         raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
-    x = x.contiguous()
+    x = _dense(x)
     B, C, H, W = x.shape
     y = torch.empty_like(x)
     check(lib.sfno_scale_shift_act(_ptr(x), _ptr(scale), _ptr(shift), _ptr(y), B * C, H * W, ACT[act], _stream(x.device)), "sfno_scale_shift_act")
@@ -174,7 +180,7 @@ def conv1x1_weight_grad(gy, x, with_bias):
     gweight[o, k] = sum_{b,p} gy[b, o, p] x[b, k, p], gbias[o] = sum_{b,p} gy[b, o, p]; bf16 operands, fp32 sums in a fixed order."""
     if not (supported(x) and supported(gy)) or gy.shape[0] != x.shape[0] or gy.shape[2:] != x.shape[2:]:
         raise RuntimeError("conv1x1_weight_grad takes two contiguous bfloat16 NCHW HIP tensors of one batch and grid size, H*W a multiple of 8")
-    x, gy = x.contiguous(), gy.contiguous()
+    x, gy = _dense(x), _dense(gy)
     B, K, H, W = x.shape
     O = gy.shape[1]
     gw = torch.empty((O, K), dtype=torch.float32, device=x.device)
@@ -192,7 +198,7 @@ class _Conv1x1(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias):
-        xb = x.detach().to(torch.bfloat16).contiguous()
+        xb = _dense(x.detach().to(torch.bfloat16))
         ctx.save_for_backward(xb, weight)
         ctx.has_bias = bias is not None
         ctx.x_dtype = x.dtype
@@ -204,7 +210,7 @@ class _Conv1x1(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, gy):
         xb, weight = ctx.saved_tensors
-        gy = gy.to(torch.bfloat16).contiguous()
+        gy = _dense(gy.to(torch.bfloat16))
         gx = gw = gb = None
         if ctx.needs_input_grad[0]:
             gx = _conv1x1(gy, weight, True).to(ctx.x_dtype)
@@ -223,7 +229,7 @@ class _ConvGeluConv(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, w1, b1, w2, b2):
-        xb = x.detach().to(torch.bfloat16).contiguous()
+        xb = _dense(x.detach().to(torch.bfloat16))
         B, K, H, W = xb.shape
         O = w1.shape[0]
         if w1.shape[1] != K or w2.shape[1] != O:
@@ -242,7 +248,7 @@ class _ConvGeluConv(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, gy):
         xb, z, a, w1, w2 = ctx.saved_tensors
-        gy = gy.to(torch.bfloat16).contiguous()
+        gy = _dense(gy.to(torch.bfloat16))
         need = ctx.needs_input_grad
         gx = gw1 = gb1 = gw2 = gb2 = None
         if need[3] or need[4]:

@@ -190,3 +190,17 @@ def test_pointwise_weight_grad_workspace_and_argument_checks(lib_built):
     assert f(ok, ok, ok, None, 1, 8, 8, 12, ok, 4096, None) != 0
     assert f(ctypes.c_void_p(base + 2), ok, ok, None, 1, 8, 8, 64, ok, 4096, None) != 0
     assert f(ok, ok, ok, None, 1, 8, 8, 64, ctypes.c_void_p(base + 4), 4096, None) != 0
+
+
+def test_training_convolutions_refuse_misaligned_tensors(lib_built):
+    """The 16-byte loads of sfno_pointwise_conv_gelu and its backward: refused on the host, whichever tensor it is."""
+    import ctypes
+
+    from makani_amd._lib import lib
+
+    buf = ctypes.create_string_buffer(4096 + 64)
+    base = (ctypes.addressof(buf) + 63) & ~63
+    for bad in range(4):
+        x, w, y, z = (ctypes.c_void_p(base + (2 if i == bad else 0)) for i in range(4))
+        assert lib.sfno_pointwise_conv_gelu(x, w, None, y, z, 1, 8, 8, 64, None) == -1
+        assert lib.sfno_pointwise_conv_gelu_grad(x, w, z, y, 1, 8, 8, 64, None) == -1

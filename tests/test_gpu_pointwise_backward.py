@@ -233,3 +233,33 @@ def test_training_gelu_and_its_derivative_on_every_bf16_value(lib_built, channel
     assert int(((got != want.to(torch.bfloat16).double()) & (xd.abs() >= 2 ** -6)).sum()) < 5
     want = Phi + xd * pdf
     assert bool(((gx.double().cpu() - want).abs() <= want.abs() * 2 ** -8 + 3e-7).all())
+
+
+def test_views_between_16_byte_boundaries(lib_built):
+    """Tensors that start in the middle of a buffer give the results of their copies, in every function that takes activations."""
+    import torch.nn as nn
+
+    from makani_amd import pointwise as pw
+    from makani_amd.sfnonet import EncoderDecoder
+
+    print("case offsets", flush=True)
+    torch.manual_seed(3)
+
+    def offset(t):
+        return torch.cat([t.new_zeros(3), t.flatten()])[3:].view(t.shape)
+
+    x, r = (torch.randn(2, 12, 8, 16, device="cuda").bfloat16() for _ in range(2))
+    w, sc, sh = torch.randn(12, 12, device="cuda"), torch.randn(2, 12, device="cuda"), torch.randn(2, 12, device="cuda")
+    wcat = torch.randn(100, 24, device="cuda")
+    calls = [lambda x, r: pw.conv1x1(x, w, None, "gelu", r, sc, sh), lambda x, r: pw.conv1x1_cat(x, r, wcat), lambda x, r: torch.stack(pw.instance_norm_coeffs(x)),
+             lambda x, r: pw.scale_shift_act(x, sc, sh, "gelu"), lambda x, r: pw.conv1x1_weight_grad(r, x, True)[0]]
+    for i, f in enumerate(calls):
+        assert torch.equal(f(offset(x), offset(r)), f(x, r)), i
+    for mod in (EncoderDecoder(1, 12, 12, 20, nn.GELU).cuda(), pw.PointwiseConv2d(12, 12).cuda()):
+        got = []
+        for view in (offset, torch.clone):
+            xi = view(x).requires_grad_()
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                y = mod(xi)
+            got.append((y, *torch.autograd.grad(y, (xi, *mod.parameters()), view(r))))
+        assert all(torch.equal(a, b) for a, b in zip(*got))
