@@ -373,10 +373,10 @@ typedef struct {
 /* tensors of a forward call inside one buffer `kept` (byte offsets; -1: not there) */
 #define SFNO_BLOCK_SPEC 0     /* spectral-layout coefficients of x (training) */
 #define SFNO_BLOCK_X 1        /* bf16 [B][embed][P] filter output (training) */
-#define SFNO_BLOCK_COEF0 2    /* float32 [4][B*embed]: scale, shift of norm0, then its (mean, 1/std) pairs */
+#define SFNO_BLOCK_COEF0 2    /* float32 [4][B*embed]: scale, shift of norm0, then its (mean, 1/std) pairs (training) */
 #define SFNO_BLOCK_H0 3       /* bf16 [B][embed][P] */
 #define SFNO_BLOCK_Z1 4       /* bf16 [B][hidden][P] W1 h0 + b1 (training) */
-#define SFNO_BLOCK_A1 5       /* bf16 [B][hidden][P] its GELU */
+#define SFNO_BLOCK_A1 5       /* bf16 [B][hidden][P] its GELU (training) */
 #define SFNO_BLOCK_Y2 6       /* bf16 [B][embed][P] */
 #define SFNO_BLOCK_COEF1 7    /* float32 [4][B*embed]: as COEF0, of norm1 */
 #define SFNO_BLOCK_RES 8      /* bf16 [B][c_in][P] the residual, where it passes through the transforms */

@@ -33,7 +33,7 @@ struct Arena {
 struct Dims {
     int B, ci, e, h, lmax, mmax, tri;
     int64_t P, Pin, rows_in, rows;            // pixels of the output and input grid; B * c_in, B * embed
-    int64_t spec_in, spec_out, xm;            // floats
+    int64_t spec_in, spec_out, xm_in, xm_out; // floats
     bool scale_residual;
     bool valid = false;
     explicit Dims(const sfno_block* b) {
@@ -50,8 +50,8 @@ struct Dims {
         scale_residual = f.nlat != i.nlat || f.nlon != i.nlon || f.grid != i.grid;
         spec_in = (int64_t)mmax * lmax * sfno_spectral_ld(rows_in);
         spec_out = (int64_t)mmax * lmax * sfno_spectral_ld(rows);
-        const int64_t nlat = std::max(f.nlat, i.nlat);
-        xm = mmax * nlat * sfno_spectral_ld(std::max(rows_in, rows));
+        xm_in = (int64_t)mmax * f.nlat * sfno_spectral_ld(rows_in);
+        xm_out = (int64_t)mmax * i.nlat * sfno_spectral_ld(std::max(rows_in, rows));
         valid = true;
     }
 };
@@ -59,52 +59,71 @@ struct Dims {
 size_t layout(const Dims& d, bool training, int64_t off[SFNO_BLOCK_TENSORS]) {
     Arena a(nullptr);
     const size_t act = sizeof(bf16) * (size_t)d.rows * d.P, hid = sizeof(bf16) * (size_t)d.B * d.h * d.P;
-    off[SFNO_BLOCK_SPEC] = a.take(sizeof(float) * (size_t)d.spec_in);
-    off[SFNO_BLOCK_X] = a.take(act);
-    off[SFNO_BLOCK_COEF0] = a.take(sizeof(float) * 4 * (size_t)d.rows);
+    // inference: the coefficients are spent (residual and channel mix) when the filter's output is stored
+    off[SFNO_BLOCK_SPEC] = a.take(std::max(sizeof(float) * (size_t)d.spec_in, training ? 0 : act));
+    off[SFNO_BLOCK_X] = training ? a.take(act) : off[SFNO_BLOCK_SPEC];
+    off[SFNO_BLOCK_COEF0] = training ? a.take(sizeof(float) * 4 * (size_t)d.rows) : -1;
     off[SFNO_BLOCK_H0] = training ? a.take(act) : off[SFNO_BLOCK_X];       // inference: norm0 and the GELU in place, the MLP's output over them
     off[SFNO_BLOCK_Z1] = training ? a.take(hid) : -1;
-    off[SFNO_BLOCK_A1] = a.take(hid);
+    off[SFNO_BLOCK_A1] = training ? a.take(hid) : -1;                      // inference: in the workspace, over the filter's buffers
     off[SFNO_BLOCK_Y2] = training ? a.take(act) : off[SFNO_BLOCK_X];
     off[SFNO_BLOCK_COEF1] = a.take(sizeof(float) * 4 * (size_t)d.rows);
     off[SFNO_BLOCK_RES] = d.scale_residual ? a.take(sizeof(bf16) * (size_t)d.rows_in * d.P) : -1;
     return a.off;
 }
 
+// The buffers of a pass are laid over each other as far as their lifetimes allow.  Beside its state a training step of the full-size
+// network with 4 layers then needs 14.0 GiB and a rollout of four samples with 8 layers 12.8; with buffers side by side 15.2 and 16.4.
 struct FwdWs {
-    float *xm, *spec;
+    float *xm_in, *xm_out, *spec, *coef0;
     float2 *stats, *partial;
+    bf16* a1;
     size_t bytes;
     FwdWs(const sfno_block* b, const Dims& d, void* base) {
         Arena a(base);
-        xm = a.get<float>(d.xm);
-        spec = a.get<float>(d.spec_out);
-        stats = a.get<float2>((size_t)d.rows * b->inv->nlat);
+        coef0 = a.get<float>(4 * (size_t)d.rows);
         partial = a.get<float2>((size_t)d.rows * row_stats_segments(d.rows, d.P));
-        bytes = a.off;
+        Arena first = a, filter = a;
+        xm_in = first.get<float>(d.xm_in);              // until the analysis
+        spec = filter.get<float>(d.spec_out);           // from the channel mix until the synthesis
+        xm_out = filter.get<float>(d.xm_out);
+        stats = filter.get<float2>((size_t)d.rows * b->inv->nlat);
+        a1 = a.get<bf16>((size_t)d.B * d.h * d.P);      // behind the filter
+        bytes = std::max({a.off, first.off, filter.off});
     }
 };
 
 struct BwdWs {
-    float *xm, *gspec_out, *gspec_in, *gspec_res, *wgrad;
+    float *xm_in, *xm_out, *gspec_out, *gspec_in, *gspec_res, *wgrad_a, *wgrad_b;
     bf16 *dy2, *dz1, *dh0, *dx;
     float2* partial;
     size_t bytes, wgrad_bytes;
     BwdWs(const Dims& d, void* base) {
         Arena a(base);
-        xm = a.get<float>(d.xm);
-        gspec_out = a.get<float>(d.spec_out);
-        gspec_in = a.get<float>(d.spec_in);
-        gspec_res = d.scale_residual ? a.get<float>(d.spec_in) : nullptr;
-        dy2 = a.get<bf16>((size_t)d.rows * d.P);
-        dz1 = a.get<bf16>((size_t)d.B * d.h * d.P);
-        dh0 = dy2;                                                        // (dy2 is spent once dz1 and the gradient of W2 exist)
-        dx = a.get<bf16>((size_t)std::max(d.rows, d.scale_residual ? d.rows_in : 0) * d.P);
         partial = a.get<float2>((size_t)d.rows * row_stats_segments(d.rows, d.P));
         wgrad_bytes = std::max({pointwise_wgrad_workspace_bytes(d.e, d.ci, 0, d.B, d.P), pointwise_wgrad_workspace_bytes(d.e, d.h, 1, d.B, d.P),
                                 pointwise_wgrad_workspace_bytes(d.h, d.e, 1, d.B, d.P)});
-        wgrad = a.get<float>(wgrad_bytes / sizeof(float) + 1);
-        bytes = a.off;
+        // two buffers in turn: dy2 -> dz1 -> dh0 -> dx, the shares of a weight gradient in the one whose tensor is not there yet or
+        // spent; the filter's buffers over what is left of them behind dx, the last transform's over dx too
+        const size_t at = a.off, dx_bytes = sizeof(bf16) * (size_t)std::max(d.rows, d.scale_residual ? d.rows_in : 0) * (size_t)d.P;
+        dz1 = a.get<bf16>(std::max({sizeof(bf16) * (size_t)d.B * d.h * (size_t)d.P, dx_bytes, wgrad_bytes}) / sizeof(bf16));
+        dy2 = a.get<bf16>(std::max(sizeof(bf16) * (size_t)d.rows * (size_t)d.P, wgrad_bytes) / sizeof(bf16));
+        dx = dz1;
+        dh0 = dy2;
+        wgrad_a = reinterpret_cast<float*>(dz1);
+        wgrad_b = reinterpret_cast<float*>(dy2);
+        Arena filter = a;
+        filter.off = at;
+        filter.take(dx_bytes);
+        xm_out = filter.get<float>(d.xm_out);
+        gspec_out = filter.get<float>(std::max(d.spec_out, d.scale_residual ? d.spec_in : 0));
+        gspec_res = gspec_out;                            // (gspec_out is spent once the input's coefficients have their gradient)
+        Arena last = filter;
+        last.off = at;
+        xm_in = last.get<float>(d.xm_in);
+        filter.off = std::max(filter.off, last.off);
+        gspec_in = filter.get<float>(d.spec_in);
+        bytes = std::max(a.off, filter.off);
     }
 };
 
@@ -184,27 +203,27 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
     hipStream_t s = (hipStream_t)stream;
     char* k = reinterpret_cast<char*>(kept);
     float* spec = reinterpret_cast<float*>(k + off[SFNO_BLOCK_SPEC]);
-    bf16 *xf = (bf16*)(k + off[SFNO_BLOCK_X]), *h0 = (bf16*)(k + off[SFNO_BLOCK_H0]), *a1 = (bf16*)(k + off[SFNO_BLOCK_A1]), *y2 = (bf16*)(k + off[SFNO_BLOCK_Y2]);
-    bf16* z1 = training ? (bf16*)(k + off[SFNO_BLOCK_Z1]) : nullptr;
-    float *c0 = (float*)(k + off[SFNO_BLOCK_COEF0]), *c1 = (float*)(k + off[SFNO_BLOCK_COEF1]);
+    bf16 *xf = (bf16*)(k + off[SFNO_BLOCK_X]), *h0 = (bf16*)(k + off[SFNO_BLOCK_H0]), *y2 = (bf16*)(k + off[SFNO_BLOCK_Y2]);
+    bf16 *z1 = training ? (bf16*)(k + off[SFNO_BLOCK_Z1]) : nullptr, *a1 = training ? (bf16*)(k + off[SFNO_BLOCK_A1]) : w.a1;
+    float *c0 = training ? (float*)(k + off[SFNO_BLOCK_COEF0]) : w.coef0, *c1 = (float*)(k + off[SFNO_BLOCK_COEF1]);
     const bf16* res = reinterpret_cast<const bf16*>(x);
 
-    TRY(sfno_rfft(b->fwd, x, SFNO_DTYPE_BF16, w.xm, d.rows_in, s));
-    TRY(sfno_legendre_analysis(b->fwd, w.xm, spec, d.rows_in, s));
+    TRY(sfno_rfft(b->fwd, x, SFNO_DTYPE_BF16, w.xm_in, d.rows_in, s));
+    TRY(sfno_legendre_analysis(b->fwd, w.xm_in, spec, d.rows_in, s));
     if (d.scale_residual) {
         bf16* r = (bf16*)(k + off[SFNO_BLOCK_RES]);
-        TRY(sfno_legendre_synthesis(b->inv, spec, w.xm, d.rows_in, s));
-        TRY(sfno_irfft(b->inv, w.xm, r, SFNO_DTYPE_BF16, d.rows_in, s));
+        TRY(sfno_legendre_synthesis(b->inv, spec, w.xm_out, d.rows_in, s));
+        TRY(sfno_irfft(b->inv, w.xm_out, r, SFNO_DTYPE_BF16, d.rows_in, s));
         res = r;
     }
     TRY(mix(b->weights, spec, w.spec, d, d.rows, s));
-    TRY(sfno_legendre_synthesis(b->inv, w.spec, w.xm, d.rows, s));
+    TRY(sfno_legendre_synthesis(b->inv, w.spec, w.xm_out, d.rows, s));
     float2* m0 = reinterpret_cast<float2*>(c0 + 2 * d.rows);
     if (d.P <= NORM_SMALL_PIXELS) {
-        TRY(sfno_irfft(b->inv, w.xm, xf, SFNO_DTYPE_BF16, d.rows, s));
+        TRY(sfno_irfft(b->inv, w.xm_out, xf, SFNO_DTYPE_BF16, d.rows, s));
         TRY(instance_norm_coeffs_launch(xf, b->gamma0, b->beta0, c0, c0 + d.rows, w.partial, d.rows, d.e, d.P, b->eps0, s, m0));
     } else {
-        TRY(irfft_launch(b->inv->fft, w.xm, xf, SFNO_DTYPE_BF16, d.rows, b->inv->nlat, d.mmax, (int)sfno_spectral_ld(d.rows), s, w.stats));
+        TRY(irfft_launch(b->inv->fft, w.xm_out, xf, SFNO_DTYPE_BF16, d.rows, b->inv->nlat, d.mmax, (int)sfno_spectral_ld(d.rows), s, w.stats));
         TRY(instance_norm_coeffs_lat_launch(w.stats, b->gamma0, b->beta0, c0, c0 + d.rows, d.rows, d.e, b->inv->nlat, b->eps0, s, m0));
     }
     TRY(scale_shift_act_launch(xf, c0, c0 + d.rows, h0, d.rows, d.P, training ? ACT_GELU_TRAIN : SFNO_ACT_GELU, s));
@@ -236,14 +255,14 @@ extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const vo
     const bf16* res = d.scale_residual ? (const bf16*)(k + off[SFNO_BLOCK_RES]) : reinterpret_cast<const bf16*>(x);
     const bf16* g = reinterpret_cast<const bf16*>(gv);
 
-    if (grads->gwskip) TRY(pointwise_wgrad_launch(g, res, grads->gwskip, nullptr, d.B, d.ci, d.e, d.P, w.wgrad, w.wgrad_bytes, s));
+    if (grads->gwskip) TRY(pointwise_wgrad_launch(g, res, grads->gwskip, nullptr, d.B, d.ci, d.e, d.P, w.wgrad_a, w.wgrad_bytes, s));
     // norm1, W2
     TRY(norm_grad_launch(g, y2, c1, c1 + d.rows, reinterpret_cast<const float2*>(c1 + 2 * d.rows), w.partial, w.dy2, grads->ggamma1, grads->gbeta1, d.B, d.e, d.P,
                          SFNO_ACT_NONE, s));
-    if (grads->gw2) TRY(pointwise_wgrad_launch(w.dy2, a1, grads->gw2, grads->gb2, d.B, d.h, d.e, d.P, w.wgrad, w.wgrad_bytes, s));
+    if (grads->gw2) TRY(pointwise_wgrad_launch(w.dy2, a1, grads->gw2, grads->gb2, d.B, d.h, d.e, d.P, w.wgrad_a, w.wgrad_bytes, s));
     // GELU, W1
     TRY(conv(w.dy2, b->w2t, nullptr, w.dz1, d.B, d.e, d.h, d.P, SFNO_ACT_NONE, z1, nullptr, nullptr, nullptr, 1, s));
-    if (grads->gw1) TRY(pointwise_wgrad_launch(w.dz1, h0, grads->gw1, grads->gb1, d.B, d.e, d.h, d.P, w.wgrad, w.wgrad_bytes, s));
+    if (grads->gw1) TRY(pointwise_wgrad_launch(w.dz1, h0, grads->gw1, grads->gb1, d.B, d.e, d.h, d.P, w.wgrad_b, w.wgrad_bytes, s));
     if (!need_h0) return SFNO_OK;
     TRY(conv(w.dz1, b->w1t, nullptr, w.dh0, d.B, d.h, d.e, d.P, SFNO_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0, s));
     // GELU, norm0
@@ -251,7 +270,7 @@ extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const vo
                          SFNO_ACT_GELU, s));
     if (!need_in) return SFNO_OK;
     // filter
-    TRY(synthesis_adjoint_launch(b->inv_adj, w.dx, SFNO_DTYPE_BF16, w.xm, w.gspec_out, d.rows, s));
+    TRY(synthesis_adjoint_launch(b->inv_adj, w.dx, SFNO_DTYPE_BF16, w.xm_out, w.gspec_out, d.rows, s));
     if (grads->gfilter) {
         DhconvWgradArgs a;
         a.X = spec;
@@ -269,11 +288,11 @@ extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const vo
     if (d.scale_residual) {
         // the residual's gradient joins in spectral space
         TRY(conv(g, b->wskipt, nullptr, w.dx, d.B, d.e, d.ci, d.P, SFNO_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0, s));
-        TRY(synthesis_adjoint_launch(b->inv_adj, w.dx, SFNO_DTYPE_BF16, w.xm, w.gspec_res, d.rows_in, s));
+        TRY(synthesis_adjoint_launch(b->inv_adj, w.dx, SFNO_DTYPE_BF16, w.xm_out, w.gspec_res, d.rows_in, s));
         TRY(spectral_add_launch(w.gspec_in, w.gspec_res, d.lmax, d.mmax, (int)sfno_spectral_ld(d.rows_in), d.tri, s));
-        return analysis_adjoint_launch(b->fwd_adj, w.gspec_in, gx, SFNO_DTYPE_BF16, w.xm, d.rows_in, s);
+        return analysis_adjoint_launch(b->fwd_adj, w.gspec_in, gx, SFNO_DTYPE_BF16, w.xm_in, d.rows_in, s);
     }
-    TRY(analysis_adjoint_launch(b->fwd_adj, w.gspec_in, gx, SFNO_DTYPE_BF16, w.xm, d.rows_in, s));
+    TRY(analysis_adjoint_launch(b->fwd_adj, w.gspec_in, gx, SFNO_DTYPE_BF16, w.xm_in, d.rows_in, s));
     // skip gradient on top, in place
     return conv(g, b->wskipt, nullptr, gx, d.B, d.e, d.ci, d.P, SFNO_ACT_NONE, gx, nullptr, nullptr, nullptr, 0, s);
 }

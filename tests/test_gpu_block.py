@@ -363,3 +363,59 @@ def test_backward_refuses_foreign_buffers_plans_and_weights(lib_built):
     assert lib.sfno_block_forward(ref, 1, x.data_ptr(), out.data_ptr(), kept.data_ptr(), kept.numel(), ws.data_ptr(), ws.numel(), c.stream) == EINVAL
     c.b.weights = keep
     torch.cuda.synchronize()
+
+
+def peak_of(call):
+    """Bytes beside what is allocated before and after the call."""
+    call()                                            # packed weights, plans
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    call()
+    torch.cuda.synchronize()
+    return torch.cuda.max_memory_allocated() - base
+
+
+@pytest.mark.parametrize("f,i", [((64, 128), (64, 128)), ((64, 128), (32, 64)), ((32, 64), (64, 128))])
+def test_peak_memory_of_inference_is_no_more_than_layer_by_layer(lib_built, f, i, monkeypatch):
+    """The call's buffers are laid over each other: what it needs beside its input does not exceed what the layers need one after
+    the other (the block may hand its last sum on)."""
+    import makani_amd as ma
+    from makani_amd import block as nb
+
+    print(f"case peak {f} -> {i}", flush=True)
+    torch.manual_seed(14)
+    lmax, mmax = min(f[0], i[0]), min(f[1], i[1]) // 2 + 1
+    fwd = ma.RealSHT(*f, lmax=lmax, mmax=mmax, grid="legendre-gauss")
+    blk = make_block(fwd, ma.InverseRealSHT(*i, lmax=lmax, mmax=mmax, grid="legendre-gauss"), 64, 2.0).eval()
+    x = torch.randn(2, 64, *f, device="cuda").to(torch.bfloat16)
+
+    @torch.autocast("cuda", dtype=torch.bfloat16)
+    @torch.no_grad()
+    def call():
+        blk(x, defer_skip=True)
+
+    native = peak_of(call)
+    monkeypatch.setattr(nb, "supported", lambda *a: False)
+    assert native <= peak_of(call) + (1 << 16)        # rounding of some dozen allocations
+
+
+def test_peak_memory_of_training_is_that_of_layer_by_layer(lib_built):
+    """What a block kept is given back at the end of its backward only, layer by layer it goes piece by piece, but with more tensors on
+    their way: a twentieth more at most (at 721 x 1440 it is less)."""
+    from makani_amd.sfnonet import SphericalFourierNeuralOperatorNet
+
+    torch.manual_seed(15)
+    net = SphericalFourierNeuralOperatorNet(inp_shape=(65, 128), out_shape=(65, 128), inp_chans=6, out_chans=6, scale_factor=2, embed_dim=64, num_layers=4).cuda()
+    x = torch.randn(2, 6, 65, 128, device="cuda")
+
+    def call():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            net(x).float().square().mean().backward()
+        net.zero_grad(set_to_none=True)
+
+    native = peak_of(call)
+    net.fused_pointwise = False
+    for b in net.blocks:
+        b.fused_pointwise = False
+    assert native <= 1.05 * peak_of(call)
