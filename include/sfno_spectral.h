@@ -289,7 +289,7 @@ int sfno_diagonal_weight_grad(const void* x, const void* gy, void* gweight, int 
  * sfno_pointwise_pack_weight; bias, addend, add_scale, add_shift may be null.  fp32 accumulation, one
  * rounding at the store.  Replaces nn.Conv2d(kernel_size=1) followed by the activation of EncoderDecoder / MLP
  * (makani/models/common/layers.py:95-116,160-216) and, with `addend`, the "norm1(x) + outer_skip(residual)"
- * and "decoder(x) + residual_transform(residual)" sums (makani/models/networks/sfnonet.py:258-262,636-638). */
+ * and "decoder(x) + residual_transform(residual)" sums (makani/models/networks/sfnonet.py:258-262,636-638).  y may be addend. */
 int sfno_pointwise_conv(const void* x, const void* w, const float* bias, void* y, int batch, int K, int O,
                         int64_t P, int act, const void* addend, const float* add_scale, const float* add_shift,
                         void* stream);
@@ -345,7 +345,7 @@ int sfno_instance_norm_coeffs_lat(const float* lat_stats, const float* gamma, co
                                   int channels, int nlat, float eps, void* stream);
 
 /* y = act(scale[row] * x + shift[row]) on bf16 rows of P pixels: the norm0 -> activation step of
- * sfnonet.py:246-251 once the coefficients above are known. */
+ * sfnonet.py:246-251 once the coefficients above are known.  y may be x. */
 int sfno_scale_shift_act(const void* x, const float* scale, const float* shift, void* y, int64_t rows, int64_t P,
                          int act, void* stream);
 

@@ -265,8 +265,9 @@ __global__ __launch_bounds__(64 * NW) void pw_gemm_kernel(PointwiseArgs a) {
     const int64_t px = pw0 + pxw + NT * q;
     const bool inside = px < a.P;
     const int64_t pxc = inside ? px : a.P - NT;
-    unsigned short* __restrict__ Y = a.Y + (int64_t)b * a.O * a.P;
-    const unsigned short* __restrict__ R = ADD ? a.addend + (int64_t)b * a.O * a.P : nullptr;
+    // (no __restrict__: the addend may be the output itself; every value is read, or its batch of rows is, before it is written)
+    unsigned short* Y = a.Y + (int64_t)b * a.O * a.P;
+    const unsigned short* R = ADD ? a.addend + (int64_t)b * a.O * a.P : nullptr;
     // value of row 8 g + 4 ko + j of a 32-row tile whose lane r holds that of row r
     auto row_value = [&](float v, int g, int j) {
         const int lo = __builtin_amdgcn_readlane(__float_as_int(v), 8 * g + j), hi = __builtin_amdgcn_readlane(__float_as_int(v), 8 * g + 4 + j);
@@ -514,8 +515,8 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
     // covers every store issued before it.  The addend itself is read half a row tile ahead.
     auto epilogue = [&](auto whole, int o0, int ko4, int b, int64_t lane_off) {
         constexpr bool WHOLE = decltype(whole)::value;
-        unsigned short* __restrict__ Y = a.Y + lane_off;
-        const unsigned short* __restrict__ R = ADD ? a.addend + lane_off : nullptr;
+        unsigned short* Y = a.Y + lane_off;                                     // (may be the addend itself, as above)
+        const unsigned short* R = ADD ? a.addend + lane_off : nullptr;
         auto row_of = [&](int mt, int v) { return 32 * mt + 8 * (v >> 2) + (v & 3); };     // without the lane's 4 ko
         u32x2 rv[2][8];
         auto load_addend = [&](int mh) {
@@ -835,9 +836,9 @@ __global__ __launch_bounds__(64) void lat_stats_finalize_kernel(const float2* __
     }
 }
 
-// y = act(scale[row] * x + shift[row]), bf16 -> bf16, 8 pixels per thread
-__global__ __launch_bounds__(256) void scale_shift_act_kernel(const unsigned short* __restrict__ x, const float* __restrict__ scale,
-                                                              const float* __restrict__ shift, unsigned short* __restrict__ y, int64_t P,
+// y = act(scale[row] * x + shift[row]), bf16 -> bf16, 8 pixels per thread; y may be x
+__global__ __launch_bounds__(256) void scale_shift_act_kernel(const unsigned short* x, const float* __restrict__ scale,
+                                                              const float* __restrict__ shift, unsigned short* y, int64_t P,
                                                               int64_t groups_per_row, int64_t total_groups, int act) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= total_groups) return;

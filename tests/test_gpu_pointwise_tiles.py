@@ -36,3 +36,26 @@ def test_tiles(lib_built, B, K, O, H, W):
         got = pw.conv1x1(x, w, bias, act, addend, sc if addend is not None else None, sh if addend is not None else None).double()
         assert float((got - want).norm() / want.norm()) < 2 ** -8
         assert float(((got - want).abs() / (want.abs() + 0.05)).max()) < 2 ** -7
+
+
+@pytest.mark.parametrize("K,O,H,W", [(24, 40, 16, 24), (40, 150, 24, 40), (33, 384, 40, 64)])
+def test_sums_in_place(lib_built, K, O, H, W):
+    """The addend may be the output, and scale_shift_act may write where it reads: bit for bit the results of separate tensors."""
+    import ctypes
+
+    from makani_amd import pointwise as pw
+    from makani_amd._lib import check, lib
+
+    print(f"case in place {K}->{O}", flush=True)
+    gen = torch.Generator().manual_seed(6)
+    x, add = torch.randn(2, K, H, W, generator=gen).cuda().to(torch.bfloat16), torch.randn(2, O, H, W, generator=gen).cuda().to(torch.bfloat16)
+    w, sc, sh = torch.randn(O, K, generator=gen).cuda(), torch.randn(2, O, generator=gen).cuda(), torch.randn(2, O, generator=gen).cuda()
+    want, act = pw.conv1x1(x, w, None, None, add, sc, sh), pw.scale_shift_act(add, sc, sh, "gelu")
+
+    def p(t):
+        return ctypes.c_void_p(t.data_ptr())
+
+    packed, y, z = pw.packed_weight(w), add.clone(), add.clone()
+    check(lib.sfno_pointwise_conv(p(x), p(packed), None, p(y), 2, K, O, H * W, 0, p(y), p(sc), p(sh), pw._stream(x.device)), "sfno_pointwise_conv")
+    check(lib.sfno_scale_shift_act(p(z), p(sc), p(sh), p(z), 2 * O, H * W, 1, pw._stream(x.device)), "sfno_scale_shift_act")
+    assert torch.equal(y, want) and torch.equal(z, act)
