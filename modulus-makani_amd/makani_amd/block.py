@@ -54,15 +54,19 @@ def shapes_fit(params, c_in, embed, lmax):
     return all(p is None or tuple(p.shape) == w for p, w in zip(params, want))
 
 
-def supported(blk, x, filter_weight=None, skip_weight=None):
+def supported(blk, x, filter_weight=None, skip_weight=None, training=False):
     """Whether the native block serves this block (whose fusable() the caller has checked) and input; filter_weight, skip_weight: as of
-    forward()."""
+    forward(); training: with its gradients, see trainable()."""
     conv, fwd, inv = blk.filter.filter, blk.filter.filter.forward_transform, blk.filter.filter.inverse_transform
-    if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or mlp_convs(blk) is None:
+    convs = mlp_convs(blk)
+    if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or convs is None:
         return False
     if type(blk.norm0) is not nn.InstanceNorm2d or type(blk.norm1) is not nn.InstanceNorm2d or inv.mmax > inv.nlon // 2 + 1:
         return False
     if type(blk.act_layer0) is not nn.GELU or type(conv) is not SpectralConv or not plain_conv(blk.outer_skip):
+        return False
+    params = _with(block_params(blk, convs), filter_weight, skip_weight)
+    if training and not trainable(x, params, *convs, blk.outer_skip):
         return False
     if tuple(x.shape[2:]) != (fwd.nlat, fwd.nlon) or (inv.nlat * inv.nlon) % 8 != 0:
         return False
@@ -70,7 +74,6 @@ def supported(blk, x, filter_weight=None, skip_weight=None):
         return False
     if x.is_contiguous() and x.data_ptr() % 16 != 0:      # a view into the middle of a buffer: the kernels load 16 bytes at a time
         return False
-    params = _with(block_params(blk), filter_weight, skip_weight)
     if not shapes_fit(params, x.shape[1], conv.out_channels, inv.lmax):
         return False
     wf, *params = [p for p in params if p is not None]
@@ -78,9 +81,9 @@ def supported(blk, x, filter_weight=None, skip_weight=None):
         blk.filter, conv, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.mlp.fwd, *blk.mlp.fwd, blk.outer_skip)
 
 
-def block_params(blk):
+def block_params(blk, convs=None):
     """The block's parameters in the order of _Call: filter, skip, W1, b1, W2, b2, gamma0, beta0, gamma1, beta1 (None where there is none)."""
-    fc1, fc2 = mlp_convs(blk)
+    fc1, fc2 = convs or mlp_convs(blk)
     n0, n1 = blk.norm0, blk.norm1
     return [blk.filter.filter.weight, blk.outer_skip.weight, fc1.weight, fc1.bias, fc2.weight, fc2.bias, n0.weight, n0.bias, n1.weight, n1.bias]
 
@@ -183,12 +186,6 @@ class _BlockFn(torch.autograd.Function):
         return (gx, None, *(t if n else None for t, n in zip(grads, need[2:])))
 
 
-def train_asked(blk, x):
-    """Whether the block (fusable, see supported) may run with its gradients on the kernels: see trainable()."""
-    convs = mlp_convs(blk)
-    return convs is not None and trainable(x, block_params(blk), *convs, blk.outer_skip)
-
-
 def train(blk, x):
-    """The block with autograd (supported() and train_asked() hold)."""
+    """The block with autograd (supported(training=True) holds)."""
     return _BlockFn.apply(x, blk, *block_params(blk))

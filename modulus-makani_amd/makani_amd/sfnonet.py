@@ -234,7 +234,7 @@ class FourierNeuralOperatorBlock(nn.Module):
         if getattr(self, "fused_pointwise", True) and x.is_cuda and x.dtype == torch.bfloat16:
             # the whole block as one native call, with its gradients while they are recorded
             if torch.is_grad_enabled():
-                if self._fusable() and native_block.train_asked(self, x) and native_block.supported(self, x):
+                if self._fusable() and native_block.supported(self, x, training=True):
                     return native_block.train(self, x)
             elif not self.training and fused_pointwise_active(x) and self._fusable() and native_block.supported(self, x):
                 return native_block.forward(self, x, defer_skip=defer_skip)

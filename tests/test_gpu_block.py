@@ -419,3 +419,17 @@ def test_peak_memory_of_training_is_that_of_layer_by_layer(lib_built):
     for b in net.blocks:
         b.fused_pointwise = False
     assert native <= 1.05 * peak_of(call)
+
+
+def test_blocks_without_a_norm_train_on_the_modules(lib_built):
+    from makani_amd.sfnonet import SphericalFourierNeuralOperatorNet
+
+    torch.manual_seed(16)
+    net = SphericalFourierNeuralOperatorNet(inp_shape=(33, 64), out_shape=(33, 64), inp_chans=3, out_chans=3, scale_factor=2, embed_dim=16, num_layers=2,
+                                            normalization_layer="none").cuda()
+    x = torch.randn(1, 3, 33, 64, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        net(x).float().square().mean().backward()
+        with torch.no_grad():
+            y = net.eval()(x)
+    assert torch.isfinite(y).all() and all(p.grad is not None for p in net.parameters())
