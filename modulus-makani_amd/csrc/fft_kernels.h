@@ -807,19 +807,18 @@ __global__ __launch_bounds__(FT) void latfft_fast_kernel(const float2* __restric
 //
 // Rows.  Two neighbouring latitudes of a channel share one complex sequence; a tile is S such pairs, persistent workgroups as in
 // the order-major kernels above (next tile requested into registers before the passes, unconditional requests and stores: a pair
-// slot past the end repeats the last pair, a last latitude without a partner is its own partner).
+// slot past the end repeats the last pair).  The number of latitudes is even: it is one of the lengths with column kernels.
 struct RowPair {
-    int64_t a, b;            // grid rows of the pair
+    int64_t a;               // first grid row of the pair, the other one follows it
     int r, lat;              // its channel and first latitude
     __device__ __forceinline__ RowPair(int pair, int npairs, int npl, int nlat) {
         const int q = pair < npairs ? pair : npairs - 1;
         r = q / npl;
         lat = 2 * (q - r * npl);
         a = (int64_t)r * nlat + lat;
-        b = lat + 1 < nlat ? a + 1 : a;
     }
     // element of y that holds order m of the first row; order m + u TP (TP a multiple of C) lies u TP nlat further on, the second
-    // row's value (b - a) C further on
+    // row's value C further on
     __device__ __forceinline__ int64_t y_index(int m, int ng, int cs, int nlat) const {
         return ((((int64_t)r * ng + (m >> cs)) * nlat + lat) << cs) + (m & ((1 << cs) - 1));
     }
@@ -848,7 +847,7 @@ __global__ __launch_bounds__(FT, 4) void rows_fwd_kernel(const float2* __restric
             const bool in = (it + 1) * TP <= Q || q0 + it * TP < Q;
             const int off = in ? 4 * (q0 + it * TP) : 0;
             a[it] = *reinterpret_cast<const float4*>(x + rp.a * N + off);
-            b[it] = *reinterpret_cast<const float4*>(x + rp.b * N + off);
+            b[it] = *reinterpret_cast<const float4*>(x + (rp.a + 1) * N + off);
         }
     };
     const float h = 0.5f * scale;
@@ -875,7 +874,7 @@ __global__ __launch_bounds__(FT, 4) void rows_fwd_kernel(const float2* __restric
         __syncthreads();
         passes_dif<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
         float2* ya = y + rp.y_index(q0, ng, cs, nlat);
-        float2* yb = ya + ((rp.b - rp.a) << cs);
+        float2* yb = ya + (1 << cs);
         const int64_t ystep = (int64_t)TP * nlat;
 #pragma unroll
         for (int u = 0; u < NSW; ++u)
@@ -909,7 +908,7 @@ __global__ __launch_bounds__(FT, 4) void rows_inv_kernel(const float2* __restric
     auto request = [&](int tile) {
         const RowPair rp(tile * S + pl, npairs, npl, nlat);
         const float2* ya = y + rp.y_index(q0, ng, cs, nlat);
-        const float2* yb = ya + ((rp.b - rp.a) << cs);
+        const float2* yb = ya + (1 << cs);
         const int64_t ystep = (int64_t)TP * nlat;
 #pragma unroll
         for (int u = 0; u < NSW; ++u) {
@@ -953,7 +952,7 @@ __global__ __launch_bounds__(FT, 4) void rows_inv_kernel(const float2* __restric
                 if ((it + 1) * TP > Q) i4 = i4 < Q ? i4 : Q - 1;
                 const float4 u0 = src[2 * i4], u1 = src[2 * i4 + 1];
                 *reinterpret_cast<float4*>(x + rp.a * N + 4 * i4) = make_float4(u0.x, u0.z, u1.x, u1.z);
-                *reinterpret_cast<float4*>(x + rp.b * N + 4 * i4) = make_float4(u0.y, u0.w, u1.y, u1.w);
+                *reinterpret_cast<float4*>(x + (rp.a + 1) * N + 4 * i4) = make_float4(u0.y, u0.w, u1.y, u1.w);
             }
         }
         if (tn >= ntiles) break;
@@ -1118,7 +1117,8 @@ int go_rows(bool inverse, const FftPlan& p, const float* in, float* out, int64_t
     constexpr int FT = (S * N >= 4096) ? 512 : 256;
     constexpr int WG_PER_CU = 1024 / FT;
     static_assert(FT / S % 16 == 0, "a sweep covers whole groups");
-    const int npl = (nlat + 1) / 2, ng = (mmax + (1 << cs) - 1) >> cs;
+    if (nlat % 2 != 0) return SFNO_EUNSUPPORTED;
+    const int npl = nlat / 2, ng = (mmax + (1 << cs) - 1) >> cs;
     const int64_t npairs = rows * npl;
     if (npairs > 0x7fffffffLL - S) return SFNO_EUNSUPPORTED;
     const dim3 grid((unsigned)std::min<int64_t>((npairs + S - 1) / S, std::max(1, WG_PER_CU * p.n_cu)));

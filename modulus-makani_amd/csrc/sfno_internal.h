@@ -192,7 +192,7 @@ int fft_fast_launch(bool inverse, const FftPlan& p, const void* in, void* out, i
 int latfft_fast_launch(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
 // planar pair on the reference layout: real FFTs along the grid rows, x [rows][nlat][n] <-> y [rows][group][nlat][2^cs] complex (groups
 // of 2^cs orders; forward scaled by 2 pi / n), and complex FFTs along latitude, y <-> coefficients [rows][lmax][mmax] (outputs times
-// mscale[m]); lengths with specialised kernels only.  cs is fft_col_shift of the latitude length, 0 if it has none
+// mscale[m]); lengths with specialised kernels only, an even number of latitudes.  cs is fft_col_shift of the latitude length, 0 if it has none
 int fft_col_shift(int n);
 int fft_rows_launch(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s);
 int fft_cols_launch(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, const float* mscale,

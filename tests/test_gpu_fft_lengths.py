@@ -27,6 +27,7 @@ def kept(nlat, lmax):
 
 @pytest.mark.parametrize("n", LENGTHS)
 def test_longitude(lib_built, n):
+    """Order-major kernels (nine latitudes have no column kernel; test_row_ordered_pair has the others)."""
     import makani_amd as ma
 
     print(f"case lon {n}", flush=True)
@@ -69,3 +70,56 @@ def test_latitude(lib_built, n):
         full[:, kept(n, lmax), :mmax] = want
         back = np.fft.irfft2(full, s=(n, nlon), norm="ortho")
         assert rel(inv(torch.from_numpy(want.astype(np.complex64)).cuda()).cpu().numpy(), back) < TOL
+
+
+def planar_reference(x, lmax, mmax):
+    """float64 coefficients of x and the field they give back"""
+    nlat, n = x.shape[-2:]
+    c = np.fft.rfft2(x.astype(np.float64), norm="ortho")[..., kept(nlat, lmax), :mmax]
+    full = np.zeros((*x.shape[:-2], nlat, n // 2 + 1), dtype=complex)
+    full[..., kept(nlat, lmax), :mmax] = c
+    return c, np.fft.irfft2(full, s=(nlat, n), norm="ortho")
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_row_ordered_pair(lib_built, n):
+    """Row kernels of every length, which take latitude counts with column kernels only (test_longitude has none): all orders and few of
+    them, groups of 16 orders that are not full; the last tile of row pairs is not either.  Adjoints by <A x, c> = <x, A^T c>."""
+    import makani_amd as ma
+
+    print(f"case rows {n}", flush=True)
+    rng = np.random.default_rng(n)
+    for rows, nlat, lmax, mmax in ((5, 12, 12, n // 2 + 1), (7, 8, 5, max(2, n // 6 + 1))):
+        x = rng.standard_normal((rows, nlat, n)).astype(np.float32)
+        fwd, inv = ma.RealFFT2(nlat, n, lmax=lmax, mmax=mmax), ma.InverseRealFFT2(nlat, n, lmax=lmax, mmax=mmax)
+        want, back = planar_reference(x, lmax, mmax)
+        xd = torch.from_numpy(x).cuda().requires_grad_()
+        got = fwd(xd)
+        assert rel(got.detach().cpu().numpy(), want) < TOL
+        cd = torch.from_numpy(want.astype(np.complex64)).cuda().requires_grad_()
+        y = inv(cd)
+        assert rel(y.detach().cpu().numpy(), back) < TOL
+        u = (rng.standard_normal(want.shape) + 1j * rng.standard_normal(want.shape)).astype(np.complex64)
+        v = rng.standard_normal(x.shape).astype(np.float32)
+        got.backward(torch.from_numpy(u).cuda())
+        y.backward(torch.from_numpy(v).cuda())
+        # real inner products; both sides are sums of products of normal numbers: the error is TOL of the vectors' norms
+        for lhs, rhs, norms in (
+            (np.sum(want.real * u.real + want.imag * u.imag), np.sum(x.astype(np.float64) * xd.grad.cpu().numpy()), np.linalg.norm(want) * np.linalg.norm(u)),
+            (np.sum(back * v), np.sum((want.conj() * cd.grad.cpu().numpy()).real), np.linalg.norm(back) * np.linalg.norm(v)),
+        ):
+            assert abs(lhs - rhs) < TOL * norms
+
+
+@pytest.mark.parametrize("rows,nlat,n", [(400, 64, 96), (140, 64, 1024)])
+def test_row_kernels_walk_many_tiles(lib_built, rows, nlat, n):
+    """More tiles of row pairs than resident workgroups (1024 of 8 pairs, 512 of 4): the second round of the persistent loops, element by
+    element.  fp32 transform pairs of normal numbers: TOL of their standard deviation, six times that at most over all elements."""
+    import makani_amd as ma
+
+    print(f"case row tiles {rows} {nlat} {n}", flush=True)
+    x = np.random.default_rng(1).standard_normal((rows, nlat, n)).astype(np.float32)
+    fwd, inv = ma.RealFFT2(nlat, n), ma.InverseRealFFT2(nlat, n)
+    want, back = planar_reference(x, nlat, n // 2 + 1)
+    assert np.abs(fwd(torch.from_numpy(x).cuda()).cpu().numpy() - want).max() < 6 * TOL
+    assert np.abs(inv(torch.from_numpy(want.astype(np.complex64)).cuda()).cpu().numpy() - back).max() < 6 * TOL
