@@ -20,9 +20,9 @@
 //
 // What bounds it: per chunk and 64 x 64 tile a wavefront issues 96 matrix instructions (3072 cycles) and about 400 vector
 // instructions, most of them cutting the 64 values it loaded, on a SIMD shared by two wavefronts; the store of gw (283 MB for
-// 384 x 384 x 240) follows the sums.  384 x 384 channels, 240 degrees: 223 / 425 / 763 us for 1 / 2 / 4 samples (on
+// 384 x 384 x 240) follows the sums.  384 x 384 channels, 240 degrees: 231 / 430 / 765 us for 1 / 2 / 4 samples (on
 // v_mfma_f32_32x32x2_f32, 512 matrix cycles per 16 rows and product instead of 192: 387 / 689 / 1322; two fp16 numbers, 96 cycles:
-// 191 / 338 / 578), 241 degrees, whose lines of gw are partial, 385 for one sample (416; 354).  Error against float64 of operands of
+// 191 / 338 / 578), 241 degrees, whose lines of gw are partial, 390 for one sample (416; 354).  Error against float64 of operands of
 // one magnitude, 1080 rows: 7.2e-7 (fp32 instruction 8.3e-7), and the same where they differ.
 #include "sfno_internal.h"
 
@@ -88,12 +88,15 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
     // Rows of a chunk: lanes of half 0 take rows first .. first + 7, half 1 the 8 rows `hr` further on.  A chunk near the end of
     // the buffer starts earlier than its turn so that no load leaves the buffer; rows of the chunk before it, and orders the
     // degree does not have (their memory is unwritten), are zeroed in both operands.
-    const int hr = p.M >= WG_KC ? 8 : max(p.M - 8, 0);
+    // A degree of at most 8 orders takes two samples per chunk, the second half the rows of the second one (the last chunk of an odd
+    // number starts a sample early): half the additions, whose rounding is what such short sums lose.
+    const bool two = nm > 0 && nm <= 8 && p.B > 1;
+    const int hr = two ? 0 : p.M >= WG_KC ? 8 : max(p.M - 8, 0);
     OFF offx[IB], offg[OB];          // byte offset of my channel (clamped to the last one) in my half of a chunk
 #pragma unroll
-    for (int ib = 0; ib < IB; ++ib) offx[ib] = (OFF)(hr * kg) * (OFF)ms_x + 8u * min(i0 + 32 * ib + jj, p.I - 1);
+    for (int ib = 0; ib < IB; ++ib) offx[ib] = (OFF)(hr * kg) * (OFF)ms_x + (two ? (OFF)(8 * kg) * (OFF)p.I : 0) + 8u * min(i0 + 32 * ib + jj, p.I - 1);
 #pragma unroll
-    for (int ob = 0; ob < OB; ++ob) offg[ob] = (OFF)(hr * kg) * (OFF)ms_g + 8u * min(o0 + 32 * ob + jj, p.O - 1);
+    for (int ob = 0; ob < OB; ++ob) offg[ob] = (OFF)(hr * kg) * (OFF)ms_g + (two ? (OFF)(8 * kg) * (OFF)p.O : 0) + 8u * min(o0 + 32 * ob + jj, p.O - 1);
 
     f32x16 re[IB][OB], im[IB][OB];
 #pragma unroll
@@ -114,10 +117,10 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
             r[j] = make_float2(z[0], z[1]);
         }
     };
-    // zeroes the rows of chunk m0 that do not count (see above)
-    auto mask = [&](int m0, float2 (&r)[8]) {
+    // zeroes the rows of chunk m0 that do not count (see above); counted: the first half's sample has had its turn
+    auto mask = [&](int m0, bool counted, float2 (&r)[8]) {
         const int first = max(min(m0, p.M - WG_KC), 0) + hr * kg;
-        const int lo = kg && p.M < WG_KC ? 8 : m0;
+        const int lo = two ? (!kg && counted ? 8 : 0) : kg && p.M < WG_KC ? 8 : m0;
 #pragma unroll
         for (int j = 0; j < 8; ++j)
             if (first + j < lo || first + j >= nm) r[j] = make_float2(0.f, 0.f);
@@ -131,7 +134,7 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
                 f.i[k][w] = take_bf16(r[2 * w].y, r[2 * w + 1].y);
             }
     };
-    const int64_t nchunks = (int64_t)nch * p.B;
+    const int64_t nchunks = two ? (p.B + 1) / 2 : (int64_t)nch * p.B;
     if (nchunks > 0) {
         float2 rx[IB][8], rg[OB][8];
         const char *Xb = X, *Gb = G;             // rows of the sample the next loads belong to
@@ -149,18 +152,20 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
         for (int64_t c = 0; c < nchunks; ++c) {
             const int mc = m0;
             if (mc + WG_KC > nm || mc > p.M - WG_KC) {
+                const bool counted = 2 * c > p.B - 2;
 #pragma unroll
-                for (int ib = 0; ib < IB; ++ib) mask(mc, rx[ib]);
+                for (int ib = 0; ib < IB; ++ib) mask(mc, counted, rx[ib]);
 #pragma unroll
-                for (int ob = 0; ob < OB; ++ob) mask(mc, rg[ob]);
+                for (int ob = 0; ob < OB; ++ob) mask(mc, counted, rg[ob]);
             }
             // the next chunk (the last one again after it) is requested into the registers of this one as they come free
             if (c + 1 < nchunks) {
                 m0 += WG_KC;
                 if (m0 >= nm) {
                     m0 = 0;
-                    Xb += 8 * (int64_t)p.I;
-                    Gb += 8 * (int64_t)p.O;
+                    const int samples = two && 2 * (int)c + 4 <= p.B ? 2 : 1;
+                    Xb += 8 * (int64_t)p.I * samples;
+                    Gb += 8 * (int64_t)p.O * samples;
                 }
             }
             Planes fx[IB];

@@ -17,7 +17,9 @@ pytestmark = pytest.mark.gpu
     [
         (1, 1, 1, 1, 1, True),
         (1, 32, 32, 8, 8, False),       # one tile, rows a half chunk
-        (2, 33, 31, 9, 7, False),       # fewer than 8 orders
+        (2, 33, 31, 9, 7, False),       # fewer than 8 orders: two samples per chunk
+        (5, 20, 33, 12, 5, True),       # an odd number of them
+        (3, 96, 64, 24, 8, False),
         (3, 31, 33, 17, 15, True),      # the second half of a chunk overlaps the first
         (1, 64, 65, 20, 16, True),      # exactly one chunk
         (2, 65, 64, 31, 17, True),      # the last chunk starts early
@@ -75,6 +77,25 @@ def test_orders_of_any_magnitude_count(lib_built, B, I, O, L, M, triangular, bit
     ref = torch.bmm(xl.conj().resolve_conj(), gl).permute(1, 2, 0)
     err = (got - ref).norm(dim=0) / ref.norm(dim=0).clamp_min(1e-300)
     assert float(err.max()) < 1.5e-6
+
+
+def test_row_strides_beyond_32_bits(lib_built):
+    """16 row strides of more than 4 GiB (one order, 66048 rows of 512 degrees): 64-bit offsets.  516 chunks of two samples make 12 * 516
+    additions: 0.5 sqrt(6192) 2^-24 = 2.4e-6 by the reckoning above, asserted."""
+    from makani_amd.contractions import _to_spectral, _weight_grad
+
+    B, I, O, L, M = 1032, 64, 33, 512, 1
+    print("case wgrad 64-bit offsets", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    x, g = (torch.view_as_complex(torch.randn(B, c, L, M, 2, device="cuda", generator=gen)) for c in (I, O))
+    sx, sg = _to_spectral(x, B * I, L, M, True), _to_spectral(g, B * O, L, M, True)
+    assert 64 * L * max(sx.shape[-1], sg.shape[-1]) > 2 ** 32
+    got = _weight_grad(sx, sg, (I, O, L), B, M, True)
+    torch.cuda.synchronize()
+    for l in (0, 1, 7, 8, 255, 511):
+        ref = torch.matmul(x[:, :, l, 0].to(torch.complex128).t().conj().resolve_conj().contiguous(), g[:, :, l, 0].to(torch.complex128).contiguous())
+        err = (got[:, :, l].to(torch.complex128) - ref).norm(dim=0) / ref.norm(dim=0)
+        assert float(err.max()) < 2.4e-6, l
 
 
 @pytest.mark.parametrize("I,O,L", [(256, 200, 333), (600, 610, 49)])
