@@ -76,6 +76,24 @@ def test_weight_gradient_counts_every_pixel_once(lib_built):
         assert torch.equal(gw.cpu(), torch.full((3, 5), float(B * P))) and torch.equal(gb.cpu(), torch.full((3,), float(B * P)))
 
 
+@pytest.mark.parametrize("B,K,O,P", [(1, 3, 5, 2 ** 23 + 8), (2, 9, 2, 2 ** 23 + 72)])
+def test_rows_too_long_for_32_bit_offsets(lib_built, B, K, O, P):
+    """From 2^23 pixels on 256 rows lie further apart than 32 bits reach: addresses in 64 bits.  fp32 sums of 1.7e7 products in shares:
+    1e-5, as above."""
+    from makani_amd import pointwise as pw
+
+    print(f"case pointwise wgrad long rows B={B} P={P}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x, gy = (torch.randn(B, c, 8, P // 8, device="cuda", generator=gen).bfloat16() for c in (K, O))
+    gw, gb = pw.conv1x1_weight_grad(gy, x, True)
+    for o in range(O):
+        go = gy[:, o].double()
+        want = torch.stack([(go * x[:, k].double()).sum() for k in range(K)])
+        # the sums of independent products cancel to sqrt(B P); relative to that
+        assert float((gw[o].double() - want).abs().max()) < 1e-5 * (B * P) ** 0.5
+        assert float((gb[o].double() - go.sum()).abs()) < 1e-5 * (B * P) ** 0.5
+
+
 AUTOGRAD_CASES = [
     # B, K, O, H, W, bias, x requires grad
     (2, 73, 384, 20, 36, True, False),      # first layer of the encoder: the input needs no gradient
