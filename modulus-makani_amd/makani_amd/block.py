@@ -173,7 +173,7 @@ class _BlockFn(torch.autograd.Function):
         blk, need = ctx.blk, ctx.needs_input_grad
         c = _Call(blk, x, params, backward=True)
         want = [p is not None and n for p, n in zip(params, need[2:])]
-        want[2], want[4] = want[2] or want[3], want[4] or want[5]          # a bias gradient is a column of its matrix's kernel
+        want[2], want[4] = want[2] or want[3], want[4] or want[5]          # a bias gradient comes with its matrix's
         grads = [torch.empty(p.shape, dtype=p.dtype, device=p.device) if w else None for p, w in zip(params, want)]
         gx = torch.empty_like(x) if need[0] else None
         s = _lib.BlockGrads()

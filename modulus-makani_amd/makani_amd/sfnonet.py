@@ -6,8 +6,9 @@ constructor keywords, same layer order and parameter names (``encoder.fwd.N``,
 ``blocks.i.{norm0,norm1,filter.filter,mlp.fwd.N,outer_skip}``, ``decoder.fwd.N``,
 ``residual_transform``), so a Makani state_dict loads with ``strict=True``.  The spectral
 filter runs on makani_amd.SpectralConv (HIP kernels).  The pointwise parts are plain PyTorch
-modules, as in the reference; for inference under bf16 autocast (no gradient recorded) the
-same modules are evaluated by the fused HIP kernels of makani_amd.pointwise instead.
+modules, as in the reference; under bf16 autocast their parameters are read by the HIP kernels
+instead, in inference by the fused ones of makani_amd.pointwise, and a whole block as one native
+call with or without its gradients (makani_amd.block).
 """
 import math
 from functools import partial
@@ -74,7 +75,7 @@ def _stamp(*tensors):
 
 def fused_pointwise_active(x):
     """The fused kernels serve inference on bf16 activations: bf16 input or bf16 autocast, and no autograd graph (the callers
-    also require ``eval()`` mode: a module in training mode always runs the PyTorch modules)."""
+    also require ``eval()`` mode: without a gradient, a module in training mode runs the PyTorch modules)."""
     if torch.is_grad_enabled() or not x.is_cuda or x.dim() != 4:
         return False
     bf16 = x.dtype == torch.bfloat16 or (torch.is_autocast_enabled() and torch.get_autocast_dtype("cuda") == torch.bfloat16)
@@ -157,8 +158,9 @@ class FourierNeuralOperatorBlock(nn.Module):
                  separable=False, inner_skip="linear", outer_skip=None, use_mlp=False, complex_activation="real", spectral_layers=1, bias=False,
                  final_activation=False, fused_pointwise=True, **kwargs):
         super().__init__()
-        # fused_pointwise (not a Makani option): evaluate the tail of the block with the fused HIP kernels when no gradient
-        # is recorded and the activations are bfloat16; False keeps the PyTorch modules in every situation
+        # fused_pointwise (not a Makani option): evaluate the block with the fused HIP kernels where the activations are bfloat16,
+        # in eval() mode without a gradient and, with its gradients, wherever something asks for them; False keeps the modules in
+        # every situation (the package's 1x1 convolutions still train on their own kernels)
         self.fused_pointwise = fused_pointwise
         if path_drop_rate > 0.0:
             raise NotImplementedError("stochastic depth is a training feature outside this path")
@@ -283,11 +285,12 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         self.merge_decoder = merge_decoder
         self._merge_cache = None
         self._tail_cache = None
-        # fused_pointwise (not a Makani option): under torch.no_grad() / inference_mode() with bf16 autocast the 1x1 convolutions,
-        # instance norms and GELUs run on the fused HIP kernels (weights rounded to bf16 once, fp32 accumulation, one rounding per
-        # layer, norm0 statistics from the unrounded field).  A forward that records gradients always runs the PyTorch modules, so
-        # a validation pass under no_grad does not follow the training forward's arithmetic to the bit: pass False (or set the
-        # attribute on the network and on every block) where train and validation numbers must come from the same path.
+        # fused_pointwise (not a Makani option): under bf16 autocast the 1x1 convolutions, instance norms and GELUs run on the fused HIP
+        # kernels (weights rounded to bf16 once, fp32 accumulation, one rounding per layer, norm0 statistics from the unrounded field
+        # where the grid is not small): under torch.no_grad() / inference_mode() the whole network, where gradients are recorded the
+        # blocks, the encoder and the decoder.  Inference folds and merges linear layers and takes a coarser fit of the GELU, so a
+        # validation pass under no_grad does not follow the training forward's arithmetic to the bit: pass False (or set the
+        # attribute on the network and on every block) where train and validation numbers must come from the same modules.
         self.fused_pointwise = fused_pointwise
         # spectral_compute = "bf16" (not a Makani option) runs the Legendre and dhconv contractions on bf16 MFMA
         self.spectral_compute = spectral_compute
