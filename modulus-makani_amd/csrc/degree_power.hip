@@ -13,7 +13,7 @@ namespace {
 // A workgroup owns one degree (the longest first) and up to 128 channel rows: nx threads side by side along the row of coefficients,
 // two rows (16 bytes) each, and as many of those as fit along the orders, each with several loads in flight.  One 8-byte load at a time by
 // four order groups of 64 rows left the 73-row transform at 721 x 1440 waiting on latency, a second workgroup with 9 of 64 lanes busy:
-// 78 us per power and 117 us per gradient for 152 MB of coefficients, DPNUM2.
+// 78 us per power and 117 us per gradient for 152 MB of coefficients; now 35 (4.4 TB/s) and 69 (read and written, 4.4 TB/s).
 constexpr int DP_THREADS = 512;
 constexpr int DP_NX = 64;     // pairs of rows per workgroup
 constexpr int DP_NY = 32;     // orders in parallel
