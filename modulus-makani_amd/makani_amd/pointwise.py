@@ -4,9 +4,9 @@
 instance norm split into its statistics (a per-(b, c) scale and shift) and their application.
 These replace the nn.Conv2d(kernel_size=1) / nn.InstanceNorm2d / nn.GELU sequences of
 makani/models/networks/sfnonet.py:246-262 and makani/models/common/layers.py:86-216 on the
-inference path under bf16 autocast.  The plain convolution (with its bias) also has a backward on the HIP
-kernels -- conv1x1_trainable, the forward of PointwiseConv2d when a gradient is asked for --, so that training under
-bf16 autocast keeps its 1x1 convolutions here; the fused epilogues have none.
+inference path under bf16 autocast.  In training the plain convolution (with its bias) has a backward on the HIP
+kernels -- conv1x1_trainable, the forward of PointwiseConv2d when a gradient is asked for --, convolution -> GELU -> convolution
+has one (conv_gelu_conv_trainable), and so has a whole block (block.py); the other epilogues have none.
 """
 import ctypes
 import weakref
@@ -18,7 +18,7 @@ from ._lib import lib, check
 
 ACT = {None: _lib.ACT_NONE, "none": _lib.ACT_NONE, "gelu": _lib.ACT_GELU}
 
-# (id(parameter), transposed) -> (weakref, stamp, packed bf16 [O, Kpad])
+# (id(parameter), transposed) -> (weakref, stamp, packed bf16 [O, Kpad], stream it was packed on, handles of the streams that may use it)
 _wcache = {}
 
 
@@ -30,6 +30,17 @@ def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+def _order(p, packed_on, streams):
+    """Puts the current stream, the first time it uses p, behind the stream that packed it, and keeps p's memory until its work is done.
+    (A capture is entered with the device idle; work outside it cannot be waited for inside.)"""
+    if torch.cuda.is_current_stream_capturing():
+        return
+    s = torch.cuda.current_stream(p.device)
+    s.wait_stream(packed_on)
+    p.record_stream(s)
+    streams.add(s.cuda_stream)
+
+
 def packed_weight(weight, transposed=False):
     """MFMA operand stream of a 1x1 convolution weight ([O, K, 1, 1] or [O, K]), or of its transpose (the weight of the
     convolution's input gradient); cached per parameter and rebuilt when the parameter changes."""
@@ -38,13 +49,16 @@ def packed_weight(weight, transposed=False):
     stamp = (weight.data_ptr(), -1 if weight.is_inference() else weight._version, weight.device)
     hit = _wcache.get(key)
     if hit is not None and hit[0]() is weight and hit[1] == stamp:
+        if torch._C._cuda_getCurrentRawStream(weight.device.index) not in hit[4]:
+            _order(*hit[2:])
         return hit[2]
     w = weight.detach().reshape(weight.shape[0], -1).float().contiguous()
     O, K = (w.shape[1], w.shape[0]) if transposed else w.shape
     p = torch.empty(lib.sfno_pointwise_weight_elems(O, K), dtype=torch.bfloat16, device=w.device)
     pack = lib.sfno_pointwise_pack_weight_transposed if transposed else lib.sfno_pointwise_pack_weight
-    check(pack(_ptr(w), _ptr(p), O, K, _stream(w.device)), "sfno_pointwise_pack_weight")
-    _wcache[key] = (weakref.ref(weight, lambda _, k=key: _wcache.pop(k, None)), stamp, p)
+    s = torch.cuda.current_stream(w.device)
+    check(pack(_ptr(w), _ptr(p), O, K, ctypes.c_void_p(s.cuda_stream)), "sfno_pointwise_pack_weight")
+    _wcache[key] = (weakref.ref(weight, lambda _, k=key: _wcache.pop(k, None)), stamp, p, s, {s.cuda_stream})
     return p
 
 

@@ -281,3 +281,28 @@ def test_views_between_16_byte_boundaries(lib_built):
                 y = mod(xi)
             got.append((y, *torch.autograd.grad(y, (xi, *mod.parameters()), view(r))))
         assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_packed_weight_on_another_stream(lib_built, transposed):
+    """A weight packed behind other work of one stream is used by the next stream at once: that stream waits for the packing."""
+    from makani_amd import pointwise as pw
+
+    print("case packed weight, two streams", transposed, flush=True)
+    torch.manual_seed(4)
+    w, x = torch.randn(24, 24, device="cuda"), torch.randn(1, 24, 16, 16, device="cuda").bfloat16()
+    pw._conv1x1(x, w, transposed)
+    pw.clear_cache(w)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(20_000_000)
+        p = pw.packed_weight(w, transposed)
+    with torch.cuda.stream(b):
+        got = pw._conv1x1(x, w, transposed)
+        again = pw._conv1x1(x, w, transposed)
+    assert pw.packed_weight(w, transposed) is p
+    torch.cuda.synchronize()
+    pw.clear_cache(w)
+    want = pw._conv1x1(x, w, transposed)
+    assert torch.equal(got, want) and torch.equal(again, want)
