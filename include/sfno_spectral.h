@@ -328,6 +328,11 @@ int sfno_pointwise_conv_gelu_grad(const void* gy, const void* wt, const void* z,
 /* Packs a 1x1 convolution weight (float32 [O][K], the nn.Conv2d parameter viewed as a matrix) into the bf16
  * MFMA operand stream sfno_pointwise_conv reads; `packed` holds sfno_pointwise_weight_elems(O, K) bf16 values. */
 int64_t sfno_pointwise_weight_elems(int O, int K);
+/* y = W2 gelu(W1 gelu(scale x + shift) + b1) + b2 in one kernel (inference): x, y bf16 [batch][E][P] (y may be x), scale and shift
+ * [batch][E], w1 ([H][E]) and w2 ([E][H]) packed, b1 and b2 may be null.  SFNO_EUNSUPPORTED outside E <= 384, E a multiple of 8, H of
+ * 16, P of 8: run the three steps by themselves there. */
+int sfno_pointwise_mlp(const void* x, const float* scale, const float* shift, const void* w1, const float* b1, const void* w2,
+                       const float* b2, void* y, int batch, int E, int H, int64_t P, void* stream);
 int sfno_pointwise_pack_weight(const float* w, void* packed, int O, int K, void* stream);
 /* the same stream from the transposed matrix: w is float32 [K][O] (the weight of an input gradient) */
 int sfno_pointwise_pack_weight_transposed(const float* w, void* packed, int O, int K, void* stream);

@@ -34,7 +34,7 @@ struct Dims {
     int B, ci, e, h, lmax, mmax, tri;
     int64_t P, Pin, rows_in, rows;            // pixels of the output and input grid; B * c_in, B * embed
     int64_t spec_in, spec_out, xm_in, xm_out; // floats
-    bool scale_residual;
+    bool scale_residual, one_mlp;
     bool valid = false;
     explicit Dims(const sfno_block* b) {
         if (!b || !b->fwd || !b->inv || b->batch < 1 || b->c_in < 1 || b->embed < 1 || b->hidden < 1) return;
@@ -52,6 +52,7 @@ struct Dims {
         spec_out = (int64_t)mmax * lmax * sfno_spectral_ld(rows);
         xm_in = (int64_t)mmax * f.nlat * sfno_spectral_ld(rows_in);
         xm_out = (int64_t)mmax * i.nlat * sfno_spectral_ld(std::max(rows_in, rows));
+        one_mlp = pointwise_mlp_preferred(B, e, h, P);
         valid = true;
     }
 };
@@ -63,7 +64,7 @@ size_t layout(const Dims& d, bool training, int64_t off[SFNO_BLOCK_TENSORS]) {
     off[SFNO_BLOCK_SPEC] = a.take(std::max(sizeof(float) * (size_t)d.spec_in, training ? 0 : act));
     off[SFNO_BLOCK_X] = training ? a.take(act) : off[SFNO_BLOCK_SPEC];
     off[SFNO_BLOCK_COEF0] = training ? a.take(sizeof(float) * 4 * (size_t)d.rows) : -1;
-    off[SFNO_BLOCK_H0] = training ? a.take(act) : off[SFNO_BLOCK_X];       // inference: norm0 and the GELU in place, the MLP's output over them
+    off[SFNO_BLOCK_H0] = training ? a.take(act) : off[SFNO_BLOCK_X];       // inference: norm0, GELU and MLP in place
     off[SFNO_BLOCK_Z1] = training ? a.take(hid) : -1;
     off[SFNO_BLOCK_A1] = training ? a.take(hid) : -1;                      // inference: in the workspace, over the filter's buffers
     off[SFNO_BLOCK_Y2] = training ? a.take(act) : off[SFNO_BLOCK_X];
@@ -77,7 +78,7 @@ size_t layout(const Dims& d, bool training, int64_t off[SFNO_BLOCK_TENSORS]) {
 struct FwdWs {
     float *xm_in, *xm_out, *spec, *coef0;
     float2 *stats, *partial;
-    bf16* a1;
+    bf16* a1;                                            // null where norm0's GELU and the MLP are one kernel
     size_t bytes;
     FwdWs(const sfno_block* b, const Dims& d, void* base) {
         Arena a(base);
@@ -88,7 +89,7 @@ struct FwdWs {
         spec = filter.get<float>(d.spec_out);           // from the channel mix until the synthesis
         xm_out = filter.get<float>(d.xm_out);
         stats = filter.get<float2>((size_t)d.rows * b->inv->nlat);
-        a1 = a.get<bf16>((size_t)d.B * d.h * d.P);      // behind the filter
+        a1 = d.one_mlp ? nullptr : a.get<bf16>((size_t)d.B * d.h * d.P);      // behind the filter
         bytes = std::max({a.off, first.off, filter.off});
     }
 };
@@ -226,9 +227,24 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
         TRY(irfft_launch(b->inv->fft, w.xm_out, xf, SFNO_DTYPE_BF16, d.rows, b->inv->nlat, d.mmax, (int)sfno_spectral_ld(d.rows), s, w.stats));
         TRY(instance_norm_coeffs_lat_launch(w.stats, b->gamma0, b->beta0, c0, c0 + d.rows, d.rows, d.e, b->inv->nlat, b->eps0, s, m0));
     }
-    TRY(scale_shift_act_launch(xf, c0, c0 + d.rows, h0, d.rows, d.P, training ? ACT_GELU_TRAIN : SFNO_ACT_GELU, s));
-    TRY(conv(h0, b->w1, b->b1, a1, d.B, d.e, d.h, d.P, SFNO_ACT_GELU, nullptr, nullptr, nullptr, z1, 0, s));
-    TRY(conv(a1, b->w2, b->b2, y2, d.B, d.h, d.e, d.P, SFNO_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0, s));
+    if (!training && d.one_mlp) {
+        MlpArgs m;
+        std::memset(&m, 0, sizeof(m));
+        m.X = xf;
+        m.scale = c0;
+        m.shift = c0 + d.rows;
+        m.W1 = reinterpret_cast<const bf16*>(b->w1);
+        m.b1 = b->b1;
+        m.W2 = reinterpret_cast<const bf16*>(b->w2);
+        m.b2 = b->b2;
+        m.Y = y2;
+        m.B = d.B; m.E = d.e; m.H = d.h; m.P = d.P;
+        TRY(pointwise_mlp_launch(m, s));
+    } else {
+        TRY(scale_shift_act_launch(xf, c0, c0 + d.rows, h0, d.rows, d.P, training ? ACT_GELU_TRAIN : SFNO_ACT_GELU, s));
+        TRY(conv(h0, b->w1, b->b1, a1, d.B, d.e, d.h, d.P, SFNO_ACT_GELU, nullptr, nullptr, nullptr, z1, 0, s));
+        TRY(conv(a1, b->w2, b->b2, y2, d.B, d.h, d.e, d.P, SFNO_ACT_NONE, nullptr, nullptr, nullptr, nullptr, 0, s));
+    }
     TRY(instance_norm_coeffs_launch(y2, b->gamma1, b->beta1, c1, c1 + d.rows, w.partial, d.rows, d.e, d.P, b->eps1, s, reinterpret_cast<float2*>(c1 + 2 * d.rows)));
     if (!out) return SFNO_OK;
     return conv(res, b->wskip, nullptr, reinterpret_cast<bf16*>(out), d.B, d.ci, d.e, d.P, SFNO_ACT_NONE, y2, c1, c1 + d.rows, nullptr, 0, s);

@@ -709,6 +709,24 @@ extern "C" int sfno_pointwise_conv(const void* x, const void* w, const float* bi
     return pointwise_gemm_launch(a, (hipStream_t)stream);
 }
 
+extern "C" int sfno_pointwise_mlp(const void* x, const float* scale, const float* shift, const void* w1, const float* b1, const void* w2, const float* b2,
+                                  void* y, int batch, int E, int H, int64_t P, void* stream) {
+    if (!x || !scale || !shift || !w1 || !w2 || !y || batch < 1 || E < 1 || H < 1 || P < 1) return SFNO_EINVAL;
+    if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(w1) | reinterpret_cast<uintptr_t>(w2)) & 15) return SFNO_EINVAL;
+    MlpArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.X = reinterpret_cast<const unsigned short*>(x);
+    a.scale = scale;
+    a.shift = shift;
+    a.W1 = reinterpret_cast<const unsigned short*>(w1);
+    a.b1 = b1;
+    a.W2 = reinterpret_cast<const unsigned short*>(w2);
+    a.b2 = b2;
+    a.Y = reinterpret_cast<unsigned short*>(y);
+    a.B = batch; a.E = E; a.H = H; a.P = P;
+    return pointwise_mlp_launch(a, (hipStream_t)stream);
+}
+
 extern "C" int sfno_pointwise_conv_cat(const void* x1, int K1, const void* x2, int K2, const void* w, const float* bias, void* y, int batch,
                                        int O, int64_t P, int act, void* stream) {
     if (!x1 || !x2 || !w || !y || batch < 1 || K1 < 1 || K2 < 1 || O < 1 || P < 1) return SFNO_EINVAL;

@@ -975,6 +975,8 @@ __global__ __launch_bounds__(64) void norm_param_grad_kernel(const float2* __res
     }
 }
 
+#include "pointwise_mlp.h"
+
 }  // namespace
 
 // compute units of the current device (256 when the query fails)
@@ -1077,6 +1079,47 @@ int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s) {
         gemm_go<2>(a, blocks, epi, s);
     else
         gemm_go<8>(a, blocks, epi, s);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+template <int MT>
+static void mlp_go(const MlpArgs& a, bool ragged, hipStream_t s) {
+    const dim3 grid((unsigned)std::min<int64_t>(a.n_strips * a.B, device_cus())), block(256);
+    if (ragged)
+        hipLaunchKernelGGL((pw_mlp_kernel<MT, true>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((pw_mlp_kernel<MT, false>), grid, block, 0, s, a);
+}
+
+bool pointwise_mlp_supported(int B, int E, int H, int64_t P) {
+    if (B < 1 || E < 8 || E > 384 || H < 16 || E % 8 != 0 || H % 16 != 0 || P < 8 || P % 8 != 0) return false;
+    // 32-bit byte offsets within a sample and within a packed weight, a 31-bit count of tiles
+    return (int64_t)E * P < (1LL << 30) && (int64_t)E * H < (1LL << 28) && (P + 127) / 128 * B < (1LL << 30);
+}
+
+// Whether the one kernel is the faster way (both give the same bits).  In us, the three kernels / this one, hidden channels 2 E, on 256
+// CUs: E = 32 with 16 tiles of 128 pixels 14.6 / 12.7, with 900 tiles 27.3 / 43.2 (rows are padded to 128); E = 64 16.5 / 12.7 and
+// 35.8 / 43.6; E = 96 18.7 / 12.8 and 53.4 / 46.0; E = 128 21.8 / 11.7 and 60.8 / 45.2; E = 256 32.0 / 25.5 and 139 / 97; E = 264
+// 33.6 / 42.8 and 171 / 156; E = 320 with 57 tiles 41.6 / 43.5, with 127 53.0 / 45.0; E = 384 42.0 / 43.6 and 240 / 177 (a tile takes 40 us
+// there, so few tiles leave CUs idle that the three kernels fill with smaller ones).
+bool pointwise_mlp_preferred(int B, int E, int H, int64_t P) {
+    const int64_t tiles = (P + 127) / 128 * B, cus = device_cus();
+    return pointwise_mlp_supported(B, E, H, P) && (E > 64 || tiles <= cus) && (E <= 256 || 4 * tiles >= cus);
+}
+
+int pointwise_mlp_launch(MlpArgs a, hipStream_t s) {
+    if (!pointwise_mlp_supported(a.B, a.E, a.H, a.P)) return SFNO_EUNSUPPORTED;
+    a.kpad1 = pointwise_kpad(a.E, a.H);
+    a.opad1 = pointwise_opad(a.H);
+    a.kpad2 = pointwise_kpad(a.H, a.E);
+    a.opad2 = pointwise_opad(a.E);
+    a.n_strips = (a.P + 127) / 128;
+    const bool ragged = a.E % 128 != 0 || a.H % 128 != 0 || a.H < 256;
+    switch ((a.E + 127) / 128) {
+        case 1: mlp_go<1>(a, ragged, s); break;
+        case 2: mlp_go<2>(a, ragged, s); break;
+        default: mlp_go<3>(a, ragged, s); break;
+    }
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

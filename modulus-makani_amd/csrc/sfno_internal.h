@@ -107,6 +107,23 @@ struct PointwiseArgs {
     int64_t n_strips;
 };
 int pointwise_gemm_launch(PointwiseArgs a, hipStream_t s);
+// y = W2 gelu(W1 gelu(scale x + shift) + b1) + b2 in one kernel (pointwise_mlp.h); W1 [H][E] and W2 [E][H] packed, Y may be X
+struct MlpArgs {
+    const unsigned short* X;       // bf16 [B][E][P]
+    const float *scale, *shift;    // [B][E]
+    const unsigned short* W1;
+    const float* b1;               // [H] or null
+    const unsigned short* W2;
+    const float* b2;               // [E] or null
+    unsigned short* Y;             // bf16 [B][E][P]
+    int B, E, H;
+    int64_t P;
+    int kpad1, opad1, kpad2, opad2;   // filled by the launcher
+    int64_t n_strips;
+};
+bool pointwise_mlp_supported(int B, int E, int H, int64_t P);
+bool pointwise_mlp_preferred(int B, int E, int H, int64_t P);
+int pointwise_mlp_launch(MlpArgs a, hipStream_t s);
 int pointwise_kpad(int K, int O);
 int pointwise_opad(int O);
 int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, int transposed, hipStream_t s);

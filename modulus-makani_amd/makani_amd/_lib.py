@@ -94,6 +94,7 @@ def _load():
         "sfno_pointwise_weight_elems": (i64, [i32, i32]),
         "sfno_pointwise_pack_weight": (i32, [vp, vp, i32, i32, vp]),
         "sfno_pointwise_conv": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, i32, vp, vp, vp, vp]),
+        "sfno_pointwise_mlp": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i64, vp]),
         "sfno_pointwise_conv_gelu": (i32, [vp, vp, vp, vp, vp, i32, i32, i32, i64, vp]),
         "sfno_pointwise_conv_gelu_grad": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, vp]),
         "sfno_pointwise_pack_weight_transposed": (i32, [vp, vp, i32, i32, vp]),

@@ -116,6 +116,23 @@ def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=
     return y
 
 
+def norm_mlp(x, scale, shift, w1, b1, w2, b2):
+    """conv1x1(gelu(conv1x1(gelu(scale[b, c] * x + shift[b, c]), w1) + b1), w2) + b2 -> bf16 [B, E, H, W] in one kernel (inference);
+    x has E <= 384 channels, a multiple of 8, and w1 [H, E] a multiple of 16 rows."""
+    if not supported(x):
+        raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
+    x = _dense(x)
+    B, E, H, W = x.shape
+    hidden = w1.shape[0]
+    if w1.reshape(hidden, -1).shape[1] != E or tuple(w2.shape[:2]) != (E, hidden) or scale.numel() != B * E or shift.numel() != B * E:
+        raise RuntimeError(f"norm_mlp: weights {tuple(w1.shape)} and {tuple(w2.shape)} do not fit {E} channels")
+    y = torch.empty_like(x)
+    scale, shift, b1, b2 = (t.detach().float().contiguous() if t is not None else None for t in (scale, shift, b1, b2))
+    check(lib.sfno_pointwise_mlp(_ptr(x), _ptr(scale), _ptr(shift), _ptr(packed_weight(w1)), _ptr(b1), _ptr(packed_weight(w2)), _ptr(b2), _ptr(y), B, E,
+                                 hidden, H * W, _stream(x.device)), "sfno_pointwise_mlp")
+    return y
+
+
 def conv1x1_cat(x1, x2, weight, bias=None, act=None, out=None):
     """act(conv1x1(cat([x1, x2], dim=1), weight) + bias) without building the concatenation  ->  bf16 [B, O, H, W];
     weight [O, K1 + K2] (or [O, K1 + K2, 1, 1]); out: a contiguous bf16 tensor of the result's shape to write into."""
