@@ -178,6 +178,10 @@ int sfno_sht_analysis(const sfno_sht_plan* plan, const void* x, int x_dtype, flo
                       void* workspace, size_t workspace_bytes, void* stream);
 int sfno_sht_synthesis(const sfno_sht_plan* plan, const float* spec, void* x, int x_dtype, int64_t rows,
                        void* workspace, size_t workspace_bytes, void* stream);
+/* sfno_sht_analysis of the float32 field x - x2, which is not stored; plans whose longitude length has specialised kernels
+ * (those that support SFNO_DTYPE_BF16 fields), otherwise SFNO_EUNSUPPORTED. */
+int sfno_sht_analysis_diff(const sfno_sht_plan* plan, const float* x, const float* x2, float* spec, int64_t rows,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 /* The four stages of the transform pair on their own (what sfno_sht_analysis and
  * sfno_sht_synthesis chain).  xm is the order-major Fourier buffer float32
@@ -268,6 +272,15 @@ int sfno_degree_power(const float* spec, float* power, int64_t rows, int lmax, i
  * gspec[r,l,m] = 2 w_m gpower[r][l] c[r,l,m], w_0 = 1, w_m = 2 otherwise */
 int sfno_degree_power_grad(const float* spec, const float* gpower, float* gspec, int64_t rows, int lmax, int mmax,
                            void* stream);
+
+/* Norms of GeometricH1Loss (makani/utils/losses.py:301-331) from the coefficients of `batch` examples of `channels` rows each:
+ * sums[b] = (a, h), a = sum over channels and degrees of the power, h the same weighted by weights[l]; norms[b] = alpha a + (1 - alpha) h if
+ * squared, else alpha sqrt(a) + (1 - alpha) sqrt(h).  The gradient takes sums and the cotangent of norms. */
+size_t sfno_degree_norm_workspace_bytes(int batch, int64_t channels, int lmax);
+int sfno_degree_norm(const float* spec, const float* weights, float* sums, float* norms, int batch, int64_t channels,
+                     int lmax, int mmax, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream);
+int sfno_degree_norm_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec,
+                          int batch, int64_t channels, int lmax, int mmax, float alpha, int squared, void* stream);
 
 /* ---- "diagonal" operator ------------------------------------------------------------- */
 

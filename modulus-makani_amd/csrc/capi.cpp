@@ -329,6 +329,16 @@ extern "C" int sfno_legendre_synthesis(const sfno_sht_plan* p, const float* spec
     return legendre_fold_launch(false, p->format, a, p->inv.n_work, (hipStream_t)stream);
 }
 
+extern "C" int sfno_sht_analysis_diff(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, int64_t rows, void* workspace,
+                                      size_t workspace_bytes, void* stream) {
+    if (!p || !x || !x2 || !spec || !rows_ok(rows)) return SFNO_EINVAL;
+    if (!(p->directions & SFNO_DIR_FORWARD)) return SFNO_EINVAL;
+    Ws w = carve(p, rows, workspace);
+    if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
+    int rc = rfft_launch(p->fft, x, SFNO_DTYPE_F32, w.xm, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream, x2);
+    if (rc != SFNO_OK) return rc;
+    return sfno_legendre_analysis(p, w.xm, spec, rows, stream);
+}
 extern "C" int sfno_sht_analysis(const sfno_sht_plan* p, const void* x, int x_dtype, float* spec, int64_t rows, void* workspace,
                                  size_t workspace_bytes, void* stream) {
     if (!p || !x || !spec || !rows_ok(rows)) return SFNO_EINVAL;
@@ -622,6 +632,27 @@ extern "C" int sfno_degree_power(const float* spec, float* power, int64_t rows, 
     return degree_power_launch(spec, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
 }
 
+extern "C" size_t sfno_degree_norm_workspace_bytes(int batch, int64_t channels, int lmax) {
+    if (batch < 1 || channels < 1 || lmax < 1) return 0;
+    return align_up(sizeof(float) * (size_t)batch * channels * lmax, 256) + sizeof(double2) * (size_t)batch * degree_norm_segments(channels, lmax);
+}
+extern "C" int sfno_degree_norm(const float* spec, const float* weights, float* sums, float* norms, int batch, int64_t channels, int lmax, int mmax,
+                                float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!spec || !weights || !sums || !norms || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
+    if (!workspace || workspace_bytes < sfno_degree_norm_workspace_bytes(batch, channels, lmax)) return SFNO_EWORKSPACE;
+    float* power = reinterpret_cast<float*>(workspace);
+    const int64_t rows = batch * channels;
+    int rc = degree_power_launch(spec, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
+    if (rc != SFNO_OK) return rc;
+    double2* partial = reinterpret_cast<double2*>(reinterpret_cast<char*>(workspace) + align_up(sizeof(float) * (size_t)rows * lmax, 256));
+    return degree_norm_launch(power, weights, partial, reinterpret_cast<float2*>(sums), norms, batch, channels, lmax, alpha, squared, (hipStream_t)stream);
+}
+extern "C" int sfno_degree_norm_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec, int batch, int64_t channels,
+                                     int lmax, int mmax, float alpha, int squared, void* stream) {
+    if (!spec || !weights || !sums || !gnorms || !gspec || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
+    return degree_norm_grad_launch(spec, weights, reinterpret_cast<const float2*>(sums), gnorms, gspec, batch, channels, lmax, mmax,
+                                   (int)sfno_spectral_ld(batch * channels), alpha, squared, (hipStream_t)stream);
+}
 extern "C" int sfno_degree_power_grad(const float* spec, const float* gpower, float* gspec, int64_t rows, int lmax, int mmax, void* stream) {
     if (!spec || !gpower || !gspec || !rows_ok(rows)) return SFNO_EINVAL;
     return degree_power_grad_launch(spec, gpower, gspec, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);

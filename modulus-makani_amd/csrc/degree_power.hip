@@ -7,6 +7,8 @@
 // the adjoint analysis consumes.  Both are bound by the one pass over the coefficients.
 #include "sfno_internal.h"
 
+#include <algorithm>
+
 namespace sfno {
 namespace {
 
@@ -65,15 +67,37 @@ __global__ __launch_bounds__(DP_THREADS) void degree_power_kernel(const float* _
     }
 }
 
-// gspec[m][l][2r..2r+1] = w_m * 2 * gpower[r][l] * c[r,l,m]  (w_0 = 1, w_m = 2 otherwise); padding columns zero
+// cotangent of the power of row r at degree l: given as a tensor ...
+struct PowerGrad {
+    const float* gpower;
+    int lmax;
+    __device__ __forceinline__ float operator()(int64_t r, int l) const { return gpower[r * lmax + l]; }
+};
+// ... or that of the norms of degree_norm_kernel
+struct NormGrad {
+    const float *weights, *gnorms;
+    const float2* sums;
+    int64_t channels;
+    float alpha;
+    int squared;
+    __device__ __forceinline__ float operator()(int64_t r, int l) const {
+        const int b = (int)(r / channels);
+        const float g = gnorms[b], a = alpha * g, h = (1.f - alpha) * g;
+        const float2 s = sums[b];
+        return squared ? fmaf(h, weights[l], a) : fmaf(h / (2.f * sqrtf(s.y)), weights[l], a / (2.f * sqrtf(s.x)));
+    }
+};
+
+// gspec[m][l][2r..2r+1] = w_m * 2 * g(r, l) * c[r,l,m]  (w_0 = 1, w_m = 2 otherwise); padding columns zero
 // grid (lmax, ceil(ld / 4 / DP_NX)), block DP_THREADS
-__global__ __launch_bounds__(DP_THREADS) void degree_power_grad_kernel(const float* __restrict__ spec, const float* __restrict__ gpower,
-                                                                       float* __restrict__ gspec, int64_t rows, int lmax, int mmax, int ld) {
+template <class Grad>
+__global__ __launch_bounds__(DP_THREADS) void degree_power_grad_kernel(const float* __restrict__ spec, Grad gpower, float* __restrict__ gspec, int64_t rows,
+                                                                       int lmax, int mmax, int ld) {
     const DpThread t = dp_thread(ld / 4, lmax, mmax);
     if (!t.on) return;
     const int64_t r = 2 * t.pair;
     const bool has0 = r < rows, has1 = r + 1 < rows;
-    const float g0 = has0 ? 2.f * gpower[r * lmax + t.l] : 0.f, g1 = has1 ? 2.f * gpower[(r + 1) * lmax + t.l] : 0.f;
+    const float g0 = has0 ? 2.f * gpower(r, t.l) : 0.f, g1 = has1 ? 2.f * gpower(r + 1, t.l) : 0.f;
     const int64_t at = (int64_t)t.l * ld + 4 * t.pair;
 #pragma unroll 4
     for (int m = t.ty; m <= t.mtop; m += t.ny) {
@@ -86,6 +110,67 @@ __global__ __launch_bounds__(DP_THREADS) void degree_power_grad_kernel(const flo
         c.w = has1 ? w * g1 * c.w : 0.f;
         *reinterpret_cast<float4*>(gspec + i) = c;
     }
+}
+
+// Sums of an example's powers, plain and weighted by degree, in double precision: one workgroup per segment of the example's channels * lmax
+// values (grid (segments, batch)); a single one also forms the norm.  With a second kernel where there are several, this takes
+// the place of nine elementwise and reduction kernels of 4 to 10 us (73 x 721 values).
+constexpr int DN_THREADS = 512;
+__device__ __forceinline__ void norm_of(double a, double h, float alpha, int squared, float2* sums, float* norm) {
+    const float2 s = make_float2((float)a, (float)h);
+    *sums = s;
+    *norm = squared ? alpha * s.x + (1.f - alpha) * s.y : alpha * sqrtf(s.x) + (1.f - alpha) * sqrtf(s.y);
+}
+
+__global__ __launch_bounds__(DN_THREADS) void degree_norm_kernel(const float* __restrict__ power, const float* __restrict__ weights,
+                                                                 double2* __restrict__ partial, float2* __restrict__ sums, float* __restrict__ norms, int64_t n,
+                                                                 int lmax, float alpha, int squared) {
+    const int b = blockIdx.y, nseg = gridDim.x;
+    const int64_t from = n * blockIdx.x / nseg, to = n * (blockIdx.x + 1) / nseg;
+    const float* __restrict__ p = power + (int64_t)b * n;
+    double a = 0.0, h = 0.0;
+    int l = (int)((from + threadIdx.x) % lmax);
+    const int step = DN_THREADS % lmax;
+#pragma unroll 4
+    for (int64_t i = from + threadIdx.x; i < to; i += DN_THREADS) {
+        const double v = p[i];
+        a += v;
+        h += v * (double)weights[l];
+        l += step;
+        if (l >= lmax) l -= lmax;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_down(a, off, 64);
+        h += __shfl_down(h, off, 64);
+    }
+    __shared__ double2 red[DN_THREADS / 64];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = make_double2(a, h);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < DN_THREADS / 64; ++w) {
+            a += red[w].x;
+            h += red[w].y;
+        }
+        if (nseg == 1)
+            norm_of(a, h, alpha, squared, sums + b, norms + b);
+        else
+            partial[(int64_t)b * nseg + blockIdx.x] = make_double2(a, h);
+    }
+}
+
+// one wavefront per example; nseg <= 64
+__global__ __launch_bounds__(64) void degree_norm_finish_kernel(const double2* __restrict__ partial, float2* __restrict__ sums, float* __restrict__ norms, int nseg,
+                                                                float alpha, int squared) {
+    const int b = blockIdx.x;
+    double2 t = make_double2(0.0, 0.0);
+    if ((int)threadIdx.x < nseg) t = partial[(int64_t)b * nseg + threadIdx.x];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        t.x += __shfl_down(t.x, off, 64);
+        t.y += __shfl_down(t.y, off, 64);
+    }
+    if (threadIdx.x == 0) norm_of(t.x, t.y, alpha, squared, sums + b, norms + b);
 }
 
 }  // namespace
@@ -101,7 +186,29 @@ int degree_power_launch(const float* spec, float* power, int64_t rows, int lmax,
 int degree_power_grad_launch(const float* spec, const float* gpower, float* gspec, int64_t rows, int lmax, int mmax, int ld, hipStream_t s) {
     const int64_t blocks = (ld / 4 + DP_NX - 1) / DP_NX;
     if (rows < 1 || lmax < 1 || mmax < 1 || ld < 2 * rows || ld % 4 != 0 || blocks > 65535) return SFNO_EINVAL;
-    hipLaunchKernelGGL(degree_power_grad_kernel, dim3(lmax, (unsigned)blocks), dim3(DP_THREADS), 0, s, spec, gpower, gspec, rows, lmax, mmax, ld);
+    hipLaunchKernelGGL(degree_power_grad_kernel<PowerGrad>, dim3(lmax, (unsigned)blocks), dim3(DP_THREADS), 0, s, spec, PowerGrad{gpower, lmax}, gspec, rows, lmax,
+                       mmax, ld);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+// some 8 thousand values per workgroup; by an example's size alone, so that it gives the same norm alone and in a batch
+int degree_norm_segments(int64_t channels, int lmax) { return (int)std::max<int64_t>(1, std::min<int64_t>(channels * lmax / 8192, 64)); }
+
+int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, int batch, int64_t channels, int lmax,
+                       float alpha, int squared, hipStream_t s) {
+    if (batch < 1 || batch > 65535 || channels < 1 || lmax < 1) return SFNO_EINVAL;
+    const int nseg = degree_norm_segments(channels, lmax);
+    hipLaunchKernelGGL(degree_norm_kernel, dim3(nseg, batch), dim3(DN_THREADS), 0, s, power, weights, partial, sums, norms, channels * lmax, lmax, alpha, squared);
+    if (nseg > 1) hipLaunchKernelGGL(degree_norm_finish_kernel, dim3(batch), dim3(64), 0, s, partial, sums, norms, nseg, alpha, squared);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+int degree_norm_grad_launch(const float* spec, const float* weights, const float2* sums, const float* gnorms, float* gspec, int batch, int64_t channels, int lmax,
+                            int mmax, int ld, float alpha, int squared, hipStream_t s) {
+    const int64_t rows = batch * channels, blocks = (ld / 4 + DP_NX - 1) / DP_NX;
+    if (batch < 1 || channels < 1 || lmax < 1 || mmax < 1 || ld < 2 * rows || ld % 4 != 0 || blocks > 65535) return SFNO_EINVAL;
+    hipLaunchKernelGGL(degree_power_grad_kernel<NormGrad>, dim3(lmax, (unsigned)blocks), dim3(DP_THREADS), 0, s, spec,
+                       NormGrad{weights, gnorms, sums, channels, alpha, squared}, gspec, rows, lmax, mmax, ld);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

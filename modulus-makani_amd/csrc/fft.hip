@@ -391,9 +391,10 @@ static int pick_pairs(int n) {
     return 0;
 }
 
-int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s) {
+int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2) {
     if (mmax > p.n / 2 + 1 || ld % 4 != 0 || ld < 2 * rows) return SFNO_EINVAL;
-    if (fft_fast_supported(p.n)) return fft_fast_launch(false, p, xv, xm, rows, nlat, mmax, ld, x_dtype, s);
+    if (fft_fast_supported(p.n)) return fft_fast_launch(false, p, xv, xm, rows, nlat, mmax, ld, x_dtype, s, nullptr, x2);
+    if (x2) return SFNO_EUNSUPPORTED;
     if (x_dtype != SFNO_DTYPE_F32) return SFNO_EUNSUPPORTED;     // the generic kernels read float only
     const float* x = reinterpret_cast<const float*>(xv);
     switch (pick_pairs(p.n)) {

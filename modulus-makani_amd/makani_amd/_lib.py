@@ -65,6 +65,7 @@ def _load():
         "sfno_sht_forward_static": (i32, [vp, vp, vp, i64, vp]),
         "sfno_sht_io_dtype_supported": (i32, [vp, i32]),
         "sfno_sht_analysis": (i32, [vp, vp, i32, vp, i64, vp, sz, vp]),
+        "sfno_sht_analysis_diff": (i32, [vp, vp, vp, vp, i64, vp, sz, vp]),
         "sfno_sht_synthesis": (i32, [vp, vp, vp, i32, i64, vp, sz, vp]),
         "sfno_sht_lat_stats_supported": (i32, [vp]),
         "sfno_sht_synthesis_lat_stats": (i32, [vp, vp, vp, i32, i64, vp, sz, vp, vp]),
@@ -89,6 +90,9 @@ def _load():
         "sfno_dhconv": (i32, [vp, vp, vp, i32, i32, i32, vp, sz, vp]),
         "sfno_degree_power": (i32, [vp, vp, i64, i32, i32, vp]),
         "sfno_degree_power_grad": (i32, [vp, vp, vp, i64, i32, i32, vp]),
+        "sfno_degree_norm_workspace_bytes": (sz, [i32, i64, i32]),
+        "sfno_degree_norm": (i32, [vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp, sz, vp]),
+        "sfno_degree_norm_grad": (i32, [vp, vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp]),
         "sfno_diagonal_contract": (i32, [vp, vp, vp, i32, i32, i32, i64, i32, vp]),
         "sfno_diagonal_weight_grad": (i32, [vp, vp, vp, i32, i32, i32, i64, vp]),
         "sfno_pointwise_weight_elems": (i64, [i32, i32]),

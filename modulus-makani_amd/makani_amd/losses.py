@@ -46,6 +46,34 @@ class _DegreePowerFn(torch.autograd.Function):
         return gspec, None, None, None
 
 
+class _DegreeNormFn(torch.autograd.Function):
+    """spectral-layout coefficients [mmax, lmax, ld] of batch * channels rows -> norms [batch] of GeometricH1Loss."""
+
+    @staticmethod
+    def forward(ctx, spec, weights, batch, channels, alpha, squared):
+        mmax, lmax, _ = spec.shape
+        sums = torch.empty((batch, 2), dtype=torch.float32, device=spec.device)
+        norms = torch.empty((batch,), dtype=torch.float32, device=spec.device)
+        nbytes = lib.sfno_degree_norm_workspace_bytes(batch, channels, lmax)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=spec.device)
+        check(lib.sfno_degree_norm(_ptr(spec), _ptr(weights), _ptr(sums), _ptr(norms), batch, channels, lmax, mmax, alpha, squared, _ptr(ws), nbytes,
+                                   _stream(spec.device)), "sfno_degree_norm")
+        ctx.save_for_backward(spec, weights, sums)
+        ctx.cfg = (batch, channels, lmax, mmax, alpha, squared)
+        return norms
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g):
+        spec, weights, sums = ctx.saved_tensors
+        batch, channels, lmax, mmax, alpha, squared = ctx.cfg
+        g = g.float().contiguous()
+        gspec = torch.empty_like(spec)
+        check(lib.sfno_degree_norm_grad(_ptr(spec), _ptr(weights), _ptr(sums), _ptr(g), _ptr(gspec), batch, channels, lmax, mmax, alpha, squared,
+                                        _stream(spec.device)), "sfno_degree_norm_grad")
+        return gspec, None, None, None, None, None
+
+
 def degree_power(sht, x):
     """|c_l0|^2 + 2 sum_{m>0} |c_lm|^2 of sht(x) for every leading index: x [..., nlat, nlon] -> [..., lmax]."""
     lead = x.shape[:-2]
@@ -72,7 +100,17 @@ class GeometricH1Loss(nn.Module):
         h1_weights = torch.arange(self.sht.lmax).float()
         self.register_buffer("h1_weights", h1_weights * (h1_weights + 1))
 
-    def _norms(self, x):
+    def _norms(self, x, minus=None):
+        """Norms of x, or of x - minus."""
+        sht, w = self.sht, self.h1_weights
+        # (a batch of channels of fields, the weights as they were registered: what the kernels form the norms of directly)
+        if type(sht) is RealSHT and x.dim() >= 3 and x.numel() > 0 and (minus is None or minus.shape == x.shape) and x.is_cuda and isinstance(self.alpha, (int, float)) \
+                and w.shape == (sht.lmax,) and w.dtype == torch.float32 and w.device == x.device and w.is_contiguous() and not w.requires_grad:
+            spec = sht.analysis(x) if minus is None else sht.analysis_diff(x, minus)
+            rows = x.numel() // (sht.nlat * sht.nlon)
+            return _DegreeNormFn.apply(spec, w, x.shape[0], rows // x.shape[0], float(self.alpha), bool(self.squared))
+        if minus is not None:
+            x = x - minus
         num_examples = x.size()[0]
         norm2 = degree_power(self.sht, x)
         l2_norm2 = norm2.reshape(num_examples, -1).sum(dim=-1)
@@ -82,13 +120,13 @@ class GeometricH1Loss(nn.Module):
         return self.alpha * l2_norm2 + (1 - self.alpha) * h1_norm2
 
     def abs(self, prd, tar):
-        all_norms = self._norms(prd - tar)
+        all_norms = self._norms(prd, tar)
         if self.reduction:
             return torch.mean(all_norms) if self.size_average else torch.sum(all_norms)
         return all_norms
 
     def rel(self, prd, tar, mask=None):
-        retval = self._norms(prd - tar) / self._norms(tar)
+        retval = self._norms(prd, tar) / self._norms(tar)
         if mask is not None:
             retval = retval * mask
         if self.reduction:

@@ -234,6 +234,33 @@ class _AnalysisFn(torch.autograd.Function):
         return gx, None, None
 
 
+class _AnalysisDiffFn(torch.autograd.Function):
+    """Spectral layout of x - x2 (float32 fields of one shape) without storing the difference; backward as of the analysis."""
+
+    @staticmethod
+    def forward(ctx, x, x2, mod):
+        ctx.mod, ctx.shape = mod, x.shape
+        rows = _rows(x.shape[:-2])
+        spec = torch.empty(mod.spectral_shape(rows), dtype=torch.float32, device=x.device)
+        plan = mod.plan(x.device)
+        ws, nbytes = mod.workspace(plan, rows, x.device)
+        check(lib.sfno_sht_analysis_diff(plan.handle, _ptr(x), _ptr(x2), _ptr(spec), rows, _ptr(ws), nbytes, _stream_ptr(x.device)), "sfno_sht_analysis_diff")
+        return spec
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g):
+        mod = ctx.mod
+        g = g.contiguous()
+        rows = _rows(ctx.shape[:-2])
+        gx = torch.empty(ctx.shape, dtype=torch.float32, device=g.device)
+        plan = mod.plan(g.device, adjoint=True)
+        ws, nbytes = mod.workspace(plan, rows, g.device)
+        check(lib.sfno_sht_analysis_adjoint(plan.handle, _ptr(g), _ptr(gx), _lib.DTYPE_F32, rows, _ptr(ws), nbytes, _stream_ptr(g.device)),
+              "sfno_sht_analysis_adjoint")
+        return (gx if ctx.needs_input_grad[0] else None), (-gx if ctx.needs_input_grad[1] else None), None
+
+
 class _InverseFn(torch.autograd.Function):
     """InverseRealSHT.forward on the reference layout; backward = sfno_sht_inverse_adjoint."""
 
@@ -324,6 +351,16 @@ class RealSHT(_SHTBase):
         if x.dtype == torch.bfloat16 and lib.sfno_sht_io_dtype_supported(plan.handle, _lib.DTYPE_BF16):
             return _AnalysisFn.apply(x.contiguous(), self, _lib.DTYPE_BF16)
         return _AnalysisFn.apply(_as_fp32_rows(x, "grid"), self, _lib.DTYPE_F32)
+
+    def analysis_diff(self, x, x2):
+        """analysis(x - x2); float32 fields of one shape and layout without a pass for the difference."""
+        plain = type(x) in (torch.Tensor, torch.nn.Parameter) and type(x2) in (torch.Tensor, torch.nn.Parameter)
+        if not (plain and x.is_cuda and x.dtype == x2.dtype == torch.float32 and x.shape == x2.shape and x.device == x2.device and x.numel() > 0
+                and x.dim() >= 2 and tuple(x.shape[-2:]) == (self.nlat, self.nlon) and x.is_contiguous() and x2.is_contiguous()
+                and x.data_ptr() % 16 == 0 and x2.data_ptr() % 16 == 0
+                and lib.sfno_sht_io_dtype_supported(self.plan(x.device).handle, _lib.DTYPE_BF16)):
+            return self.analysis(x - x2)
+        return _AnalysisDiffFn.apply(x, x2, self)
 
     def _analysis(self, x, dt):
         plan = self.plan(x.device)
