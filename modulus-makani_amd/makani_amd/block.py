@@ -55,18 +55,20 @@ def shapes_fit(params, c_in, embed, lmax):
 
 
 def supported(blk, x, filter_weight=None, skip_weight=None, training=False):
-    """Whether the native block serves this block (whose fusable() the caller has checked) and input; filter_weight, skip_weight: as of
-    forward(); training: with its gradients, see trainable()."""
-    conv, fwd, inv = blk.filter.filter, blk.filter.filter.forward_transform, blk.filter.filter.inverse_transform
+    """The block's parameters (true) where the native block serves this block (whose fusable() the caller has checked) and input, else False;
+    filter_weight, skip_weight: as of forward(); training: with its gradients, see trainable()."""
+    layer, norm0, norm1, act, mlp, skip = blk.filter, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.outer_skip
+    conv = layer.filter
+    fwd, inv = conv.forward_transform, conv.inverse_transform
     convs = mlp_convs(blk)
     if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or convs is None:
         return False
-    if type(blk.norm0) is not nn.InstanceNorm2d or type(blk.norm1) is not nn.InstanceNorm2d or inv.mmax > inv.nlon // 2 + 1:
+    if type(norm0) is not nn.InstanceNorm2d or type(norm1) is not nn.InstanceNorm2d or inv.mmax > inv.nlon // 2 + 1:
         return False
-    if type(blk.act_layer0) is not nn.GELU or type(conv) is not SpectralConv or not plain_conv(blk.outer_skip):
+    if type(act) is not nn.GELU or type(conv) is not SpectralConv or not plain_conv(skip):
         return False
     params = _with(block_params(blk, convs), filter_weight, skip_weight)
-    if training and not trainable(x, params, *convs, blk.outer_skip):
+    if training and not trainable(x, params, *convs, skip):
         return False
     if tuple(x.shape[2:]) != (fwd.nlat, fwd.nlon) or (inv.nlat * inv.nlon) % 8 != 0:
         return False
@@ -76,9 +78,10 @@ def supported(blk, x, filter_weight=None, skip_weight=None, training=False):
         return False
     if not shapes_fit(params, x.shape[1], conv.out_channels, inv.lmax):
         return False
-    wf, *params = [p for p in params if p is not None]
-    return wf.dtype == torch.complex64 and wf.is_cuda and all(p.dtype == torch.float32 and p.is_cuda for p in params) and _no_hooks(
-        blk.filter, conv, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.mlp.fwd, *blk.mlp.fwd, blk.outer_skip)
+    wf, *rest = [p for p in params if p is not None]
+    if wf.dtype != torch.complex64 or not wf.is_cuda or not all(p.dtype == torch.float32 and p.is_cuda for p in rest):
+        return False
+    return params if _no_hooks(layer, conv, norm0, norm1, act, mlp, mlp.fwd, *mlp.fwd, skip) else False
 
 
 def block_params(blk, convs=None):
@@ -131,11 +134,11 @@ class _Call:
         return kept
 
 
-def forward(blk, x, filter_weight=None, skip_weight=None, defer_skip=False):
-    """The block without autograd.  filter_weight, skip_weight: in place of the block's own.  defer_skip: returns (y2, residual, scale,
-    shift) of the last sum scale * y2 + shift + skip(residual) instead of running it."""
+def forward(blk, x, filter_weight=None, skip_weight=None, defer_skip=False, params=None):
+    """The block without autograd.  filter_weight, skip_weight: in place of the block's own (params: what supported() returned for them).
+    defer_skip: returns (y2, residual, scale, shift) of the last sum scale * y2 + shift + skip(residual) instead of running it."""
     x = x.contiguous()
-    c = _Call(blk, x, _with(block_params(blk), filter_weight, skip_weight))
+    c = _Call(blk, x, params or _with(block_params(blk), filter_weight, skip_weight))
     B, E = x.shape[0], c.b.embed
     if not defer_skip:
         out = torch.empty((B, E, *c.P), dtype=torch.bfloat16, device=x.device)
@@ -186,6 +189,6 @@ class _BlockFn(torch.autograd.Function):
         return (gx, None, *(t if n else None for t, n in zip(grads, need[2:])))
 
 
-def train(blk, x):
-    """The block with autograd (supported(training=True) holds)."""
-    return _BlockFn.apply(x, blk, *block_params(blk))
+def train(blk, x, params=None):
+    """The block with autograd (supported(training=True) holds; params: what it returned)."""
+    return _BlockFn.apply(x, blk, *(params or block_params(blk)))

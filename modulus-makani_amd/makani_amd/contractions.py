@@ -11,6 +11,7 @@ from torch.autograd.function import once_differentiable
 
 from . import _lib
 from ._lib import lib, check
+from .sht import _stream_ptr as _stream
 
 
 class PackedWeights:
@@ -35,7 +36,7 @@ class PackedWeights:
             if w.dtype != torch.complex64:
                 raise TypeError(f"dhconv weight must be complex64, got {w.dtype}")
             w = w.contiguous()
-            s = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
+            s = _stream(self.device)
             if adjoint:
                 check(lib.sfno_dhconv_weights_update_adjoint(self.handle, ctypes.c_void_p(w.data_ptr()), s), "sfno_dhconv_weights_update_adjoint")
             else:
@@ -87,10 +88,6 @@ def clear_cache(weight=None):
         _cache.pop(key, None)
 
 
-def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
-
-
 def _weight_grad(spec_in, gspec_out, shape, batch, mmax, triangular):
     """gw[i,o,l] = sum_{b,m} conj(x[b,i,l,m]) g[b,o,l,m] from spectral-layout buffers."""
     I, O, L = shape
@@ -140,7 +137,7 @@ def _dhconv_spectral(spec_in, weight, batch, mmax, triangular, compute, adjoint)
         out.zero_()
     if batch == 0:
         return out
-    s = ctypes.c_void_p(torch.cuda.current_stream(spec_in.device).cuda_stream)
+    s = _stream(spec_in.device)
     check(
         lib.sfno_dhconv_spectral(pw.handle, ctypes.c_void_p(spec_in.data_ptr()), ctypes.c_void_p(out.data_ptr()), batch, mmax, int(triangular), s),
         "sfno_dhconv_spectral",
@@ -199,7 +196,7 @@ def _dhconv(ac, bc, triangular, compute, adjoint):
         return out
     nbytes = lib.sfno_dhconv_workspace_bytes(pw.handle, B, M)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=ac.device)
-    s = ctypes.c_void_p(torch.cuda.current_stream(ac.device).cuda_stream)
+    s = _stream(ac.device)
     check(
         lib.sfno_dhconv(pw.handle, ctypes.c_void_p(ac.data_ptr()), ctypes.c_void_p(out.data_ptr()), B, M, int(triangular),
                         ctypes.c_void_p(ws.data_ptr()), nbytes, s),

@@ -5,22 +5,12 @@ to a per-degree power |c_l0|^2 + 2 sum_{m>0} |c_lm|^2 and weights the degrees wi
 Here the power comes from one kernel that reads the output of the Legendre analysis in place (no pass to the reference
 coefficient layout, no intermediate tensors of the coefficients' size); its gradient feeds the adjoint transform.
 """
-import ctypes
-
 import torch
 from torch import nn
 from torch.autograd.function import once_differentiable
 
 from ._lib import lib, check
-from .sht import RealSHT
-
-
-def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
-
-
-def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+from .sht import RealSHT, _ptr, _stream_ptr as _stream
 
 
 class _DegreePowerFn(torch.autograd.Function):

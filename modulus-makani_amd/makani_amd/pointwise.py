@@ -15,6 +15,7 @@ import torch
 
 from . import _lib
 from ._lib import lib, check
+from .sht import _stream_ptr as _stream
 
 ACT = {None: _lib.ACT_NONE, "none": _lib.ACT_NONE, "gelu": _lib.ACT_GELU}
 
@@ -23,11 +24,7 @@ _wcache = {}
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
-
-
-def _stream(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return t.data_ptr() if t is not None else None
 
 
 def _order(p, packed_on, streams):
@@ -57,7 +54,7 @@ def packed_weight(weight, transposed=False):
     p = torch.empty(lib.sfno_pointwise_weight_elems(O, K), dtype=torch.bfloat16, device=w.device)
     pack = lib.sfno_pointwise_pack_weight_transposed if transposed else lib.sfno_pointwise_pack_weight
     s = torch.cuda.current_stream(w.device)
-    check(pack(_ptr(w), _ptr(p), O, K, ctypes.c_void_p(s.cuda_stream)), "sfno_pointwise_pack_weight")
+    check(pack(_ptr(w), _ptr(p), O, K, s.cuda_stream), "sfno_pointwise_pack_weight")
     _wcache[key] = (weakref.ref(weight, lambda _, k=key: _wcache.pop(k, None)), stamp, p, s, {s.cuda_stream})
     return p
 

@@ -236,10 +236,13 @@ class FourierNeuralOperatorBlock(nn.Module):
         if getattr(self, "fused_pointwise", True) and x.is_cuda and x.dtype == torch.bfloat16:
             # the whole block as one native call, with its gradients while they are recorded
             if torch.is_grad_enabled():
-                if self._fusable() and native_block.supported(self, x, training=True):
-                    return native_block.train(self, x)
-            elif not self.training and fused_pointwise_active(x) and self._fusable() and native_block.supported(self, x):
-                return native_block.forward(self, x, defer_skip=defer_skip)
+                params = self._fusable() and native_block.supported(self, x, training=True)
+                if params:
+                    return native_block.train(self, x, params)
+            elif not self.training and fused_pointwise_active(x):
+                params = self._fusable() and native_block.supported(self, x)
+                if params:
+                    return native_block.forward(self, x, defer_skip=defer_skip, params=params)
         # on the fused inference path the inverse transform hands over the moments norm0 needs together with its output
         want_stats = getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x) and x.dtype == torch.bfloat16 \
             and self._norm0_from_transform() and self._fusable()
@@ -395,12 +398,12 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
     # into the block's spectral weight (w'[j, o, l] = sum_i W2[i, j] w[i, o, l], computed once per weight update) and into the
     # skip convolution of the residual (W_skip W2).  W2 enters with its bf16-rounded values, as autocast would use it; what
     # differs from the layer-by-layer evaluation is one bf16 rounding of the 384-channel field that is no longer made.
-    def _encoder_fold(self):
+    def _encoder_fold(self, enc=None):
         """(encoder steps without the last convolution, folded spectral weight, folded skip weight), or None where the
         shortcut does not apply."""
         if not getattr(self, "fold_encoder", True) or self.repeat_layers != 1 or len(self.blocks) == 0:
             return None
-        enc = _fused_chain(self.encoder.fwd)
+        enc = enc or _fused_chain(self.encoder.fwd)
         blk = self.blocks[0]
         conv = blk.filter.filter
         if enc is None or len(enc) < 2 or enc[-1][1] is not None or enc[-1][0].bias is not None:
@@ -422,7 +425,8 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
                 w2b = w2.detach().reshape(w2.shape[0], w2.shape[1]).to(torch.bfloat16).float()        # [i, j]
                 wf = torch.einsum("ij,iol->jol", w2b.to(torch.complex64), w0.detach()).contiguous()
                 wsb = ws.detach().reshape(ws.shape[0], ws.shape[1]).to(torch.bfloat16).float()
-                wsk = (wsb @ w2b).reshape(ws.shape[0], w2.shape[1], 1, 1).contiguous()
+                # (under autocast the product comes out as bfloat16, which the native block does not take)
+                wsk = (wsb @ w2b).float().reshape(ws.shape[0], w2.shape[1], 1, 1).contiguous()
             cached = (stamp, wf, wsk)
             self._fold_cache = cached
         return enc[:-1], cached[1], cached[2]
@@ -438,8 +442,9 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         blk = self.blocks[0]
         conv = blk.filter.filter
         B = h.shape[0]
-        if native_block.supported(blk, h, wf, wsk):
-            return native_block.forward(blk, h, wf, wsk)
+        params = native_block.supported(blk, h, wf, wsk)
+        if params:
+            return native_block.forward(blk, h, wf, wsk, params=params)
         spec = conv.forward_transform.analysis(h)
         residual = conv.inverse_transform.synthesis(spec, (B, h.shape[1]), dtype=torch.bfloat16)
         spec = dhconv_spectral(spec, wf, B, conv.modes_lon, triangular=conv._triangular, compute=conv.compute)
@@ -453,18 +458,18 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
     # linear, so they are one convolution over the two tensors m and r, with the weight [W_d diag(scale) | W_d W_skip] and the
     # bias W_d shift + b_d of each sample: the sum is never written and the skip convolution's 384 x 384 products per pixel at
     # full resolution are not computed.  W_d and W_skip enter with their bf16-rounded values, as autocast would use them.
-    def _decoder_merge_ok(self):
+    def _decoder_merge_ok(self, dec=None):
         if not getattr(self, "merge_decoder", True) or self.repeat_layers != 1 or len(self.blocks) < 2:
             return False
-        dec = _fused_chain(self.decoder.fwd)
+        dec = dec or _fused_chain(self.decoder.fwd)
         blk = self.blocks[-1]
         if dec is None or not (isinstance(blk, FourierNeuralOperatorBlock) and blk._fusable() and getattr(blk, "fused_pointwise", True)):
             return False
         wd = dec[0][0].weight
         return wd.shape[0] > 96 and wd.shape[1] == blk.outer_skip.weight.shape[0]
 
-    def _tail_cat_ok(self):
-        dec = _fused_chain(self.decoder.fwd)
+    def _tail_cat_ok(self, dec=None):
+        dec = dec or _fused_chain(self.decoder.fwd)
         return bool(self.big_skip and getattr(self, "merge_decoder", True) and dec and dec[-1][1] is None)
 
     def _tail_weight(self, conv):
@@ -479,10 +484,10 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
             self._tail_cache = cached
         return cached[1]
 
-    def _decoder_merged(self, x):
+    def _decoder_merged(self, x, dec):
         """Last block and the decoder's first step for the output x of the block before it; returns the result and the decoder
         steps still to run."""
-        blk, dec = self.blocks[-1], _fused_chain(self.decoder.fwd)
+        blk = self.blocks[-1]
         conv_d = dec[0][0]
         out = blk(x, defer_skip=True)
         if not isinstance(out, tuple):           # the block could not take its fused path after all: layer by layer from here
@@ -512,9 +517,9 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
             pw.conv1x1_cat(m[b:b + 1], r[b:b + 1], wcat[b], bias[b], dec[0][1], out=y[b:b + 1])
         return y, dec[1:]
 
-    def _forward_fused(self, x):
-        """Encoder, blocks and decoder with every 1x1 convolution on the fused bf16 kernels (inference under bf16 autocast)."""
-        enc, dec = _fused_chain(self.encoder.fwd), _fused_chain(self.decoder.fwd)
+    def _forward_fused(self, x, enc, dec):
+        """Encoder, blocks and decoder with every 1x1 convolution on the fused bf16 kernels (inference under bf16 autocast); enc, dec:
+        their steps, see _fusable."""
         xb = x.to(torch.bfloat16).contiguous()
         cat_tail = False
         if self.big_skip:
@@ -524,11 +529,11 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
                 residual = xb
             # the decoder's last convolution and residual_transform feed one sum (sfnonet.py:636-638): one convolution over
             # the two tensors with the weight [W_last | W_res]; where that does not apply the residual is convolved here
-            cat_tail = self._tail_cat_ok()
+            cat_tail = self._tail_cat_ok(dec)
             if not cat_tail:
                 residual = pw.conv1x1(residual, self.residual_transform.weight)
-        fold = self._encoder_fold()
-        merge = self._decoder_merge_ok()
+        fold = self._encoder_fold(enc)
+        merge = self._decoder_merge_ok(dec)
         if fold is not None:
             x = self._block0_folded(_run_chain(fold[0], xb), fold[1], fold[2])
             rest = self.blocks[1:]
@@ -542,7 +547,7 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         for blk in (rest[:-1] if merge else rest):
             x = blk(x)
         if merge:
-            x, dec = self._decoder_merged(x.to(torch.bfloat16).contiguous())
+            x, dec = self._decoder_merged(x.to(torch.bfloat16).contiguous(), dec)
         x = x.to(torch.bfloat16).contiguous()
         if self.big_skip and cat_tail:
             if not dec:                           # the merged convolution was the decoder's last step: the residual is still to be added
@@ -555,17 +560,20 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         return _run_chain(dec, x, residual if self.big_skip else None)
 
     def _fusable(self, x):
+        """(encoder steps, decoder steps) where the fused path serves the network and the input, else None."""
         if not (getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x)) or hasattr(self, "pos_embed"):
-            return False
+            return None
         if not isinstance(self.pos_drop, nn.Identity) or (self.out_shape[0] * self.out_shape[1]) % 8 != 0:
-            return False
+            return None
         if self.big_skip and not (_is_conv1x1(self.residual_transform) and self.residual_transform.bias is None):
-            return False
-        return _fused_chain(self.encoder.fwd) is not None and _fused_chain(self.decoder.fwd) is not None
+            return None
+        enc, dec = _fused_chain(self.encoder.fwd), _fused_chain(self.decoder.fwd)
+        return (enc, dec) if enc is not None and dec is not None else None
 
     def forward(self, x):
-        if self._fusable(x):
-            return self._forward_fused(x)
+        steps = self._fusable(x)
+        if steps is not None:
+            return self._forward_fused(x, *steps)
         if self.big_skip:
             if self.out_shape != self.inp_shape:
                 xtype = x.dtype

@@ -11,6 +11,7 @@ buffers, so the modules add nothing to a state_dict -- like the non-persistent b
 of the reference modules.
 """
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -82,11 +83,12 @@ class _Plan:
 
 
 def _stream_ptr(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """Handle of the device's current stream, without the Stream object that torch.cuda.current_stream builds around it."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 class _SHTBase(nn.Module):
@@ -129,7 +131,8 @@ class _SHTBase(nn.Module):
 
     def plan(self, device, adjoint=False):
         """Device plan of the transform, or (built on the first backward pass) of its adjoint."""
-        device = torch.device(device)
+        if type(device) is not torch.device:
+            device = torch.device(device)
         if device.type != "cuda":
             raise RuntimeError("the SFNO spectral kernels run on a HIP device only; move the input to the GPU")
         index = device.index if device.index is not None else torch.cuda.current_device()
@@ -184,7 +187,7 @@ def _as_fp32_rows(x, tail):
 
 
 def _rows(lead):
-    return int(np.prod(lead)) if len(lead) else 1
+    return math.prod(lead)
 
 
 class _ForwardFn(torch.autograd.Function):

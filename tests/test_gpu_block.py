@@ -433,3 +433,28 @@ def test_blocks_without_a_norm_train_on_the_modules(lib_built):
         with torch.no_grad():
             y = net.eval()(x)
     assert torch.isfinite(y).all() and all(p.grad is not None for p in net.parameters())
+
+
+def test_every_block_of_a_network_is_one_native_call(lib_built):
+    """Under autocast the skip weight folded with the encoder stays float32, so the first block is served like the others."""
+    import makani_amd as ma
+    from makani_amd import block as nb
+
+    torch.manual_seed(8)
+    net = ma.SphericalFourierNeuralOperatorNet(inp_shape=(32, 64), out_shape=(32, 64), scale_factor=4, inp_chans=3, out_chans=3, embed_dim=16, num_layers=3,
+                                               operator_type="dhconv").cuda().eval()
+    x = torch.randn(2, 3, 32, 64, device="cuda")
+    calls = []
+    keep = nb.forward
+    nb.forward = lambda *a, **k: calls.append(1) or keep(*a, **k)
+    try:
+        with torch.inference_mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+            got = net(x)
+    finally:
+        nb.forward = keep
+    assert len(calls) == 3 and net._fold_cache[2].dtype == torch.float32
+    net.fused_pointwise = False
+    for b in net.blocks:
+        b.fused_pointwise = False
+    with torch.inference_mode():
+        assert rel(got, net(x)) < 3e-2
