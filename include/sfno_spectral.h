@@ -237,6 +237,9 @@ int sfno_dhconv_weights_destroy(sfno_dhconv_weights* w);
  * map the gradient of the output to the gradient of the input: gx[b,i,l,m] = sum_o gy[b,o,l,m]
  * conj(w[i,o,l]) -- the backward of the einsum at contractions.py:130-136 with respect to `ac`. */
 int sfno_dhconv_weights_update_adjoint(sfno_dhconv_weights* w, const void* weight, void* stream);
+/* Both of the above for a training step: fills w (in_channels, out_channels, lmax) and adj (out_channels, in_channels, lmax), two handles of
+ * one device, from one reading of the parameter where their compute mode has a kernel for it. */
+int sfno_dhconv_weights_update_both(sfno_dhconv_weights* w, sfno_dhconv_weights* adj, const void* weight, void* stream);
 
 /* y[b,o,l,m] = sum_i x[b,i,l,m] w[i,o,l] on spectral-layout buffers:
  * spec_in rows = batch*in_channels, spec_out rows = batch*out_channels.  With

@@ -557,6 +557,16 @@ extern "C" int sfno_dhconv_weights_update_adjoint(sfno_dhconv_weights* w, const 
     return pack_weights(w, weight, 1, stream);
 }
 
+extern "C" int sfno_dhconv_weights_update_both(sfno_dhconv_weights* w, sfno_dhconv_weights* adj, const void* weight, void* stream) {
+    if (!w || !adj || !weight || w == adj || adj->I != w->O || adj->O != w->I || adj->L != w->L || adj->device != w->device) return SFNO_EINVAL;
+    if (w->f16 && adj->f16) {
+        const int rc = dhconv_pack_both_f16_launch(reinterpret_cast<const float2*>(weight), *w, *adj, (hipStream_t)stream);
+        if (rc != SFNO_EUNSUPPORTED) return rc;
+    }
+    const int rc = pack_weights(w, weight, 0, stream);
+    return rc == SFNO_OK ? pack_weights(adj, weight, 1, stream) : rc;
+}
+
 extern "C" int sfno_dhconv_weight_grad(int I, int O, int L, const float* spec_in, const float* gspec_out, void* gweight, int batch,
                                        int mmax, int triangular, void* stream) {
     if (I < 1 || O < 1 || L < 1 || !spec_in || !gspec_out || !gweight || batch < 1 || mmax < 1) return SFNO_EINVAL;

@@ -409,6 +409,164 @@ int dhconv_pack_f16_launch(const float2* w, void* packed, float* cinv, float* cm
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
+// A weight w[i][o][l] and its conjugate transpose packed together (training: the backward wants the second one).  HBM bounds this: one
+// reading for both maxima and one for both packings instead of two each, and the writes.  384 x 384 x 240 (283 MB) 370 -> 272 us for the pair
+// (maxima 94, packing 174), 128 x 128 x 90 30 -> 17.4, 32 x 32 x 4 18.7 -> 11.5 (launches).
+//
+// cmax[o][l] over the input channels and amax[i][l] over the output channels: a workgroup takes 16 x 16 channel pairs of 64 degrees, a
+// wavefront two input channels and a lane one degree (runs of 512 bytes: 384 x 384 x 240 in 94 us; 32 x 32 pairs of 16 degrees, runs of 128 bytes: 213).  The
+// maxima leave as above.  Degrees [lb, lb + ln).  grid (ceil(O / 16), ceil(I / 16), ceil(ln / 64)), block 512
+__global__ __launch_bounds__(256) void dhconv_bothmax_clear_kernel(float* __restrict__ cmax, int64_t n, float* __restrict__ amax, int64_t na) {
+    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx < n) cmax[idx] = 0.f;
+    if (idx < na) amax[idx] = 0.f;
+}
+__global__ __launch_bounds__(512) void dhconv_bothmax_kernel(const float2* __restrict__ w, float* __restrict__ cmax, float* __restrict__ amax, int I, int O,
+                                                             int L, int lb, int ln) {
+    __shared__ float part[8][16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int o0 = 16 * blockIdx.x, i0 = 16 * blockIdx.y + 2 * wave;
+    const int l = lb + 64 * blockIdx.z + lane;
+    const bool in = l < lb + ln;
+    // (no load under a branch: channels past the end repeat the last one's values)
+    const int lc = in ? l : lb;
+    float2 z[2][16];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) z[e][k] = w[((int64_t)min(i0 + e, I - 1) * O + min(o0 + k, O - 1)) * L + lc];
+    float cm[16], rm[2] = {0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        cm[k] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = fmaxf(fabsf(z[e][k].x), fabsf(z[e][k].y));
+            cm[k] = fmaxf(cm[k], v);
+            rm[e] = fmaxf(rm[e], v);
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        if (in && i0 + e < I) atomicMax(reinterpret_cast<unsigned int*>(amax) + (int64_t)(i0 + e) * L + l, __float_as_uint(rm[e]));
+#pragma unroll
+    for (int k = 0; k < 16; ++k) part[wave][k][lane] = cm[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = wave; k < 16; k += 8) {
+        float v = part[0][k][lane];
+#pragma unroll
+        for (int p = 1; p < 8; ++p) v = fmaxf(v, part[p][k][lane]);
+        if (in && o0 + k < O) atomicMax(reinterpret_cast<unsigned int*>(cmax) + (int64_t)(o0 + k) * L + l, __float_as_uint(v));
+    }
+}
+
+// One operand stream of dhconv_pack_both_kernel (layout as dhconv_pack_f16_kernel writes it).
+struct DhfStream {
+    unsigned char* packed;
+    float* cinv;
+    const float* cmax;
+    int nob, nc, co;                // column blocks, chunks of 16 input channels, channels per column block
+};
+__device__ __forceinline__ int dhf_shift(const float* __restrict__ cmax, int64_t idx) {
+    const unsigned int mb = __builtin_bit_cast(unsigned int, cmax[idx]);
+    return mb != 0 ? DHF_SH - (int)(mb >> 23) : 0;
+}
+// eight values of a column, scaled by 2^sh, as the four pieces of their half chunk
+template <class Get>
+__device__ __forceinline__ void dhf_store_pieces(unsigned char* dst, int co, int sh, float sign, Get get) {
+    unsigned short h[2][2][8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float2 z = get(e);
+#pragma unroll
+        for (int part = 0; part < 2; ++part) {
+            const float v = __builtin_ldexpf(part ? sign * z.y : z.x, sh);
+            const _Float16 v0 = (_Float16)v;
+            h[part][0][e] = __builtin_bit_cast(unsigned short, v0);
+            h[part][1][e] = __builtin_bit_cast(unsigned short, (_Float16)(v - (float)v0));
+        }
+    }
+#pragma unroll
+    for (int pp = 0; pp < 4; ++pp) {
+        u4 piece;
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2)
+            piece[e2] = (unsigned int)h[pp >> 1][pp & 1][2 * e2] | ((unsigned int)h[pp >> 1][pp & 1][2 * e2 + 1] << 16);
+        *reinterpret_cast<u4*>(dst + pp * co * 32) = piece;
+    }
+}
+// A workgroup moves 16 input x 32 output channels of 16 degrees through LDS: as a chunk of the weight (f, lane = half chunk and output
+// channel) and as 16 columns of two chunks of its conjugate transpose (t, lane = half chunk and input channel; the input channels' pitch
+// spreads them over all banks).  Tiles that only one of the streams has, in its padding, are zeros.
+// grid (tiles of 16 input channels, tiles of 32 output channels, ceil(ln / 16)), block 512
+constexpr int DHF_PITCH = 32 * (DHF_PL + 1) + 1;
+__global__ __launch_bounds__(512) void dhconv_pack_both_kernel(const float2* __restrict__ w, DhfStream f, DhfStream t, int I, int O, int L, int lb) {
+    __shared__ float2 tile[DHF_KC * DHF_PITCH];
+    const int ti = blockIdx.x, to = blockIdx.y;
+    const int l0 = lb + blockIdx.z * DHF_PL;
+    const int tid = threadIdx.x, dl = tid & (DHF_PL - 1);
+#pragma unroll
+    for (int pass = 0; pass < DHF_PL; ++pass) {
+        const int pr = pass * (512 / DHF_PL) + tid / DHF_PL;     // sixteen lanes per pair: one 128-byte segment
+        const int ii = pr >> 5, o = pr & 31;
+        const int i = DHF_KC * ti + ii, oo = 32 * to + o, l = l0 + dl;
+        float2 z = make_float2(0.f, 0.f);
+        if (i < I && oo < O && l < L) z = w[((int64_t)i * O + oo) * L + l];
+        tile[ii * DHF_PITCH + o * (DHF_PL + 1) + dl] = z;
+    }
+    const int lane = tid & 63, wave = tid >> 6;                  // wavefront -> degrees wave and wave + 8
+    const int of = lane & 31, kf = lane >> 5, it = lane & 15, ot = lane >> 4;
+    const int oo = 32 * to + of, ii = DHF_KC * ti + it, ct = 2 * to + (ot >> 1);
+    const bool has_f = ti < f.nc && 32 * to < f.nob * f.co, has_t = ct < t.nc && DHF_KC * ti < t.nob * t.co;
+    int sf[2], st[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int l = l0 + 8 * k + wave;
+        sf[k] = oo < O && l < L ? dhf_shift(f.cmax, (int64_t)oo * L + l) : 0;
+        st[k] = ii < I && l < L ? dhf_shift(t.cmax, (int64_t)ii * L + l) : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const int d = 8 * k + wave, l = l0 + d;
+        if (l >= L) break;
+        if (has_f) {
+            if (ti == 0 && kf == 0) f.cinv[(int64_t)l * (f.nob * f.co) + oo] = __builtin_ldexpf(1.0f, -sf[k]);
+            unsigned char* dst = f.packed + (((int64_t)l * f.nob + oo / f.co) * f.nc + ti) * (f.co * 128) + dhf_piece(oo % f.co, kf);
+            dhf_store_pieces(dst, f.co, sf[k], 1.f, [&](int e) { return tile[(8 * kf + e) * DHF_PITCH + of * (DHF_PL + 1) + d]; });
+        }
+        if (has_t) {
+            if (to == 0 && ot == 0) t.cinv[(int64_t)l * (t.nob * t.co) + ii] = __builtin_ldexpf(1.0f, -st[k]);
+            unsigned char* dst = t.packed + (((int64_t)l * t.nob + ii / t.co) * t.nc + ct) * (t.co * 128) + dhf_piece(ii % t.co, ot & 1);
+            dhf_store_pieces(dst, t.co, st[k], -1.f, [&](int e) { return tile[it * DHF_PITCH + (8 * ot + e) * (DHF_PL + 1) + d]; });
+        }
+    }
+}
+
+// weight bytes of a slab here, where twice as much is written; whole groups of 64 degrees
+constexpr int64_t DHF_SLAB_BOTH_BYTES = 80 << 20;
+int dhconv_pack_both_f16_launch(const float2* w, const sfno_dhconv_weights& fw, const sfno_dhconv_weights& tw, hipStream_t s) {
+    const int I = fw.I, O = fw.O, L = fw.L;
+    auto stream = [](const sfno_dhconv_weights& h) {
+        return DhfStream{reinterpret_cast<unsigned char*>(h.d_W), h.d_cinv, h.d_cmax, h.nob, h.nc, 32 * dhconv_f16_ntc(h.O)};
+    };
+    const DhfStream f = stream(fw), t = stream(tw);
+    const int64_t nti = std::max<int64_t>(f.nc, (int64_t)t.nob * t.co / 16), nto = std::max<int64_t>((int64_t)f.nob * f.co / 32, (t.nc + 1) / 2);
+    const int64_t cols = (int64_t)std::max(I, O) * L;
+    if (nto > 65535 || (I + 15) / 16 > 65535 || (cols + 255) / 256 > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
+    const int64_t per64 = (int64_t)sizeof(float2) * I * O * 64;
+    // (a grid has at most 65535 layers of 16 degrees)
+    const int slab = 64 * (int)std::max<int64_t>(1, std::min({(int64_t)(L + 63) / 64, DHF_SLAB_BOTH_BYTES / per64, (int64_t)16383}));
+    hipLaunchKernelGGL(dhconv_bothmax_clear_kernel, dim3((unsigned)((cols + 255) / 256)), dim3(256), 0, s, fw.d_cmax, (int64_t)O * L, tw.d_cmax, (int64_t)I * L);
+    for (int lb = 0; lb < L; lb += slab) {
+        const int ln = std::min(slab, L - lb), nl = (ln + DHF_PL - 1) / DHF_PL;
+        hipLaunchKernelGGL(dhconv_bothmax_kernel, dim3((O + 15) / 16, (I + 15) / 16, (ln + 63) / 64), dim3(512), 0, s, w, fw.d_cmax, tw.d_cmax, I, O, L, lb, ln);
+        hipLaunchKernelGGL(dhconv_pack_both_kernel, dim3((unsigned)nti, (unsigned)nto, nl), dim3(512), 0, s, w, f, t, I, O, L, lb);
+    }
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
 int dhconv_f16_launch(const DhconvArgs& a, hipStream_t s) {
     const int64_t rows_max = (int64_t)a.M * a.B;
     if (rows_max <= 0 || a.L <= 0) return SFNO_OK;

@@ -72,6 +72,8 @@ int dhconv_pack_split_launch(const float2* w, void* packed, int I, int O, int L,
 int dhconv_f16_ntc(int O);
 int dhconv_f16_launch(const DhconvArgs& a, hipStream_t s);
 int dhconv_pack_f16_launch(const float2* w, void* packed, float* cinv, float* cmax, int I, int O, int L, int adjoint, hipStream_t s);
+// both handles f16, tw of shape (O, I, L): the weight into fw, its conjugate transpose into tw
+int dhconv_pack_both_f16_launch(const float2* w, const sfno_dhconv_weights& fw, const sfno_dhconv_weights& tw, hipStream_t s);
 // adjoint = 1 packs the conjugate transpose: w then has shape [O][I][L] and element (i, o) is conj(w[o][i])
 int dhconv_pack_bf16_launch(const float2* w, void* packed, int I, int O, int L, int adjoint, hipStream_t s);
 // gradient of the contraction with respect to its weight:

@@ -84,6 +84,7 @@ def _load():
         "sfno_dhconv_weights_update": (i32, [vp, vp, vp]),
         "sfno_dhconv_weights_destroy": (i32, [vp]),
         "sfno_dhconv_weights_update_adjoint": (i32, [vp, vp, vp]),
+        "sfno_dhconv_weights_update_both": (i32, [vp, vp, vp, vp]),
         "sfno_dhconv_weight_grad": (i32, [i32, i32, i32, vp, vp, vp, i32, i32, i32, vp]),
         "sfno_dhconv_spectral": (i32, [vp, vp, vp, i32, i32, i32, vp]),
         "sfno_dhconv_workspace_bytes": (sz, [vp, i32, i32]),

@@ -100,13 +100,13 @@ class _Call:
     """The sfno_block structure of one call, and what has to stay alive while it is used.  The values come from `params` alone: the
     modules may hold others by the time of the backward (functional calls, parametrisations)."""
 
-    def __init__(self, blk, x, params, backward=False):
+    def __init__(self, blk, x, params, backward=False, training=False):
         conv = blk.filter.filter
         fwd, inv = conv.forward_transform, conv.inverse_transform
         wf, wskip, w1, b1, w2, b2, g0, be0, g1, be1 = params
         dev = x.device
         b = _lib.Block()
-        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(wf, conv.compute), pw.packed_weight(w1), pw.packed_weight(w2), pw.packed_weight(wskip)]
+        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(wf, conv.compute, both=training), pw.packed_weight(w1), pw.packed_weight(w2), pw.packed_weight(wskip)]
         b.fwd, b.inv, b.weights = keep[0].handle, keep[1].handle, keep[2].handle
         b.w1, b.w2, b.wskip = (t.data_ptr() for t in keep[3:6])
         if backward:
@@ -161,7 +161,7 @@ class _BlockFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, blk, *params):
         x = x.detach().contiguous()
-        c = _Call(blk, x, params)
+        c = _Call(blk, x, params, training=any(ctx.needs_input_grad))
         out = torch.empty((x.shape[0], c.b.embed, *c.P), dtype=torch.bfloat16, device=x.device)
         kept = c.forward(x, 1, out)
         ctx.blk = blk

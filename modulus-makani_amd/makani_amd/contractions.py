@@ -26,10 +26,11 @@ class PackedWeights:
         with torch.cuda.device(self.device):
             check(lib.sfno_dhconv_weights_create(in_channels, out_channels, lmax, COMPUTE[compute], ctypes.byref(self.handle)), "sfno_dhconv_weights_create")
 
-    def refresh(self, weight, adjoint=False):
+    def refresh(self, weight, adjoint=False, partner=None):
         """Re-pack if the parameter changed (in-place updates bump ``_version``).
 
-        adjoint: this handle has shape (O, I, L) and is filled with the conjugate transpose of ``weight`` [I, O, L]."""
+        adjoint: this handle has shape (O, I, L) and is filled with the conjugate transpose of ``weight`` [I, O, L].
+        partner: the weight's adjoint handle, filled along with this one if it is out of date as well."""
         stamp = (weight.data_ptr(), -1 if weight.is_inference() else weight._version)
         if stamp != self.stamp:
             w = weight.detach()
@@ -37,7 +38,10 @@ class PackedWeights:
                 raise TypeError(f"dhconv weight must be complex64, got {w.dtype}")
             w = w.contiguous()
             s = _stream(self.device)
-            if adjoint:
+            if partner is not None and partner.stamp != stamp:
+                check(lib.sfno_dhconv_weights_update_both(self.handle, partner.handle, ctypes.c_void_p(w.data_ptr()), s), "sfno_dhconv_weights_update_both")
+                partner.stamp = stamp
+            elif adjoint:
                 check(lib.sfno_dhconv_weights_update_adjoint(self.handle, ctypes.c_void_p(w.data_ptr()), s), "sfno_dhconv_weights_update_adjoint")
             else:
                 check(lib.sfno_dhconv_weights_update(self.handle, ctypes.c_void_p(w.data_ptr()), s), "sfno_dhconv_weights_update")
@@ -58,9 +62,16 @@ COMPUTE = {"fp32": _lib.COMPUTE_FP32, "bf16": _lib.COMPUTE_BF16, "fp32_bf16x3": 
 _cache = {}
 
 
-def packed_for(weight, compute="fp32", adjoint=False):
+def packed_for(weight, compute="fp32", adjoint=False, both=False):
     """Packed handle for a weight tensor (or, for the backward pass, for its conjugate transpose), cached per
-    tensor object and refreshed when it changes."""
+    tensor object and refreshed when it changes.
+
+    both: a backward pass will follow, so the conjugate transpose is packed in the same pass over the weight."""
+    p = _handle_for(weight, compute, adjoint)
+    return p.refresh(weight, adjoint, _handle_for(weight, compute, True) if both and not adjoint else None)
+
+
+def _handle_for(weight, compute, adjoint):
     if weight.device.type != "cuda":
         raise RuntimeError("the dhconv kernel runs on a HIP device only")
     if compute not in COMPUTE:
@@ -72,7 +83,7 @@ def packed_for(weight, compute="fp32", adjoint=False):
     if p is None or p.device != weight.device or p.shape != shape:
         p = PackedWeights(shape[0], shape[1], shape[2], weight.device, compute)
         _cache[key] = (weakref.ref(weight, lambda _, k=key: _cache.pop(k, None)), p)
-    return p.refresh(weight, adjoint)
+    return p
 
 
 def clear_cache(weight=None):
@@ -107,7 +118,7 @@ class _DhconvSpectralFn(torch.autograd.Function):
     def forward(ctx, spec_in, weight, batch, mmax, triangular, compute):
         ctx.save_for_backward(spec_in, weight)
         ctx.cfg = (batch, mmax, triangular, compute)
-        return _dhconv_spectral(spec_in, weight, batch, mmax, triangular, compute, False)
+        return _dhconv_spectral(spec_in, weight, batch, mmax, triangular, compute, False, ctx.needs_input_grad[0])
 
     @staticmethod
     @once_differentiable
@@ -128,8 +139,8 @@ def dhconv_spectral(spec_in, weight, batch, mmax, triangular=True, compute="fp32
     return _DhconvSpectralFn.apply(spec_in.contiguous(), weight, batch, mmax, triangular, compute)
 
 
-def _dhconv_spectral(spec_in, weight, batch, mmax, triangular, compute, adjoint):
-    pw = packed_for(weight, compute, adjoint)
+def _dhconv_spectral(spec_in, weight, batch, mmax, triangular, compute, adjoint, both=False):
+    pw = packed_for(weight, compute, adjoint, both)
     I, O, L = pw.shape
     ld_out = int(lib.sfno_spectral_ld(batch * O))
     out = torch.empty((mmax, L, ld_out), dtype=torch.float32, device=spec_in.device)

@@ -231,3 +231,26 @@ def test_real_weight_contractions_and_their_gradients(lib_built, operator_type):
     assert wg.grad.dtype == torch.float32 and rel_l2(wg.grad.cpu().numpy(), wr.grad.numpy()) < TOL
     with pytest.raises(NotImplementedError):
         ma.get_contract_fun(wg, separable=True, complex=False, operator_type=operator_type)(ag, wg)
+
+
+@pytest.mark.parametrize("I,O,L,M", [(2, 4, 1, 2), (8, 6, 5, 6), (64, 48, 40, 41), (70, 130, 17, 9), (34, 258, 33, 12), (256, 20, 16, 17), (5, 8, 6, 6)])
+def test_weight_and_adjoint_packed_together(lib_built, I, O, L, M):
+    """Both operand streams from one reading of the weight hold what the two separate packings hold: the contractions with them
+    give the same bits (tiles of 16 x 32 channels x 16 degrees with remainders; the last case has no joint kernel)."""
+    from makani_amd import contractions as C
+
+    print(f"case pack both I={I} O={O} L={L} M={M}", flush=True)
+    g = torch.Generator().manual_seed(6)
+    w = (torch.randn(I, O, L, dtype=torch.complex64, generator=g) * torch.exp(3.0 * torch.randn(I, O, L, generator=g)))
+    w[:, O // 2] = 0                                                     # a column without a scale
+    w[I // 2, :, L - 1] = 0                                              # and one of the adjoint
+    w = w.cuda()
+    x = torch.randn(2, I, L, M, dtype=torch.complex64, generator=g).cuda()
+    y = torch.randn(2, O, L, M, dtype=torch.complex64, generator=g).cuda()
+    want = [C._dhconv(x, w, False, "fp32", False), C._dhconv(y, w, False, "fp32", True)]
+    C.clear_cache(w)
+    C.packed_for(w, both=True)
+    assert C._handle_for(w, "fp32", True).stamp == C._handle_for(w, "fp32", False).stamp
+    got = [C._dhconv(x, w, False, "fp32", False), C._dhconv(y, w, False, "fp32", True)]
+    assert all(torch.isfinite(t).all() for t in got)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
