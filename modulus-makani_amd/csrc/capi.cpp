@@ -385,6 +385,12 @@ extern "C" int sfno_sht_forward(const sfno_sht_plan* p, const float* x, void* co
         const int rc = planar_direct(p, MS_FWD, false, x, coeffs, rows, workspace, w.bytes, (hipStream_t)stream);
         if (rc != SFNO_EUNSUPPORTED) return rc;
     }
+    if (!planar(p) && x && rows_ok(rows) && (p->directions & SFNO_DIR_FORWARD) && legendre_coeffs_fit(true, p->format, rows, p->lmax, p->mmax)) {
+        const int rc = sfno_rfft(p, x, SFNO_DTYPE_F32, w.xm, rows, stream);
+        if (rc != SFNO_OK) return rc;
+        const PgemmArgs a = legendre_args(p, p->fwd, w.xm, reinterpret_cast<float*>(coeffs), sfno_spectral_ld(rows));
+        return legendre_coeffs_launch(true, a, rows, p->fwd.n_work, (hipStream_t)stream);
+    }
     int rc = sfno_sht_analysis(p, x, SFNO_DTYPE_F32, w.spec, rows, workspace, workspace_bytes, stream);
     if (rc != SFNO_OK) return rc;
     return spectral_to_coeffs_launch(w.spec, reinterpret_cast<float2*>(coeffs), rows, p->lmax, p->mmax,
@@ -399,6 +405,12 @@ extern "C" int sfno_sht_inverse(const sfno_sht_plan* p, const void* coeffs, floa
     if (planar(p) && coeffs && (p->directions & SFNO_DIR_INVERSE)) {
         const int rc = planar_direct(p, MS_INV, true, coeffs, x, rows, workspace, w.bytes, (hipStream_t)stream);
         if (rc != SFNO_EUNSUPPORTED) return rc;
+    }
+    if (!planar(p) && x && rows_ok(rows) && (p->directions & SFNO_DIR_INVERSE) && legendre_coeffs_fit(false, p->format, rows, p->lmax, p->mmax)) {
+        const PgemmArgs a = legendre_args(p, p->inv, reinterpret_cast<const float*>(coeffs), w.xm, sfno_spectral_ld(rows));
+        const int rc = legendre_coeffs_launch(false, a, rows, p->inv.n_work, (hipStream_t)stream);
+        if (rc != SFNO_OK) return rc;
+        return sfno_irfft(p, w.xm, x, SFNO_DTYPE_F32, rows, stream);
     }
     int rc = coeffs_to_spectral_launch(reinterpret_cast<const float2*>(coeffs), w.spec, rows, p->lmax, p->mmax,
                                        (int)sfno_spectral_ld(rows), planar(p) ? 0 : 1, (hipStream_t)stream);

@@ -42,7 +42,9 @@ constexpr int lh_occupancy(int nt, bool analysis) { return nt <= 4 ? 4 : analysi
 
 __device__ __forceinline__ unsigned int lh_pk(float a, float b) { return __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(a, b)); }
 
-template <int NT, bool ANALYSIS>
+// COEFFS: the spectral side is the reference layout, complex [rows][lmax][mmax] (zeros above the diagonal included), and no layout pass
+// runs: an order's values lie 8 mmax bytes apart there, eight bytes at a time, so this is for small transforms only (legendre_coeffs_fit).
+template <int NT, bool ANALYSIS, bool COEFFS>
 __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_kernel(PgemmArgs a) {
     constexpr int TN = 32 * NT;            // columns per workgroup
     constexpr int QN = TN / 4;             // column quads
@@ -89,7 +91,10 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     const bool active = rb < nrb;
 
     const float* xm_m = (ANALYSIS ? a.Q : a.Out) + (int64_t)m * nlat * ld;     // Fourier panel of order m
-    const float* sp_m = (ANALYSIS ? a.Out : a.Q) + (int64_t)m * lmax * ld;     // spectral panel of order m
+    const float* sp_m = (ANALYSIS ? a.Out : a.Q) + (COEFFS ? 2 * (int64_t)m : (int64_t)m * lmax * ld);     // spectral panel of order m
+    const int nval = COEFFS ? a.ncol : ld;         // columns with values on the spectral side
+    const uint32_t srow = COEFFS ? 2u * a.mmax : (uint32_t)ld;       // floats from degree to degree, and the column's offset
+    auto scolumn = [&](int n) { return COEFFS ? (uint32_t)(n >> 1) * (uint32_t)lmax * srow + (uint32_t)(n & 1) : (uint32_t)n; };
     // Index entry of a row block: first block of its stream | leading chunks left out << 48 (their entries are negligible:
     // towards the poles the table falls off like sin^m(theta)).  The K loop of the workgroup starts at the smallest such
     // count of its (up to) four row blocks; a wavefront joins in at its own.
@@ -126,9 +131,11 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     int E0 = 0, E1 = 0;                    // exponent bounds of my column, panel 0 and 1 (equal in the lanes that share it)
     // uniform panel base + 32-bit byte offset per lane (a panel is far smaller than 4 GiB): one address register per load
     const char* qpanel = reinterpret_cast<const char*>(ANALYSIS ? xm_m : sp_m);
-    const int sn = min(n0 + scol, ld - 1);
-    const bool col_ok = n0 + scol < ld;
-    auto q_at = [&](int row) { return *reinterpret_cast<const float*>(qpanel + (size_t)(((uint32_t)row * (uint32_t)ld + (uint32_t)sn) * 4u)); };
+    const int nq = ANALYSIS ? ld : nval;
+    const int sn = min(n0 + scol, nq - 1);
+    const bool col_ok = n0 + scol < nq;
+    const uint32_t qrow = ANALYSIS ? (uint32_t)ld : srow, qcol = ANALYSIS ? (uint32_t)sn : scolumn(sn);
+    auto q_at = [&](int row) { return *reinterpret_cast<const float*>(qpanel + (size_t)(((uint32_t)row * qrow + qcol) * 4u)); };
     // raw rows into registers (indices clamped into the panel); masking, the mirror sum/difference and the cut happen when
     // the chunk is written to LDS, one chunk of matrix instructions later
     auto q_load = [&](int c) {
@@ -304,7 +311,32 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[t][v] = __builtin_ldexpf(acc[t][v], erun[t] - LH_SH) * rinv[v >> 2][v & 3];
     }
-    if (ANALYSIS) {
+    if (ANALYSIS && COEFFS) {
+        float* out = a.Out + 2 * (int64_t)m;
+        if (rb - (wslot & 1) == 0) {
+            // the order's first workgroups write its zeros, those of the last order with degrees also the orders past it
+            for (int i = tid; i < m * TN; i += 256) {
+                const int n = n0 + i % TN;
+                if (n < nval) out[scolumn(n) + (uint32_t)(i / TN) * srow] = 0.f;
+            }
+            if (m == min(lmax, a.mmax) - 1)
+                for (int i = tid; i < (a.mmax - 1 - m) * lmax * TN; i += 256) {
+                    const int n = n0 + i % TN, l = i / TN % lmax, mm = 1 + i / TN / lmax;
+                    if (n < nval) out[scolumn(n) + (uint32_t)l * srow + 2 * mm] = 0.f;
+                }
+        }
+        if (!active) return;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int n = n0 + 32 * t + cl;
+            float* o = out + scolumn(n);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int r = PG_ROWS * rb + 8 * (v >> 2) + 4 * kg + (v & 3);
+                if (r < nrows && n < nval) o[(uint32_t)(m + par + 2 * r) * srow] = acc[t][v];
+            }
+        }
+    } else if (ANALYSIS) {
         if (!active) return;
         float* out = a.Out + (int64_t)m * lmax * ld;
         if (PG_ROWS * (rb + 1) <= nrows && n0 + TN <= ld) {
@@ -371,7 +403,7 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     }
 }
 
-template <bool ANALYSIS>
+template <bool ANALYSIS, bool COEFFS>
 static int launch_f16(const PgemmArgs& a, int n_work, hipStream_t s) {
     const int64_t ncols = a.ld;
     if (n_work <= 0 || ncols <= 0) return SFNO_OK;
@@ -391,7 +423,7 @@ static int launch_f16(const PgemmArgs& a, int n_work, hipStream_t s) {
         const int64_t nwg = (int64_t)n_work * ((ncols + 32 * NT_ - 1) / (32 * NT_));             \
         if (nwg > 0x7fffffffLL) return SFNO_EUNSUPPORTED;                                        \
         dim3 grid((unsigned)nwg);                                                                \
-        hipLaunchKernelGGL((legendre_f16_kernel<NT_, ANALYSIS>), grid, dim3(256), 0, s, a);      \
+        hipLaunchKernelGGL((legendre_f16_kernel<NT_, ANALYSIS, COEFFS>), grid, dim3(256), 0, s, a); \
         break;                                                                                   \
     }
     switch (best) {
@@ -403,7 +435,20 @@ static int launch_f16(const PgemmArgs& a, int n_work, hipStream_t s) {
 }
 
 int legendre_f16_launch(bool analysis, const PgemmArgs& a, int n_work, hipStream_t s) {
-    return analysis ? launch_f16<true>(a, n_work, s) : launch_f16<false>(a, n_work, s);
+    return analysis ? launch_f16<true, false>(a, n_work, s) : launch_f16<false, false>(a, n_work, s);
+}
+
+// A launch less against eight-byte accesses.  Coefficients of 0.06 MiB (32 x 64, 8 rows): analysis 9.6 -> 7.5 us, synthesis 10.6 -> 7.5; 0.64 MiB
+// (20 degrees, 200 rows) 13.9 -> 11.4 and 14.6 -> 11.2; 1.3 MiB (64 x 128, 40 rows) 13.8 -> 15.1 and 16.2 -> 14.2; 1.6 MiB (91 x 180, 26 rows) 15.0 -> 14.0
+// and 16.1 -> 13.3; 3.9 MiB (160 x 320, 20 rows) 21.6 -> 23.7 and 24.3 -> 22.5; 14.5 MiB 32 -> 51 and 37 -> 43.  (One workgroup writes the zeros of the orders
+// past the last degree: there may be one such order, not many.)
+bool legendre_coeffs_fit(bool analysis, int format, int64_t rows, int lmax, int mmax) {
+    return format == PG_FORMAT_F16X2 && mmax <= lmax + 1 && 8 * rows * lmax * mmax <= (analysis ? 1 << 20 : 2 << 20);
+}
+
+int legendre_coeffs_launch(bool analysis, PgemmArgs a, int64_t rows, int n_work, hipStream_t s) {
+    a.ncol = (int)(2 * rows);
+    return analysis ? launch_f16<true, true>(a, n_work, s) : launch_f16<false, true>(a, n_work, s);
 }
 
 }  // namespace sfno

@@ -47,6 +47,7 @@ struct PgemmArgs {
     const float* rinv;             // two-part fp16 format: row factors, [entry position - 2 mmax][32]
     int lmax, nlat, mmax;          // Legendre modes
     int ld;                        // channel leading dimension of Q and Out (Legendre modes)
+    int ncol;                      // the spectral side in the reference layout: columns, 2 rows
 };
 
 // dhconv: output columns o' per workgroup, and the kernel arguments
@@ -184,6 +185,9 @@ void pack_legendre_fold(const LegendreGen& g, const double* lat_w, const double*
                         std::vector<float>* rinv = nullptr);
 int legendre_fold_launch(bool analysis, int format, const PgemmArgs& a, int n_work, hipStream_t s);
 int legendre_f16_launch(bool analysis, const PgemmArgs& a, int n_work, hipStream_t s);
+// the same with coefficients complex [rows][lmax][mmax] as the analysis' output or the synthesis' input, where they fit
+bool legendre_coeffs_fit(bool analysis, int format, int64_t rows, int lmax, int mmax);
+int legendre_coeffs_launch(bool analysis, PgemmArgs a, int64_t rows, int n_work, hipStream_t s);
 
 // ---- FFT (fft.hip) -----------------------------------------------------------------------
 struct FftPlan {
