@@ -352,6 +352,8 @@ int sfno_pointwise_mlp(const void* x, const float* scale, const float* shift, co
 int sfno_pointwise_pack_weight(const float* w, void* packed, int O, int K, void* stream);
 /* the same stream from the transposed matrix: w is float32 [K][O] (the weight of an input gradient) */
 int sfno_pointwise_pack_weight_transposed(const float* w, void* packed, int O, int K, void* stream);
+/* both in one launch: the weight w [O][K], and its transpose as sfno_pointwise_pack_weight_transposed(w, ..., K, O) packs it */
+int sfno_pointwise_pack_weight_both(const float* w, void* packed, void* packed_transposed, int O, int K, void* stream);
 
 /* Instance norm as a per-(b, c) affine: scale = gamma[c] / sqrt(var + eps), shift = beta[c] - mean * scale over
  * the P pixels of each of the `rows` = B*C rows of x (bf16), statistics in fp32 with the biased variance

@@ -712,6 +712,11 @@ extern "C" int sfno_pointwise_pack_weight_transposed(const float* w, void* packe
     if (!w || !packed || O < 1 || K < 1) return SFNO_EINVAL;
     return pointwise_pack_launch(w, reinterpret_cast<unsigned short*>(packed), O, K, 1, (hipStream_t)stream);
 }
+extern "C" int sfno_pointwise_pack_weight_both(const float* w, void* packed, void* packed_transposed, int O, int K, void* stream) {
+    if (!w || !packed || !packed_transposed || O < 1 || K < 1) return SFNO_EINVAL;
+    return pointwise_pack_both_launch(w, reinterpret_cast<unsigned short*>(packed), reinterpret_cast<unsigned short*>(packed_transposed), O, K,
+                                      (hipStream_t)stream);
+}
 
 // 16-byte loads of eight bf16 values
 static bool on16(const void* a, const void* b, const void* c, const void* d) {

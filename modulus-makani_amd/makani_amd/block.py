@@ -106,7 +106,7 @@ class _Call:
         wf, wskip, w1, b1, w2, b2, g0, be0, g1, be1 = params
         dev = x.device
         b = _lib.Block()
-        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(wf, conv.compute, both=training), pw.packed_weight(w1), pw.packed_weight(w2), pw.packed_weight(wskip)]
+        keep = self.keep = [fwd.plan(dev), inv.plan(dev), packed_for(wf, conv.compute, both=training), *(pw.packed_weight(w, both=training) for w in (w1, w2, wskip))]
         b.fwd, b.inv, b.weights = keep[0].handle, keep[1].handle, keep[2].handle
         b.w1, b.w2, b.wskip = (t.data_ptr() for t in keep[3:6])
         if backward:

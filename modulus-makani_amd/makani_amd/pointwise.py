@@ -38,9 +38,11 @@ def _order(p, packed_on, streams):
     streams.add(s.cuda_stream)
 
 
-def packed_weight(weight, transposed=False):
+def packed_weight(weight, transposed=False, both=False):
     """MFMA operand stream of a 1x1 convolution weight ([O, K, 1, 1] or [O, K]), or of its transpose (the weight of the
-    convolution's input gradient); cached per parameter and rebuilt when the parameter changes."""
+    convolution's input gradient); cached per parameter and rebuilt when the parameter changes.
+
+    both: the input gradient will follow, so the transpose is packed by the same launch."""
     key = (id(weight), transposed)
     # (tensors made under inference_mode carry no version counter: they are packed once per tensor object)
     stamp = (weight.data_ptr(), -1 if weight.is_inference() else weight._version, weight.device)
@@ -52,10 +54,19 @@ def packed_weight(weight, transposed=False):
     w = weight.detach().reshape(weight.shape[0], -1).float().contiguous()
     O, K = (w.shape[1], w.shape[0]) if transposed else w.shape
     p = torch.empty(lib.sfno_pointwise_weight_elems(O, K), dtype=torch.bfloat16, device=w.device)
-    pack = lib.sfno_pointwise_pack_weight_transposed if transposed else lib.sfno_pointwise_pack_weight
     s = torch.cuda.current_stream(w.device)
-    check(pack(_ptr(w), _ptr(p), O, K, s.cuda_stream), "sfno_pointwise_pack_weight")
-    _wcache[key] = (weakref.ref(weight, lambda _, k=key: _wcache.pop(k, None)), stamp, p, s, {s.cuda_stream})
+
+    def keep(key, p):
+        _wcache[key] = (weakref.ref(weight, lambda _, k=key: _wcache.pop(k, None)), stamp, p, s, {s.cuda_stream})
+
+    if both and not transposed:
+        pt = torch.empty(lib.sfno_pointwise_weight_elems(K, O), dtype=torch.bfloat16, device=w.device)
+        check(lib.sfno_pointwise_pack_weight_both(_ptr(w), _ptr(p), _ptr(pt), O, K, s.cuda_stream), "sfno_pointwise_pack_weight_both")
+        keep((id(weight), True), pt)
+    else:
+        pack = lib.sfno_pointwise_pack_weight_transposed if transposed else lib.sfno_pointwise_pack_weight
+        check(pack(_ptr(w), _ptr(p), O, K, s.cuda_stream), "sfno_pointwise_pack_weight")
+    keep(key, p)
     return p
 
 
@@ -85,7 +96,7 @@ def conv1x1(x, weight, bias=None, act=None, addend=None, add_scale=None, add_shi
     return _conv1x1(x, weight, False, bias, act, addend, add_scale, add_shift)
 
 
-def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
+def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=None, add_shift=None, both=False):
     O, K_weight = (weight.shape[1], weight.shape[0]) if transposed else weight.shape[:2]
     if not supported(x):
         raise RuntimeError("the fused pointwise kernels take contiguous bfloat16 NCHW HIP tensors with H*W a multiple of 8")
@@ -93,7 +104,7 @@ def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=
     B, K, H, W = x.shape
     if K_weight != K:
         raise RuntimeError(f"conv1x1: input has {K} channels, weight expects {K_weight}")
-    pw = packed_weight(weight, transposed)
+    pw = packed_weight(weight, transposed, both)
     y = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
     if bias is not None:
         bias = bias.detach().float().contiguous()
@@ -232,7 +243,7 @@ class _Conv1x1(torch.autograd.Function):
         ctx.x_dtype = x.dtype
         ctx.b_dtype = bias.dtype if bias is not None else None
         # (the parameter itself goes in: its packed copy is cached per parameter object and version)
-        return conv1x1(xb, weight, bias)
+        return _conv1x1(xb, weight, False, bias, both=ctx.needs_input_grad[0])
 
     @staticmethod
     @torch.autograd.function.once_differentiable
@@ -265,12 +276,13 @@ class _ConvGeluConv(torch.autograd.Function):
         z = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
         a = torch.empty_like(z)
         bias = b1.detach().float().contiguous() if b1 is not None else None
-        check(lib.sfno_pointwise_conv_gelu(_ptr(xb), _ptr(packed_weight(w1)), _ptr(bias), _ptr(a), _ptr(z), B, K, O, H * W, _stream(x.device)),
+        need = ctx.needs_input_grad
+        check(lib.sfno_pointwise_conv_gelu(_ptr(xb), _ptr(packed_weight(w1, both=need[0])), _ptr(bias), _ptr(a), _ptr(z), B, K, O, H * W, _stream(x.device)),
               "sfno_pointwise_conv_gelu")
         ctx.save_for_backward(xb, z, a, w1, w2)
         ctx.biases = (b1 is not None, b2 is not None)
         ctx.x_dtype = x.dtype
-        return conv1x1(a, w2, b2)
+        return _conv1x1(a, w2, False, b2, both=need[0] or need[1] or need[2])
 
     @staticmethod
     @torch.autograd.function.once_differentiable

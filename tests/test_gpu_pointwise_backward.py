@@ -306,3 +306,17 @@ def test_packed_weight_on_another_stream(lib_built, transposed):
     pw.clear_cache(w)
     want = pw._conv1x1(x, w, transposed)
     assert torch.equal(got, want) and torch.equal(again, want)
+
+
+@pytest.mark.parametrize("O,K", [(1, 1), (73, 384), (384, 73), (97, 128), (130, 260), (31, 64)])
+def test_weight_and_transpose_packed_together(lib_built, O, K):
+    """One launch writes what the two separate packings write, padding included."""
+    from makani_amd import pointwise as pw
+
+    w = torch.randn(O, K, 1, 1, generator=torch.Generator().manual_seed(8)).cuda()
+    want = [pw.packed_weight(w, transposed=t).clone() for t in (False, True)]
+    pw.clear_cache(w)
+    p = pw.packed_weight(w, both=True)
+    hit = [pw._wcache[(id(w), t)][2] for t in (False, True)]
+    assert hit[0] is p and pw.packed_weight(w, transposed=True) is hit[1]
+    assert torch.equal(hit[0], want[0]) and torch.equal(hit[1], want[1])
