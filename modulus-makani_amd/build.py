@@ -16,7 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 OUT = os.path.join(HERE, "makani_amd", "libsfno_spectral.so")
 SOURCES = ["tables.cpp", "capi.cpp", "block.cpp", "dhconv.hip", "dhconv_f16.hip", "dhconv_wgrad.hip", "pointwise.hip", "pointwise_wgrad.hip", "diagonal.hip", "degree_power.hip", "legendre_fold.hip", "legendre_f16.hip", "fft.hip",
-           "fft_fast.hip", "fft_fast_a.hip", "fft_fast_b.hip", "fft_fast_c.hip", "fft_fast_d.hip", "fft_fast_e.hip", "fft_fast_f.hip", "layout.hip",
+           "fft_fast.hip", "fft_fast_a.hip", "fft_fast_b.hip", "fft_fast_c.hip", "fft_fast_d.hip", "fft_fast_e.hip", "fft_fast_f.hip", "fft_matrix.hip", "layout.hip",
            "static_scratch.hip"]
 HEADERS = [os.path.join(CSRC, h) for h in ("sfno_internal.h", "dhconv_map.h", "fft_kernels.h", "fft_fast.h", "fft_lengths.h", "pointwise_mlp.h")] + [os.path.join(ROOT, "include", "sfno_spectral.h")]
 

@@ -435,7 +435,10 @@ int sfno::analysis_adjoint_launch(const sfno_sht_plan* p, const float* gspec, vo
 
 int sfno::synthesis_adjoint_launch(const sfno_sht_plan* p, const void* gx, int x_dtype, float* xm, float* gspec, int64_t rows, hipStream_t s) {
     if (!(p->directions & SFNO_DIR_INVERSE_ADJOINT)) return SFNO_EINVAL;
-    const int rc = sfno_rfft(p, gx, x_dtype, xm, rows, s);
+    // (gradients only: the forward transforms keep the rounding of the vector kernel, for a network in bf16 carries a difference in the last
+    // place of its first spectrum to some percent of a forecast a few steps on)
+    const bool matrix = x_dtype == SFNO_DTYPE_BF16 && rfft_matrix_supported(p->fft, gx, rows, p->nlat, p->mmax);
+    const int rc = matrix ? rfft_matrix_launch(p->fft, gx, xm, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), s) : sfno_rfft(p, gx, x_dtype, xm, rows, s);
     if (rc != SFNO_OK) return rc;
     if (planar(p)) return planar_stage(p, MS_INV_ADJ, false, xm, gspec, rows, s);
     PgemmArgs a = legendre_args(p, p->inv_adj, xm, gspec, sfno_spectral_ld(rows));

@@ -262,7 +262,8 @@ int fft_plan_init(FftPlan& p, int n) {
     }
     if (hipMalloc(&p.d_tw, sizeof(float2) * n) != hipSuccess) return SFNO_ENOMEM;
     if (hipMemcpy(p.d_tw, tw.data(), sizeof(float2) * n, hipMemcpyHostToDevice) != hipSuccess) return SFNO_EHIP;
-    return fft_fast_plan_init(p);
+    const int rc = fft_matrix_plan_init(p);
+    return rc == SFNO_OK ? fft_fast_plan_init(p) : rc;
 }
 
 void fft_plan_free(FftPlan& p) {
@@ -272,6 +273,10 @@ void fft_plan_free(FftPlan& p) {
     if (p.d_chirp) (void)hipFree(p.d_chirp);
     if (p.d_vhat) (void)hipFree(p.d_vhat);
     if (p.d_post) (void)hipFree(p.d_post);
+    if (p.d_mfrag) (void)hipFree(p.d_mfrag);
+    if (p.d_mtw) (void)hipFree(p.d_mtw);
+    p.d_mfrag = nullptr;
+    p.d_mtw = nullptr;
     p.d_tw = p.d_tw0 = p.d_tw1 = p.d_chirp = p.d_vhat = nullptr;
     p.d_post = nullptr;
     p.chirp_m = 0;

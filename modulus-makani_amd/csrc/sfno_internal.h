@@ -201,6 +201,8 @@ struct FftPlan {
     float2* d_tw0 = nullptr;       // inter-pass twiddles of the specialised kernels (fft_kernels.h)
     float2* d_tw1 = nullptr;
     unsigned* d_post = nullptr;    // [n/2+1] LDS slot of bin m (low half) and of bin n - m (high half) around the specialised passes
+    unsigned short* d_mfrag = nullptr;   // matrix operands and twiddles of fft_matrix.hip, for the lengths it has kernels for
+    float2* d_mtw = nullptr;
     // latitude plans of lengths with a large prime factor (fft_chirp_plan_init): the DFT as a circular convolution of
     // length chirp_m with a chirp; d_tw0 / d_tw1 then belong to the specialised passes of length chirp_m
     int chirp_m = 0;
@@ -213,6 +215,10 @@ int fft_fast_plan_init(FftPlan& p);
 // lat_stats (inverse only, may be null): float2 [rows][nlat] = mean over longitude of the output row and of its squared deviation from that mean
 int fft_fast_launch(bool inverse, const FftPlan& p, const void* in, void* out, int64_t rows, int nlat, int mmax, int ld, int grid_dtype,
                     hipStream_t s, float2* lat_stats = nullptr, const void* in2 = nullptr);
+// bf16 rows of which the lowest orders are kept (fft_matrix.hip)
+int fft_matrix_plan_init(FftPlan& p);
+bool rfft_matrix_supported(const FftPlan& p, const void* x, int64_t rows, int nlat, int mmax);
+int rfft_matrix_launch(const FftPlan& p, const void* x, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s);
 // latitude FFT on the specialised passes; SFNO_EUNSUPPORTED for a length without them
 int latfft_fast_launch(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
 // planar pair on the reference layout: real FFTs along the grid rows, x [rows][nlat][n] <-> y [rows][group][nlat][2^cs] complex (groups
