@@ -68,17 +68,25 @@ __device__ __forceinline__ void wg_dma16(const void* base, unsigned offset, unsi
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds_byte_addr) : "memory");
 }
 
+// tile of the second kernel: eight wavefronts of 96 x 96, 4 x 2
+constexpr int WW_MT = 3, WW_NT = 3, WW_WO = 4, WW_WK = 2;
+constexpr int WW_THREADS = 64 * WW_WO * WW_WK;
+constexpr int WW_TO = 32 * WW_MT * WW_WO, WW_TK = 32 * WW_NT * WW_WK;
+
 struct WgradShape {
     int n_ot, n_kt, splits;
     int64_t cps, chunks;               // chunks per sample, chunks in all
+    bool wide;                         // tiles of pw_wgrad_wide_kernel
 };
 
 // how the launcher and the workspace query divide the work: shares of at least four chunks, one workgroup per CU (all
 // workgroups resident at once, the tiles of a share side by side on one XCD)
-static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
+static WgradShape wgrad_shape(int O, int K, int B, int64_t P, bool wide) {
+    const int to = wide ? WW_TO : WG_TO, tk = wide ? WW_TK : WG_TK;
     WgradShape s;
-    s.n_ot = (O + WG_TO - 1) / WG_TO;
-    s.n_kt = (K + WG_TK - 1) / WG_TK;
+    s.wide = wide;
+    s.n_ot = (O + to - 1) / to;
+    s.n_kt = (K + tk - 1) / tk;
     s.cps = (P + WG_PX - 1) / WG_PX;
     s.chunks = s.cps * B;
     const int tiles = s.n_ot * s.n_kt;
@@ -91,6 +99,11 @@ static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
     return s;
 }
 
+static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
+    const WgradShape s = wgrad_shape(O, K, B, P, false), w = wgrad_shape(O, K, B, P, true);
+    return (int64_t)(WW_TO + WW_TK) * s.splits < (int64_t)(WG_TO + WG_TK) * w.splits ? w : s;
+}
+
 struct WgradArgs {
     const unsigned short* G;           // bf16 [B][O][P]
     const unsigned short* X;           // bf16 [B][K][P]
@@ -99,6 +112,53 @@ struct WgradArgs {
     int64_t P;
     int n_ot, n_kt, splits;
     int64_t cps, chunks;
+};
+
+// One stream per operand: the next chunk to ask for lies in sample ib at chunk ic of the sample.  Thread t asks for the piece at
+// slot t + THREADS j of the rows' image in LDS (16 bytes a slot, eight to a row), j < PIECES: the thread's rows lie THREADS / 8 apart, a
+// multiple of 16, and share their permutation.  Inside a sample the addresses are
+// a scalar base and the lane's 32-bit offsets from the tile's first row; they are worked out in 64 bits for the last chunk of a
+// sample, whose pieces may lie outside, and where the rows of a tile lie further apart than 32 bits reach.
+template <int PIECES, int THREADS>
+struct WgStream {
+    static_assert(THREADS % 128 == 0, "a thread's pieces share the permutation of their rows");
+    static constexpr int ROWS = PIECES * THREADS / 8;
+    static_assert(ROWS <= 512, "32-bit offsets");
+    static constexpr int64_t NEAR = ROWS <= 256 ? 1 << 23 : 1 << 22;      // ROWS rows of fewer values lie within 2^32 bytes
+    const unsigned short* base;
+    int r0, last;                  // first row of the tile, last row of the tensor
+    int64_t ib, ic;
+    unsigned off[PIECES];
+    static __device__ __forceinline__ int part(int tid) { return (tid & 7) ^ ((tid >> 4) & 7); }
+    __device__ __forceinline__ WgStream(const unsigned short* t, int first, int rows, const WgradArgs& a, int64_t c_begin, int tid)
+        : base(t), r0(first), last(rows - 1), ib(c_begin / a.cps), ic(c_begin - ib * a.cps) {
+        const unsigned row_bytes = (unsigned)(2 * a.P);
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j) off[j] = (unsigned)min((tid >> 3) + THREADS / 8 * j, last - r0) * row_bytes + 16 * part(tid);
+    }
+    // dst: LDS address of the wavefront's first slot
+    __device__ __forceinline__ void issue(const WgradArgs& a, unsigned dst, int tid) {
+        const unsigned short* b = base + ((ib * (last + 1) + r0) * a.P + ic * WG_PX);
+        if (a.P < NEAR && (ic + 1) * WG_PX <= a.P) {
+            // (uniform, but the division by the chunks per sample left it in vector registers)
+            const uint64_t bits = reinterpret_cast<uint64_t>(b);
+            const void* ubase = reinterpret_cast<const void*>((uint64_t)__builtin_amdgcn_readfirstlane((int)(bits >> 32)) << 32 |
+                                                              (unsigned)__builtin_amdgcn_readfirstlane((int)bits));
+#pragma unroll
+            for (int j = 0; j < PIECES; ++j) wg_dma16(ubase, off[j], dst + j * (THREADS * 16));
+        } else {
+            const bool in = ic * WG_PX + 8 * part(tid) < a.P;      // P is a multiple of 8: a piece lies inside the row or outside
+#pragma unroll
+            for (int j = 0; j < PIECES; ++j) {
+                const unsigned short* p = b + (int64_t)min((tid >> 3) + THREADS / 8 * j, last - r0) * a.P + 8 * part(tid);
+                wg_dma16(in ? p : reinterpret_cast<const unsigned short*>(wg_zero16), dst + j * (THREADS * 16));
+            }
+        }
+        if (++ic == a.cps) {
+            ic = 0;
+            ++ib;
+        }
+    }
 };
 
 // grid = 8 * ceil(splits / 8) * n_ot * n_kt workgroups of 512 threads
@@ -119,50 +179,8 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
 
     // ---- loads: LDS slot s = 512 j + tid of a half (16 bytes) holds row s >> 3, piece (s & 7) ^ ((row >> 1) & 7).  A thread's four
     // slots lie 64 rows apart: same piece, same permutation.  Rows past the matrix are its last row, whose products are never stored.
-    const int part = (tid & 7) ^ ((tid >> 4) & 7), row0 = tid >> 3;
-    const unsigned short* zero16 = reinterpret_cast<const unsigned short*>(wg_zero16);
-    // One stream per operand: the next chunk to ask for lies in sample ib at chunk ic of the sample.  Inside a sample the addresses are
-    // a scalar base and the lane's 32-bit offsets from the tile's first row; they are worked out in 64 bits for the last chunk of a
-    // sample, whose pieces may lie outside, and where the rows of a tile lie further apart than 32 bits reach.
-    struct Stream {
-        const unsigned short* base;
-        int r0, last;                  // first row of the tile, last row of the tensor
-        int64_t ib, ic;
-        unsigned off[WG_PIECES];
-    };
-    const unsigned row_bytes = (unsigned)(2 * a.P);
-    const bool near = a.P < (1 << 23);
-    auto stream = [&](const unsigned short* base, int r0, int rows) {
-        Stream t{base, r0, rows - 1, c_begin / a.cps, 0, {}};
-        t.ic = c_begin - t.ib * a.cps;
-#pragma unroll
-        for (int j = 0; j < WG_PIECES; ++j) t.off[j] = (unsigned)min(row0 + WG_RSTEP * j, t.last - r0) * row_bytes + 16 * part;
-        return t;
-    };
-    Stream sg = stream(a.G, o0, a.O), sx = stream(a.X, k0, a.K);
-    auto issue = [&](Stream& t, int slot) {
-        const unsigned dst = lds0 + slot * WG_HALF + wave * 1024;
-        const unsigned short* base = t.base + ((t.ib * (t.last + 1) + t.r0) * a.P + t.ic * WG_PX);
-        if (near && (t.ic + 1) * WG_PX <= a.P) {
-            // (uniform, but the division by the chunks per sample left it in vector registers)
-            const uint64_t bits = reinterpret_cast<uint64_t>(base);
-            const void* ubase = reinterpret_cast<const void*>((uint64_t)__builtin_amdgcn_readfirstlane((int)(bits >> 32)) << 32 |
-                                                              (unsigned)__builtin_amdgcn_readfirstlane((int)bits));
-#pragma unroll
-            for (int j = 0; j < WG_PIECES; ++j) wg_dma16(ubase, t.off[j], dst + j * (WG_THREADS * 16));
-        } else {
-            const bool in = t.ic * WG_PX + 8 * part < a.P;         // P is a multiple of 8: a piece lies inside the row or outside
-#pragma unroll
-            for (int j = 0; j < WG_PIECES; ++j) {
-                const unsigned short* p = base + (int64_t)min(row0 + WG_RSTEP * j, t.last - t.r0) * a.P + 8 * part;
-                wg_dma16(in ? p : zero16, dst + j * (WG_THREADS * 16));
-            }
-        }
-        if (++t.ic == a.cps) {
-            t.ic = 0;
-            ++t.ib;
-        }
-    };
+    WgStream<WG_PIECES, WG_THREADS> sg(a.G, o0, a.O, a, c_begin, tid), sx(a.X, k0, a.K, a, c_begin, tid);
+    auto issue = [&](WgStream<WG_PIECES, WG_THREADS>& t, int slot) { t.issue(a, lds0 + slot * WG_HALF + wave * 1024, tid); };
 
     f32x16 acc[2][4];
     float accb[2] = {0.f, 0.f}, chunkb[2] = {0.f, 0.f};       // sums of the lane's pixels of its two rows: all chunks, this chunk
@@ -285,6 +303,132 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     }
 }
 
+// The same with tiles of 384 x 192 and wavefronts of 96 x 96 (3 x 3 matrix instructions from six fragments instead of 2 x 4 from six).
+// LDS holds two chunks of 576 rows; the one after next is asked for when the last fragments of a chunk have been read, and has a whole
+// chunk's products to land.
+__global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs a) {
+    constexpr int MT = WW_MT, NT = WW_NT, ROW = 2 * WG_PX, BUF = (WW_TO + WW_TK) * ROW;
+    constexpr int PA = WW_TO * ROW / (16 * WW_THREADS), PB = WW_TK * ROW / (16 * WW_THREADS);
+    static_assert(PA * 16 * WW_THREADS == WW_TO * ROW && PB * 16 * WW_THREADS == WW_TK * ROW && 2 * BUF <= 160 * 1024, "whole pieces, two chunks in LDS");
+    __shared__ __align__(16) unsigned char lds[2 * BUF];
+    const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+    const int tiles = a.n_ot * a.n_kt;
+    const int split = (q / tiles) * 8 + xcd, tile = q % tiles;
+    if (split >= a.splits) return;
+    const int o0 = (tile % a.n_ot) * WW_TO, k0 = (tile / a.n_ot) * WW_TK;
+    const int64_t c_begin = (int64_t)split * a.chunks / a.splits, c_end = (int64_t)(split + 1) * a.chunks / a.splits;
+    const int nch = (int)(c_end - c_begin);
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wo = wave % WW_WO, wk = wave / WW_WO;
+    const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)lds) + wave * 1024;
+    WgStream<PA, WW_THREADS> sg(a.G, o0, a.O, a, c_begin, tid);
+    WgStream<PB, WW_THREADS> sx(a.X, k0, a.K, a, c_begin, tid);
+    auto issue = [&](int buf) {
+        sg.issue(a, lds0 + buf * BUF, tid);
+        sx.issue(a, lds0 + buf * BUF + WW_TO * ROW, tid);
+    };
+
+    f32x16 acc[MT][NT];
+    float accb[MT], chunkb[MT];               // sums of the lane's pixels of its rows: all chunks, this chunk
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        accb[mt] = chunkb[mt] = 0.f;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.f;
+    }
+    const int ro = wo * MT * 32, rk = wk * NT * 32;
+    const int sw = (lane >> 1) & 7, kg = lane >> 5;
+    const unsigned fa = (ro + (lane & 31)) * ROW, fb = (WW_TO + rk + (lane & 31)) * ROW;
+    const bool live = o0 + ro < a.O && k0 + rk < a.K;
+    const bool bias = a.Kext > a.K && k0 + rk == 0;
+    bf16x8 af[2][MT], bf[2][NT];              // [step & 1][32-row block]
+    auto fragments = [&](int buf, int ks) {
+        const unsigned char* p = lds + buf * BUF + (unsigned)(((2 * ks + kg) ^ sw) * 16);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) af[ks & 1][mt] = *reinterpret_cast<const bf16x8*>(p + fa + mt * 32 * ROW);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) bf[ks & 1][nt] = *reinterpret_cast<const bf16x8*>(p + fb + nt * 32 * ROW);
+    };
+    auto products = [&](int ks) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][mt], bf[ks & 1][nt], acc[mt][nt], 0, 0, 0);
+        if (bias) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const u32x4 p = __builtin_bit_cast(u32x4, af[ks & 1][mt]);
+                float lo = 0.f, hi = 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    lo += __uint_as_float(p[i] << 16);
+                    hi += __uint_as_float(p[i] & 0xffff0000u);
+                }
+                chunkb[mt] += lo + hi;
+                if (ks == 3) {
+                    accb[mt] += chunkb[mt];
+                    chunkb[mt] = 0.f;
+                }
+            }
+        }
+    };
+    issue(0);
+    if (nch > 1) issue(1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (nch > 1)
+        __builtin_amdgcn_s_waitcnt(wg_wait(PA + PB));
+    else
+        __builtin_amdgcn_s_waitcnt(wg_wait(0));
+    wg_barrier();
+    if (live) fragments(0, 0);
+    for (int i = 0; i < nch; ++i) {
+        if (live) {
+#pragma unroll
+            for (int ks = 0; ks < 3; ++ks) {
+                fragments(i & 1, ks + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                products(ks);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // this wavefront holds all it needs of chunk i, and its pieces of chunk i + 1 (all that is under way) have landed
+        __builtin_amdgcn_s_waitcnt(wg_wait(0));
+        wg_barrier();
+        if (i + 2 < nch) issue(i & 1);
+        if (live) {
+            fragments((i + 1) & 1, 0);        // (past the last chunk: whatever that buffer holds, and not used)
+            __builtin_amdgcn_sched_barrier(0);
+            products(3);
+        }
+    }
+
+    float* out = a.ws + (int64_t)split * a.O * a.Kext;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int kk = k0 + rk + nt * 32 + (lane & 31);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int o = o0 + ro + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                if (o < a.O && kk < a.K) out[(int64_t)o * a.Kext + kk] = acc[mt][nt][v];
+            }
+        }
+    if (bias) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int o = o0 + ro + mt * 32 + (lane & 31);
+            const float b = accb[mt] + __shfl_xor(accb[mt], 32, 64);
+            if (lane < 32 && o < a.O) out[(int64_t)o * a.Kext + a.K] = b;
+        }
+    }
+}
+
 // dW[o][k] = sum over the shares, in a fixed order; column K goes to db.  A workgroup's 16 wavefronts take every 16th share each of
 // the same 64 V entries and meet in LDS: latency is what bounds small matrices (up to 256 shares of 73 x 73 entries; one thread per
 // four entries walked all shares in turn: both kernels 145 us for 73 -> 73 channels at 2 x 181 x 360, now 20; 128 -> 256 with bias 45 -> 35).  V = 4 entries per lane (16-byte loads; a share must then start on
@@ -335,7 +479,10 @@ int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, flo
     a.n_ot = sh.n_ot; a.n_kt = sh.n_kt; a.splits = sh.splits; a.cps = sh.cps; a.chunks = sh.chunks;
     const int64_t nwg = 8 * (int64_t)((sh.splits + 7) / 8) * sh.n_ot * sh.n_kt;
     if (nwg > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
-    hipLaunchKernelGGL(pw_wgrad_kernel, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
+    if (sh.wide)
+        hipLaunchKernelGGL(pw_wgrad_wide_kernel, dim3((unsigned)nwg), dim3(WW_THREADS), 0, s, a);
+    else
+        hipLaunchKernelGGL(pw_wgrad_kernel, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
     if (hipGetLastError() != hipSuccess) return SFNO_EHIP;
     const int64_t n = (int64_t)O * Kext;
     if (n % 4 == 0 && n >= 256 * 256)

@@ -30,6 +30,13 @@ WGRAD_CASES = [
     (1, 257, 70, 24, 16, True),        # one column in the second column tile: the bias belongs to the first only
     (2, 73, 73, 64, 96, False),        # an odd number of entries, 48 shares: the reduction's single loads
     (1, 256, 256, 16, 40, True),       # 65792 entries: its 16-byte loads, few shares (fewer than its wavefronts)
+    # tiles of 384 x 192
+    (1, 1, 257, 1, 8, True),           # one chunk, one piece of it; wavefronts without rows or columns
+    (3, 192, 384, 9, 8, True),         # one full tile, chunks of 64 and 8 pixels: two buffers from the first share on
+    (1, 193, 385, 40, 48, True),       # a row and a column in tiles of their own
+    (2, 384, 384, 24, 40, False),      # two column tiles
+    (1, 320, 640, 16, 40, True),       # two row tiles and two column tiles, neither full
+    (1, 768, 384, 241, 480, True),     # shares of many chunks, the last chunk of the sample a part
 ]
 
 
@@ -76,9 +83,9 @@ def test_weight_gradient_counts_every_pixel_once(lib_built):
         assert torch.equal(gw.cpu(), torch.full((3, 5), float(B * P))) and torch.equal(gb.cpu(), torch.full((3,), float(B * P)))
 
 
-@pytest.mark.parametrize("B,K,O,P", [(1, 3, 5, 2 ** 23 + 8), (2, 9, 2, 2 ** 23 + 72)])
+@pytest.mark.parametrize("B,K,O,P", [(1, 3, 5, 2 ** 23 + 8), (2, 9, 2, 2 ** 23 + 72), (1, 2, 384, 2 ** 22 - 8), (1, 2, 384, 2 ** 22 + 8)])
 def test_rows_too_long_for_32_bit_offsets(lib_built, B, K, O, P):
-    """From 2^23 pixels on 256 rows lie further apart than 32 bits reach: addresses in 64 bits.  fp32 sums of 1.7e7 products in shares:
+    """From 2^23 pixels on 256 rows, from 2^22 on 384, lie further apart than 32 bits reach: addresses in 64 bits.  fp32 sums of 1.7e7 products in shares:
     1e-5, as above."""
     from makani_amd import pointwise as pw
 
