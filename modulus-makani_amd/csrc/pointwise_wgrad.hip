@@ -9,7 +9,7 @@
 // tiles it took a column of tiles to itself where K is a multiple of 256 (eight instead of six for 768 -> 384 channels with bias:
 // 1249 -> 997 us at 721 x 1440).
 //
-// A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile of dW and a contiguous share of the (sample, 64-pixel chunk)
+// A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile (wide layers: 384 x 192, pw_wgrad_wide_kernel) of dW and a contiguous share of the (sample, 64-pixel chunk)
 // sequence.  Per chunk 256 rows of g and 256 rows of x, a whole 128-byte line each (with 64-byte pieces of 32-pixel chunks the
 // same bytes were 1.4 times as long on their way, 989 against 704 us without the products for 384 -> 768 channels at 721 x 1440, and
 // the kernel took as long as its loads: 1029 -> 902 us in all, 768 -> 384 with bias 997 -> 858),
@@ -99,6 +99,8 @@ static WgradShape wgrad_shape(int O, int K, int B, int64_t P, bool wide) {
     return s;
 }
 
+// Whichever kernel's workgroups ask for fewer rows, per pixel of the tensor, is the faster (figures at pw_wgrad_wide_kernel); 256 x 256 where O <= 256,
+// and where a few channels on the wide side would fill a 384 by little (384 -> 73 channels).
 static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
     const WgradShape s = wgrad_shape(O, K, B, P, false), w = wgrad_shape(O, K, B, P, true);
     return (int64_t)(WW_TO + WW_TK) * s.splits < (int64_t)(WG_TO + WG_TK) * w.splits ? w : s;
@@ -306,6 +308,11 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
 // The same with tiles of 384 x 192 and wavefronts of 96 x 96 (3 x 3 matrix instructions from six fragments instead of 2 x 4 from six).
 // LDS holds two chunks of 576 rows; the one after next is asked for when the last fragments of a chunk have been read, and has a whole
 // chunk's products to land.
+// A CU's intake bounds both kernels: memory is read once (2.40 GB for 768 -> 384 channels at 721 x 1440, 736 us), yet a chunk's 72 KiB take 2.7 us
+// with nothing else in the loop (694 us), the products alone 425; lines in L2 ahead of their requests, or a share's lines next to
+// its neighbours', made it no faster.  So the tile that asks for fewer rows is the better one: four tiles of 576 rows for 384 x 768 where the other
+// kernel has six of 512 (384 -> 768 1034 -> 843 us, 768 -> 384 873 -> 736, 384 -> 384 546 -> 407, all at 721 x 1440; 320 -> 640 at
+// 2 x 90 x 180 43 us as before).  Larger tiles (384 x 256) do not fit the registers.
 __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs a) {
     constexpr int MT = WW_MT, NT = WW_NT, ROW = 2 * WG_PX, BUF = (WW_TO + WW_TK) * ROW;
     constexpr int PA = WW_TO * ROW / (16 * WW_THREADS), PB = WW_TK * ROW / (16 * WW_THREADS);
