@@ -73,18 +73,20 @@ constexpr int WW_MT = 3, WW_NT = 3, WW_WO = 4, WW_WK = 2;
 constexpr int WW_THREADS = 64 * WW_WO * WW_WK;
 constexpr int WW_TO = 32 * WW_MT * WW_WO, WW_TK = 32 * WW_NT * WW_WK;
 
+enum WgradKind { WG_SQUARE, WG_WIDE, WG_WIDE_SWAP };      // pw_wgrad_kernel, pw_wgrad_wide_kernel<false>, <true>
 struct WgradShape {
     int n_ot, n_kt, splits;
     int64_t cps, chunks;               // chunks per sample, chunks in all
-    bool wide;                         // tiles of pw_wgrad_wide_kernel
+    WgradKind kind;
+    int rows() const { return kind == WG_SQUARE ? WG_TO + WG_TK : WW_TO + WW_TK; }     // that a workgroup asks for
 };
 
 // how the launcher and the workspace query divide the work: shares of at least four chunks, one workgroup per CU (all
 // workgroups resident at once, the tiles of a share side by side on one XCD)
-static WgradShape wgrad_shape(int O, int K, int B, int64_t P, bool wide) {
-    const int to = wide ? WW_TO : WG_TO, tk = wide ? WW_TK : WG_TK;
+static WgradShape wgrad_shape(int O, int K, int B, int64_t P, WgradKind kind) {
+    const int to = kind == WG_SQUARE ? WG_TO : kind == WG_WIDE ? WW_TO : WW_TK, tk = kind == WG_SQUARE ? WG_TK : kind == WG_WIDE ? WW_TK : WW_TO;
     WgradShape s;
-    s.wide = wide;
+    s.kind = kind;
     s.n_ot = (O + to - 1) / to;
     s.n_kt = (K + tk - 1) / tk;
     s.cps = (P + WG_PX - 1) / WG_PX;
@@ -99,11 +101,20 @@ static WgradShape wgrad_shape(int O, int K, int B, int64_t P, bool wide) {
     return s;
 }
 
-// Whichever kernel's workgroups ask for fewer rows, per pixel of the tensor, is the faster (figures at pw_wgrad_wide_kernel); 256 x 256 where O <= 256,
-// and where a few channels on the wide side would fill a 384 by little (384 -> 73 channels).
+// Bytes a CU takes in: the rows its workgroup asks for, and its part of the partial sums, written and read by a kernel of their own (twice their
+// bytes).  The kernel with fewer is the faster: 256 x 256 where both sides are at most 256 and where more shares cost more than fewer rows save
+// (384 -> 192 channels at 4 x 120 x 240 45 us, 51 with 192 x 384), else the side of 384 on the output or the input channels (384 -> 384 at 240 x 480
+// 65 -> 59 us; more at pw_wgrad_wide_kernel).
+static double wgrad_cost(const WgradShape& s, int O, int K) {
+    return 2.0 * s.rows() * WG_PX * (double)s.chunks / s.splits + 16.0 * O * K * s.splits / 256;
+}
 static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
-    const WgradShape s = wgrad_shape(O, K, B, P, false), w = wgrad_shape(O, K, B, P, true);
-    return (int64_t)(WW_TO + WW_TK) * s.splits < (int64_t)(WG_TO + WG_TK) * w.splits ? w : s;
+    WgradShape best = wgrad_shape(O, K, B, P, WG_SQUARE);
+    for (WgradKind kind : {WG_WIDE, WG_WIDE_SWAP}) {
+        const WgradShape s = wgrad_shape(O, K, B, P, kind);
+        if (wgrad_cost(s, O, K) < wgrad_cost(best, O, K)) best = s;
+    }
+    return best;
 }
 
 struct WgradArgs {
@@ -311,8 +322,11 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
 // A CU's intake bounds both kernels: memory is read once (2.40 GB for 768 -> 384 channels at 721 x 1440, 736 us), yet a chunk's 72 KiB take 2.7 us
 // with nothing else in the loop (694 us), the products alone 425; lines in L2 ahead of their requests, or a share's lines next to
 // its neighbours', made it no faster.  So the tile that asks for fewer rows is the better one: four tiles of 576 rows for 384 x 768 where the other
-// kernel has six of 512 (384 -> 768 1034 -> 843 us, 768 -> 384 873 -> 736, 384 -> 384 546 -> 407, all at 721 x 1440; 320 -> 640 at
-// 2 x 90 x 180 43 us as before).  Larger tiles (384 x 256) do not fit the registers.
+// kernel has six of 512 (384 -> 768 1034 -> 843 us, 768 -> 384 873 -> 736, 384 -> 384 546 -> 407, 384 -> 73 265 -> 198, all at
+// 721 x 1440).  Larger tiles (384 x 256) do not fit the registers.
+// SWAP: the 384 are input channels, the 192 output channels; a share's partial sums are stored transposed, [K (+ 1 with bias)][O], so that a
+// wavefront writes whole lines (written to [O][K] 384 -> 192 at 4 x 120 x 240 took 92 us).
+template <bool SWAP>
 __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs a) {
     constexpr int MT = WW_MT, NT = WW_NT, ROW = 2 * WG_PX, BUF = (WW_TO + WW_TK) * ROW;
     constexpr int PA = WW_TO * ROW / (16 * WW_THREADS), PB = WW_TK * ROW / (16 * WW_THREADS);
@@ -322,7 +336,10 @@ __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs 
     const int tiles = a.n_ot * a.n_kt;
     const int split = (q / tiles) * 8 + xcd, tile = q % tiles;
     if (split >= a.splits) return;
-    const int o0 = (tile % a.n_ot) * WW_TO, k0 = (tile / a.n_ot) * WW_TK;
+    const int ot = tile % a.n_ot, kt = tile / a.n_ot;
+    // rows of the first operand (384 of them) and of the second, and the tile's first ones
+    const int RA = SWAP ? a.K : a.O, RB = SWAP ? a.O : a.K;
+    const int a0 = (SWAP ? kt : ot) * WW_TO, b0 = (SWAP ? ot : kt) * WW_TK;
     const int64_t c_begin = (int64_t)split * a.chunks / a.splits, c_end = (int64_t)(split + 1) * a.chunks / a.splits;
     const int nch = (int)(c_end - c_begin);
 
@@ -330,15 +347,16 @@ __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wo = wave % WW_WO, wk = wave / WW_WO;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)lds) + wave * 1024;
-    WgStream<PA, WW_THREADS> sg(a.G, o0, a.O, a, c_begin, tid);
-    WgStream<PB, WW_THREADS> sx(a.X, k0, a.K, a, c_begin, tid);
+    WgStream<PA, WW_THREADS> sa(SWAP ? a.X : a.G, a0, RA, a, c_begin, tid);
+    WgStream<PB, WW_THREADS> sb(SWAP ? a.G : a.X, b0, RB, a, c_begin, tid);
     auto issue = [&](int buf) {
-        sg.issue(a, lds0 + buf * BUF, tid);
-        sx.issue(a, lds0 + buf * BUF + WW_TO * ROW, tid);
+        sa.issue(a, lds0 + buf * BUF, tid);
+        sb.issue(a, lds0 + buf * BUF + WW_TO * ROW, tid);
     };
 
     f32x16 acc[MT][NT];
-    float accb[MT], chunkb[MT];               // sums of the lane's pixels of its rows: all chunks, this chunk
+    static_assert(MT == NT, "as many row blocks of g in either order");
+    float accb[MT], chunkb[MT];               // sums of the lane's pixels of its rows of g: all chunks, this chunk
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         accb[mt] = chunkb[mt] = 0.f;
@@ -350,8 +368,8 @@ __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs 
     const int ro = wo * MT * 32, rk = wk * NT * 32;
     const int sw = (lane >> 1) & 7, kg = lane >> 5;
     const unsigned fa = (ro + (lane & 31)) * ROW, fb = (WW_TO + rk + (lane & 31)) * ROW;
-    const bool live = o0 + ro < a.O && k0 + rk < a.K;
-    const bool bias = a.Kext > a.K && k0 + rk == 0;
+    const bool live = a0 + ro < RA && b0 + rk < RB;
+    const bool bias = a.Kext > a.K && (SWAP ? a0 + ro : b0 + rk) == 0;
     bf16x8 af[2][MT], bf[2][NT];              // [step & 1][32-row block]
     auto fragments = [&](int buf, int ks) {
         const unsigned char* p = lds + buf * BUF + (unsigned)(((2 * ks + kg) ^ sw) * 16);
@@ -368,7 +386,7 @@ __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs 
         if (bias) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
-                const u32x4 p = __builtin_bit_cast(u32x4, af[ks & 1][mt]);
+                const u32x4 p = __builtin_bit_cast(u32x4, SWAP ? bf[ks & 1][mt] : af[ks & 1][mt]);
                 float lo = 0.f, hi = 0.f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -419,19 +437,19 @@ __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs 
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const int kk = k0 + rk + nt * 32 + (lane & 31);
+            const int rb = b0 + rk + nt * 32 + (lane & 31);
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int o = o0 + ro + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (o < a.O && kk < a.K) out[(int64_t)o * a.Kext + kk] = acc[mt][nt][v];
+                const int ra = a0 + ro + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                if (ra < RA && rb < RB) out[(int64_t)ra * (SWAP ? a.O : a.Kext) + rb] = acc[mt][nt][v];
             }
         }
     if (bias) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const int o = o0 + ro + mt * 32 + (lane & 31);
+            const int o = (SWAP ? b0 + rk : a0 + ro) + mt * 32 + (lane & 31);
             const float b = accb[mt] + __shfl_xor(accb[mt], 32, 64);
-            if (lane < 32 && o < a.O) out[(int64_t)o * a.Kext + a.K] = b;
+            if (lane < 32 && o < a.O) out[SWAP ? (int64_t)a.K * a.O + o : (int64_t)o * a.Kext + a.K] = b;
         }
     }
 }
@@ -442,8 +460,8 @@ __global__ __launch_bounds__(WW_THREADS, 2) void pw_wgrad_wide_kernel(WgradArgs 
 // 16 bytes) where that still makes 256 workgroups, else one.
 constexpr int WR_WAVES = 16;
 template <int V>
-__global__ __launch_bounds__(64 * WR_WAVES) void pw_wgrad_reduce_kernel(const float* __restrict__ ws, float* __restrict__ dW, float* __restrict__ db, int K,
-                                                                        int Kext, int64_t n, int splits) {
+__global__ __launch_bounds__(64 * WR_WAVES) void pw_wgrad_reduce_kernel(const float* __restrict__ ws, float* __restrict__ dW, float* __restrict__ db, int O,
+                                                                        int K, int Kext, int64_t n, int splits, bool swap) {
     typedef float vec __attribute__((ext_vector_type(V)));
     __shared__ __align__(16) float part[WR_WAVES][64 * V];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -460,8 +478,8 @@ __global__ __launch_bounds__(64 * WR_WAVES) void pw_wgrad_reduce_kernel(const fl
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < WR_WAVES; ++w) s += part[w][threadIdx.x];
-    const int64_t o = e / Kext;
-    const int k = (int)(e - o * Kext);
+    const int inner = swap ? O : Kext;             // partial sums lie as [O][Kext] or [Kext][O]
+    const int64_t i = e / inner, j = e - i * inner, o = swap ? j : i, k = swap ? i : j;
     if (k < K)
         dW[o * K + k] = s;
     else if (db)
@@ -486,16 +504,18 @@ int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, flo
     a.n_ot = sh.n_ot; a.n_kt = sh.n_kt; a.splits = sh.splits; a.cps = sh.cps; a.chunks = sh.chunks;
     const int64_t nwg = 8 * (int64_t)((sh.splits + 7) / 8) * sh.n_ot * sh.n_kt;
     if (nwg > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
-    if (sh.wide)
-        hipLaunchKernelGGL(pw_wgrad_wide_kernel, dim3((unsigned)nwg), dim3(WW_THREADS), 0, s, a);
+    if (sh.kind == WG_WIDE)
+        hipLaunchKernelGGL(pw_wgrad_wide_kernel<false>, dim3((unsigned)nwg), dim3(WW_THREADS), 0, s, a);
+    else if (sh.kind == WG_WIDE_SWAP)
+        hipLaunchKernelGGL(pw_wgrad_wide_kernel<true>, dim3((unsigned)nwg), dim3(WW_THREADS), 0, s, a);
     else
         hipLaunchKernelGGL(pw_wgrad_kernel, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
     if (hipGetLastError() != hipSuccess) return SFNO_EHIP;
     const int64_t n = (int64_t)O * Kext;
     if (n % 4 == 0 && n >= 256 * 256)
-        hipLaunchKernelGGL(pw_wgrad_reduce_kernel<4>, dim3((unsigned)((n + 255) / 256)), dim3(64 * WR_WAVES), 0, s, ws, dW, db, K, Kext, n, sh.splits);
+        hipLaunchKernelGGL(pw_wgrad_reduce_kernel<4>, dim3((unsigned)((n + 255) / 256)), dim3(64 * WR_WAVES), 0, s, ws, dW, db, O, K, Kext, n, sh.splits, sh.kind == WG_WIDE_SWAP);
     else
-        hipLaunchKernelGGL(pw_wgrad_reduce_kernel<1>, dim3((unsigned)((n + 63) / 64)), dim3(64 * WR_WAVES), 0, s, ws, dW, db, K, Kext, n, sh.splits);
+        hipLaunchKernelGGL(pw_wgrad_reduce_kernel<1>, dim3((unsigned)((n + 63) / 64)), dim3(64 * WR_WAVES), 0, s, ws, dW, db, O, K, Kext, n, sh.splits, sh.kind == WG_WIDE_SWAP);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

@@ -30,13 +30,16 @@ WGRAD_CASES = [
     (1, 257, 70, 24, 16, True),        # one column in the second column tile: the bias belongs to the first only
     (2, 73, 73, 64, 96, False),        # an odd number of entries, 48 shares: the reduction's single loads
     (1, 256, 256, 16, 40, True),       # 65792 entries: its 16-byte loads, few shares (fewer than its wavefronts)
-    # tiles of 384 x 192
-    (1, 1, 257, 1, 8, True),           # one chunk, one piece of it; wavefronts without rows or columns
-    (3, 192, 384, 9, 8, True),         # one full tile, chunks of 64 and 8 pixels: two buffers from the first share on
-    (1, 193, 385, 40, 48, True),       # a row and a column in tiles of their own
-    (2, 384, 384, 24, 40, False),      # two column tiles
-    (1, 320, 640, 16, 40, True),       # two row tiles and two column tiles, neither full
-    (1, 768, 384, 241, 480, True),     # shares of many chunks, the last chunk of the sample a part
+    # enough pixels for tiles of 384 x 192
+    (1, 1, 257, 260, 160, True),       # wavefronts without rows or columns, shares of four chunks
+    (3, 192, 384, 240, 241, True),     # one full tile, the last chunk of a sample a part
+    (2, 384, 384, 200, 212, False),    # two column tiles
+    (1, 320, 640, 161, 256, True),     # two row tiles and two column tiles, neither full
+    (1, 768, 384, 241, 480, True),     # shares of many chunks
+    # and of 192 x 384
+    (1, 257, 1, 260, 160, True),
+    (3, 384, 192, 240, 241, True),
+    (1, 384, 73, 241, 480, True),
 ]
 
 
