@@ -54,6 +54,10 @@ int build_legendre_table(const sfno_sht_plan& p, const double* theta, const doub
             nrb[m] = (K2 + PG_ROWS - 1) / PG_ROWS;       // orders without any degree still zero-fill their rows
         }
         cost[m] = 1.0 + kept[m];
+        const int nc = analysis ? (K2 + PG_KC - 1) / PG_KC : (nl0 + PG_KC - 1) / PG_KC, items = (nrb[m] + 1) / 2;
+        t.items += items;
+        t.chunks += (int64_t)items * nc;
+        if (items > 0) t.longest = std::max(t.longest, nc);
     }
     std::vector<int2> work;
     build_worklist(nrb, cost, work, 2);
@@ -121,6 +125,9 @@ PgemmArgs legendre_args(const sfno_sht_plan* p, const PgemmTable& t, const float
     a.nlat = p->nlat;
     a.mmax = p->mmax;
     a.ld = (int)ld;
+    a.items = t.items;
+    a.chunks = t.chunks;
+    a.longest = t.longest;
     return a;
 }
 

@@ -11,17 +11,25 @@
 // accumulator, where three exact bf16 parts need six.
 //   table: cut on the host from the float64 value (both parts rounded to nearest, so 23 bits are kept), one power-of-two
 //          scale per table row that brings the row's largest entry to [2^14, 2^15); 4 bytes per entry in the stream;
-//   panel: cut once per workgroup by the threads that stage it (one thread per column, which holds the column's 16 rows
-//          of the chunk: no cross-lane work) -- sums and differences of mirrored latitude rows (analysis) or the degree
-//          rows of the two parities (synthesis) go to LDS as two fp16 planes in the order the matrix instruction wants
-//          its B operand (16-byte fragment reads, no arithmetic in the matrix phase) -- with one power-of-two scale per column.  The scale of a column is found while the
-//          column streams by: the staging threads keep a bound on its exponent, raise it (leaving a few bits of
-//          headroom) when a chunk exceeds it and publish the bound with the chunk; a wavefront whose column's bound
-//          moved rescales that column's partial sums, which is exact.
+//   panel: cut once per workgroup by the wavefronts that stage it -- sums and differences of mirrored latitude rows
+//          (analysis) or the degree rows of the two parities (synthesis) go to LDS as two fp16 planes in the order the
+//          matrix instruction wants its B operand (16-byte fragment reads, no arithmetic in the matrix phase) -- with one
+//          power-of-two scale per column.  The scale of a column is found while the column streams by: the staging
+//          wavefronts keep a bound on its exponent, raise it (leaving a few bits of headroom) when a chunk exceeds it and
+//          publish the bound with the chunk; a wavefront whose column's bound moved rescales that column's partial sums,
+//          which is exact.
+// What bounds it: the panels' way from L2.  With the panel loads left out a kernel of 200 us took 157 (no matrix
+// instructions: 180; no cut: 180; loads two chunks ahead: no gain), so a lane asks for four columns at once and a
+// wavefront for whole 128-byte pieces of a row (a float per lane before): analysis of 384 rows, 721 latitudes, 240
+// degrees 162 -> 134 us, synthesis 199 -> 171; 240 latitudes 62 -> 55 and 76 -> 62; 73 rows, 721 degrees 196 -> 185
+// and 200 -> 205, before the choice of tiles (see launch_f16).
 // Entries more than 2^17 below the largest entry of their column (row) keep fewer bits, so the error bound is
 // 2^-21 |t q| + 2^-38 max|t| max|q| per product where fp32 arithmetic has 2^-24 |t q|; the transform's own longitude
 // FFT has an error of that second kind already (relative to the largest value of a latitude row).
 #include "sfno_internal.h"
+
+#include <algorithm>
+#include <cmath>
 
 namespace sfno {
 
@@ -36,9 +44,10 @@ typedef int i4 __attribute__((ext_vector_type(4)));
 constexpr int LH_TOP = 14;             // scaled magnitudes stay below 2^(TOP + 1)
 constexpr int LH_HEAD = 3;             // bits of headroom left when a column's exponent bound is raised
 constexpr int LH_SH = LH_TOP + 127;    // scaled = x * 2^(SH - E), E = biased exponent bound of the column
+constexpr int LH_EMIN = LH_SH - 127;   // smallest bound: its scale is the largest power of two of fp32 (columns below 2^-112 keep 25 bits above 2^-151)
 
 // resident workgroups per CU: set by the 16 NT accumulator registers and the staged rows held across the matrix phase
-constexpr int lh_occupancy(int nt, bool analysis) { return nt <= 4 ? 4 : analysis ? 2 : 3; }
+constexpr int lh_occupancy(int nt, bool analysis) { return nt <= 4 ? 4 : 3; }
 
 __device__ __forceinline__ unsigned int lh_pk(float a, float b) { return __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(a, b)); }
 
@@ -48,13 +57,12 @@ template <int NT, bool ANALYSIS, bool COEFFS>
 __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_kernel(PgemmArgs a) {
     constexpr int TN = 32 * NT;            // columns per workgroup
     constexpr int QN = TN / 4;             // column quads
-    constexpr int QW = QN / 4;             // column quads staged per wavefront
     // LDS image of one (buffer, panel, plane): column c = 4 j + cc lives in class cc at slot j; a slot is the column's 16 k
     // values (32 bytes); classes are CS bytes apart with CS = 128 mod 256, and the two 16-byte halves of a slot swap places in
     // classes 2 and 3, so that the 16-byte fragment reads of 16 consecutive columns cover all banks
     constexpr int CS = QN * 32 + 128;
     constexpr int PLANE = 4 * CS;
-    constexpr int PLANES = 2 * 2 * 2 * PLANE < 16384 ? 16384 : 2 * 2 * 2 * PLANE;      // [buffer][panel][plane]; at least the 16 KiB of the parity exchange
+    constexpr int PLANES = 2 * 2 * 2 * PLANE < 18432 ? 18432 : 2 * 2 * 2 * PLANE;      // [buffer][panel][plane]; at least the 16 KiB of the parity exchange
     __shared__ __align__(16) unsigned char planes[PLANES];
     __shared__ __align__(16) int expo[2][2][TN];   // [buffer][panel][column]: exponent bound the chunk was cut with
 
@@ -72,6 +80,7 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     const int m = (int)rec[PG_WREC_M];
     if (m < 0) return;
     const int2 wi = make_int2(m, (int)rec[PG_WREC_RB]);
+    __builtin_amdgcn_s_setreg((1 << 11) | (2 << 6) | 1, 3);      // MODE[3:2]: conversions to fp16 round toward zero
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     // wavefront w runs on SIMD w; alternate which SIMDs get the (possibly absent) second row block
     // and the (one row shorter) odd parity from workgroup to workgroup
@@ -94,6 +103,7 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     const float* sp_m = (ANALYSIS ? a.Out : a.Q) + (COEFFS ? 2 * (int64_t)m : (int64_t)m * lmax * ld);     // spectral panel of order m
     const int nval = COEFFS ? a.ncol : ld;         // columns with values on the spectral side
     const uint32_t srow = COEFFS ? 2u * a.mmax : (uint32_t)ld;       // floats from degree to degree, and the column's offset
+    const int live = min(NT, (ld - n0 + 31) >> 5);         // tiles with columns
     auto scolumn = [&](int n) { return COEFFS ? (uint32_t)(n >> 1) * (uint32_t)lmax * srow + (uint32_t)(n & 1) : (uint32_t)n; };
     // Index entry of a row block: first block of its stream | leading chunks left out << 48 (their entries are negligible:
     // towards the poles the table falls off like sin^m(theta)).  The K loop of the workgroup starts at the smallest such
@@ -117,114 +127,161 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
         for (int v = 0; v < 16; ++v) acc[t][v] = 0.0f;
     int erun[NT];                          // exponent bound my partial sums of tile t are scaled with (per lane = column)
 #pragma unroll
-    for (int t = 0; t < NT; ++t) erun[t] = 0;
+    for (int t = 0; t < NT; ++t) erun[t] = LH_EMIN;
 
-    // ---- staging: thread = one column of the tile and RPT consecutive rows of the chunk, both panels.  Up to four tiles a
-    // column is shared by two neighbouring lanes (8 rows each: all 256 threads at four tiles); five tiles give a thread the
-    // column's 16 rows (160 threads, dealt out over the four wavefronts).
-    constexpr int RPT = NT <= 4 ? 8 : 16;  // rows per thread
-    constexpr int TPC = PG_KC / RPT;       // threads per column
-    constexpr int CW = TN / 4;             // columns staged per wavefront
-    const bool stager = lane < CW * TPC;
-    const int scol = wave * CW + min(lane / TPC, CW - 1), shalf = lane % TPC;
-    float q0[RPT], q1[RPT];
-    int E0 = 0, E1 = 0;                    // exponent bounds of my column, panel 0 and 1 (equal in the lanes that share it)
-    // uniform panel base + 32-bit byte offset per lane (a panel is far smaller than 4 GiB): one address register per load
+    // ---- staging: a wavefront takes a column tile, a lane four columns and RPL consecutive rows of the chunk in both panels: eight
+    // lanes ask for one 128-byte piece of a row.  Up to four tiles there is a wavefront for each; of five the first wavefront takes
+    // two, 32 lanes and four rows each.
+    constexpr int RPL = NT <= 4 ? 2 : 4;   // rows per lane
+    constexpr int RG = PG_KC / RPL;        // row groups: lanes that share a column
+    const int stile = NT <= 4 ? wave : lane < 32 ? wave : wave + 4;
+    const bool stager = stile < live;
+    const int rg = (lane >> 3) & (RG - 1);
+    const int slot = min(stile, NT - 1) * 8 + (lane & 7);      // column quad of the tile
+    float q[2][RPL][4];
     const char* qpanel = reinterpret_cast<const char*>(ANALYSIS ? xm_m : sp_m);
-    const int nq = ANALYSIS ? ld : nval;
-    const int sn = min(n0 + scol, nq - 1);
-    const bool col_ok = n0 + scol < nq;
-    const uint32_t qrow = ANALYSIS ? (uint32_t)ld : srow, qcol = ANALYSIS ? (uint32_t)sn : scolumn(sn);
-    auto q_at = [&](int row) { return *reinterpret_cast<const float*>(qpanel + (size_t)(((uint32_t)row * qrow + qcol) * 4u)); };
-    // raw rows into registers (indices clamped into the panel); masking, the mirror sum/difference and the cut happen when
-    // the chunk is written to LDS, one chunk of matrix instructions later
+    const uint32_t qstep = (ANALYSIS ? (uint32_t)ld : srow) * 4u;
+    const int sn = n0 + 4 * slot;
+    constexpr bool PAIRS = COEFFS && !ANALYSIS;                // columns come as (re, im) pairs of a row
+    const int sna = PAIRS ? min(sn, nval - 2) : min(sn, ld - 4), snb = PAIRS ? min(sn + 2, nval - 2) : 0;
+    const uint32_t qca = (PAIRS ? scolumn(sna) : (uint32_t)sna) * 4u, qcb = PAIRS ? scolumn(snb) * 4u : 0u;
+    // offsets of my first row in chunk 0 and of the last row walked; a wavefront without a tile reads row 0 only
+    const uint32_t qfirst = (uint32_t)(ANALYSIS ? RPL * rg : m + 2 * RPL * rg) * qstep, qlast = stager ? (uint32_t)(ANALYSIS ? K2 - 1 : lmax - 1) * qstep : 0u;
+    const uint32_t qtop = (uint32_t)(nlat - 1) * qstep;
+    auto q_at = [&](uint32_t off, float (&v)[4]) {
+        if constexpr (PAIRS) {
+            const float2 x = *reinterpret_cast<const float2*>(qpanel + (size_t)(off + qca)), y = *reinterpret_cast<const float2*>(qpanel + (size_t)(off + qcb));
+            v[0] = x.x; v[1] = x.y; v[2] = y.x; v[3] = y.y;
+        } else {
+            const float4 x = *reinterpret_cast<const float4*>(qpanel + (size_t)(off + qca));
+            v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+        }
+    };
     auto q_load = [&](int c) {
-        if (!stager) return;
+        const uint32_t off = qfirst + (uint32_t)((ANALYSIS ? PG_KC : 2 * PG_KC) * c) * qstep;
 #pragma unroll
-        for (int rr = 0; rr < RPT; ++rr) {
-            const int i = c * PG_KC + RPT * shalf + rr;
+        for (int r = 0; r < RPL; ++r) {
             if (ANALYSIS) {
-                const int k = min(i, K2 - 1);
-                q0[rr] = q_at(k);
-                q1[rr] = q_at(nlat - 1 - k);
+                const uint32_t o = min(off + r * qstep, qlast);
+                q_at(o, q[0][r]);
+                q_at(qtop - o, q[1][r]);
             } else {
-                q0[rr] = q_at(min(m + 2 * i, lmax - 1));
-                q1[rr] = q_at(min(m + 2 * i + 1, lmax - 1));
+                q_at(min(off + 2 * r * qstep, qlast), q[0][r]);
+                q_at(min(off + (2 * r + 1) * qstep, qlast), q[1][r]);
             }
         }
     };
-    // my column's slot within a plane (class scol & 3, slot scol >> 2; the 16-byte halves swap in classes 2 and 3)
-    const int st_lo = (scol & 3) * CS + (scol >> 2) * 32 + ((((scol & 3) >> 1) ^ (RPT == 8 ? shalf : 0)) * 16), st_hi = st_lo ^ 16;
-    // one panel's values of my column: bound, scale, cut, one 16-byte write per plane and 8 rows
-    auto cut_store = [&](unsigned char* pl0, const float (&v)[RPT], int& E) {
-        float mx = __builtin_fabsf(v[0]);
+    // largest exponent of my values of a column; an excess over the bound of any column of the wavefront is rare
+    auto exponents = [&](const float (&v)[RPL][4], int (&eb)[4]) {
 #pragma unroll
-        for (int rr = 1; rr < RPT; ++rr) mx = __builtin_fmaxf(mx, __builtin_fabsf(v[rr]));
-        int mb = __builtin_bit_cast(int, mx);
-        if (TPC == 2) mb = max(mb, __builtin_amdgcn_mov_dpp(mb, 0xB1, 0xF, 0xF, true));      // the neighbour's eight rows (quad_perm [1,0,3,2])
-        const int eb = mb >> 23;
-        E = eb > E ? eb + LH_HEAD : E;
-        const int sh = LH_SH - E;
-        u4 hi[RPT / 8], lo[RPT / 8];
+        for (int cc = 0; cc < 4; ++cc) {
+            float mx;
+            asm("v_max_f32 %0, |%1|, |%2|" : "=v"(mx) : "v"(v[0][cc]), "v"(v[1][cc]));
 #pragma unroll
-        for (int e = 0; e < RPT / 2; ++e) {
-            const float xa = __builtin_ldexpf(v[2 * e], sh), xb = __builtin_ldexpf(v[2 * e + 1], sh);
-            const unsigned int h = lh_pk(xa, xb);
-            float ra, rb2;
-            // remainder = x - (float)h in one instruction each: the fp16 operand is read as it stands
-            asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(h), "v"(xa));
-            asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb2) : "v"(h), "v"(xb));
-            hi[e >> 2][e & 3] = h;
-            lo[e >> 2][e & 3] = lh_pk(ra, rb2);
+            for (int r = 2; r < RPL; ++r) asm("v_max_f32 %0, %1, |%2|" : "=v"(mx) : "v"(mx), "v"(v[r][cc]));
+            eb[cc] = __builtin_bit_cast(int, mx) >> 23;
         }
-        *reinterpret_cast<u4*>(pl0 + st_lo) = hi[0];
-        *reinterpret_cast<u4*>(pl0 + PLANE + st_lo) = lo[0];
-        if constexpr (RPT == 16) {
-            *reinterpret_cast<u4*>(pl0 + st_hi) = hi[1];
-            *reinterpret_cast<u4*>(pl0 + PLANE + st_hi) = lo[1];
+    };
+    auto raise = [&](const int (&eb_)[4], i4& E) {
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+            int eb = eb_[cc];
+#pragma unroll
+            for (int d = 8; d < 8 * RG; d <<= 1) eb = max(eb, __shfl_xor(eb, d, 64));
+            E[cc] = eb > E[cc] ? eb + LH_HEAD : E[cc];
+        }
+    };
+    const uint32_t dpos = slot * 32 + (RPL == 2 ? (rg & 3) * 4 : (rg & 1) * 8), dhalf = (RPL == 2 ? rg >> 2 : rg >> 1) * 16;
+    const uint32_t dst01 = dpos + dhalf, dst23 = dpos + (dhalf ^ 16);
+    // one panel's values of my columns: scale, cut, write
+    auto cut_store = [&](unsigned char* pl0, const float (&v)[RPL][4], const i4& E) {
+#pragma unroll
+        for (int cc = 0; cc < 4; ++cc) {
+            const float sc = __builtin_bit_cast(float, (unsigned)(LH_SH + 127 - E[cc]) << 23);
+            unsigned char* dst = pl0 + cc * CS + (cc < 2 ? dst01 : dst23);
+            unsigned hi[RPL / 2], lo[RPL / 2];
+#pragma unroll
+            for (int e = 0; e < RPL / 2; ++e) {
+                asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hi[e]) : "v"(v[2 * e][cc]), "v"(sc));
+                asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hi[e]) : "v"(v[2 * e + 1][cc]), "v"(sc));
+                asm("v_fma_mixlo_f16 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(lo[e]) : "v"(v[2 * e][cc]), "v"(sc), "v"(hi[e]));
+                asm("v_fma_mixhi_f16 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(lo[e]) : "v"(v[2 * e + 1][cc]), "v"(sc), "v"(hi[e]));
+            }
+            if constexpr (RPL == 2) {
+                *reinterpret_cast<unsigned*>(dst) = hi[0];
+                *reinterpret_cast<unsigned*>(dst + PLANE) = lo[0];
+            } else {
+                *reinterpret_cast<uint2*>(dst) = make_uint2(hi[0], hi[RPL / 2 - 1]);
+                *reinterpret_cast<uint2*>(dst + PLANE) = make_uint2(lo[0], lo[RPL / 2 - 1]);
+            }
         }
     };
     auto q_store = [&](int buf, int c) {
         if (!stager) return;
-        // chunks that touch neither end of the K range nor the column tail need no masks
-        const bool plain = col_ok && (ANALYSIS ? (c + 1) * PG_KC < K2 : m + 2 * (c + 1) * PG_KC < lmax);
+        // chunks that touch neither end of the K range need no masks
+        const bool plain = ANALYSIS ? (c + 1) * PG_KC < K2 : m + 2 * (c + 1) * PG_KC < lmax;
+        if (PAIRS && sn + 2 >= nval) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int r = 0; r < RPL; ++r)
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc)
+                        if (sn + cc >= nval) q[p][r][cc] = 0.f;
+        }
         if constexpr (ANALYSIS) {
             // i = latitude k; panel 0 = X[k] + X[k'], panel 1 = X[k] - X[k']; the equator row is its own mirror
-            float v0[RPT], v1[RPT];
-            if (plain) {
-#pragma unroll
-                for (int rr = 0; rr < RPT; ++rr) {
-                    v0[rr] = q0[rr] + q1[rr];
-                    v1[rr] = q0[rr] - q1[rr];
-                }
-            } else {
-#pragma unroll
-                for (int rr = 0; rr < RPT; ++rr) {
-                    const int i = c * PG_KC + RPT * shalf + rr;
-                    const bool ok = col_ok && i < K2, mirror = (nlat - 1 - i) != i;
-                    v0[rr] = ok ? (mirror ? q0[rr] + q1[rr] : q0[rr]) : 0.f;
-                    v1[rr] = ok && mirror ? q0[rr] - q1[rr] : 0.f;
-                }
-            }
-            cut_store(planes + ((buf * 2 + 0) * 2) * PLANE, v0, E0);
-            cut_store(planes + ((buf * 2 + 1) * 2) * PLANE, v1, E1);
-        } else {
-            // i = index within a parity; panel 0 = degree m+2i, panel 1 = degree m+2i+1.  What lies outside is zeroed in place (the
-            // raw rows are not needed again), so that the common case carries no copies of the 32 values
             if (!plain) {
 #pragma unroll
-                for (int rr = 0; rr < RPT; ++rr) {
-                    const int i = c * PG_KC + RPT * shalf + rr;
-                    q0[rr] = (col_ok && m + 2 * i < lmax) ? q0[rr] : 0.f;
-                    q1[rr] = (col_ok && m + 2 * i + 1 < lmax) ? q1[rr] : 0.f;
+                for (int r = 0; r < RPL; ++r) {
+                    const int i = c * PG_KC + RPL * rg + r;
+                    const bool ok = i < K2, mirror = (nlat - 1 - i) != i;
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc) {
+                        q[0][r][cc] = ok ? q[0][r][cc] : 0.f;
+                        q[1][r][cc] = ok && mirror ? q[1][r][cc] : 0.f;
+                    }
                 }
             }
-            cut_store(planes + ((buf * 2 + 0) * 2) * PLANE, q0, E0);
-            cut_store(planes + ((buf * 2 + 1) * 2) * PLANE, q1, E1);
+#pragma unroll
+            for (int r = 0; r < RPL; ++r)
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc) {
+                    const float a_ = q[0][r][cc], b_ = q[1][r][cc];
+                    q[0][r][cc] = a_ + b_;
+                    q[1][r][cc] = a_ - b_;
+                }
+            if (!plain) {
+#pragma unroll
+                for (int r = 0; r < RPL; ++r) {
+                    const int i = c * PG_KC + RPL * rg + r;
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc) q[1][r][cc] = (nlat - 1 - i) != i ? q[1][r][cc] : 0.f;
+                }
+            }
+        } else if (!plain) {
+            // i = index within a parity; panel 0 = degree m+2i, panel 1 = degree m+2i+1
+#pragma unroll
+            for (int r = 0; r < RPL; ++r) {
+                const int i = c * PG_KC + RPL * rg + r;
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc) {
+                    q[0][r][cc] = m + 2 * i < lmax ? q[0][r][cc] : 0.f;
+                    q[1][r][cc] = m + 2 * i + 1 < lmax ? q[1][r][cc] : 0.f;
+                }
+            }
         }
-        if (shalf == 0) {
-            expo[buf][0][scol] = E0;
-            expo[buf][1][scol] = E1;
+        // the bounds live in the other buffer's array between chunks: they would cost eight registers across the matrix phase
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            i4 E = *reinterpret_cast<const i4*>(&expo[buf ^ 1][p][4 * slot]);
+            int eb[4];
+            exponents(q[p], eb);
+            const int over = max(max(eb[0] - E[0], eb[1] - E[1]), max(eb[2] - E[2], eb[3] - E[3]));
+            if (__builtin_amdgcn_ballot_w64(over > 0) != 0) raise(eb, E);
+            cut_store(planes + ((buf * 2 + p) * 2) * PLANE, q[p], E);
+            if (rg == 0) *reinterpret_cast<i4*>(&expo[buf][p][4 * slot]) = E;
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -263,40 +320,39 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     auto a_load = [&](int c, f4 (&ar)[2]) {
         // (chunks past the end repeat the last one: the stream of the next row block, or the end of the buffer, follows)
 #pragma unroll
-        for (int p = 0; p < 2; ++p) ar[p] = apv[(int64_t)max(min(c, nc - 1) - c0w, 0) * APB + 64 * p];
+        for (int p = 0; p < 2; ++p) ar[p] = apv[(int64_t)min(max(c - c0w, 0), max(nc - 1 - c0w, 0)) * APB + 64 * p];
     };
 
-    // Software pipeline, one chunk deep: the loads of the next chunk (raw panel rows and table fragments) are issued before
-    // the matrix instructions of the current one and are first touched after them.  (Table fragments requested three chunks
-    // ahead, in rotating register sets, changed nothing at any shape and cost a resident workgroup at four tiles.)
+    // Software pipeline, one chunk deep: the panel rows of the next chunk are requested before the matrix instructions of the current
+    // one and its table fragments after them (into the same registers); the rows are cut once those instructions are issued.
     // The analysis walks the latitudes from the equator to the pole: Fourier coefficients of order m fall off towards the
     // poles like sin^m(theta), so the first chunk sets the column scales and later ones rarely move them; the synthesis
     // walks the degrees upwards, the direction in which spectra decay.
     constexpr int cstep = ANALYSIS ? -1 : 1;
     const int cfirst = ANALYSIS ? nc - 1 : cstart;
-    f4 acur[2], anext[2];
+    f4 acur[2];
     if (cstart < nc) {
+        if (stager && rg == 0) {
+            const i4 e0 = {LH_EMIN, LH_EMIN, LH_EMIN, LH_EMIN};
+            *reinterpret_cast<i4*>(&expo[(cfirst & 1) ^ 1][0][4 * slot]) = e0;
+            *reinterpret_cast<i4*>(&expo[(cfirst & 1) ^ 1][1][4 * slot]) = e0;
+        }
         q_load(cfirst);
         a_load(cfirst, acur);
         q_store(cfirst & 1, cfirst);
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0): the first table fragments too
     __syncthreads();
     for (int c = cfirst, left = nc - cstart; left > 0; --left, c += cstep) {
         const int buf = c & 1;
         const bool more = left > 1;
-        if (more) {
-            q_load(c + cstep);
-            a_load(c + cstep, anext);
-        }
+        q_load(c + cstep);      // (past the end: the nearest row; unconditional, so that what is waited for can be counted)
         __builtin_amdgcn_sched_barrier(0);
         if (c >= c0w) compute(buf, acur);
         __builtin_amdgcn_sched_barrier(0);
+        a_load(c + cstep, acur);
+        __builtin_amdgcn_sched_barrier(0);
         if (more) q_store(buf ^ 1, c + cstep);
-        __builtin_amdgcn_s_waitcnt(0x0F70);       // vmcnt(0): everything issued above has landed
         __syncthreads();
-#pragma unroll
-        for (int p = 0; p < 2; ++p) acur[p] = anext[p];
     }
 
     // ---- epilogue: undo the scales (row factor stored with the table, column bound erun), store ------------------------------
@@ -360,47 +416,67 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
             }
         }
     } else {
-        // X[k] = E[k] + O[k] and X[k'] = E[k] - O[k]: the two wavefronts of a row block swap their sums through LDS, one column
-        // tile at a time, and each stores one of the two rows -- the even-parity wavefront the northern row k, the odd-parity
-        // one the mirrored row k' -- so that all four wavefronts share the stores
-        static_assert(4 * 16 * 64 * 4 <= PLANES, "the parity exchange reuses the plane buffers");
+        // X[k] = E[k] + O[k] and X[k'] = E[k] - O[k]: the two wavefronts of a row block leave their sums in LDS, TB column tiles at a
+        // time, and each stores one of the two rows -- the even-parity wavefront the northern row k, the odd-parity one the mirrored
+        // row k' -- so that all four wavefronts share the stores; read back by rows, four columns to a lane
+        constexpr int TP = 32 * 36;                   // floats of a tile: rows 36 apart keep the 16-byte reads aligned and off each other's banks
+        constexpr int TB = NT >= 2 && PLANES >= 2 * 4 * TP * 4 ? 2 : 1;
+        static_assert(TB * 4 * TP * 4 <= PLANES, "the parity exchange reuses the plane buffers");
         float* exch = reinterpret_cast<float*>(planes);
-        float* mine = exch + wslot * (16 * 64) + lane;
-        const float* theirs = exch + (wslot ^ 2) * (16 * 64) + lane;
+        float* mine = exch + wslot * (TB * TP) + 4 * kg * 36 + cl;
+        const int er = lane >> 3, ec = 4 * (lane & 7);
+        const float* pe = exch + (wslot & 1) * (TB * TP) + er * 36 + ec;
+        const float* po = pe + 2 * (TB * TP);
         float* out = a.Out + (int64_t)m * nlat * ld;
-        const int k0 = PG_ROWS * rb + 4 * kg;
-        const bool whole = active && PG_ROWS * (rb + 1) <= K2 - 1 && n0 + TN <= ld;      // no row or column of my tile needs a check
+        const int k0 = PG_ROWS * rb;
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            if (t > 0) __syncthreads();               // the previous tile has been read
+        for (int t0 = 0; t0 < NT; t0 += TB) {
+            if (t0 > 0) __syncthreads();               // the previous tiles have been read
             if (active) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) mine[v * 64] = acc[t][v];
+                for (int t = t0; t < t0 + TB && t < NT; ++t)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) mine[(t - t0) * TP + (8 * (v >> 2) + (v & 3)) * 36] = acc[t][v];
             }
             __syncthreads();
-            if (whole) {
-                // one address per wavefront tile, rows at multiples of +-ld from it, no checks
-                float* o = out + (int64_t)(par ? nlat - 1 - k0 : k0) * ld + n0 + 32 * t + cl;
-                const int64_t rstep = par ? -(int64_t)ld : (int64_t)ld;
+            if (active) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const float other = theirs[v * 64];
-                    o[(8 * (v >> 2) + (v & 3)) * rstep] = par ? other - acc[t][v] : acc[t][v] + other;
-                }
-            } else if (active) {
-                const int n = n0 + 32 * t + cl;
+                for (int t = t0; t < t0 + TB && t < NT; ++t) {
+                    const int n = n0 + 32 * t + ec;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int k = k0 + 8 * (v >> 2) + (v & 3);
-                    const float other = theirs[v * 64];
-                    // even parity: E + O to row k; odd parity: E - O to row k' (the equator row is its own mirror and has O = 0)
-                    const float x = par ? other - acc[t][v] : acc[t][v] + other;
-                    const int row = par ? nlat - 1 - k : k;
-                    if (k < K2 && n < ld && !(par && row == k)) out[(int64_t)row * ld + n] = x;
+                    for (int u = 0; u < 4; ++u) {
+                        const int k = k0 + 8 * u + er;
+                        const f4 e = *reinterpret_cast<const f4*>(pe + (t - t0) * TP + 8 * u * 36), o = *reinterpret_cast<const f4*>(po + (t - t0) * TP + 8 * u * 36);
+                        const int row = par ? nlat - 1 - k : k;
+                        // even parity: E + O to row k; odd parity: E - O to row k' (the equator row is its own mirror and has O = 0)
+                        if (k < K2 && n < ld && !(par && row == k)) *reinterpret_cast<f4*>(out + (int64_t)row * ld + n) = par ? e - o : e + o;
+                    }
                 }
             }
         }
     }
+}
+
+// Column tiles per workgroup (1 to 5).  Wide workgroups read the table once for more columns and spread the cut of the panels, narrow
+// ones are more in number (small grids leave CUs idle) and pad less.  Estimated time in us: a launch, and the longer of one workgroup
+// alone (longest chunk loop and epilogue) and a CU's share of all of them, the coefficients fitted to 4000 measured shapes per
+// direction (8 to 720 latitudes, 2 to 720 degrees, 1 to 3072 rows, all five tile counts): the choice is 0.6 % (analysis) and 0.8 % (synthesis) from the
+// best tile count on average, 11 % at worst above 30 us.  By the least padding alone it was 10 % and 85 %: 74 rows of 160 x 320 went
+// 14.4 -> 11.4 us and 17.2 -> 12.7, 384 rows of 721 latitudes and 240 degrees keep four tiles.
+int legendre_f16_tiles(bool analysis, int64_t ncols, int64_t items, int64_t chunks, int longest, int cus) {
+    static const double alone[2][4] = {{0.626, 0.139, 0.0, 0.328}, {0.619, 0.161, 0.0, 0.294}};      // per chunk: + per tile; epilogue: + per tile
+    static const double per_chunk[2][5] = {{0.259, 0.291, 0.297, 0.278, 0.377}, {0.247, 0.348, 0.435, 0.480, 0.673}};
+    static const double per_item[2][5] = {{0.673, 1.338, 2.152, 2.769, 3.901}, {0.488, 0.871, 1.352, 1.920, 3.060}};
+    int best = 1;
+    double best_t = 0.0;
+    for (int nt = 1; nt <= 5; ++nt) {
+        const double groups = (double)((ncols + 32 * nt - 1) / (32 * nt));
+        const double one = longest * (alone[analysis][0] + alone[analysis][1] * nt) + alone[analysis][2] + alone[analysis][3] * nt;
+        const double all = groups * ((double)chunks * per_chunk[analysis][nt - 1] + (double)items * per_item[analysis][nt - 1]) / cus;
+        const double t = std::pow(std::pow(one, 4) + std::pow(all, 4), 0.25);
+        if (nt == 1 || t < best_t) { best_t = t; best = nt; }
+    }
+    return best;
 }
 
 template <bool ANALYSIS, bool COEFFS>
@@ -410,14 +486,7 @@ static int launch_f16(const PgemmArgs& a, int n_work, hipStream_t s) {
     if (!a.rinv || !a.wrec) return SFNO_EINVAL;
     // the kernel addresses a panel (one order: nlat or lmax rows of ld floats) with 32-bit byte offsets
     if ((int64_t)(a.nlat > a.lmax ? a.nlat : a.lmax) * a.ld >= ((int64_t)1 << 30)) return SFNO_EUNSUPPORTED;
-    // prefer the least padding, then the tile count listed first
-    static const int cand[] = {4, 3, 5, 2, 1};
-    int best = 1;
-    int64_t best_pad = INT64_MAX;
-    for (int nt : cand) {
-        int64_t pad = (ncols + 32 * nt - 1) / (32 * nt) * (32 * nt);
-        if (pad < best_pad) { best_pad = pad; best = nt; }
-    }
+    const int best = legendre_f16_tiles(ANALYSIS, ncols, a.items, a.chunks, a.longest, device_cus());
 #define LH_CASE(NT_)                                                                             \
     case NT_: {                                                                                  \
         const int64_t nwg = (int64_t)n_work * ((ncols + 32 * NT_ - 1) / (32 * NT_));             \

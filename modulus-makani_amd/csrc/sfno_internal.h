@@ -35,6 +35,8 @@ struct PgemmTable {
     int64_t* d_wrec = nullptr;     // two-part fp16 format: [n_work][8] everything a workgroup needs of the index, see PG_WREC_*
     int n_work = 0;                // multiple of 8 (one queue per XCD, interleaved)
     int64_t n_blocks = 0;
+    int64_t items = 0, chunks = 0; // entries of the work list and K chunks of all of them (leading chunks that are left out included)
+    int longest = 0;               // K chunks of the longest one
 };
 
 struct PgemmArgs {
@@ -47,6 +49,8 @@ struct PgemmArgs {
     const float* rinv;             // two-part fp16 format: row factors, [entry position - 2 mmax][32]
     int lmax, nlat, mmax;          // Legendre modes
     int ld;                        // channel leading dimension of Q and Out (Legendre modes)
+    int64_t items, chunks;         // as in PgemmTable
+    int longest;
     int ncol;                      // the spectral side in the reference layout: columns, 2 rows
 };
 
@@ -188,6 +192,7 @@ void pack_legendre_fold(const LegendreGen& g, const double* lat_w, const double*
                         std::vector<float>* rinv = nullptr);
 int legendre_fold_launch(bool analysis, int format, const PgemmArgs& a, int n_work, hipStream_t s);
 int legendre_f16_launch(bool analysis, const PgemmArgs& a, int n_work, hipStream_t s);
+int legendre_f16_tiles(bool analysis, int64_t ncols, int64_t items, int64_t chunks, int longest, int cus);
 // the same with coefficients complex [rows][lmax][mmax] as the analysis' output or the synthesis' input, where they fit
 bool legendre_coeffs_fit(bool analysis, int format, int64_t rows, int lmax, int mmax);
 int legendre_coeffs_launch(bool analysis, PgemmArgs a, int64_t rows, int n_work, hipStream_t s);
