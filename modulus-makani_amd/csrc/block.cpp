@@ -209,22 +209,19 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
     float *c0 = training ? (float*)(k + off[SFNO_BLOCK_COEF0]) : w.coef0, *c1 = (float*)(k + off[SFNO_BLOCK_COEF1]);
     const bf16* res = reinterpret_cast<const bf16*>(x);
 
-    TRY(sfno_rfft(b->fwd, x, SFNO_DTYPE_BF16, w.xm_in, d.rows_in, s));
-    TRY(sfno_legendre_analysis(b->fwd, w.xm_in, spec, d.rows_in, s));
+    TRY(analysis_launch(b->fwd, x, SFNO_DTYPE_BF16, nullptr, w.xm_in, spec, d.rows_in, s));
     if (d.scale_residual) {
         bf16* r = (bf16*)(k + off[SFNO_BLOCK_RES]);
-        TRY(sfno_legendre_synthesis(b->inv, spec, w.xm_out, d.rows_in, s));
-        TRY(sfno_irfft(b->inv, w.xm_out, r, SFNO_DTYPE_BF16, d.rows_in, s));
+        TRY(synthesis_launch(b->inv, spec, w.xm_out, r, SFNO_DTYPE_BF16, nullptr, d.rows_in, s));
         res = r;
     }
     TRY(mix(b->weights, spec, w.spec, d, d.rows, s));
-    TRY(sfno_legendre_synthesis(b->inv, w.spec, w.xm_out, d.rows, s));
     float2* m0 = reinterpret_cast<float2*>(c0 + 2 * d.rows);
     if (d.P <= NORM_SMALL_PIXELS) {
-        TRY(sfno_irfft(b->inv, w.xm_out, xf, SFNO_DTYPE_BF16, d.rows, s));
+        TRY(synthesis_launch(b->inv, w.spec, w.xm_out, xf, SFNO_DTYPE_BF16, nullptr, d.rows, s));
         TRY(instance_norm_coeffs_launch(xf, b->gamma0, b->beta0, c0, c0 + d.rows, w.partial, d.rows, d.e, d.P, b->eps0, s, m0));
     } else {
-        TRY(irfft_launch(b->inv->fft, w.xm_out, xf, SFNO_DTYPE_BF16, d.rows, b->inv->nlat, d.mmax, (int)sfno_spectral_ld(d.rows), s, w.stats));
+        TRY(synthesis_launch(b->inv, w.spec, w.xm_out, xf, SFNO_DTYPE_BF16, w.stats, d.rows, s));
         TRY(instance_norm_coeffs_lat_launch(w.stats, b->gamma0, b->beta0, c0, c0 + d.rows, d.rows, d.e, b->inv->nlat, b->eps0, s, m0));
     }
     if (!training && d.one_mlp) {

@@ -30,6 +30,7 @@ void free_table(PgemmTable& t) {
     if (t.d_aoff) (void)hipFree(t.d_aoff);
     if (t.d_work) (void)hipFree(t.d_work);
     if (t.d_wrec) (void)hipFree(t.d_wrec);
+    if (t.d_kept) (void)hipFree(t.d_kept);
     t = PgemmTable();
 }
 
@@ -59,6 +60,37 @@ int build_legendre_table(const sfno_sht_plan& p, const double* theta, const doub
         t.chunks += (int64_t)items * nc;
         if (items > 0) t.longest = std::max(t.longest, nc);
     }
+    // Orders that matter at a latitude: row k = min(latitude, its mirror) of the Fourier buffer of order m is read by an analysis from the first K chunk on that
+    // a row block of the order keeps, and is zero behind a synthesis in the row blocks that keep no chunk in either parity; both grow with the
+    // order, so the others are the last ones.  (The smallest such row of this and all higher orders, should they not grow somewhere.)
+    std::vector<int> blocks(p.mmax);       // synthesis: leading row blocks that do not matter
+    std::vector<int> kept_orders(p.nlat);
+    {
+        std::vector<int> row(p.mmax);
+        for (int m = p.mmax - 1; m >= 0; --m) {
+            const int nl[2] = {(p.lmax - m > 0) ? (p.lmax - m + 1) / 2 : 0, (p.lmax - m - 1 > 0) ? (p.lmax - m) / 2 : 0};
+            auto skip = [&](int par, int rb) { return (int)(aoff[(size_t)(aoff[2 * m + par] + rb)] >> 48); };
+            if (analysis) {
+                int c = (K2 + PG_KC - 1) / PG_KC;
+                for (int par = 0; par < 2; ++par)
+                    for (int rb = 0; rb * PG_ROWS < nl[par]; ++rb) c = std::min(c, skip(par, rb));
+                row[m] = c * PG_KC;
+            } else {
+                const int nc = (nl[0] + PG_KC - 1) / PG_KC;
+                int rb = 0;
+                while (rb < nrb[m] && (nc == 0 || (skip(0, rb) >= nc && skip(1, rb) >= nc))) ++rb;
+                blocks[m] = m + 1 < p.mmax ? std::min(rb, blocks[m + 1]) : rb;
+                row[m] = blocks[m] * PG_ROWS;
+            }
+            if (m + 1 < p.mmax) row[m] = std::min(row[m], row[m + 1]);
+        }
+        row[0] = 0;
+        blocks[0] = 0;
+        for (int k = 0, n = 0; k < K2; ++k) {
+            while (n < p.mmax && row[n] <= k) ++n;
+            kept_orders[k] = kept_orders[p.nlat - 1 - k] = n;
+        }
+    }
     std::vector<int2> work;
     build_worklist(nrb, cost, work, 2);
     t.n_work = (int)work.size();
@@ -68,6 +100,7 @@ int build_legendre_table(const sfno_sht_plan& p, const double* theta, const doub
     if (p.format == PG_FORMAT_F16X2 && (rc = upload(&t.d_rinv, rinv)) != SFNO_OK) return rc;
     if ((rc = upload(&t.d_aoff, aoff)) != SFNO_OK) return rc;
     if ((rc = upload(&t.d_work, work)) != SFNO_OK) return rc;
+    if ((rc = upload(&t.d_kept, kept_orders)) != SFNO_OK) return rc;
     if (p.format == PG_FORMAT_F16X2) {
         std::vector<int64_t> wrec(work.size() * PG_WREC, 0);
         for (size_t w = 0; w < work.size(); ++w) {
@@ -76,6 +109,7 @@ int build_legendre_table(const sfno_sht_plan& p, const double* theta, const doub
             r[PG_WREC_M] = m;
             r[PG_WREC_RB] = rb0;
             if (m < 0) continue;
+            if (!analysis) r[PG_WREC_M] |= (int64_t)blocks[m] << 32;
             const int nl0 = (p.lmax - m > 0) ? (p.lmax - m + 1) / 2 : 0;
             const int nl1 = (p.lmax - m - 1 > 0) ? (p.lmax - m) / 2 : 0;
             const int nc = analysis ? (K2 + PG_KC - 1) / PG_KC : (nl0 + PG_KC - 1) / PG_KC;
@@ -336,15 +370,47 @@ extern "C" int sfno_legendre_synthesis(const sfno_sht_plan* p, const float* spec
     return legendre_fold_launch(false, p->format, a, p->inv.n_work, (hipStream_t)stream);
 }
 
+// orders that matter at each latitude, where the longitude kernels can leave the others out
+static const int* kept_orders(const sfno_sht_plan* p, const PgemmTable& t) { return !planar(p) && fft_fast_supported(p->nlon) ? t.d_kept : nullptr; }
+
+// Legendre synthesis from `table` and the longitude transform behind it
+static int synthesis_from(const sfno_sht_plan* p, const PgemmTable& table, const float* spec, float* xm, void* x, int x_dtype, float2* lat_stats, int64_t rows,
+                          hipStream_t s) {
+    const int64_t ld = sfno_spectral_ld(rows);
+    const int* kept = kept_orders(p, table);
+    PgemmArgs a = legendre_args(p, table, spec, xm, ld);
+    a.drop = kept != nullptr;
+    const int rc = legendre_fold_launch(false, p->format, a, table.n_work, s);
+    return rc != SFNO_OK ? rc : irfft_launch(p->fft, xm, x, x_dtype, rows, p->nlat, p->mmax, (int)ld, s, lat_stats, kept);
+}
+
+// longitude transform and the Legendre analysis with `table` behind it
+static int analysis_with(const sfno_sht_plan* p, const PgemmTable& table, const void* x, int x_dtype, const float* x2, float* xm, float* spec, int64_t rows,
+                         hipStream_t s) {
+    const int64_t ld = sfno_spectral_ld(rows);
+    const int rc = rfft_launch(p->fft, x, x_dtype, xm, rows, p->nlat, p->mmax, (int)ld, s, x2, kept_orders(p, table));
+    return rc != SFNO_OK ? rc : legendre_fold_launch(true, p->format, legendre_args(p, table, xm, spec, ld), table.n_work, s);
+}
+
+int sfno::analysis_launch(const sfno_sht_plan* p, const void* x, int x_dtype, const float* x2, float* xm, float* spec, int64_t rows, hipStream_t s) {
+    if (!planar(p)) return analysis_with(p, p->fwd, x, x_dtype, x2, xm, spec, rows, s);
+    const int rc = rfft_launch(p->fft, x, x_dtype, xm, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), s, x2);
+    return rc != SFNO_OK ? rc : planar_stage(p, MS_FWD, false, xm, spec, rows, s);
+}
+
+int sfno::synthesis_launch(const sfno_sht_plan* p, const float* spec, float* xm, void* x, int x_dtype, float2* lat_stats, int64_t rows, hipStream_t s) {
+    if (!planar(p)) return synthesis_from(p, p->inv, spec, xm, x, x_dtype, lat_stats, rows, s);
+    const int rc = planar_stage(p, MS_INV, true, spec, xm, rows, s);
+    return rc != SFNO_OK ? rc : irfft_launch(p->fft, xm, x, x_dtype, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), s, lat_stats);
+}
+
 extern "C" int sfno_sht_analysis_diff(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, int64_t rows, void* workspace,
                                       size_t workspace_bytes, void* stream) {
     if (!p || !x || !x2 || !spec || !rows_ok(rows)) return SFNO_EINVAL;
     if (!(p->directions & SFNO_DIR_FORWARD)) return SFNO_EINVAL;
     Ws w = carve(p, rows, workspace);
     if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
-    int rc = rfft_launch(p->fft, x, SFNO_DTYPE_F32, w.xm, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream, x2);
-    if (rc != SFNO_OK) return rc;
-    return sfno_legendre_analysis(p, w.xm, spec, rows, stream);
+    return analysis_launch(p, x, SFNO_DTYPE_F32, x2, w.xm, spec, rows, (hipStream_t)stream);
 }
 extern "C" int sfno_sht_analysis(const sfno_sht_plan* p, const void* x, int x_dtype, float* spec, int64_t rows, void* workspace,
                                  size_t workspace_bytes, void* stream) {
@@ -352,9 +418,7 @@ extern "C" int sfno_sht_analysis(const sfno_sht_plan* p, const void* x, int x_dt
     if (!(p->directions & SFNO_DIR_FORWARD)) return SFNO_EINVAL;
     Ws w = carve(p, rows, workspace);
     if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
-    int rc = sfno_rfft(p, x, x_dtype, w.xm, rows, stream);
-    if (rc != SFNO_OK) return rc;
-    return sfno_legendre_analysis(p, w.xm, spec, rows, stream);
+    return analysis_launch(p, x, x_dtype, nullptr, w.xm, spec, rows, (hipStream_t)stream);
 }
 
 extern "C" int sfno_sht_synthesis(const sfno_sht_plan* p, const float* spec, void* x, int x_dtype, int64_t rows, void* workspace,
@@ -363,9 +427,7 @@ extern "C" int sfno_sht_synthesis(const sfno_sht_plan* p, const float* spec, voi
     if (!(p->directions & SFNO_DIR_INVERSE)) return SFNO_EINVAL;
     Ws w = carve(p, rows, workspace);
     if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
-    int rc = sfno_legendre_synthesis(p, spec, w.xm, rows, stream);
-    if (rc != SFNO_OK) return rc;
-    return sfno_irfft(p, w.xm, x, x_dtype, rows, stream);
+    return synthesis_launch(p, spec, w.xm, x, x_dtype, nullptr, rows, (hipStream_t)stream);
 }
 
 extern "C" int sfno_sht_lat_stats_supported(const sfno_sht_plan* p) { return p && fft_fast_supported(p->nlon) ? 1 : 0; }
@@ -377,10 +439,7 @@ extern "C" int sfno_sht_synthesis_lat_stats(const sfno_sht_plan* p, const float*
     if (!sfno_sht_lat_stats_supported(p)) return SFNO_EUNSUPPORTED;
     Ws w = carve(p, rows, workspace);
     if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
-    int rc = sfno_legendre_synthesis(p, spec, w.xm, rows, stream);
-    if (rc != SFNO_OK) return rc;
-    return irfft_launch(p->fft, w.xm, x, x_dtype, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream,
-                        reinterpret_cast<float2*>(lat_stats));
+    return synthesis_launch(p, spec, w.xm, x, x_dtype, reinterpret_cast<float2*>(lat_stats), rows, (hipStream_t)stream);
 }
 
 extern "C" int sfno_sht_forward(const sfno_sht_plan* p, const float* x, void* coeffs, int64_t rows, void* workspace,
@@ -393,7 +452,8 @@ extern "C" int sfno_sht_forward(const sfno_sht_plan* p, const float* x, void* co
         if (rc != SFNO_EUNSUPPORTED) return rc;
     }
     if (!planar(p) && x && rows_ok(rows) && (p->directions & SFNO_DIR_FORWARD) && legendre_coeffs_fit(true, p->format, rows, p->lmax, p->mmax)) {
-        const int rc = sfno_rfft(p, x, SFNO_DTYPE_F32, w.xm, rows, stream);
+        const int rc = rfft_launch(p->fft, x, SFNO_DTYPE_F32, w.xm, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream, nullptr,
+                                   kept_orders(p, p->fwd));
         if (rc != SFNO_OK) return rc;
         const PgemmArgs a = legendre_args(p, p->fwd, w.xm, reinterpret_cast<float*>(coeffs), sfno_spectral_ld(rows));
         return legendre_coeffs_launch(true, a, rows, p->fwd.n_work, (hipStream_t)stream);
@@ -414,10 +474,12 @@ extern "C" int sfno_sht_inverse(const sfno_sht_plan* p, const void* coeffs, floa
         if (rc != SFNO_EUNSUPPORTED) return rc;
     }
     if (!planar(p) && x && rows_ok(rows) && (p->directions & SFNO_DIR_INVERSE) && legendre_coeffs_fit(false, p->format, rows, p->lmax, p->mmax)) {
-        const PgemmArgs a = legendre_args(p, p->inv, reinterpret_cast<const float*>(coeffs), w.xm, sfno_spectral_ld(rows));
+        PgemmArgs a = legendre_args(p, p->inv, reinterpret_cast<const float*>(coeffs), w.xm, sfno_spectral_ld(rows));
+        const int* kept = kept_orders(p, p->inv);
+        a.drop = kept != nullptr;
         const int rc = legendre_coeffs_launch(false, a, rows, p->inv.n_work, (hipStream_t)stream);
         if (rc != SFNO_OK) return rc;
-        return sfno_irfft(p, w.xm, x, SFNO_DTYPE_F32, rows, stream);
+        return irfft_launch(p->fft, w.xm, x, SFNO_DTYPE_F32, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream, nullptr, kept);
     }
     int rc = coeffs_to_spectral_launch(reinterpret_cast<const float2*>(coeffs), w.spec, rows, p->lmax, p->mmax,
                                        (int)sfno_spectral_ld(rows), planar(p) ? 0 : 1, (hipStream_t)stream);
@@ -430,23 +492,16 @@ extern "C" int sfno_sht_inverse(const sfno_sht_plan* p, const void* coeffs, floa
 // spectral layout -> grid / grid -> spectral layout with the Fourier buffer passed in
 int sfno::analysis_adjoint_launch(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, float* xm, int64_t rows, hipStream_t s) {
     if (!(p->directions & SFNO_DIR_FORWARD_ADJOINT)) return SFNO_EINVAL;
-    int rc;
-    if (planar(p)) {
-        rc = planar_stage(p, MS_FWD_ADJ, true, gspec, xm, rows, s);
-    } else {
-        PgemmArgs a = legendre_args(p, p->fwd_adj, gspec, xm, sfno_spectral_ld(rows));
-        rc = legendre_fold_launch(false, p->format, a, p->fwd_adj.n_work, s);
-    }
+    if (!planar(p)) return synthesis_from(p, p->fwd_adj, gspec, xm, gx, x_dtype, nullptr, rows, s);
+    const int rc = planar_stage(p, MS_FWD_ADJ, true, gspec, xm, rows, s);
     return rc != SFNO_OK ? rc : sfno_irfft(p, xm, gx, x_dtype, rows, s);
 }
 
 int sfno::synthesis_adjoint_launch(const sfno_sht_plan* p, const void* gx, int x_dtype, float* xm, float* gspec, int64_t rows, hipStream_t s) {
     if (!(p->directions & SFNO_DIR_INVERSE_ADJOINT)) return SFNO_EINVAL;
+    if (!planar(p)) return analysis_with(p, p->inv_adj, gx, x_dtype, nullptr, xm, gspec, rows, s);
     const int rc = sfno_rfft(p, gx, x_dtype, xm, rows, s);
-    if (rc != SFNO_OK) return rc;
-    if (planar(p)) return planar_stage(p, MS_INV_ADJ, false, xm, gspec, rows, s);
-    PgemmArgs a = legendre_args(p, p->inv_adj, xm, gspec, sfno_spectral_ld(rows));
-    return legendre_fold_launch(true, p->format, a, p->inv_adj.n_work, s);
+    return rc != SFNO_OK ? rc : planar_stage(p, MS_INV_ADJ, false, xm, gspec, rows, s);
 }
 
 extern "C" int sfno_sht_analysis_adjoint(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, int64_t rows, void* workspace,

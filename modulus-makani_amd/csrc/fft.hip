@@ -391,10 +391,10 @@ static int pick_pairs(int n) {
     return 0;
 }
 
-int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2) {
+int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2, const int* kept) {
     if (mmax > p.n / 2 + 1 || ld % 4 != 0 || ld < 2 * rows) return SFNO_EINVAL;
-    if (fft_fast_supported(p.n)) return fft_fast_launch(false, p, xv, xm, rows, nlat, mmax, ld, x_dtype, s, nullptr, x2);
-    if (x2) return SFNO_EUNSUPPORTED;
+    if (fft_fast_supported(p.n)) return fft_fast_launch(false, p, xv, xm, rows, nlat, mmax, ld, x_dtype, s, nullptr, x2, kept);
+    if (x2 || kept) return SFNO_EUNSUPPORTED;
     if (x_dtype != SFNO_DTYPE_F32) return SFNO_EUNSUPPORTED;     // the generic kernels read float only
     const float* x = reinterpret_cast<const float*>(xv);
     switch (pick_pairs(p.n)) {
@@ -405,11 +405,12 @@ int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_
     return SFNO_EUNSUPPORTED;
 }
 
-int irfft_launch(const FftPlan& p, const float* xm, void* xv, int x_dtype, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, float2* lat_stats) {
+int irfft_launch(const FftPlan& p, const float* xm, void* xv, int x_dtype, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, float2* lat_stats,
+                 const int* kept) {
     // orders above nlon/2 are dropped, as torch.fft.irfft(n=nlon) drops surplus input bins
     if (ld % 4 != 0 || ld < 2 * rows) return SFNO_EINVAL;
-    if (fft_fast_supported(p.n)) return fft_fast_launch(true, p, xm, xv, rows, nlat, mmax, ld, x_dtype, s, lat_stats);
-    if (lat_stats) return SFNO_EUNSUPPORTED;                      // only the specialised kernels produce the moments
+    if (fft_fast_supported(p.n)) return fft_fast_launch(true, p, xm, xv, rows, nlat, mmax, ld, x_dtype, s, lat_stats, nullptr, kept);
+    if (lat_stats || kept) return SFNO_EUNSUPPORTED;              // only the specialised kernels produce the moments and leave orders out
     if (x_dtype != SFNO_DTYPE_F32) return SFNO_EUNSUPPORTED;
     float* x = reinterpret_cast<float*>(xv);
     switch (pick_pairs(p.n)) {

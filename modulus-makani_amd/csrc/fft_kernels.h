@@ -447,6 +447,14 @@ struct TileWalk {
     }
 };
 
+// Orders of a latitude that are exchanged with the order-major buffer.  Towards the poles the Legendre functions of high order vanish and the Legendre stage
+// neither reads nor writes those entries; at 721 latitudes and degrees a quarter of the buffer, 15 to 20 % of it where the degrees are truncated.
+// (Through the scalar unit: a vector load would have to be waited for together with the requested tile.)
+__device__ __forceinline__ int tile_orders(const int* kept, int lat, int mmax) {
+    if (!kept) return mmax;
+    return reinterpret_cast<const __attribute__((address_space(4))) int*>(reinterpret_cast<uintptr_t>(kept))[__builtin_amdgcn_readfirstlane(lat)];
+}
+
 // A tile is one latitude and S * H channel pairs: H = 2 batches of S = 4 pairs for the long rows, one batch of 8 for the
 // shorter ones, so that per order a tile owns one whole 128-byte line of the order-major buffer (8 pairs x 16 bytes).
 // Lines written or read in halves by different workgroups cost a third of the achievable bandwidth here (the two halves
@@ -461,7 +469,7 @@ struct TileWalk {
 template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, bool DIFF>
 __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
                                                           const void* __restrict__ x, const void* __restrict__ x2, float* __restrict__ xm, int64_t rows,
-                                                          int nlat, int mmax, int ld, int ngroups, float scale) {
+                                                          int nlat, int mmax, const int* kept, int ld, int ngroups, float scale) {
     using G = Geo<N, R0, R1, R2>;
     static_assert((S & (S - 1)) == 0 && FT % S == 0 && N % 4 == 0, "a power-of-two number of channel pairs shares the threads evenly");
     static_assert(H == 1 || H == 2, "one or two batches per tile");
@@ -552,6 +560,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
         const int tn = t + walk.step;
         const int tq = tn < walk.ntiles ? tn : t;       // the last tile requests itself again: always a request, never a branch around one
         const int pair = group * H * S + pp_;
+        const int mleft = tile_orders(kept, lat, mmax) - mfirst;     // (of the orders from my first one on)
         float* o = xm + ((int64_t)mfirst * nlat + lat) * ld + 4 * (int64_t)pair;
         fill(lat, group, 0);
         if (H == 2)
@@ -564,13 +573,13 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
             if (pair < ld / 4) {
 #pragma unroll
                 for (int u = 0; u < NSW; ++u)
-                    if (mfirst + u * TP < mmax) *reinterpret_cast<float4*>(o + u * mstep) = split(mfirst + u * TP);
+                    if (u * TP < mleft) *reinterpret_cast<float4*>(o + u * mstep) = split(mfirst + u * TP);
             }
         } else {
             float4 first[NSW];
 #pragma unroll
             for (int u = 0; u < NSW; ++u)
-                if (mfirst + u * TP < mmax) first[u] = split(mfirst + u * TP);
+                if (u * TP < mleft) first[u] = split(mfirst + u * TP);
             __syncthreads();
             fill(lat, group, 1);
             request(tq, 0);
@@ -579,7 +588,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
             const bool va = pair < ld / 4, vb = pair + S < ld / 4;
 #pragma unroll
             for (int u = 0; u < NSW; ++u) {
-                if (mfirst + u * TP < mmax) {
+                if (u * TP < mleft) {
                     const float4 second = split(mfirst + u * TP);
                     if (va) *reinterpret_cast<float4*>(o + u * mstep) = first[u];
                     if (vb) *reinterpret_cast<float4*>(o + u * mstep + 4 * S) = second;
@@ -602,7 +611,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
 // to the first one's row, and the lanes past the end of a row store its last four values again.
 template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, int NSWA, bool LS>
 __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
-                                                           const float* __restrict__ xm, void* __restrict__ x, int64_t rows, int nlat, int mmax, int ld,
+                                                           const float* __restrict__ xm, void* __restrict__ x, int64_t rows, int nlat, int mmax, const int* kept, int ld,
                                                            int ngroups, float2* __restrict__ lat_stats) {
     using G = Geo<N, R0, R1, R2>;
     static_assert(N % 4 == 0, "even length");
@@ -635,10 +644,11 @@ __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restr
         int lat, group;
         walk.locate(tile, lat, group);
         const float* src = xm + (int64_t)lat * ld;
+        const int morders = tile_orders(kept, lat, mmax);
 #pragma unroll
         for (int u = 0; u < NSWA; ++u) {
             const int m = mfirst + u * TP;
-            const float* row = src + (int64_t)(m < mmax ? m : 0) * nlat * ld;
+            const float* row = src + (int64_t)(m < morders ? m : 0) * nlat * ld;
 #pragma unroll
             for (int hh = 0; hh < HV; ++hh) {
                 const int pair = (group * H + half + hh) * S + pp_;
@@ -653,6 +663,7 @@ __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restr
         walk.locate(t, lat, group);
         const int tn = t + walk.step;
         const int tq = tn < walk.ntiles ? tn : t;         // the last tile requests itself again: always a request, never a branch around one
+        const int morders = tile_orders(kept, lat, mmax);
 #pragma unroll
         for (int hh = 0; hh < H; ++hh) {
             const int pair0 = (group * H + hh) * S;
@@ -674,7 +685,7 @@ __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restr
                         float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
                         if (u < NSWA) {
                             w = vv[u < NSWA ? u : 0];
-                            if (m >= mmax) w = make_float4(0.f, 0.f, 0.f, 0.f);
+                            if (m >= morders) w = make_float4(0.f, 0.f, 0.f, 0.f);
                             if (!hb) {
                                 w.z = w.x;
                                 w.w = w.y;
@@ -1082,7 +1093,7 @@ __global__ __launch_bounds__(FT) void latfft_chirp_kernel(const float2* __restri
 
 template <int N, int R0, int R1, int R2, bool BF16>
 int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, void* out, int64_t rows, int nlat, int mmax, int ld, float2* lat_stats,
-            hipStream_t s) {
+            const int* kept, hipStream_t s) {
     constexpr int S = (N >= 1024) ? 4 : 8;              // channel pairs in LDS at a time
     constexpr int H = 8 / S;                            // batches per tile: a tile owns 8 pairs = one 128-byte line per order
     constexpr int FT = (S * N >= 4096) ? 512 : 256;     // threads per workgroup
@@ -1097,10 +1108,10 @@ int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, voi
         float scale = (float)(kTwoPi / (double)N);
         if (!in2) {
             hipLaunchKernelGGL((rfft_fast_kernel<N, R0, R1, R2, S, H, FT, BF16, false>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, in2,
-                               reinterpret_cast<float*>(out), rows, nlat, mmax, ld, ngroups, scale);
+                               reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, ngroups, scale);
         } else if constexpr (!BF16) {
             hipLaunchKernelGGL((rfft_fast_kernel<N, R0, R1, R2, S, H, FT, false, true>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, in2,
-                               reinterpret_cast<float*>(out), rows, nlat, mmax, ld, ngroups, scale);
+                               reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, ngroups, scale);
         } else {
             return SFNO_EUNSUPPORTED;      // a difference of bf16 fields would be rounded before it is transformed
         }
@@ -1115,7 +1126,7 @@ int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, voi
         const int per = (int)std::min<int64_t>((int64_t)((nlat + 7) / 8) * ng, std::max(1, WG_PER_CU * p.n_cu / 8));
 #define IRFFT_GO(H_, NSWA_, LS_)                                                                                                            \
     hipLaunchKernelGGL((irfft_fast_kernel<N, R0, R1, R2, S, H_, FT, BF16, NSWA_, LS_>), dim3((unsigned)(8 * per)), dim3(FT), 0, s, p.d_tw0, \
-                       p.d_tw1, p.d_post, xm, out, rows, nlat, mmax, ld, ng, lat_stats)
+                       p.d_tw1, p.d_post, xm, out, rows, nlat, mmax, kept, ld, ng, lat_stats)
         if (lat_stats) {
             if (small) IRFFT_GO(H, NSMALL, true); else IRFFT_GO(1, NSW, true);
         } else {

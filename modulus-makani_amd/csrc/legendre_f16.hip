@@ -79,6 +79,9 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     for (int i = 0; i < PG_WREC; ++i) rec[i] = wrec[i];
     const int m = (int)rec[PG_WREC_M];
     if (m < 0) return;
+    // (leading row blocks of the order that its consumer takes for zero)
+    const int dropped = !ANALYSIS && a.drop ? (int)(rec[PG_WREC_M] >> 32) : 0;
+    if (!ANALYSIS && (int)rec[PG_WREC_RB] + 2 <= dropped) return;
     const int2 wi = make_int2(m, (int)rec[PG_WREC_RB]);
     __builtin_amdgcn_s_setreg((1 << 11) | (2 << 6) | 1, 3);      // MODE[3:2]: conversions to fp16 round toward zero
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     const int nrows = ANALYSIS ? nlp : K2;
     const int nrb = (nrows + PG_ROWS - 1) / PG_ROWS;
     const int nc = ANALYSIS ? (K2 + PG_KC - 1) / PG_KC : (nl0 + PG_KC - 1) / PG_KC;
-    const bool active = rb < nrb;
+    const bool active = rb < nrb && rb >= dropped;
 
     const float* xm_m = (ANALYSIS ? a.Q : a.Out) + (int64_t)m * nlat * ld;     // Fourier panel of order m
     const float* sp_m = (ANALYSIS ? a.Out : a.Q) + (COEFFS ? 2 * (int64_t)m : (int64_t)m * lmax * ld);     // spectral panel of order m

@@ -25,6 +25,7 @@ constexpr int PG_WAVES = 4;        // wavefronts (= row blocks) per workgroup
 // entries of the workgroup's four (parity, row block) streams (an absent one reads nc << 48: nothing to do) and the
 // positions of the two parities' first entries -- one 64-byte read instead of a chain of dependent look-ups.
 constexpr int PG_WREC = 8;
+// (PG_WREC_M: the order in the low half, in the high half the number of leading row blocks that do not matter, synthesis only)
 constexpr int PG_WREC_M = 0, PG_WREC_RB = 1, PG_WREC_ENTRY = 2, PG_WREC_POS = 6;
 
 struct PgemmTable {
@@ -37,6 +38,7 @@ struct PgemmTable {
     int64_t n_blocks = 0;
     int64_t items = 0, chunks = 0; // entries of the work list and K chunks of all of them (leading chunks that are left out included)
     int longest = 0;               // K chunks of the longest one
+    int* d_kept = nullptr;         // [nlat] orders of the Fourier buffer that matter at each latitude, see build_legendre_table
 };
 
 struct PgemmArgs {
@@ -49,6 +51,7 @@ struct PgemmArgs {
     const float* rinv;             // two-part fp16 format: row factors, [entry position - 2 mmax][32]
     int lmax, nlat, mmax;          // Legendre modes
     int ld;                        // channel leading dimension of Q and Out (Legendre modes)
+    int drop;                      // synthesis: rows of orders that do not matter there (PgemmTable::d_kept) are not written
     int64_t items, chunks;         // as in PgemmTable
     int longest;
     int ncol;                      // the spectral side in the reference layout: columns, 2 rows
@@ -217,8 +220,10 @@ bool fft_fast_supported(int n);
 int fft_fast_plan_init(FftPlan& p);
 // grid_dtype: element type of the grid-side tensor (SFNO_DTYPE_*); the Fourier side is always float
 // lat_stats (inverse only, may be null): float2 [rows][nlat] = mean over longitude of the output row and of its squared deviation from that mean
+// kept (may be null: all of mmax): [nlat] orders that are exchanged with the Fourier buffer at each latitude, the first ones; at least one.  Forward leaves
+// the others as they are, inverse takes them for zero
 int fft_fast_launch(bool inverse, const FftPlan& p, const void* in, void* out, int64_t rows, int nlat, int mmax, int ld, int grid_dtype,
-                    hipStream_t s, float2* lat_stats = nullptr, const void* in2 = nullptr);
+                    hipStream_t s, float2* lat_stats = nullptr, const void* in2 = nullptr, const int* kept = nullptr);
 // latitude FFT on the specialised passes; SFNO_EUNSUPPORTED for a length without them
 int latfft_fast_launch(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
 // planar pair on the reference layout: real FFTs along the grid rows, x [rows][nlat][n] <-> y [rows][group][nlat][2^cs] complex (groups
@@ -234,9 +239,11 @@ int fft_chirp_plan_init(FftPlan& p);
 void fft_plan_free(FftPlan& p);
 // x [rows][nlat][nlon] -> xm [mmax][nlat][ld] (re,im of row r at 2r,2r+1), scaled by 2 pi / nlon
 // (x2 given: of x - x2, float32 fields and lengths with specialised kernels only)
-int rfft_launch(const FftPlan& p, const void* x, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2 = nullptr);
+int rfft_launch(const FftPlan& p, const void* x, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2 = nullptr,
+                const int* kept = nullptr);
 // xm [mmax][nlat][ld] -> x [rows][nlat][nlon]
-int irfft_launch(const FftPlan& p, const float* xm, void* x, int x_dtype, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, float2* lat_stats = nullptr);
+int irfft_launch(const FftPlan& p, const float* xm, void* x, int x_dtype, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, float2* lat_stats = nullptr,
+                 const int* kept = nullptr);
 // latitude FFT of the planar transforms on the order-major layout: in[m][nlat | lmax][ld] -> out[m][lmax | nlat][ld]
 // (forward keeps lmax frequencies, inverse zero-fills the dropped ones); outputs are multiplied by mscale[m] (device array)
 int latfft_launch(const FftPlan& p, bool inverse, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
@@ -257,7 +264,10 @@ int degree_power_grad_launch(const float* spec, const float* gpower, float* gspe
 // looks up, once per device, the device address of the array on the current device; called at plan creation
 int static_scratch_prepare();
 
-// ---- adjoint transforms with the Fourier buffer passed in (capi.cpp) ----------------------------
+// ---- transforms and their adjoints with the Fourier buffer passed in (capi.cpp) -----------------
+// the buffer holds only what the transform needs of it (PgemmTable::d_kept)
+int analysis_launch(const sfno_sht_plan* p, const void* x, int x_dtype, const float* x2, float* xm, float* spec, int64_t rows, hipStream_t s);
+int synthesis_launch(const sfno_sht_plan* p, const float* spec, float* xm, void* x, int x_dtype, float2* lat_stats, int64_t rows, hipStream_t s);
 int analysis_adjoint_launch(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, float* xm, int64_t rows, hipStream_t s);
 int synthesis_adjoint_launch(const sfno_sht_plan* p, const void* gx, int x_dtype, float* xm, float* gspec, int64_t rows, hipStream_t s);
 
