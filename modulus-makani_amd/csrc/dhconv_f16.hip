@@ -9,11 +9,18 @@
 //
 // Per degree l the contraction is four real GEMMs on the real and imaginary parts,
 //   Yr = Xr Wr + (-Xi) Wi,   Yi = Xr Wi + Xi Wr,
-// with rows (m, b) of the spectral layout as A operands (read straight from HBM/L2, de-interleaved and cut in
+// with rows (m, b) of the spectral layout as A operands (moved to LDS as they are, in whole 128-byte lines, de-interleaved and cut in
 // registers; -Xi costs one sign flip per packed pair) and the weights as B operands: the packed stream holds, per
 // (degree, block of 32 NTC output channels, chunk of 16 input channels), the image of one LDS stage -- (Wr, Wi) x two
-// fp16 planes x output channel x 16 input channels -- which the wavefronts move with global_load_lds_dwordx4 into a
-// ring of three stages, two chunks ahead of the matrix instructions.  8 bytes per complex weight, read once.
+// fp16 planes x output channel x 16 input channels.  The wavefronts move both with global_load_lds_dwordx4, the weights into a
+// ring of three stages, the activations into two, two chunks ahead of the matrix instructions.  8 bytes per complex weight, read once.
+//
+// What bounds it: at one sample the stream of weights (283 of 460 MB for 384 x 384 channels and 240 degrees) and the three rounds that 132 workgroups to an
+// XCD take on its 64 places; at four samples the matrix pipe, 425 GFLOP at 1050 TFLOP/s where a large bf16 product reaches 1350 here (the
+// clock falls to 1.6 GHz under either).  The vector instructions of a chunk were a third of its time and are 70 for 48 matrix instructions now, and a request
+// had one contraction to land where it has two now (activations waited in registers, a lane asking for 64 bytes of its own row in four pieces).
+// 384 x 384 channels, 240 degrees, 1 / 2 / 4 samples 160 / 242 / 428 -> 139 / 233 / 404 us; 120 degrees 58 / 85 -> 49 / 66; 128 x 128 channels,
+// 90 degrees, 2 samples 22.5 -> 19.2.  Same bits.
 //
 // Scales.  fp16 keeps 11 significant bits only above 2^-14, so every operand row is brought close to the top of the
 // range (magnitudes below 2^15) by a power of two, which costs no accuracy and is undone when the result is stored:
@@ -35,18 +42,16 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __fp16 fp16x2 __attribute__((ext_vector_type(2)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 
 constexpr int DHF_KC = 16;             // complex input channels per chunk: one matrix K step per part
 constexpr int DHF_TOP = 14;            // scaled magnitudes stay below 2^(TOP + 1)
 constexpr int DHF_HEAD = 3;            // bits of headroom left when a row's exponent bound is raised
 constexpr int DHF_SH = DHF_TOP + 127;  // scaled = x * 2^(SH - E), E = biased exponent bound of the row
-constexpr int DHF_STAGES = 3;
+constexpr int DHF_EMIN = DHF_SH - 127; // smallest bound: its scale is the largest power of two of fp32 (rows below 2^-112 keep 25 bits above 2^-151)
+constexpr int DHF_STAGES = 3;          // of weights
+constexpr int DHF_XSTAGES = 2, DHF_XBYTES = 32 * 128;      // of activations: 32 rows x 16 complex fp32 per wavefront
 
-__device__ __forceinline__ unsigned int pk_rtz(float a, float b) {
-    return __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(a, b));
-}
 // 16 bytes per lane from global memory to LDS base + 16 lane (M0 carries the base; the compiler reserves M0 and does not
 // accept it on a clobber list: nothing else in this file may depend on M0 -- no indexed register arrays, no LDS-DMA builtins)
 __device__ __forceinline__ void dhf_dma16(const void* g, unsigned lds_byte_addr) {
@@ -56,96 +61,128 @@ __device__ __forceinline__ void dhf_dma16(const void* g, unsigned lds_byte_addr)
 // the halves swap places every 8 channels so that the 16-byte reads of 16 consecutive lanes cover all banks
 __host__ __device__ constexpr int dhf_piece(int o, int kg) { return o * 32 + ((kg ^ ((o >> 3) & 1)) * 16); }
 
-// grid = dh_blocks workgroups (see dh_map), row groups of 128; a.nob = ceil(O / (32 NTC)); requires 2*I % 4 == 0
-template <int NTC>
-__global__ __launch_bounds__(256, 2) void dhconv_f16_kernel(DhconvArgs a) {
+// One row group of up to 128 rows against one block of CO output channels: this wavefront has 32 rows and T tiles of 32 channels, tile t0 first.
+template <int NTC, int T>
+__device__ __forceinline__ void dhf_rows(const DhconvArgs& a, unsigned char* lds, int l, int ob, int first, int t0, bool active, int ncols, int wslot) {
     constexpr int CO = 32 * NTC;                     // complex output channels per workgroup
     constexpr int STAGE = 4 * CO * 32;               // bytes: (Wr, Wi) x 2 planes x CO x 16 fp16
-    constexpr int ND = STAGE / 4096;                 // direct-to-LDS loads per wavefront and chunk
-    constexpr int NX = 4;                            // activation loads per lane and chunk
-    __shared__ __align__(16) unsigned char lds[DHF_STAGES * STAGE];
-
-    int l, ob, r0, ncols, rot;
-    if (!dh_map(a, 128, l, ob, r0, ncols, rot)) return;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wslot = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave = (wslot + rot) & 3;
-    const bool active = r0 + 32 * wave < ncols;
+    constexpr int ND = STAGE / 4096;                 // weight requests per wavefront and chunk
+    constexpr int NX = 4;                            // activation requests per wavefront and chunk
+    const int lane = threadIdx.x & 63;
     const int nc = a.nc;                                           // chunks of 16 complex input channels
     const int kg = lane >> 5, cl = lane & 31;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)lds);
 
-    const int n = min(r0 + 32 * wave + cl, ncols - 1);
-    const int mm = n / a.B, bb = n - mm * a.B;
-    const float* xrow = a.X + ((int64_t)mm * a.L + l) * a.ld_in + (int64_t)bb * a.I2;
     // packed weights of (l, ob): nc stage images; this wavefront moves bytes [ND wslot KiB, ND (wslot + 1) KiB) of each
     const unsigned char* wsrc = reinterpret_cast<const unsigned char*>(a.W) + ((int64_t)l * a.nob + ob) * nc * STAGE + wslot * (ND * 1024) + lane * 16;
     const unsigned wdst = lds0 + wslot * (ND * 1024);
-
-    floatx16 yr[NTC], yi[NTC];
+    // Activations: request j brings 8 whole 128-byte lines, chunk c of rows 8 j .. 8 j + 7, into this wavefront's two KiB x 4 of LDS.  Slot s of
+    // row r holds piece s ^ (r / 2 % 8) of the line, so that 16 lanes that read the same piece of 16 rows cover all banks.
+    const unsigned xdst = lds0 + DHF_STAGES * STAGE + wslot * (DHF_XSTAGES * DHF_XBYTES);
+    const unsigned char* xraw = lds + DHF_STAGES * STAGE + wslot * (DHF_XSTAGES * DHF_XBYTES) + cl * 128;
+    const int rr = lane >> 3, ps = (lane & 7) ^ (rr >> 1);
+    int64_t xoff[NX];          // my piece of chunk 0 of the rows
+    const bool aligned = (reinterpret_cast<uintptr_t>(a.X) & 15) == 0;       // (16 bytes at a time go to LDS directly from aligned addresses only)
 #pragma unroll
-    for (int t = 0; t < NTC; ++t)
+    for (int j = 0; j < NX; ++j) {
+        const int n = min(first + 8 * j + rr, ncols - 1);
+        const int mm = n / a.B, bb = n - mm * a.B;
+        xoff[j] = ((int64_t)mm * a.L + l) * a.ld_in + (int64_t)bb * a.I2 + 4 * (ps ^ (4 * (j & 1)));
+    }
+    // (pieces past the last channel, in the last chunk only, repeat the last one: the weights are zero there)
+    auto x_dma = [&](int c, int stage) {
+        const unsigned dst = xdst + stage * DHF_XBYTES;
+        if (!aligned) {
+            // (these loads retire behind the weights requested before them, so the counted waits below hold)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            yr[t][v] = 0.0f;
-            yi[t][v] = 0.0f;
+            for (int j = 0; j < NX; ++j) {
+                const int k = 4 * (ps ^ (4 * (j & 1)));
+                const f4 x = *reinterpret_cast<const f4*>(a.X + xoff[j] + (min(2 * DHF_KC * c + k, a.I2 - 4) - k));
+                *reinterpret_cast<f4*>(lds + (dst - lds0) + j * 1024 + 16 * lane) = x;
+            }
+        } else if (c + 1 < nc) {
+            const float* base = a.X + 2 * DHF_KC * c;
+#pragma unroll
+            for (int j = 0; j < NX; ++j) dhf_dma16(base + xoff[j], dst + j * 1024);
+        } else {
+#pragma unroll
+            for (int j = 0; j < NX; ++j) {
+                const int k = 4 * (ps ^ (4 * (j & 1)));
+                dhf_dma16(a.X + xoff[j] + (min(2 * DHF_KC * c + k, a.I2 - 4) - k), dst + j * 1024);
+            }
         }
-    int E = 0;                 // biased exponent bound of my row (lanes cl and cl + 32 hold the same row and agree)
-    int pend = 0;              // change of E by the last chunk that was cut, not yet applied to the partial sums
-
-    // my 8 complex activations of chunk c: i = 16c + 8kg .. +7, (re, im) interleaved (clamped in groups of two complex
-    // values; the weights are zero past I)
-    auto x_load = [&](int c, f4 (&xr)[NX]) {
-        const int k = 2 * DHF_KC * c + 16 * kg;
-#pragma unroll
-        for (int j = 0; j < NX; ++j) xr[j] = *reinterpret_cast<const f4*>(xrow + min(k + 4 * j, a.I2 - 4));
     };
     auto w_dma = [&](int c, int stage) {
 #pragma unroll
         for (int j = 0; j < ND; ++j) dhf_dma16(wsrc + (int64_t)c * STAGE + j * 1024, wdst + stage * STAGE + j * 1024);
     };
-    // exponent bound of the row after this chunk
-    auto bound = [&](const f4 (&xr)[NX]) {
-        float mx = 0.f;
+
+    floatx16 yr[T], yi[T];
 #pragma unroll
-        for (int j = 0; j < NX; ++j)
-            mx = __builtin_fmaxf(__builtin_fmaxf(mx, __builtin_fmaxf(__builtin_fabsf(xr[j][0]), __builtin_fabsf(xr[j][1]))),
-                                 __builtin_fmaxf(__builtin_fabsf(xr[j][2]), __builtin_fabsf(xr[j][3])));
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            yr[t][v] = 0.0f;
+            yi[t][v] = 0.0f;
+        }
+    int E = DHF_EMIN;          // biased exponent bound of my row (lanes cl and cl + 32 hold the same row and agree)
+    const int xs = 4 * kg ^ (cl >> 1 & 7);
+    // my 8 complex activations of the chunk in stage `stage`: i = 16c + 8kg .. +7, (re, im) interleaved
+    auto x_read = [&](int stage, f4 (&xr)[NX]) {
+#pragma unroll
+        for (int j = 0; j < NX; ++j) xr[j] = *reinterpret_cast<const f4*>(xraw + stage * DHF_XBYTES + 16 * (xs ^ j));
+    };
+    // raises the exponent bound of the row to this chunk's values, and the scale of the partial sums with it: D row
+    // 8 (v / 4) + 4 kg + v % 4 belongs to the lanes of that number
+    auto bound = [&](const f4 (&xr)[NX]) {
+        // (written out: the compiler would bring every magnitude to canonical form first)
+        float mx;
+        asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(mx) : "v"(xr[0][0]), "v"(xr[0][1]), "v"(xr[0][2]));
+        asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(mx) : "v"(mx), "v"(xr[0][3]), "v"(xr[1][0]));
+        asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(mx) : "v"(mx), "v"(xr[1][1]), "v"(xr[1][2]));
+        asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(mx) : "v"(mx), "v"(xr[1][3]), "v"(xr[2][0]));
+        asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(mx) : "v"(mx), "v"(xr[2][1]), "v"(xr[2][2]));
+        asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(mx) : "v"(mx), "v"(xr[2][3]), "v"(xr[3][0]));
+        asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(mx) : "v"(mx), "v"(xr[3][1]), "v"(xr[3][2]));
+        asm("v_max_f32 %0, %1, |%2|" : "=v"(mx) : "v"(mx), "v"(xr[3][3]));
         const unsigned int mb = __builtin_bit_cast(unsigned int, mx);
+        if (__builtin_amdgcn_ballot_w64((int)(mb >> 23) > E) == 0) return;
         // the other half of the row's chunk sits 32 lanes away
         const auto sw = __builtin_amdgcn_permlane32_swap(mb, mb, false, false);
         const int eb = (int)(max(sw[0], sw[1]) >> 23);
         const int en = eb > E ? eb + DHF_HEAD : E;
-        pend = E - en;
+        const int pend = E - en;
         E = en;
-    };
-    // planes of the chunk: pl[0], pl[1] = Xr (upper, lower part), pl[2], pl[3] = Xi; word e of a plane holds the channels
-    // 2e, 2e + 1 of the lane's eight
-    auto cut_quad = [&](const f4 (&xr)[NX], int e, u4 (&pl)[4]) {
-        const f4 s = xr[e];
-        const int sh = DHF_SH - E;
-        const float ra = __builtin_ldexpf(s[0], sh), ia = __builtin_ldexpf(s[1], sh), rb = __builtin_ldexpf(s[2], sh), ib = __builtin_ldexpf(s[3], sh);
-        const fp16x2 hr = __builtin_amdgcn_cvt_pkrtz(ra, rb), hi = __builtin_amdgcn_cvt_pkrtz(ia, ib);
-        pl[0][e] = __builtin_bit_cast(unsigned int, hr);
-        pl[1][e] = pk_rtz(__builtin_fmaf((float)hr[0], -1.0f, ra), __builtin_fmaf((float)hr[1], -1.0f, rb));
-        pl[2][e] = __builtin_bit_cast(unsigned int, hi);
-        pl[3][e] = pk_rtz(__builtin_fmaf((float)hi[0], -1.0f, ia), __builtin_fmaf((float)hi[1], -1.0f, ib));
-    };
-    // partial sums follow their row's scale: D row 8 (v / 4) + 4 kg + v % 4 belongs to the lanes of that number
-    auto rescale = [&]() {
-        if (__builtin_amdgcn_ballot_w64(pend != 0) == 0) return;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int d = __builtin_amdgcn_ds_bpermute(4 * (8 * (v >> 2) + 4 * kg + (v & 3)), pend);
 #pragma unroll
-            for (int t = 0; t < NTC; ++t) {
+            for (int t = 0; t < T; ++t) {
                 yr[t][v] = __builtin_ldexpf(yr[t][v], d);
                 yi[t][v] = __builtin_ldexpf(yi[t][v], d);
             }
         }
     };
+    // planes of the chunk: pl[0], pl[1] = Xr (upper, lower part), pl[2], pl[3] = Xi; word e of a plane holds the channels
+    // 2e, 2e + 1 of the lane's eight.  (The conversions round toward zero, see MODE below.)
+    auto cut = [&](const f4 (&xr)[NX], u4 (&pl)[4]) {
+        const float sc = __builtin_bit_cast(float, (unsigned)(DHF_SH + 127 - E) << 23);
+#pragma unroll
+        for (int e = 0; e < NX; ++e)
+#pragma unroll
+            for (int part = 0; part < 2; ++part) {
+                const float u = xr[e][part], v = xr[e][2 + part];
+                unsigned hi, lo;
+                asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hi) : "v"(u), "v"(sc));
+                asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hi) : "v"(v), "v"(sc));
+                asm("v_fma_mixlo_f16 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(lo) : "v"(u), "v"(sc), "v"(hi));
+                asm("v_fma_mixhi_f16 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(lo) : "v"(v), "v"(sc), "v"(hi));
+                pl[2 * part][e] = hi;
+                pl[2 * part + 1][e] = lo;
+            }
+    };
     // one chunk of matrix instructions on stage `stage` with the planes pc
-    const int frag = dhf_piece(cl, kg);
+    const int frag = dhf_piece(32 * t0 + cl, kg);
     auto contract = [&](int stage, const u4 (&pc)[4]) {
         const unsigned char* sb = lds + stage * STAGE + frag;
         const f16x8 xr0 = __builtin_bit_cast(f16x8, pc[0]), xr1 = __builtin_bit_cast(f16x8, pc[1]);
@@ -153,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void dhconv_f16_kernel(DhconvArgs a) {
         // -Xi: one sign flip per packed pair
         const f16x8 ni0 = __builtin_bit_cast(f16x8, pc[2] ^ 0x80008000u), ni1 = __builtin_bit_cast(f16x8, pc[3] ^ 0x80008000u);
 #pragma unroll
-        for (int t = 0; t < NTC; ++t) {
+        for (int t = 0; t < T; ++t) {
             const f16x8 wr0 = *reinterpret_cast<const f16x8*>(sb + (0 * CO + 32 * t) * 32), wr1 = *reinterpret_cast<const f16x8*>(sb + (1 * CO + 32 * t) * 32);
             const f16x8 wi0 = *reinterpret_cast<const f16x8*>(sb + (2 * CO + 32 * t) * 32), wi1 = *reinterpret_cast<const f16x8*>(sb + (3 * CO + 32 * t) * 32);
             // smallest terms first; the two sums alternate so that no instruction waits for the one before it
@@ -172,92 +209,86 @@ __global__ __launch_bounds__(256, 2) void dhconv_f16_kernel(DhconvArgs a) {
         }
     };
 
-    // Pipeline, three weight stages.  Iteration c: cut the activations of chunk c + 1 (requested during iteration c - 1;
-    // the compiler's wait for them also covers this wavefront's pieces of the weights of chunk c + 1, which were requested
-    // before them), barrier (every wavefront's pieces of chunk c + 1 have landed and every wavefront is done reading
-    // chunk c - 1), request chunk c + 2 into the stage of chunk c - 1, contract chunk c, and let the partial sums follow
-    // the scale chunk c + 1 was cut with.  The requests thus have one contraction (48 or 24 matrix instructions) to land.
-    // Only the weight requests are written in assembly (the compiler would make every LDS read wait for them); their
-    // wait is the explicit one before the barrier.
-    f4 X0[NX], X1[NX];
-    u4 P0[4], P1[4];
-    if (active) x_load(0, X0);
+    // Pipeline, three weight stages and two of activations.  Iteration c: wait for this wavefront's pieces of chunk c (those of chunk c + 1
+    // stay in flight), take its activations out of LDS, barrier (every wavefront's pieces of the weights of chunk c have landed and every wavefront
+    // is done reading chunk c - 1), request chunk c + 2 into the stages that came free, cut the activations and contract.  A request has two
+    // contractions to land.  All requests are written in assembly (the compiler would make every LDS read wait for them) and none has a
+    // result register; the explicit waits count them.
     w_dma(0, 0);
+    if (active) x_dma(0, 0);
     if (nc > 1) {
-        if (active) x_load(1, X1);
         w_dma(1, 1);
+        if (active) x_dma(1, 1);
     }
-    if (active) {
-        bound(X0);
-#pragma unroll
-        for (int e = 0; e < NX; ++e) cut_quad(X0, e, P0);
-    }
-    pend = 0;                                                       // nothing has been summed yet
-
-    auto iter = [&](int c, int stage, const u4 (&pc)[4], u4 (&pn)[4], f4 (&xc)[NX], const f4 (&xn)[NX]) {
+    __builtin_amdgcn_s_setreg((1 << 11) | (2 << 6) | 1, 3);        // MODE[3:2]: conversions to fp16 round toward zero
+    for (int c = 0, stage = 0; c < nc; ++c, stage = stage == 2 ? 0 : stage + 1) {
         const bool more1 = c + 1 < nc, more2 = c + 2 < nc;         // uniform over the workgroup
-        if (active && more1) {
-            bound(xn);
-#pragma unroll
-            for (int e = 0; e < NX; ++e) cut_quad(xn, e, pn);
+        f4 xc[NX];
+        __builtin_amdgcn_sched_barrier(0);
+        if (active) {
+            if (more1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(ND + NX) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            x_read(c & 1, xc);
+        } else {
+            if (more1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(ND) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         }
         __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
-        if (more2) {
-            // xc held chunk c, cut during the previous iteration
-            if (active) x_load(c + 2, xc);
-            w_dma(c + 2, stage == 0 ? 2 : stage - 1);
-        }
+        if (more2) w_dma(c + 2, stage == 0 ? 2 : stage - 1);
         if (active) {
+            if (more2) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");         // (the stage has been read)
+                x_dma(c + 2, c & 1);
+            }
+            u4 pc[4];
+            bound(xc);
+            cut(xc, pc);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
             contract(stage, pc);
-            rescale();
-            pend = 0;
+            __builtin_amdgcn_s_setprio(0);
         }
-    };
-    int c = 0, stage = 0;
-    for (; c + 1 < nc; c += 2) {
-        iter(c, stage, P0, P1, X0, X1);
-        stage = stage == 2 ? 0 : stage + 1;
-        iter(c + 1, stage, P1, P0, X1, X0);
-        stage = stage == 2 ? 0 : stage + 1;
     }
-    if (c < nc) iter(c, stage, P0, P1, X0, X1);
 
     if (!active) return;
     // Undo the scales: row by 2^(E - SH) (the partial sums carry the scale of the last cut), column by the factor stored
     // with the weights.
-    float cinv[NTC];
+    const int ch0 = CO * ob + 32 * t0;                             // my first channel
+    float cinv[T];
 #pragma unroll
-    for (int t = 0; t < NTC; ++t) cinv[t] = a.cinv[(int64_t)l * (a.nob * CO) + CO * ob + 32 * t + cl];
+    for (int t = 0; t < T; ++t) cinv[t] = a.cinv[(int64_t)l * (a.nob * CO) + ch0 + 32 * t + cl];
+    // (waited for here and not where they are used: on some way around the uses they would count as on their way in the loops of the other T,
+    // whose registers they share, and hold up every iteration there)
+    __builtin_amdgcn_s_waitcnt(0x0F70);                            // vmcnt(0)
     const int Efinal = E;
-    const int nn0 = r0 + 32 * wave + 4 * kg;                       // my first row; the others are 8 (v / 4) + v % 4 further on
-    if (a.B == 1 && r0 + 32 * wave + 32 <= ncols && 2 * (CO * ob + CO) <= a.O2) {
+    const int nn0 = first + 4 * kg;                                // my first row; the others are 8 (v / 4) + v % 4 further on
+    if (a.B == 1 && first + 32 <= ncols && 2 * (ch0 + 32 * T) <= a.O2) {
         // one sample and no row or channel of my tile outside the tensor: row = order, one address, constant steps
-        float* o = a.Y + ((int64_t)nn0 * a.L + l) * a.ld_out + 2 * (CO * ob + cl);
+        float* o = a.Y + ((int64_t)nn0 * a.L + l) * a.ld_out + 2 * (ch0 + cl);
         const int64_t rstep = (int64_t)a.L * a.ld_out;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int er = __builtin_amdgcn_ds_bpermute(4 * (8 * (v >> 2) + 4 * kg + (v & 3)), Efinal);
             float* orow = o + (8 * (v >> 2) + (v & 3)) * rstep;
 #pragma unroll
-            for (int t = 0; t < NTC; ++t)
+            for (int t = 0; t < T; ++t)
                 *reinterpret_cast<f2*>(orow + 64 * t) = f2{__builtin_ldexpf(yr[t][v], er - DHF_SH) * cinv[t], __builtin_ldexpf(yi[t][v], er - DHF_SH) * cinv[t]};
         }
         return;
     }
-    if ((a.B & (a.B - 1)) == 0 && r0 + 32 * wave + 32 <= ncols && 2 * (CO * ob + CO) <= a.O2) {
+    if ((a.B & (a.B - 1)) == 0 && first + 32 <= ncols && 2 * (ch0 + 32 * T) <= a.O2) {
         // a power-of-two number of samples, whole tile inside: (order, sample) of a row by shift and mask, no checks
         const int lb = 31 - __builtin_clz(a.B);
-        float* o = a.Y + (int64_t)l * a.ld_out + 2 * (CO * ob + cl);
+        float* o = a.Y + (int64_t)l * a.ld_out + 2 * (ch0 + cl);
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const int er = __builtin_amdgcn_ds_bpermute(4 * (8 * (v >> 2) + 4 * kg + (v & 3)), Efinal);
             const int nn = nn0 + 8 * (v >> 2) + (v & 3);
             float* orow = o + (int64_t)(nn >> lb) * a.L * a.ld_out + (int64_t)(nn & (a.B - 1)) * a.O2;
 #pragma unroll
-            for (int t = 0; t < NTC; ++t)
+            for (int t = 0; t < T; ++t)
                 *reinterpret_cast<f2*>(orow + 64 * t) = f2{__builtin_ldexpf(yr[t][v], er - DHF_SH) * cinv[t], __builtin_ldexpf(yi[t][v], er - DHF_SH) * cinv[t]};
         }
         return;
@@ -270,12 +301,32 @@ __global__ __launch_bounds__(256, 2) void dhconv_f16_kernel(DhconvArgs a) {
         const int m2 = nn / a.B, b2 = nn - m2 * a.B;
         float* orow = a.Y + ((int64_t)m2 * a.L + l) * a.ld_out + (int64_t)b2 * a.O2;
 #pragma unroll
-        for (int t = 0; t < NTC; ++t) {
-            const int oc = 2 * (CO * ob + 32 * t + cl);
+        for (int t = 0; t < T; ++t) {
+            const int oc = 2 * (ch0 + 32 * t + cl);
             if (oc < a.O2)
                 *reinterpret_cast<f2*>(orow + oc) = f2{__builtin_ldexpf(yr[t][v], er - DHF_SH) * cinv[t], __builtin_ldexpf(yi[t][v], er - DHF_SH) * cinv[t]};
         }
     }
+}
+
+// grid = dh_blocks workgroups (see dh_map), row groups of 128; a.nob = ceil(O / (32 NTC)); requires 2*I % 4 == 0
+template <int NTC>
+__global__ __launch_bounds__(256, 2) void dhconv_f16_kernel(DhconvArgs a) {
+    __shared__ __align__(16) unsigned char lds[DHF_STAGES * 4 * 32 * NTC * 32 + 4 * DHF_XSTAGES * DHF_XBYTES];
+    int l, ob, r0, ncols, rot;
+    if (!dh_map(a, 128, l, ob, r0, ncols, rot)) return;
+    const int wslot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = (wslot + rot) & 3;
+    // A group of at most 32 or 64 rows shares its tiles out to the wavefronts instead of leaving three or two of them idle: the lowest degrees
+    // run last and mostly alone, and a wavefront's matrix instructions one after the other (384 x 384 channels, one sample: 32 degrees 35 -> 22 us,
+    // 64 degrees and 33 orders 36 -> 26, 34 without the sharing of two blocks; 240 degrees 145 -> 140 of it for two blocks).
+    const int blocks = (ncols - r0 + 31) >> 5;
+    if (blocks == 1)
+        dhf_rows<NTC, 1>(a, lds, l, ob, r0, wave & (NTC - 1), wave < NTC, ncols, wslot);
+    else if (blocks == 2)
+        dhf_rows<NTC, NTC / 2>(a, lds, l, ob, r0 + 32 * (wave >> 1), (wave & 1) * (NTC / 2), true, ncols, wslot);
+    else
+        dhf_rows<NTC, NTC>(a, lds, l, ob, r0 + 32 * wave, 0, wave < blocks, ncols, wslot);
 }
 
 // cmax[o][l] = largest |Re|, |Im| of w[.][o][l] over the input channels (adjoint: of w[o][.][l], w being [O][I][L]).  A thread
