@@ -28,16 +28,17 @@ const FastEntry* find_fast(int n) {
 // inter-pass twiddles of the specialised passes of length f.n
 int upload_pass_twiddles(const FastEntry& f, FftPlan& p) {
     const int N = f.n, nb = N / f.r0;
-    std::vector<float2> tw0((size_t)f.r0 * nb, make_float2(1.f, 0.f)), tw1((size_t)std::max(1, f.r1 * f.r2), make_float2(1.f, 0.f));
+    // (one slab per factor index, see fft_kernels.h)
+    std::vector<float2> tw0((size_t)std::max(1, (f.r0 - 1) * nb), make_float2(1.f, 0.f)), tw1((size_t)std::max(1, (f.r1 - 1) * f.r2), make_float2(1.f, 0.f));
     for (int k0 = 1; k0 < f.r0; ++k0)
         for (int j = 0; j < nb; ++j) {
             double a = -kTwoPi * (double)(((int64_t)k0 * j) % N) / (double)N;
-            tw0[(size_t)j * f.r0 + k0] = make_float2((float)std::cos(a), (float)std::sin(a));
+            tw0[(size_t)(k0 - 1) * nb + j] = make_float2((float)std::cos(a), (float)std::sin(a));
         }
     for (int k1 = 1; k1 < f.r1; ++k1)
         for (int n2 = 0; n2 < f.r2; ++n2) {
             double a = -kTwoPi * (double)(((int64_t)f.r0 * k1 * n2) % N) / (double)N;
-            tw1[(size_t)n2 * f.r1 + k1] = make_float2((float)std::cos(a), (float)std::sin(a));
+            tw1[(size_t)(k1 - 1) * f.r2 + n2] = make_float2((float)std::cos(a), (float)std::sin(a));
         }
     // slots of bin m and of bin N - m after the decimation-in-frequency passes (= before the decimation-in-time passes)
     std::vector<unsigned> post((size_t)N / 2 + 1);

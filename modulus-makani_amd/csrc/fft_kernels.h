@@ -235,12 +235,11 @@ __device__ __forceinline__ bool map_block(int nlat, int ngroups, int& lat, int& 
     return lat < nlat;
 }
 
-// Twiddle look-up of the passes.  TL = false: the per-plan tables in global memory, factors of one butterfly adjacent
-// (tw0[j * R0 + r], tw1[n2 * R1 + r]).  TL = true: copies in LDS, one slab per factor index so that neighbouring lanes
-// read neighbouring words (tw0[(r - 1) * NB + j], tw1[(r - 1) * R2 + n2]); see lds_tables.
-template <bool TL, int R, int NJ>
+// Twiddle look-up of the passes, in global memory or in a copy in LDS (see lds_tables): one slab per factor index, so that neighbouring lanes read
+// neighbouring words (tw0[(r - 1) * NB + j], tw1[(r - 1) * R2 + n2]).
+template <int NJ>
 __device__ __forceinline__ float2 twiddle(const float2* __restrict__ tw, int j, int r) {
-    return TL ? tw[(r - 1) * NJ + j] : tw[j * R + r];
+    return tw[(r - 1) * NJ + j];
 }
 
 // Butterfly index of thread `tid` in round `it` of a pass with TOT butterflies.  A last, partial round is not given to the
@@ -261,7 +260,7 @@ struct PassRounds {
 };
 
 // ---- forward: decimation in frequency ---------------------------------------------------------------
-template <int N, int R0, int R1, int R2, int S, int FT, bool TL = false>
+template <int N, int R0, int R1, int R2, int S, int FT>
 __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__ tw0, const float2* __restrict__ tw1, int tid) {
     using G = Geo<N, R0, R1, R2>;
     {
@@ -278,7 +277,7 @@ __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__
                 dft<R0, 0>(v);
                 base[0] = v[0];
 #pragma unroll
-                for (int r = 1; r < R0; ++r) base[r * NB] = cmul(v[r], twiddle<TL, R0, NB>(tw0, j, r));
+                for (int r = 1; r < R0; ++r) base[r * NB] = cmul(v[r], twiddle<NB>(tw0, j, r));
             }
         }
     }
@@ -298,7 +297,7 @@ __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__
                 dft<R1, 0>(v);
                 base[0] = v[0];
 #pragma unroll
-                for (int r = 1; r < R1; ++r) base[r * R2] = cmul(v[r], twiddle<TL, R1, R2>(tw1, n2, r));
+                for (int r = 1; r < R1; ++r) base[r * R2] = cmul(v[r], twiddle<R2>(tw1, n2, r));
             }
         }
         __syncthreads();
@@ -325,7 +324,7 @@ __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__
 }
 
 // ---- inverse: decimation in time -------------------------------------------------------------------------
-template <int N, int R0, int R1, int R2, int S, int FT, bool TL = false>
+template <int N, int R0, int R1, int R2, int S, int FT>
 __device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__ tw0, const float2* __restrict__ tw1, int tid) {
     using G = Geo<N, R0, R1, R2>;
     {
@@ -359,7 +358,7 @@ __device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__
                 float2 v[R1];
                 v[0] = base[0];
 #pragma unroll
-                for (int r = 1; r < R1; ++r) v[r] = cmul_tw<1>(base[r * R2], twiddle<TL, R1, R2>(tw1, n2, r));
+                for (int r = 1; r < R1; ++r) v[r] = cmul_tw<1>(base[r * R2], twiddle<R2>(tw1, n2, r));
                 dft<R1, 1>(v);
 #pragma unroll
                 for (int r = 0; r < R1; ++r) base[r * R2] = v[r];
@@ -378,7 +377,7 @@ __device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__
                 float2 v[R0];
                 v[0] = base[0];
 #pragma unroll
-                for (int r = 1; r < R0; ++r) v[r] = cmul_tw<1>(base[r * NB], twiddle<TL, R0, NB>(tw0, j, r));
+                for (int r = 1; r < R0; ++r) v[r] = cmul_tw<1>(base[r * NB], twiddle<NB>(tw0, j, r));
                 dft<R0, 1>(v);
 #pragma unroll
                 for (int r = 0; r < R0; ++r) base[r * NB] = v[r];
@@ -418,16 +417,9 @@ struct LdsTables {
 template <int N, int R0, int R1, int R2, int FT>
 __device__ __forceinline__ void lds_tables(LdsTables<N, R0, R1, R2>& t, const float2* __restrict__ tw0, const float2* __restrict__ tw1,
                                            const unsigned* __restrict__ post, int tid) {
-    constexpr int NB = N / R0;
-    for (int i = tid; i < (R0 - 1) * NB; i += FT) {
-        const int r = i / NB, j = i - r * NB;
-        t.tw0[i] = tw0[j * R0 + r + 1];
-    }
+    for (int i = tid; i < (R0 - 1) * (N / R0); i += FT) t.tw0[i] = tw0[i];
     if constexpr (R2 > 1)
-        for (int i = tid; i < (R1 - 1) * R2; i += FT) {
-            const int r = i / R2, n2 = i - r * R2;
-            t.tw1[i] = tw1[n2 * R1 + r + 1];
-        }
+        for (int i = tid; i < (R1 - 1) * R2; i += FT) t.tw1[i] = tw1[i];
     for (int i = tid; i <= N / 2; i += FT) t.post[i] = post[i];
 }
 
@@ -568,7 +560,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
         else
             request(tq, 0);
         __syncthreads();
-        passes_dif<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+        passes_dif<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
         if constexpr (H == 1) {
             if (pair < ld / 4) {
 #pragma unroll
@@ -584,7 +576,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
             fill(lat, group, 1);
             request(tq, 0);
             __syncthreads();
-            passes_dif<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+            passes_dif<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
             const bool va = pair < ld / 4, vb = pair + S < ld / 4;
 #pragma unroll
             for (int u = 0; u < NSW; ++u) {
@@ -746,7 +738,7 @@ __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restr
                 else
                     request(tq, 0);
             }
-            passes_dit<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+            passes_dit<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
             {
                 // rows leave LDS in natural order: TP threads walk the two rows of one channel pair, constant offsets from one address
                 constexpr int Q = N / 4, ITS = (Q + TP - 1) / TP;
@@ -904,7 +896,7 @@ __global__ __launch_bounds__(FT, 4) void rows_fwd_kernel(const float2* __restric
         }
         request(tn < ntiles ? tn : t);
         __syncthreads();
-        passes_dif<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+        passes_dif<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
         float2* ya = y + rp.y_index(q0, ng, cs, nlat);
         float2* yb = ya + (1 << cs);
         const int64_t ystep = (int64_t)TP * nlat;
@@ -974,7 +966,7 @@ __global__ __launch_bounds__(FT, 4) void rows_inv_kernel(const float2* __restric
         }
         __syncthreads();
         request(tn < ntiles ? tn : t);
-        passes_dit<N, R0, R1, R2, S, FT, true>(z, tab.tw0, tab.tw1, tid);
+        passes_dit<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
         {
             constexpr int Q = N / 4, ITS = (Q + TP - 1) / TP;
             const float4* src = reinterpret_cast<const float4*>(z + pl * G::PITCH);
@@ -1005,6 +997,14 @@ __global__ __launch_bounds__(FT) void cols_kernel(const float2* __restrict__ tw0
                                                   const float* __restrict__ mscale) {
     using G = Geo<N, R0, R1, R2>;
     __shared__ __align__(16) float2 z[C * G::PITCH];
+    // Twiddles from LDS, unless the tables cost a resident workgroup (400 points: two instead of three, 37.7 -> 41 us for 21 channels of 400 x 800).  From
+    // global memory, factors of a butterfly adjacent, a look-up asked for 64 lines a wavefront and bounded the kernel: 720 x 1440, 73 channels, forward
+    // 186 -> 180 us (the lines that neighbouring workgroups write in parts bound it now), inverse 140 -> 121 (5 TB/s).
+    constexpr int NT0 = (R0 - 1) * (N / R0), NT1 = R2 > 1 ? (R1 - 1) * R2 : 0;
+    constexpr size_t ZB = sizeof(z), TB = sizeof(float2) * (NT0 + NT1);
+    constexpr bool TL = (160 * 1024) / (ZB + TB) == (160 * 1024) / ZB;
+    __shared__ float2 tab[TL ? NT0 + NT1 : 1];
+    const float2 *t0 = TL ? tab : tw0, *t1 = TL ? tab + NT0 : tw1;
     const int tid = threadIdx.x;
     const int q = blockIdx.x >> 3, nu = (ngroups + kColUnit - 1) / kColUnit;
     const int unit = (q / kColUnit) * 8 + (blockIdx.x & 7);
@@ -1028,6 +1028,10 @@ __global__ __launch_bounds__(FT) void cols_kernel(const float2* __restrict__ tw0
             v[it] = make_float2(0.f, 0.f);
             if (i < N && k >= 0 && live) v[it] = src[(int64_t)k * pin];
         }
+        if constexpr (TL) {
+            for (int i = tid; i < NT0; i += FT) tab[i] = tw0[i];
+            for (int i = tid; i < NT1; i += FT) tab[NT0 + i] = tw1[i];
+        }
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int i = (tid + it * FT) / C;
@@ -1036,9 +1040,9 @@ __global__ __launch_bounds__(FT) void cols_kernel(const float2* __restrict__ tw0
     }
     __syncthreads();
     if (INV)
-        passes_dit<N, R0, R1, R2, C, FT>(z, tw0, tw1, tid);
+        passes_dit<N, R0, R1, R2, C, FT>(z, t0, t1, tid);
     else
-        passes_dif<N, R0, R1, R2, C, FT>(z, tw0, tw1, tid);
+        passes_dif<N, R0, R1, R2, C, FT>(z, t0, t1, tid);
     if (!live) return;
     const float sc = mscale[m];
     float2* dst = out + (INV ? block : (int64_t)row * nout * mmax + m);
