@@ -259,16 +259,17 @@ struct PassRounds {
     }
 };
 
+// SHORT: only the first `seqs` of the S sequences are there; the butterflies of the others, whole wavefronts of them, are left out.
 // ---- forward: decimation in frequency ---------------------------------------------------------------
-template <int N, int R0, int R1, int R2, int S, int FT>
-__device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__ tw0, const float2* __restrict__ tw1, int tid) {
+template <int N, int R0, int R1, int R2, int S, int FT, bool SHORT = false>
+__device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__ tw0, const float2* __restrict__ tw1, int tid, int seqs = S) {
     using G = Geo<N, R0, R1, R2>;
     {
         constexpr int NB = N / R0, TOT = S * NB;
 #pragma unroll
         for (int it = 0; it < (TOT + FT - 1) / FT; ++it) {
             const int e = PassRounds<N, R0, R1, R2, S, FT>::template index<TOT>(tid, it);
-            if (e < TOT) {
+            if (e < (SHORT ? seqs * NB : TOT)) {
                 const int p = e / NB, j = e - p * NB;
                 float2* base = z + p * G::PITCH + j;
                 float2 v[R0];
@@ -287,7 +288,7 @@ __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__
 #pragma unroll
         for (int it = 0; it < (TOT + FT - 1) / FT; ++it) {
             const int e = PassRounds<N, R0, R1, R2, S, FT>::template index<TOT>(tid, it);
-            if (e < TOT) {
+            if (e < (SHORT ? seqs * NB : TOT)) {
                 const int p = e / NB, j = e - p * NB;
                 const int k0 = j / R2, n2 = j - k0 * R2;
                 float2* base = z + p * G::PITCH + k0 * (R1 * R2) + n2;
@@ -308,7 +309,7 @@ __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__
 #pragma unroll
         for (int it = 0; it < (TOT + FT - 1) / FT; ++it) {
             const int e = PassRounds<N, R0, R1, R2, S, FT>::template index<TOT>(tid, it);
-            if (e < TOT) {
+            if (e < (SHORT ? seqs * NB : TOT)) {
                 const int p = e / NB, j = e - p * NB;
                 float2* base = z + p * G::PITCH + j * RL;
                 float2 v[RL];
@@ -324,8 +325,8 @@ __device__ __forceinline__ void passes_dif(float2* z, const float2* __restrict__
 }
 
 // ---- inverse: decimation in time -------------------------------------------------------------------------
-template <int N, int R0, int R1, int R2, int S, int FT>
-__device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__ tw0, const float2* __restrict__ tw1, int tid) {
+template <int N, int R0, int R1, int R2, int S, int FT, bool SHORT = false>
+__device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__ tw0, const float2* __restrict__ tw1, int tid, int seqs = S) {
     using G = Geo<N, R0, R1, R2>;
     {
         constexpr int RL = (R2 > 1) ? R2 : R1;
@@ -333,7 +334,7 @@ __device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__
 #pragma unroll
         for (int it = 0; it < (TOT + FT - 1) / FT; ++it) {
             const int e = PassRounds<N, R0, R1, R2, S, FT>::template index<TOT>(tid, it);
-            if (e < TOT) {
+            if (e < (SHORT ? seqs * NB : TOT)) {
                 const int p = e / NB, j = e - p * NB;
                 float2* base = z + p * G::PITCH + j * RL;
                 float2 v[RL];
@@ -351,7 +352,7 @@ __device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__
 #pragma unroll
         for (int it = 0; it < (TOT + FT - 1) / FT; ++it) {
             const int e = PassRounds<N, R0, R1, R2, S, FT>::template index<TOT>(tid, it);
-            if (e < TOT) {
+            if (e < (SHORT ? seqs * NB : TOT)) {
                 const int p = e / NB, j = e - p * NB;
                 const int k0 = j / R2, n2 = j - k0 * R2;
                 float2* base = z + p * G::PITCH + k0 * (R1 * R2) + n2;
@@ -371,7 +372,7 @@ __device__ __forceinline__ void passes_dit(float2* z, const float2* __restrict__
 #pragma unroll
         for (int it = 0; it < (TOT + FT - 1) / FT; ++it) {
             const int e = PassRounds<N, R0, R1, R2, S, FT>::template index<TOT>(tid, it);
-            if (e < TOT) {
+            if (e < (SHORT ? seqs * NB : TOT)) {
                 const int p = e / NB, j = e - p * NB;
                 float2* base = z + p * G::PITCH + j;
                 float2 v[R0];
@@ -457,8 +458,11 @@ __device__ __forceinline__ int tile_orders(const int* kept, int lat, int mmax) {
 // registers are at their limit), their latency is the other workgroups' to hide: 73 x 721 x 1440 in 210 us (0.93 GB, 4.4 TB/s), where the
 // transform of a stored difference took 137 and the pass that stores it 183.
 //
+// SHORT: the last batch of a latitude is not full (73 channels are 36.5 pairs in batches of 4).  A kernel of its own, for float32 fields: the comparisons cost
+// whole batches up to 2 % (721 x 1440: 73 channels 146 -> 145 us, inverse 154 -> 150; 9 channels 31.5 -> 28.8; 3 channels of 360 x 720 12.0 -> 9.9).
+//
 // grid = 8 * (workgroups per XCD) workgroups, see go_fast
-template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, bool DIFF>
+template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, bool DIFF, bool SHORT = false>
 __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
                                                           const void* __restrict__ x, const void* __restrict__ x2, float* __restrict__ xm, int64_t rows,
                                                           int nlat, int mmax, const int* kept, int ld, int ngroups, float scale) {
@@ -554,13 +558,14 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
         const int pair = group * H * S + pp_;
         const int mleft = tile_orders(kept, lat, mmax) - mfirst;     // (of the orders from my first one on)
         float* o = xm + ((int64_t)mfirst * nlat + lat) * ld + 4 * (int64_t)pair;
+        const int left = (int)((rows + 1) / 2) - group * H * S;      // pairs from here on; those that are not there are zeros in LDS and stay zeros
         fill(lat, group, 0);
         if (H == 2)
             request(t, 1);
         else
             request(tq, 0);
         __syncthreads();
-        passes_dif<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
+        passes_dif<N, R0, R1, R2, S, FT, SHORT>(z, tab.tw0, tab.tw1, tid, min(left, S));
         if constexpr (H == 1) {
             if (pair < ld / 4) {
 #pragma unroll
@@ -576,7 +581,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
             fill(lat, group, 1);
             request(tq, 0);
             __syncthreads();
-            passes_dif<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
+            passes_dif<N, R0, R1, R2, S, FT, SHORT>(z, tab.tw0, tab.tw1, tid, min(left - S, S));
             const bool va = pair < ld / 4, vb = pair + S < ld / 4;
 #pragma unroll
             for (int u = 0; u < NSW; ++u) {
@@ -601,7 +606,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
 // a pair slot beyond the last pair of the tensor does the work of the last pair once more (same loads, same sequence,
 // same stores of the same values), the missing second channel of an odd row count is a copy of the first and is stored
 // to the first one's row, and the lanes past the end of a row store its last four values again.
-template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, int NSWA, bool LS>
+template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, int NSWA, bool LS, bool SHORT = false>
 __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
                                                            const float* __restrict__ xm, void* __restrict__ x, int64_t rows, int nlat, int mmax, const int* kept, int ld,
                                                            int ngroups, float2* __restrict__ lat_stats) {
@@ -738,13 +743,15 @@ __global__ __launch_bounds__(FT, 4) void irfft_fast_kernel(const float2* __restr
                 else
                     request(tq, 0);
             }
-            passes_dit<N, R0, R1, R2, S, FT>(z, tab.tw0, tab.tw1, tid);
+            // (the slots of pairs that repeat the last one need no transform: their rows are stored from its slot)
+            const int seqs = SHORT ? max(min(last_pair + 1 - pair0, S), 1) : S;
+            passes_dit<N, R0, R1, R2, S, FT, SHORT>(z, tab.tw0, tab.tw1, tid, seqs);
             {
                 // rows leave LDS in natural order: TP threads walk the two rows of one channel pair, constant offsets from one address
                 constexpr int Q = N / 4, ITS = (Q + TP - 1) / TP;
                 const int pe = pair0 + pl < last_pair ? pair0 + pl : last_pair;
                 const int64_t ra = 2 * (int64_t)pe, rb = ra + 1 < rows ? ra + 1 : ra;
-                const float4* src = reinterpret_cast<const float4*>(z + pl * G::PITCH);
+                const float4* src = reinterpret_cast<const float4*>(z + (SHORT ? min(pl, seqs - 1) : pl) * G::PITCH);
 #pragma unroll
                 for (int it = 0; it < ITS; ++it) {
                     int i4 = q0 + it * TP;
@@ -1108,17 +1115,21 @@ int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, voi
     const int64_t tiles_xcd = (int64_t)((nlat + 7) / 8) * ngroups;
     const int per_xcd = (int)std::min<int64_t>(tiles_xcd, std::max(1, WG_PER_CU * p.n_cu / 8));
     dim3 grid((unsigned)(8 * per_xcd));
+    const int64_t npairs = (rows + 1) / 2;
     if (!inverse) {
         float scale = (float)(kTwoPi / (double)N);
+        const bool full = BF16 || npairs % (S * H) == 0;
+#define RFFT_GO(DIFF_, SHORT_)                                                                                                                   \
+    hipLaunchKernelGGL((rfft_fast_kernel<N, R0, R1, R2, S, H, FT, BF16, DIFF_, SHORT_>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, \
+                       in2, reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, ngroups, scale)
         if (!in2) {
-            hipLaunchKernelGGL((rfft_fast_kernel<N, R0, R1, R2, S, H, FT, BF16, false>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, in2,
-                               reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, ngroups, scale);
+            if (full) RFFT_GO(false, false); else RFFT_GO(false, !BF16);
         } else if constexpr (!BF16) {
-            hipLaunchKernelGGL((rfft_fast_kernel<N, R0, R1, R2, S, H, FT, false, true>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, in2,
-                               reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, ngroups, scale);
+            if (full) RFFT_GO(true, false); else RFFT_GO(true, true);
         } else {
             return SFNO_EUNSUPPORTED;      // a difference of bf16 fields would be rounded before it is transformed
         }
+#undef RFFT_GO
     } else {
         // sweeps of FT / S orders the kernel reads: all of 0..N/2, or a third of them for truncated plans.  Only the truncated
         // plans afford the registers to request both batches of a tile at once (whole-line reads); the others walk tiles of one
@@ -1128,13 +1139,16 @@ int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, voi
         const bool small = mmax <= NSMALL * TP;
         const int ng = small ? ngroups : (ld / 4 + S - 1) / S;
         const int per = (int)std::min<int64_t>((int64_t)((nlat + 7) / 8) * ng, std::max(1, WG_PER_CU * p.n_cu / 8));
-#define IRFFT_GO(H_, NSWA_, LS_)                                                                                                            \
-    hipLaunchKernelGGL((irfft_fast_kernel<N, R0, R1, R2, S, H_, FT, BF16, NSWA_, LS_>), dim3((unsigned)(8 * per)), dim3(FT), 0, s, p.d_tw0, \
+        const bool full = BF16 || npairs % (small ? S * H : S) == 0;
+#define IRFFT_GO(H_, NSWA_, LS_, SHORT_)                                                                                                          \
+    hipLaunchKernelGGL((irfft_fast_kernel<N, R0, R1, R2, S, H_, FT, BF16, NSWA_, LS_, SHORT_>), dim3((unsigned)(8 * per)), dim3(FT), 0, s, p.d_tw0, \
                        p.d_tw1, p.d_post, xm, out, rows, nlat, mmax, kept, ld, ng, lat_stats)
         if (lat_stats) {
-            if (small) IRFFT_GO(H, NSMALL, true); else IRFFT_GO(1, NSW, true);
+            if (small) IRFFT_GO(H, NSMALL, true, false); else IRFFT_GO(1, NSW, true, false);
+        } else if (full) {
+            if (small) IRFFT_GO(H, NSMALL, false, false); else IRFFT_GO(1, NSW, false, false);
         } else {
-            if (small) IRFFT_GO(H, NSMALL, false); else IRFFT_GO(1, NSW, false);
+            if (small) IRFFT_GO(H, NSMALL, false, !BF16); else IRFFT_GO(1, NSW, false, !BF16);
         }
 #undef IRFFT_GO
     }
