@@ -24,6 +24,8 @@
 // v_mfma_f32_32x32x2_f32, 512 matrix cycles per 16 rows and product instead of 192: 387 / 689 / 1322; two fp16 numbers, 96 cycles:
 // 191 / 338 / 578), 241 degrees, whose lines of gw are partial, 390 for one sample (416; 354).  Error against float64 of operands of
 // one magnitude, 1080 rows: 7.2e-7 (fp32 instruction 8.3e-7), and the same where they differ.
+#include <algorithm>
+
 #include "sfno_internal.h"
 
 namespace sfno {
@@ -59,19 +61,32 @@ struct Planes {                      // a channel's 8 rows: real and imaginary p
 // IB, OB: 32-channel blocks of i and o per workgroup: 2 x 2, or 1 x 1 (half of the registers and LDS) where those leave CUs idle
 // OFF: type of a lane's byte offset within a row chunk (64 bits only where 16 row strides do not fit 32)
 template <int IB, int OB, typename OFF>
-__global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) void dhconv_wgrad_kernel(DhconvWgradArgs p, int ni, int no) {
+__global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) void dhconv_wgrad_kernel(DhconvWgradArgs p, int ni, int no, int split) {
     constexpr int WG_TI = 32 * IB, WG_TO = 32 * OB;      // channels per workgroup
     __shared__ float2 stage[32 * WG_TO * WG_PITCH];
 
-    // Workgroups are dealt to the 8 XCDs round-robin by linear id.  All tiles of one group of 8 degrees run
-    // as neighbours in one XCD's queue, where they share the rows of X and G in that XCD's L2.  The groups go
-    // to the XCDs highest degrees (most rows) first, in alternating direction round by round: the work of a
-    // group grows linearly with its degree, and dealing every round in the same direction would give the
-    // first XCD a quarter more rows than the average.
-    const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-    const int tiles = ni * no;
-    const int t = q % tiles, gl = q / tiles;
-    const int lg = (p.L + WG_DEG - 1) / WG_DEG - 1 - (gl * 8 + ((gl & 1) ? 7 - xcd : xcd));
+    // Workgroups are dealt to the 8 XCDs round-robin by linear id.  A unit is the tiles of one group of 8 degrees, or (split = 2) of its upper or
+    // lower half of the input channels; its tiles run as neighbours in one XCD's queue, where they share the rows of X and G in
+    // that XCD's L2.  The units go to the XCDs highest degrees (most rows) first, in alternating direction round by round: the
+    // work of a group grows linearly with its degree, and dealing every round in the same direction would give the first XCD a
+    // quarter more rows than the average.
+    const int xcd = blockIdx.x & 7, tiles = ni * no;
+    int k = (int)(blockIdx.x >> 3) / tiles, t = (int)(blockIdx.x >> 3) - k * tiles;      // turn of dealing, tile in the unit
+    int half = 0;
+    if (split == 2) {
+        // (two turns in a row are one lower and one upper half)
+        const int low = ni / 2 * no, first = xcd & 1 ? tiles - low : low;
+        half = xcd & 1;
+        k *= 2;
+        if (t >= first) {
+            t -= first;
+            half ^= 1;
+            ++k;
+        }
+        if (half) t += low;
+    }
+    const int u = 8 * k + ((k & 1) ? 7 - xcd : xcd);
+    const int lg = (p.L + WG_DEG - 1) / WG_DEG - 1 - (split == 2 ? u >> 1 : u);
     if (lg < 0) return;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int l = lg * WG_DEG + wave;
@@ -247,6 +262,18 @@ __global__ __launch_bounds__(64 * WG_DEG, OB == 1 && sizeof(OFF) == 4 ? 4 : 2) v
     }
 }
 
+// the fullest XCD's queue, in chunks of rows, of the units of dhconv_wgrad_kernel; a tile's way to its first chunk and its stores take about 2.5
+int64_t fullest_queue(const DhconvWgradArgs& a, int ni, int no, int split) {
+    const int groups = (a.L + WG_DEG - 1) / WG_DEG;
+    int64_t q[8] = {};
+    for (int u = 0; u < groups * split; ++u) {
+        const int g = u / split, s = u - g * split, top = std::min(WG_DEG * (groups - g), a.tri ? a.M : a.L), rows = a.tri ? top : a.M;
+        const int64_t tiles = (int64_t)(ni * (s + 1) / split - ni * s / split) * no;
+        q[(u >> 3) & 1 ? 7 - (u & 7) : u & 7] += tiles * (2 * (int64_t)((rows + WG_KC - 1) / WG_KC) * a.B + 5);
+    }
+    return *std::max_element(q, q + 8);
+}
+
 }  // namespace
 
 int dhconv_wgrad_launch(const DhconvWgradArgs& a, hipStream_t s) {
@@ -261,15 +288,20 @@ int dhconv_wgrad_launch(const DhconvWgradArgs& a, hipStream_t s) {
     const bool narrow = !wide && ((a.I <= 32 && a.O <= 32) || groups * n2 < 768);
     const int tile = narrow ? 32 : 64;
     const int ni = (a.I + tile - 1) / tile, no = (a.O + tile - 1) / tile;
+    // Two units per group: as many queues as XCDs where there are few groups (384 x 384 channels, 45 degrees, eight samples 158 -> 107 us; 190 x 190 and 60
+    // degrees, two samples, 28 -> 22.5), more shares than 32 CUs can take at a time where there are many (36 tiles of 64 x 64 of a group; 240 degrees
+    // with 2 samples 425 -> 411, 241 with one 387 -> 353; 232 with one lose 2 %).  Small tiles whose queues are even keep one unit, whose tiles share all
+    // rows (120 degrees 75.5 against 77).
+    const int split = ni < 2 ? 1 : !narrow || 10 * fullest_queue(a, ni, no, 1) > 11 * fullest_queue(a, ni, no, 2) ? 2 : 1;
     const int64_t blocks = groups * ni * no;
     if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
     const dim3 grid((unsigned)blocks), block(64 * WG_DEG);
     if (wide)
-        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, uint64_t>), grid, block, 0, s, a, ni, no);
+        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, uint64_t>), grid, block, 0, s, a, ni, no, split);
     else if (narrow)
-        hipLaunchKernelGGL((dhconv_wgrad_kernel<1, 1, unsigned>), grid, block, 0, s, a, ni, no);
+        hipLaunchKernelGGL((dhconv_wgrad_kernel<1, 1, unsigned>), grid, block, 0, s, a, ni, no, split);
     else
-        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, unsigned>), grid, block, 0, s, a, ni, no);
+        hipLaunchKernelGGL((dhconv_wgrad_kernel<2, 2, unsigned>), grid, block, 0, s, a, ni, no, split);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

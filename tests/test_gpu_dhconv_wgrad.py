@@ -117,3 +117,19 @@ def test_weights_packed_in_slabs_of_degrees(lib_built, I, O, L):
     for got, ref in ((y.detach(), torch.matmul(xl, wl)), (xd.grad, torch.matmul(gl, wl.conj().transpose(1, 2)))):
         d = got[0].cpu().permute(1, 2, 0).to(torch.complex128) - ref
         assert float((d.abs().square().sum((1, 2)) / ref.abs().square().sum((1, 2))).max()) ** 0.5 < 1.5e-6
+
+
+@pytest.mark.parametrize("L", [5, 16, 50, 72])
+@pytest.mark.parametrize("I,O", [(64, 20), (70, 40), (130, 33)])
+def test_units_of_half_a_group(lib_built, L, I, O):
+    """One to nine groups of degrees whose tiles (an even and odd number of input blocks) are dealt to the XCDs whole or in halves."""
+    from makani_amd.contractions import _to_spectral, _weight_grad
+
+    print(f"case wgrad units L={L} I={I} O={O}", flush=True)
+    gen = torch.Generator().manual_seed(L)
+    x, g = (torch.randn(2, c, L, L, dtype=torch.complex64, generator=gen).tril().cuda() for c in (I, O))
+    got = _weight_grad(_to_spectral(x, 2 * I, L, L, True), _to_spectral(g, 2 * O, L, L, True), (I, O, L), 2, L, True).to(torch.complex128)
+    torch.cuda.synchronize()
+    xl, gl = (t.to(torch.complex128).permute(2, 0, 3, 1).reshape(L, 2 * L, -1).contiguous() for t in (x, g))
+    ref = torch.bmm(xl.transpose(1, 2).conj().resolve_conj().contiguous(), gl).permute(1, 2, 0)
+    assert float((got - ref).norm() / ref.norm()) < 1.5e-6
