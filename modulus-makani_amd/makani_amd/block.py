@@ -22,10 +22,32 @@ def _ptr(t):
     return t.data_ptr() if t is not None else None
 
 
+# The checks of a call read some forty attributes of modules, and for small grids they take longer than the kernels.  nn.Module finds a parameter
+# or submodule only after the ordinary look-up has failed (and builds a message where there is none), so these look in its tables first.
+
+def member(m, name):
+    """m.name of a module"""
+    mods = m._modules
+    if name in mods:
+        return mods[name]
+    params = m._parameters
+    return params[name] if name in params else getattr(m, name)
+
+
+def has_member(m, name):
+    """hasattr(m, name) of a module"""
+    if type(m).__getattr__ is not nn.Module.__getattr__:
+        return hasattr(m, name)
+    return name in m._modules or name in m._parameters or name in m._buffers or name in m.__dict__ or hasattr(type(m), name)
+
+
 def _no_hooks(*mods):
     if torch.nn.modules.module._has_any_global_hook():
         return False
-    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in mods)
+    for m in mods:
+        if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            return False
+    return True
 
 
 def plain_conv(m):
@@ -41,7 +63,7 @@ def trainable(x, params, *convs):
 
 def mlp_convs(blk):
     """(fc1, fc2) of a conv -> GELU -> conv MLP, or None."""
-    m = [f for f in blk.mlp.fwd if not isinstance(f, nn.Identity)]
+    m = [f for f in member(member(blk, "mlp"), "fwd") if not isinstance(f, nn.Identity)]
     ok = len(m) == 3 and plain_conv(m[0]) and plain_conv(m[2]) and type(m[1]) is nn.GELU and m[1].approximate == "none"
     return (m[0], m[2]) if ok else None
 
@@ -49,19 +71,21 @@ def mlp_convs(blk):
 def shapes_fit(params, c_in, embed, lmax):
     """Whether the parameters (in the order of block_params) belong to one block: the native calls address all of them by c_in, embed,
     hidden and lmax, so anything else is left to the modules, which raise their own errors."""
-    hidden = params[2].shape[0]
-    want = [(c_in, embed, lmax), (embed, c_in, 1, 1), (hidden, embed, 1, 1), (hidden,), (embed, hidden, 1, 1)] + 5 * [(embed,)]
-    return all(p is None or tuple(p.shape) == w for p, w in zip(params, want))
+    hidden, e = params[2].shape[0], (embed,)
+    for p, w in zip(params, ((c_in, embed, lmax), (embed, c_in, 1, 1), (hidden, embed, 1, 1), (hidden,), (embed, hidden, 1, 1), e, e, e, e, e)):
+        if p is not None and p.shape != w:
+            return False
+    return True
 
 
 def supported(blk, x, filter_weight=None, skip_weight=None, training=False):
     """The block's parameters (true) where the native block serves this block (whose fusable() the caller has checked) and input, else False;
     filter_weight, skip_weight: as of forward(); training: with its gradients, see trainable()."""
-    layer, norm0, norm1, act, mlp, skip = blk.filter, blk.norm0, blk.norm1, blk.act_layer0, blk.mlp, blk.outer_skip
-    conv = layer.filter
-    fwd, inv = conv.forward_transform, conv.inverse_transform
+    layer, norm0, norm1, act, mlp, skip = (member(blk, n) for n in ("filter", "norm0", "norm1", "act_layer0", "mlp", "outer_skip"))
+    conv = member(layer, "filter")
+    fwd, inv = member(conv, "forward_transform"), member(conv, "inverse_transform")
     convs = mlp_convs(blk)
-    if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or hasattr(conv, "bias") or convs is None:
+    if x.dtype != torch.bfloat16 or x.dim() != 4 or x.shape[0] == 0 or not conv._fused or has_member(conv, "bias") or convs is None:
         return False
     if type(norm0) is not nn.InstanceNorm2d or type(norm1) is not nn.InstanceNorm2d or inv.mmax > inv.nlon // 2 + 1:
         return False
@@ -79,16 +103,21 @@ def supported(blk, x, filter_weight=None, skip_weight=None, training=False):
     if not shapes_fit(params, x.shape[1], conv.out_channels, inv.lmax):
         return False
     wf, *rest = [p for p in params if p is not None]
-    if wf.dtype != torch.complex64 or not wf.is_cuda or not all(p.dtype == torch.float32 and p.is_cuda for p in rest):
+    if wf.dtype != torch.complex64 or not wf.is_cuda:
         return False
-    return params if _no_hooks(layer, conv, norm0, norm1, act, mlp, mlp.fwd, *mlp.fwd, skip) else False
+    for p in rest:
+        if p.dtype != torch.float32 or not p.is_cuda:
+            return False
+    chain = member(mlp, "fwd")
+    return params if _no_hooks(layer, conv, norm0, norm1, act, mlp, chain, *chain, skip) else False
 
 
 def block_params(blk, convs=None):
     """The block's parameters in the order of _Call: filter, skip, W1, b1, W2, b2, gamma0, beta0, gamma1, beta1 (None where there is none)."""
     fc1, fc2 = convs or mlp_convs(blk)
-    n0, n1 = blk.norm0, blk.norm1
-    return [blk.filter.filter.weight, blk.outer_skip.weight, fc1.weight, fc1.bias, fc2.weight, fc2.bias, n0.weight, n0.bias, n1.weight, n1.bias]
+    n0, n1 = member(blk, "norm0"), member(blk, "norm1")
+    return [member(member(member(blk, "filter"), "filter"), "weight"), member(member(blk, "outer_skip"), "weight"),
+            *(member(m, n) for m in (fc1, fc2, n0, n1) for n in ("weight", "bias"))]
 
 
 def _with(params, filter_weight, skip_weight):
@@ -103,8 +132,8 @@ class _Call:
     training: a forward that records gradients; backward: of the input and the parameters (input_grad) or of the parameters alone."""
 
     def __init__(self, blk, x, params, backward=False, training=False, input_grad=True):
-        conv = blk.filter.filter
-        fwd, inv = conv.forward_transform, conv.inverse_transform
+        conv = member(member(blk, "filter"), "filter")
+        fwd, inv = member(conv, "forward_transform"), member(conv, "inverse_transform")
         wf, wskip, w1, b1, w2, b2, g0, be0, g1, be1 = params
         dev = x.device
         b = _lib.Block()
@@ -119,10 +148,10 @@ class _Call:
                 adj += [packed_for(wf, conv.compute, adjoint=True), pw.packed_weight(wskip, transposed=True)]
                 b.weights_adj, b.wskipt = adj[4].handle, adj[5].data_ptr()
             keep += adj
-        vectors = [t.detach().contiguous() if t is not None else None for t in (b1, b2, g0, be0, g1, be1)]
+        vectors = [t if t is None or t.is_contiguous() else t.detach().contiguous() for t in (b1, b2, g0, be0, g1, be1)]
         keep += vectors
         b.b1, b.b2, b.gamma0, b.beta0, b.gamma1, b.beta1 = (_ptr(t) for t in vectors)
-        b.eps0, b.eps1 = blk.norm0.eps, blk.norm1.eps
+        b.eps0, b.eps1 = member(blk, "norm0").eps, member(blk, "norm1").eps
         b.batch, b.c_in, b.embed, b.hidden = x.shape[0], x.shape[1], conv.out_channels, w1.shape[0]
         self.b = b
         self.P = (inv.nlat, inv.nlon)
@@ -132,9 +161,13 @@ class _Call:
     def forward(self, x, training, out):
         ref = ctypes.byref(self.b)
         nkept, nws = lib.sfno_block_layout(ref, training, self.offsets), lib.sfno_block_workspace_bytes(ref, 0)
-        kept = torch.empty(nkept, dtype=torch.uint8, device=x.device)
-        ws = torch.empty(nws, dtype=torch.uint8, device=x.device)
-        check(lib.sfno_block_forward(ref, training, x.data_ptr(), _ptr(out), kept.data_ptr(), nkept, ws.data_ptr(), nws, self.stream), "sfno_block_forward")
+        if training or out is None:
+            kept = torch.empty(nkept, dtype=torch.uint8, device=x.device)
+            at = (ws := torch.empty(nws, dtype=torch.uint8, device=x.device)).data_ptr()
+        else:                 # nothing outlives the call: one buffer (pieces of whole 256 bytes)
+            kept = torch.empty(nkept + nws, dtype=torch.uint8, device=x.device)
+            at = kept.data_ptr() + nkept
+        check(lib.sfno_block_forward(ref, training, x.data_ptr(), _ptr(out), kept.data_ptr(), nkept, at, nws, self.stream), "sfno_block_forward")
         return kept
 
 

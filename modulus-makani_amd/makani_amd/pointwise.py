@@ -97,6 +97,11 @@ def _dense(x):
     return x if x.data_ptr() % 16 == 0 else x.clone()
 
 
+def _vector(t):
+    """A parameter vector as the kernels read it: float32 and contiguous (None where there is none)."""
+    return t if t is None or (t.dtype == torch.float32 and t.is_contiguous()) else t.detach().float().contiguous()
+
+
 def conv1x1(x, weight, bias=None, act=None, addend=None, add_scale=None, add_shift=None):
     """act(conv1x1(x, weight) + bias) + add_scale * addend + add_shift  ->  bf16 [B, O, H, W]."""
     return _conv1x1(x, weight, False, bias, act, addend, add_scale, add_shift)
@@ -112,8 +117,7 @@ def _conv1x1(x, weight, transposed, bias=None, act=None, addend=None, add_scale=
         raise RuntimeError(f"conv1x1: input has {K} channels, weight expects {K_weight}")
     pw = packed_weight(weight, transposed, both)
     y = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
-    if bias is not None:
-        bias = bias.detach().float().contiguous()
+    bias = _vector(bias)
     if addend is not None:
         if addend.shape != y.shape or addend.dtype != torch.bfloat16:
             raise RuntimeError("conv1x1: addend must be a bfloat16 tensor of the output's shape")
@@ -165,8 +169,7 @@ def conv1x1_cat(x1, x2, weight, bias=None, act=None, out=None):
         if tuple(out.shape) != (B, O, H, W) or out.dtype != torch.bfloat16 or not out.is_contiguous() or out.device != x1.device:
             raise RuntimeError("conv1x1_cat: out must be a contiguous bfloat16 tensor of the result's shape")
         y = out
-    if bias is not None:
-        bias = bias.detach().float().contiguous()
+    bias = _vector(bias)
     check(lib.sfno_pointwise_conv_cat(_ptr(x1), K1, _ptr(x2), K2, _ptr(pw), _ptr(bias), _ptr(y), B, O, H * W, ACT[act], _stream(x1.device)),
           "sfno_pointwise_conv_cat")
     return y
@@ -281,7 +284,7 @@ class _ConvGeluConv(torch.autograd.Function):
             raise RuntimeError(f"conv1x1: input has {K} channels, weights expect {w1.shape[1]} and {w2.shape[1]} (of {O})")
         z = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x.device)
         a = torch.empty_like(z)
-        bias = b1.detach().float().contiguous() if b1 is not None else None
+        bias = _vector(b1)
         need = ctx.needs_input_grad
         check(lib.sfno_pointwise_conv_gelu(_ptr(xb), _ptr(packed_weight(w1, both=need[0] and transposed_used(w1))), _ptr(bias), _ptr(a), _ptr(z), B, K, O, H * W,
                                            _stream(x.device)), "sfno_pointwise_conv_gelu")

@@ -201,11 +201,13 @@ class FourierNeuralOperatorBlock(nn.Module):
             self.act_layer1 = act_layer()
 
     def _fusable(self):
-        if not (hasattr(self, "mlp") and _fused_chain(self.mlp.fwd) and _is_gelu(self.act_layer0)):
+        has, get = native_block.has_member, native_block.member
+        if not (has(self, "mlp") and _fused_chain(get(get(self, "mlp"), "fwd")) and _is_gelu(get(self, "act_layer0"))):
             return False
-        if hasattr(self, "inner_skip") or hasattr(self, "act_layer1") or not _norm_fusable(self.norm0) or not _norm_fusable(self.norm1):
+        if has(self, "inner_skip") or has(self, "act_layer1") or not _norm_fusable(get(self, "norm0")) or not _norm_fusable(get(self, "norm1")):
             return False
-        return hasattr(self, "outer_skip") and _is_conv1x1(self.outer_skip) and self.outer_skip.bias is None
+        skip = get(self, "outer_skip") if has(self, "outer_skip") else None
+        return skip is not None and _is_conv1x1(skip) and get(skip, "bias") is None
 
     def _norm0_from_transform(self):
         return self.output_shape_loc[0] * self.output_shape_loc[1] > pw.NORM_SMALL_PIXELS
@@ -404,9 +406,10 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         if not getattr(self, "fold_encoder", True) or self.repeat_layers != 1 or len(self.blocks) == 0:
             return None
         enc = enc or _fused_chain(self.encoder.fwd)
-        blk = self.blocks[0]
-        conv = blk.filter.filter
-        if enc is None or len(enc) < 2 or enc[-1][1] is not None or enc[-1][0].bias is not None:
+        has, get = native_block.has_member, native_block.member
+        blk = get(self, "blocks")[0]
+        conv = get(get(blk, "filter"), "filter")
+        if enc is None or len(enc) < 2 or enc[-1][1] is not None or get(enc[-1][0], "bias") is not None:
             return None
         # the fold moves the first block's transforms, channel mix and skip convolution from the encoder's output channels to
         # its hidden channels: worth it only if those are not more
@@ -414,9 +417,9 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
             return None
         if not (isinstance(blk, FourierNeuralOperatorBlock) and blk._fusable() and getattr(blk, "fused_pointwise", True)):
             return None
-        if not (conv._fused and conv.scale_residual and not hasattr(conv, "bias") and conv.in_channels == enc[-1][0].out_channels):
+        if not (conv._fused and conv.scale_residual and not has(conv, "bias") and conv.in_channels == enc[-1][0].out_channels):
             return None
-        w2, w0, ws = enc[-1][0].weight, conv.weight, blk.outer_skip.weight
+        w2, w0, ws = get(enc[-1][0], "weight"), get(conv, "weight"), get(get(blk, "outer_skip"), "weight")
         stamp = _stamp(w2, w0, ws)
         cached = getattr(self, "_fold_cache", None)
         if cached is None or cached[0] != stamp:
@@ -561,7 +564,7 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
 
     def _fusable(self, x):
         """(encoder steps, decoder steps) where the fused path serves the network and the input, else None."""
-        if not (getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x)) or hasattr(self, "pos_embed"):
+        if not (getattr(self, "fused_pointwise", True) and not self.training and fused_pointwise_active(x)) or native_block.has_member(self, "pos_embed"):
             return None
         if not isinstance(self.pos_drop, nn.Identity) or (self.out_shape[0] * self.out_shape[1]) % 8 != 0:
             return None
