@@ -9,7 +9,7 @@
 // tiles it took a column of tiles to itself where K is a multiple of 256 (eight instead of six for 768 -> 384 channels with bias:
 // 1249 -> 997 us at 721 x 1440).
 //
-// A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile (wide layers: 384 x 192, pw_wgrad_wide_kernel) of dW and a contiguous share of the (sample, 64-pixel chunk)
+// A workgroup (eight wavefronts, 4 x 2) owns a 256 x 256 tile (small layers: 128 x 128; wide ones: 384 x 192, pw_wgrad_wide_kernel) of dW and a contiguous share of the (sample, 64-pixel chunk)
 // sequence.  Per chunk 256 rows of g and 256 rows of x, a whole 128-byte line each (with 64-byte pieces of 32-pixel chunks the
 // same bytes were 1.4 times as long on their way, 989 against 704 us without the products for 384 -> 768 channels at 721 x 1440, and
 // the kernel took as long as its loads: 1029 -> 902 us in all, 768 -> 384 with bias 997 -> 858),
@@ -31,17 +31,22 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int WG_THREADS = 512;
-constexpr int WG_TO = 256;            // rows of dW (output channels) per workgroup
-constexpr int WG_TK = 256;            // columns of dW (input channels) per workgroup
 constexpr int WG_PX = 64;             // pixels per chunk: eight 16-byte pieces per row
-constexpr int WG_HALF = WG_TO * 2 * WG_PX;                    // bytes of the rows of g, or of x, of a chunk
 constexpr int WG_HALVES = 5;                                  // ring of halves
-constexpr int WG_PIECES = WG_HALF / (16 * WG_THREADS);        // 16-byte pieces per thread and half
 constexpr int WG_RSTEP = WG_THREADS / (WG_PX / 8);            // rows between a thread's pieces
 static_assert(WG_PX == 64, "eight pieces per row: the permutation and the slot arithmetic below");
-static_assert(WG_TO == WG_TK, "halves of one size");
 static_assert(WG_RSTEP % 16 == 0, "a thread's pieces share the permutation of their rows");
-static_assert(WG_HALVES * WG_HALF <= 160 * 1024, "one workgroup per CU");
+
+// tile of TILE rows (output channels) and columns (input channels) of dW per workgroup: 256, or 128 where the layer has no more or the
+// tiles of 256 are few
+template <int TILE>
+struct WgTile {
+    static constexpr int HALF = TILE * 2 * WG_PX;                    // bytes of the rows of g, or of x, of a chunk
+    static constexpr int PIECES = HALF / (16 * WG_THREADS);          // 16-byte pieces per thread and half
+    static constexpr int PER_CU = TILE == 256 ? 1 : 2;               // resident workgroups
+    static constexpr int MT = TILE / 128, NT = TILE / 64;            // 32-row blocks of a wavefront (4 x 2 of them)
+    static_assert(PER_CU * WG_HALVES * HALF <= 160 * 1024, "resident workgroups");
+};
 
 // source of the pieces that are not read from the tensors
 __device__ __align__(16) const unsigned int wg_zero16[4] = {0u, 0u, 0u, 0u};
@@ -73,18 +78,19 @@ constexpr int WW_MT = 3, WW_NT = 3, WW_WO = 4, WW_WK = 2;
 constexpr int WW_THREADS = 64 * WW_WO * WW_WK;
 constexpr int WW_TO = 32 * WW_MT * WW_WO, WW_TK = 32 * WW_NT * WW_WK;
 
-enum WgradKind { WG_SQUARE, WG_WIDE, WG_WIDE_SWAP };      // pw_wgrad_kernel, pw_wgrad_wide_kernel<false>, <true>
+enum WgradKind { WG_SQUARE, WG_SMALL, WG_WIDE, WG_WIDE_SWAP };      // pw_wgrad_kernel<256>, <128>, pw_wgrad_wide_kernel<false>, <true>
 struct WgradShape {
     int n_ot, n_kt, splits;
     int64_t cps, chunks;               // chunks per sample, chunks in all
     WgradKind kind;
-    int rows() const { return kind == WG_SQUARE ? WG_TO + WG_TK : WW_TO + WW_TK; }     // that a workgroup asks for
+    int rows() const { return kind == WG_SQUARE ? 512 : WW_TO + WW_TK; }     // that a workgroup asks for
 };
 
 // how the launcher and the workspace query divide the work: shares of at least four chunks, one workgroup per CU (all
-// workgroups resident at once, the tiles of a share side by side on one XCD)
+// workgroups resident at once, the tiles of a share side by side on one XCD; small tiles: see wgrad_shape below)
 static WgradShape wgrad_shape(int O, int K, int B, int64_t P, WgradKind kind) {
-    const int to = kind == WG_SQUARE ? WG_TO : kind == WG_WIDE ? WW_TO : WW_TK, tk = kind == WG_SQUARE ? WG_TK : kind == WG_WIDE ? WW_TK : WW_TO;
+    const int to = kind == WG_SQUARE ? 256 : kind == WG_SMALL ? 128 : kind == WG_WIDE ? WW_TO : WW_TK;
+    const int tk = kind == WG_SQUARE ? 256 : kind == WG_SMALL ? 128 : kind == WG_WIDE ? WW_TK : WW_TO;
     WgradShape s;
     s.kind = kind;
     s.n_ot = (O + to - 1) / to;
@@ -92,7 +98,7 @@ static WgradShape wgrad_shape(int O, int K, int B, int64_t P, WgradKind kind) {
     s.cps = (P + WG_PX - 1) / WG_PX;
     s.chunks = s.cps * B;
     const int tiles = s.n_ot * s.n_kt;
-    int64_t want = device_cus() / tiles / 8 * 8;
+    int64_t want = device_cus() / (kind == WG_SMALL ? ((O + 255) / 256) * ((K + 255) / 256) : tiles) / 8 * 8;
     if (want < 8) want = 8;
     const int64_t most = (s.chunks + 3) / 4;       // at least four chunks per share
     if (want > most) want = most;
@@ -112,11 +118,23 @@ static double wgrad_cost(const WgradShape& s, int O, int K) {
     return 2.0 * s.rows() * WG_PX * (double)(share + 3) + 16.0 * O * K * s.splits / device_cus();
 }
 static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
-    WgradShape best = wgrad_shape(O, K, B, P, WG_SQUARE);
+    const WgradShape square = wgrad_shape(O, K, B, P, WG_SQUARE);
+    WgradShape best = square;
     for (WgradKind kind : {WG_WIDE, WG_WIDE_SWAP}) {
         const WgradShape s = wgrad_shape(O, K, B, P, kind);
         if (wgrad_cost(s, O, K) < wgrad_cost(best, O, K)) best = s;
     }
+    // Tiles of 128 x 128 over the shares of the 256 x 256 ones (the same sums in the same order), two workgroups to a CU: a layer of at most 128
+    // channels asks for half the rows, and the way to the first chunk and the stores of a short share are spread over twice the workgroups.
+    // 1000 shapes (2 to 768 channels, 1024 to 1.5 million pixels), times against the larger tiles: 0.66 where a tile takes the place of one, 0.74 to 0.95
+    // for three in place of two, for two in place of one 0.75 with shares of less than 24 chunks and up to 1.19 with longer ones (but 0.7 with at most 64
+    // output channels), for four 0.8 with less than 6 chunks and 1.2 with longer ones.  20 % faster on average, 10 % slower at worst.
+    // 128 channels of 2 x 90 x 180 18.4 -> 12.6 us, 96 of 4 x 128 x 247 51 -> 36.
+    const WgradShape small = wgrad_shape(O, K, B, P, WG_SMALL);
+    const int n = small.n_ot * small.n_kt, n2 = square.n_ot * square.n_kt;
+    const int64_t share = (square.chunks + square.splits - 1) / square.splits;
+    const bool few = 2 * n <= 3 * n2;
+    if (best.kind == WG_SQUARE ? few || (n <= 2 * n2 && (share < 24 || O <= 64)) || (share < 6 && n2 <= 6) : few && share < 32) return small;
     return best;
 }
 
@@ -177,14 +195,16 @@ struct WgStream {
     }
 };
 
-// grid = 8 * ceil(splits / 8) * n_ot * n_kt workgroups of 512 threads
-__global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
-    __shared__ __align__(16) unsigned char lds[WG_HALVES * WG_HALF];
+// (The comments speak of the 256 x 256 tile.)  grid = 8 * ceil(splits / 8) * n_ot * n_kt workgroups of 512 threads
+template <int TILE>
+__global__ __launch_bounds__(WG_THREADS, 2 * WgTile<TILE>::PER_CU) void pw_wgrad_kernel(WgradArgs a) {
+    constexpr int HALF = WgTile<TILE>::HALF, PIECES = WgTile<TILE>::PIECES, MT = WgTile<TILE>::MT, NT = WgTile<TILE>::NT;
+    __shared__ __align__(16) unsigned char lds[WG_HALVES * HALF];
     const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
     const int tiles = a.n_ot * a.n_kt;
     const int split = (q / tiles) * 8 + xcd, tile = q % tiles;
     if (split >= a.splits) return;
-    const int o0 = (tile % a.n_ot) * WG_TO, k0 = (tile / a.n_ot) * WG_TK;
+    const int o0 = (tile % a.n_ot) * TILE, k0 = (tile / a.n_ot) * TILE;
     const int64_t c_begin = (int64_t)split * a.chunks / a.splits, c_end = (int64_t)(split + 1) * a.chunks / a.splits;
     const int nch = (int)(c_end - c_begin);
 
@@ -193,50 +213,50 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     const int wo = wave & 3, wk = wave >> 2;
     const unsigned lds0 = (unsigned)(size_t)((__attribute__((address_space(3))) unsigned char*)lds);
 
-    // ---- loads: LDS slot s = 512 j + tid of a half (16 bytes) holds row s >> 3, piece (s & 7) ^ ((row >> 1) & 7).  A thread's four
+    // ---- loads: LDS slot s = 512 j + tid of a half (16 bytes) holds row s >> 3, piece (s & 7) ^ ((row >> 1) & 7).  A thread's
     // slots lie 64 rows apart: same piece, same permutation.  Rows past the matrix are its last row, whose products are never stored.
-    WgStream<WG_PIECES, WG_THREADS> sg(a.G, o0, a.O, a, c_begin, tid), sx(a.X, k0, a.K, a, c_begin, tid);
-    auto issue = [&](WgStream<WG_PIECES, WG_THREADS>& t, int slot) { t.issue(a, lds0 + slot * WG_HALF + wave * 1024, tid); };
+    WgStream<PIECES, WG_THREADS> sg(a.G, o0, a.O, a, c_begin, tid), sx(a.X, k0, a.K, a, c_begin, tid);
+    auto issue = [&](WgStream<PIECES, WG_THREADS>& t, int slot) { t.issue(a, lds0 + slot * HALF + wave * 1024, tid); };
 
-    f32x16 acc[2][4];
-    float accb[2] = {0.f, 0.f}, chunkb[2] = {0.f, 0.f};       // sums of the lane's pixels of its two rows: all chunks, this chunk
+    f32x16 acc[MT][NT];
+    float accb[MT] = {}, chunkb[MT] = {};       // sums of the lane's pixels of its two rows: all chunks, this chunk
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[mt][nt][v] = 0.f;
 
     // fragments of this lane: row (lane & 31) of a 32-row block, pieces 2 ks + (lane >> 5) of the row (pixels 8 (lane >> 5) .. + 7 of
     // the 16-pixel step ks), at their permuted places
     const int sw = (lane >> 1) & 7, kg = lane >> 5;
-    const unsigned fa = (wo * 64 + (lane & 31)) * 128, fb = (wk * 128 + (lane & 31)) * 128;
+    const unsigned fa = (wo * 32 * MT + (lane & 31)) * 128, fb = (wk * 32 * NT + (lane & 31)) * 128;
 
-    const bool live = o0 + wo * 64 < a.O && k0 + wk * 128 < a.K;
-    const bool bias = a.Kext > a.K && k0 + wk * 128 == 0;
+    const bool live = o0 + wo * 32 * MT < a.O && k0 + wk * 32 * NT < a.K;
+    const bool bias = a.Kext > a.K && k0 + wk * 32 * NT == 0;
     // Half h (chunk h / 2; g, then x) lives in slot h % 5.  Fragments are read one 16-pixel step ahead of the matrix instructions, those of
     // a chunk's first step under the products of the last step of the chunk before.  In front of that, once a wavefront holds all it
     // needs of chunk i, it waits for its pieces of chunk i + 1 and meets the others: chunk i's slots take halves 2 i + 5 (x of chunk
-    // i + 2) and 2 i + 6 (g of chunk i + 3), chunk i + 1 may be read.  The only vector memory operations of the loop are the four loads per
-    // wavefront and half, so "at most four outstanding" leaves half 2 i + 4 under way.
-    static_assert(WG_HALVES == 5 && WG_PIECES == 4, "the wait counts below");
-    bf16x8 af[2][2], bf[2][4];                // [step & 1][32-row block]
+    // i + 2) and 2 i + 6 (g of chunk i + 3), chunk i + 1 may be read.  The only vector memory operations of the loop are the PIECES loads per
+    // wavefront and half, so "at most PIECES outstanding" leaves half 2 i + 4 under way.
+    static_assert(WG_HALVES == 5, "the wait counts below");
+    bf16x8 af[2][MT], bf[2][NT];               // [step & 1][32-row block]
     auto fragments = [&](int slot_g, int slot_x, int ks) {
         const unsigned pk = (unsigned)(((2 * ks + kg) ^ sw) * 16);
-        const unsigned char *pa = lds + slot_g * WG_HALF + fa + pk, *pb = lds + slot_x * WG_HALF + fb + pk;
+        const unsigned char *pa = lds + slot_g * HALF + fa + pk, *pb = lds + slot_x * HALF + fb + pk;
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) af[ks & 1][mt] = *reinterpret_cast<const bf16x8*>(pa + mt * 32 * 128);
+        for (int mt = 0; mt < MT; ++mt) af[ks & 1][mt] = *reinterpret_cast<const bf16x8*>(pa + mt * 32 * 128);
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) bf[ks & 1][nt] = *reinterpret_cast<const bf16x8*>(pb + nt * 32 * 128);
+        for (int nt = 0; nt < NT; ++nt) bf[ks & 1][nt] = *reinterpret_cast<const bf16x8*>(pb + nt * 32 * 128);
     };
     auto products = [&](int ks) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
+        for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][mt], bf[ks & 1][nt], acc[mt][nt], 0, 0, 0);
+            for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][mt], bf[ks & 1][nt], acc[mt][nt], 0, 0, 0);
         if (bias) {
 #pragma unroll
-            for (int mt = 0; mt < 2; ++mt) {
+            for (int mt = 0; mt < MT; ++mt) {
                 const u32x4 p = __builtin_bit_cast(u32x4, af[ks & 1][mt]);
                 float lo = 0.f, hi = 0.f;
 #pragma unroll
@@ -261,7 +281,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     if (nch > 2) issue(sg, 4);
     __builtin_amdgcn_sched_barrier(0);
     if (nch > 2)
-        __builtin_amdgcn_s_waitcnt(wg_wait(12));
+        __builtin_amdgcn_s_waitcnt(wg_wait(3 * PIECES));
     else
         __builtin_amdgcn_s_waitcnt(wg_wait(0));
     wg_barrier();
@@ -281,7 +301,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
         __builtin_amdgcn_sched_barrier(0);
         // (the builtin and not inline assembly: the compiler then knows that the fragments have arrived)
         if (i + 3 <= nch)
-            __builtin_amdgcn_s_waitcnt(wg_wait(4));
+            __builtin_amdgcn_s_waitcnt(wg_wait(PIECES));
         else
             __builtin_amdgcn_s_waitcnt(wg_wait(0));
         wg_barrier();
@@ -299,20 +319,20 @@ __global__ __launch_bounds__(WG_THREADS, 2) void pw_wgrad_kernel(WgradArgs a) {
     // D layout of the 32x32 MFMA: register v of lane j holds D[8 (v / 4) + 4 (j / 32) + v % 4][j % 32]
     float* out = a.ws + (int64_t)split * a.O * a.Kext;
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            const int kk = k0 + wk * 128 + nt * 32 + (lane & 31);
+        for (int nt = 0; nt < NT; ++nt) {
+            const int kk = k0 + wk * 32 * NT + nt * 32 + (lane & 31);
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int o = o0 + wo * 64 + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                const int o = o0 + wo * 32 * MT + mt * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
                 if (o < a.O && kk < a.K) out[(int64_t)o * a.Kext + kk] = acc[mt][nt][v];
             }
         }
     if (bias) {
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt) {
-            const int o = o0 + wo * 64 + mt * 32 + (lane & 31);
+        for (int mt = 0; mt < MT; ++mt) {
+            const int o = o0 + wo * 32 * MT + mt * 32 + (lane & 31);
             const float b = accb[mt] + __shfl_xor(accb[mt], 32, 64);
             if (lane < 32 && o < a.O) out[(int64_t)o * a.Kext + a.K] = b;
         }
@@ -511,8 +531,10 @@ int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, flo
         hipLaunchKernelGGL(pw_wgrad_wide_kernel<false>, dim3((unsigned)nwg), dim3(WW_THREADS), 0, s, a);
     else if (sh.kind == WG_WIDE_SWAP)
         hipLaunchKernelGGL(pw_wgrad_wide_kernel<true>, dim3((unsigned)nwg), dim3(WW_THREADS), 0, s, a);
+    else if (sh.kind == WG_SMALL)
+        hipLaunchKernelGGL(pw_wgrad_kernel<128>, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
     else
-        hipLaunchKernelGGL(pw_wgrad_kernel, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
+        hipLaunchKernelGGL(pw_wgrad_kernel<256>, dim3((unsigned)nwg), dim3(WG_THREADS), 0, s, a);
     if (hipGetLastError() != hipSuccess) return SFNO_EHIP;
     const int64_t n = (int64_t)O * Kext;
     if (n % 4 == 0 && n >= 256 * 256)
