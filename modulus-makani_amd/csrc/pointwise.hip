@@ -91,10 +91,28 @@ __device__ __forceinline__ float gelu_train(float x) {
 }
 
 // derivative of the GELU: Phi(x) + x phi(x), phi(x) = 2^(-x^2 log2(e) / 2) / sqrt(2 pi)
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float e = phi_neg(x);
+// (e = phi_neg(x))
+__device__ __forceinline__ float gelu_grad(float x, float e) {
     const float phi = 0.39894228040143267794f * __builtin_amdgcn_exp2f(-0.72134752044448170368f * x * x);
     return fmaf(x, phi, x > 0.f ? 1.f - e : e);
+}
+__device__ __forceinline__ float gelu_grad(float x) { return gelu_grad(x, phi_neg(x)); }
+
+// Training applies both to numbers that were rounded to bf16.  From 2^-11 to the clamp at 6.5 these are 1728 magnitudes, and the convolutions in
+// front of and behind a GELU look phi_neg up in LDS: the same bits with 8 vector instructions a value where the GELU takes 18, and 17 where its derivative
+// takes 27.  The vector instructions of the epilogue find no matrix instruction to hide behind and bounded both kernels; now memory nearly does, as it does
+// the epilogue with an addend.  721 x 1440: derivative 384 -> 768 channels 1258 -> 1136 us, 384 -> 384 645 -> 588, 73 -> 384 425 -> 398; GELU 384 -> 768 1215 -> 1141,
+// 384 -> 384 606 -> 570, but 73 -> 384 446 -> 463 (at 240 x 480 43.8 -> 41.3).
+constexpr int GT_HI = 0x40d0, GT_N = 1728, GT_LO = GT_HI - GT_N + 1;             // 6.5 as bf16
+constexpr int GT_BYTES = 4 * GT_N;
+// phi_neg of a bf16 number's magnitude, of the nearest one in the table where it is smaller
+__device__ __forceinline__ float gelu_look_up(const unsigned char* table, int magnitude) {
+    return *reinterpret_cast<const float*>(table + 4 * (min(max(magnitude, GT_LO), GT_HI) - GT_LO));
+}
+// gelu_train(x) from the entry of |x|; below the table Phi(-|x|) is a straight line in fp32
+__device__ __forceinline__ float gelu_from(float x, int magnitude, float entry) {
+    const float e = magnitude < GT_LO ? fmaf(fabsf(x), -0.39894228040143267794f, 0.5f) : entry;
+    return fmaf(-fabsf(x), e, __builtin_amdgcn_fmed3f(x, 0.f, __builtin_inff()));
 }
 
 // Epilogues: exact GELU on the output and / or "+ scale * addend + shift"; for training GELU_PRE (the output before the GELU is stored as
@@ -382,7 +400,9 @@ template <int MT, int EPI>
 __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_kernel(PointwiseArgs a) {
     using DM = DmGeo<MT>;
     constexpr bool GELU = EPI & (PW_GELU | PW_GELU_PRE), AFF = EPI & PW_ADD, ADD = EPI & (PW_ADD | PW_GELU_BWD);
-    __shared__ __align__(16) unsigned char lds[DM::LDS];
+    constexpr bool TAB = EPI & (PW_GELU_PRE | PW_GELU_BWD);
+    static_assert(DM::WG_PER_CU * (DM::LDS + GT_BYTES) <= 160 * 1024, "resident workgroups");
+    __shared__ __align__(16) unsigned char lds[DM::LDS + (TAB ? GT_BYTES : 0)];
     // tiles of this XCD, row block fastest: q -> (row block q % n_oblk, strip (q / n_oblk) * 8 + xcd); the workgroups of the
     // XCD deal them out round robin, so the row blocks of one strip run at the same time on one L2
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, nslot = gridDim.x >> 3;
@@ -461,6 +481,8 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
 
     f32x16 acc[MT][DM_NT];
 
+    if constexpr (TAB)
+        for (int i = tid; i < GT_BYTES / 4; i += 512) *reinterpret_cast<float*>(lds + DM::LDS + 4 * i) = phi_neg(__uint_as_float((unsigned)(GT_LO + i) << 16));
     // fill the pipeline: three weight chunks or the activation stages, then chunk 0 must have landed
     bool full = true;
     for (int i = 0; i < (wload ? DM_WSTAGES : DM::XSTAGES); ++i) full = issue() && full;
@@ -568,25 +590,40 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
                     for (int t = 0; t < 4; ++t) y[t] = acc[mt][t][v] + bs;
                     if constexpr (EPI & PW_GELU_PRE) {
                         u32x2 z;
+                        float e[4];
 #pragma unroll
                         for (int pp = 0; pp < 2; ++pp) {
                             z[pp] = bf16_pair(y[2 * pp], y[2 * pp + 1]);
-                            y[2 * pp] = __uint_as_float(z[pp] << 16);
-                            y[2 * pp + 1] = __uint_as_float(z[pp] & 0xffff0000u);
+                            e[2 * pp] = gelu_look_up(lds + DM::LDS, z[pp] & 0x7fffu);
+                            e[2 * pp + 1] = gelu_look_up(lds + DM::LDS, z[pp] >> 16 & 0x7fffu);
                         }
                         *reinterpret_cast<u32x2*>(a.Z + lane_off + (int64_t)row_of(mt, v) * a.P) = z;
-                    }
-                    if constexpr (GELU) {
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) y[t] = EPI & PW_GELU_PRE ? gelu_train(y[t]) : gelu(y[t]);
+                        for (int pp = 0; pp < 2; ++pp) {
+                            y[2 * pp] = gelu_from(__uint_as_float(z[pp] << 16), z[pp] & 0x7fffu, e[2 * pp]);
+                            y[2 * pp + 1] = gelu_from(__uint_as_float(z[pp] & 0xffff0000u), z[pp] >> 16 & 0x7fffu, e[2 * pp + 1]);
+                        }
+                    } else if constexpr (GELU) {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) y[t] = gelu(y[t]);
                     }
                     if constexpr (EPI & PW_GELU_BWD) {
                         const u32x2 r = rv[mh & 1][4 * g + jj];
+                        float e[4], x[4];
+                        int m[4];
 #pragma unroll
-                        for (int pp = 0; pp < 2; ++pp) {
-                            y[2 * pp] *= gelu_grad(__uint_as_float(r[pp] << 16));
-                            y[2 * pp + 1] *= gelu_grad(__uint_as_float(r[pp] & 0xffff0000u));
+                        for (int t = 0; t < 4; ++t) {
+                            m[t] = r[t >> 1] >> 16 * (t & 1) & 0x7fffu;
+                            x[t] = __uint_as_float(t & 1 ? r[t >> 1] & 0xffff0000u : r[t >> 1] << 16);
+                            e[t] = gelu_look_up(lds + DM::LDS, m[t]);
                         }
+                        // (one value in two thousand is below the table, one group of 256 in ten has such a value)
+                        if (__builtin_amdgcn_ballot_w64(min(min(m[0], m[1]), min(m[2], m[3])) < GT_LO)) {
+#pragma unroll
+                            for (int t = 0; t < 4; ++t) e[t] = phi_neg(x[t]);
+                        }
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) y[t] *= gelu_grad(x[t], e[t]);
                     }
                     if constexpr (AFF) {
                         const float sc = ko4 ? usc[qq & 1][4 + jj] : usc[qq & 1][jj], sh = ko4 ? ush[qq & 1][4 + jj] : ush[qq & 1][jj];

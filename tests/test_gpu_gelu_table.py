@@ -1,0 +1,41 @@
+"""The training GELU and its derivative by table (convolutions of more than 96 output channels, one to three row tiles per wavefront) against the formulas that narrower
+convolutions evaluate, on every bf16 value: the same activations and derivatives, NaN at the same places."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(channels, z):
+    from makani_amd import pointwise as pw
+    from makani_amd._lib import check, lib
+
+    n = z.numel()
+    P = (-(-n // channels) + 7) // 8 * 8
+    x = torch.zeros(channels * P, dtype=torch.bfloat16)
+    x[:n] = z
+    x = x.reshape(1, channels, 1, P).cuda()
+    finite = torch.where(torch.isfinite(x), x, torch.zeros_like(x))          # (an infinity would meet the zeros of the identity)
+    eye, ones = torch.eye(channels, device="cuda"), torch.ones_like(x)
+    y, pre, gx = (torch.empty_like(x) for _ in range(3))
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    check(lib.sfno_pointwise_conv_gelu(ptr(finite), ptr(pw.packed_weight(eye)), None, ptr(y), ptr(pre), 1, channels, channels, P, pw._stream(x.device)), "forward")
+    check(lib.sfno_pointwise_conv_gelu_grad(ptr(ones), ptr(pw.packed_weight(eye, transposed=True)), ptr(x), ptr(gx), 1, channels, channels, P,
+                                            pw._stream(x.device)), "backward")
+    torch.cuda.synchronize()
+    return y.reshape(-1)[:n].cpu(), gx.reshape(-1)[:n].cpu()
+
+
+@pytest.mark.parametrize("channels", [97, 128, 200, 300, 384])
+def test_table_is_the_formula(lib_built, channels):
+    print(f"case gelu table {channels}", flush=True)
+    z = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    (y0, g0), (y1, g1) = _both(64, z), _both(channels, z)
+    # (half of a subnormal number is a rounding boundary: the formula's 0.5 is off by 4e-10, the table's straight line is not)
+    big = ~(z.abs() < 2.0**-120)
+    assert torch.equal(y0[big].view(torch.int16), y1[big].view(torch.int16))
+    assert torch.equal(torch.isnan(g0), torch.isnan(g1))
+    ok = ~torch.isnan(g0)
+    assert torch.equal(g0[ok].view(torch.int16), g1[ok].view(torch.int16))
