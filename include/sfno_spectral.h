@@ -244,7 +244,8 @@ int sfno_dhconv_weights_update_both(sfno_dhconv_weights* w, sfno_dhconv_weights*
 /* y[b,o,l,m] = sum_i x[b,i,l,m] w[i,o,l] on spectral-layout buffers:
  * spec_in rows = batch*in_channels, spec_out rows = batch*out_channels.  With
  * `triangular` != 0 only m <= l is read and written (coefficients of a forward
- * transform are zero elsewhere).  Replaces _contract_dhconv (contractions.py:130-136). */
+ * transform are zero elsewhere).  The row slots of spec_out past its rows become zeros wherever
+ * its rows are written.  Replaces _contract_dhconv (contractions.py:130-136). */
 int sfno_dhconv_spectral(const sfno_dhconv_weights* w, const float* spec_in, float* spec_out,
                          int batch, int mmax, int triangular, void* stream);
 

@@ -145,16 +145,6 @@ int conv(const bf16* x, const void* w, const float* bias, bf16* y, int B, int K,
     return pointwise_gemm_launch(a, s);
 }
 
-// channel mix; row slots between the channels and ld are padding and become zeros (the transform reads whole rows)
-int mix(const sfno_dhconv_weights* w, const float* in, float* out, const Dims& d, int64_t rows_out, hipStream_t s) {
-    const int64_t ld = sfno_spectral_ld(rows_out);
-    if (ld != 2 * rows_out) {
-        const int rc = spectral_zero_padding_launch(out, rows_out, (int64_t)d.mmax * d.lmax, (int)ld, s);
-        if (rc != SFNO_OK) return rc;
-    }
-    return sfno_dhconv_spectral(w, in, out, d.B, d.mmax, d.tri, s);
-}
-
 // the kernels load and store 16 bytes at a time
 template <class... T>
 bool aligned(const T*... p) {
@@ -215,7 +205,7 @@ extern "C" int sfno_block_forward(const sfno_block* b, int training, const void*
         TRY(synthesis_launch(b->inv, spec, w.xm_out, r, SFNO_DTYPE_BF16, nullptr, d.rows_in, s));
         res = r;
     }
-    TRY(mix(b->weights, spec, w.spec, d, d.rows, s));
+    TRY(sfno_dhconv_spectral(b->weights, spec, w.spec, d.B, d.mmax, d.tri, s));
     float2* m0 = reinterpret_cast<float2*>(c0 + 2 * d.rows);
     if (d.P <= NORM_SMALL_PIXELS) {
         TRY(synthesis_launch(b->inv, w.spec, w.xm_out, xf, SFNO_DTYPE_BF16, nullptr, d.rows, s));
@@ -296,7 +286,7 @@ extern "C" int sfno_block_backward(const sfno_block* b, const void* gv, const vo
         TRY(dhconv_wgrad_launch(a, s));
     }
     if (!grads->gx) return SFNO_OK;
-    TRY(mix(b->weights_adj, w.gspec_out, w.gspec_in, d, d.rows_in, s));
+    TRY(sfno_dhconv_spectral(b->weights_adj, w.gspec_out, w.gspec_in, d.B, d.mmax, d.tri, s));
     bf16* gx = reinterpret_cast<bf16*>(grads->gx);
     if (d.scale_residual) {
         // the residual's gradient joins in spectral space

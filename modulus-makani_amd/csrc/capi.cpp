@@ -682,7 +682,9 @@ extern "C" int sfno_dhconv_spectral(const sfno_dhconv_weights* w, const float* s
     a.nob = w->nob;
     a.nc = w->nc;
     a.cinv = w->d_cinv;
-    if (w->f16) return dhconv_f16_launch(a, (hipStream_t)stream);
+    if (w->f16) return dhconv_f16_launch(a, (hipStream_t)stream);              // (clears the padding itself)
+    const int rc = spectral_zero_padding_launch(spec_out, (int64_t)batch * w->O, (int64_t)mmax * w->L, a.ld_out, (hipStream_t)stream);
+    if (rc != SFNO_OK) return rc;
     if (w->split) return dhconv_split_launch(a, (hipStream_t)stream);
     if (w->compute == SFNO_COMPUTE_BF16) return dhconv_bf16_launch(a, (hipStream_t)stream);
     return dhconv_launch(a, (hipStream_t)stream);

@@ -151,8 +151,6 @@ def _dhconv_spectral(spec_in, weight, batch, mmax, triangular, compute, adjoint,
     I, O, L = pw.shape
     ld_out = int(lib.sfno_spectral_ld(batch * O))
     out = torch.empty((mmax, L, ld_out), dtype=torch.float32, device=spec_in.device)
-    if ld_out != 2 * batch * O:
-        out.zero_()
     if batch == 0:
         return out
     s = _stream(spec_in.device)
