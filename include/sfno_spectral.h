@@ -357,6 +357,13 @@ int sfno_pointwise_pack_weight(const float* w, void* packed, int O, int K, void*
 int sfno_pointwise_pack_weight_transposed(const float* w, void* packed, int O, int K, void* stream);
 /* both in one launch: the weight w [O][K], and its transpose as sfno_pointwise_pack_weight_transposed(w, ..., K, O) packs it */
 int sfno_pointwise_pack_weight_both(const float* w, void* packed, void* packed_transposed, int O, int K, void* stream);
+/* The layer w (scale m + shift) + ws r + bias as one convolution of (m, r) by sfno_pointwise_conv_cat, for `batch` samples with a scale and
+ * a shift [K] each (null: 1 and 0): packed receives `batch` streams of sfno_pointwise_weight_elems(O, 2 K) elements, the weight [w diag(scale) | ws]
+ * of a sample, shifted float32 [batch][O] its bias w shift + bias.  w and ws are float32 [O][K], bias float32 [O] or null.  No counterpart in
+ * the reference; it merges norm1 and outer_skip of the last block with the decoder's first convolution (makani/models/networks/sfnonet.py:258-262,
+ * makani/models/common/layers.py:95-116). */
+int sfno_pointwise_merge_weight(const float* w, const float* ws, const float* scale, const float* shift, const float* bias, void* packed,
+                                float* shifted, int O, int K, int batch, void* stream);
 
 /* Instance norm as a per-(b, c) affine: scale = gamma[c] / sqrt(var + eps), shift = beta[c] - mean * scale over
  * the P pixels of each of the `rows` = B*C rows of x (bf16), statistics in fp32 with the biased variance

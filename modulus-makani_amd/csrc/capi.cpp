@@ -782,6 +782,12 @@ extern "C" int sfno_pointwise_pack_weight_both(const float* w, void* packed, voi
                                       (hipStream_t)stream);
 }
 
+extern "C" int sfno_pointwise_merge_weight(const float* w, const float* ws, const float* scale, const float* shift, const float* bias, void* packed,
+                                           float* shifted, int O, int K, int batch, void* stream) {
+    if (!w || !ws || !packed || !shifted || O < 1 || K < 1 || K > (1 << 29) || batch < 1) return SFNO_EINVAL;
+    return pointwise_merge_launch(w, ws, scale, shift, bias, reinterpret_cast<unsigned short*>(packed), shifted, O, K, batch, (hipStream_t)stream);
+}
+
 // 16-byte loads of eight bf16 values
 static bool on16(const void* a, const void* b, const void* c, const void* d) {
     return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) | reinterpret_cast<uintptr_t>(d)) & 15) == 0;

@@ -737,6 +737,43 @@ __global__ __launch_bounds__(256) void pointwise_pack_both_kernel(const float* _
         pack_element(w, packed_t, K, O, nc_t, idx - total, 1);
 }
 
+// The merged layer W (scale . m + shift) + W W_skip r + bias of a network's tail (O x K weight W), for every sample b: packed[b], the stream of
+// [W diag(scale_b) | W W_skip] as pack_element writes it, and shifted[b] = W shift_b + bias.  The first blocks of a sample pack, the others
+// take four output rows each, a wavefront one (lanes over k, sums folded in halves).  grid (pack + ceil(O / 4), samples, at most 256).  Nothing but latency at
+// these sizes; as separate products, concatenation, matrix product, sum and packing it was eleven launches and 70 us a call.
+__global__ __launch_bounds__(256) void pointwise_merge_kernel(const float* __restrict__ w, const float* __restrict__ ws, const float* __restrict__ scale,
+                                                              const float* __restrict__ shift, const float* __restrict__ bias,
+                                                              unsigned short* __restrict__ packed, float* __restrict__ shifted, int O, int K, int B,
+                                                              int nc, int64_t total, int pack) {
+    if ((int)blockIdx.x < pack) {
+        const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (idx >= total) return;
+        const int e = (int)(idx & 7), lane = (int)((idx >> 3) & 63);
+        const int64_t blk = idx >> 9;
+        const int c = (int)(blk % nc), rb = (int)(blk / nc);
+        const int o = 32 * rb + (lane & 31), k = 16 * c + 8 * (lane >> 5) + e;
+        for (int b = blockIdx.y; b < B; b += gridDim.y) {
+            float v = 0.f;
+            if (o < O && k < K)
+                v = scale ? w[(int64_t)o * K + k] * scale[(int64_t)b * K + k] : w[(int64_t)o * K + k];
+            else if (o < O && k < 2 * K)
+                v = ws[(int64_t)o * K + k - K];
+            packed[b * total + idx] = f_to_bf16(v);
+        }
+        return;
+    }
+    const int o = 4 * ((int)blockIdx.x - pack) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (o >= O) return;
+    for (int b = blockIdx.y; b < B; b += gridDim.y) {
+        float sum = 0.f;
+        if (shift)
+            for (int k = lane; k < K; k += 64) sum = fmaf(w[(int64_t)o * K + k], shift[(int64_t)b * K + k], sum);
+#pragma unroll
+        for (int d = 32; d; d >>= 1) sum += __shfl_xor(sum, d);
+        if (lane == 0) shifted[(int64_t)b * O + o] = bias ? sum + bias[o] : sum;
+    }
+}
+
 // ---- instance-norm statistics ------------------------------------------------------------------
 // partial[row][seg] = (sum d, sum d^2), d = x - x[row][0] (the pivot keeps the variance formula from cancelling)
 constexpr int ST_THREADS = 256;
@@ -1074,6 +1111,16 @@ int pointwise_pack_both_launch(const float* w, unsigned short* packed, unsigned 
     const int64_t blocks = (total + total_t + 255) / 256;
     if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
     hipLaunchKernelGGL(pointwise_pack_both_kernel, dim3((unsigned)blocks), dim3(256), 0, s, w, packed, nc, total, packed_t, nc_t, total_t, O, K);
+    return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
+}
+
+int pointwise_merge_launch(const float* w, const float* ws, const float* scale, const float* shift, const float* bias, unsigned short* packed, float* shifted,
+                           int O, int K, int B, hipStream_t s) {
+    const int nc = pointwise_kpad(2 * K, O) / PW_KC;
+    const int64_t total = (int64_t)(pointwise_opad(O) / 32) * nc * 512, pack = (total + 255) / 256, blocks = pack + (O + 3) / 4;
+    if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
+    hipLaunchKernelGGL(pointwise_merge_kernel, dim3((unsigned)blocks, (unsigned)std::min(B, 256)), dim3(256), 0, s, w, ws, scale, shift, bias, packed, shifted, O, K,
+                       B, nc, total, (int)pack);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

@@ -140,6 +140,9 @@ int pointwise_opad(int O);
 int pointwise_pack_launch(const float* w, unsigned short* packed, int O, int K, int transposed, hipStream_t s);
 // w [O][K] and its transpose, the latter as pointwise_pack_launch(w, packed_t, K, O, 1, s) writes it
 int pointwise_pack_both_launch(const float* w, unsigned short* packed, unsigned short* packed_t, int O, int K, hipStream_t s);
+// B streams of [w diag(scale_b) | ws] (O x 2 K) and the vectors w shift_b + bias
+int pointwise_merge_launch(const float* w, const float* ws, const float* scale, const float* shift, const float* bias, unsigned short* packed, float* shifted,
+                           int O, int K, int B, hipStream_t s);
 // weight and bias gradient of the 1x1 convolution (pointwise_wgrad.hip); db null: no bias column
 size_t pointwise_wgrad_workspace_bytes(int O, int K, int has_bias, int B, int64_t P);
 int pointwise_wgrad_launch(const unsigned short* g, const unsigned short* x, float* dW, float* db, int B, int K, int O, int64_t P, float* ws,

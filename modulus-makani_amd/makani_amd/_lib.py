@@ -105,6 +105,7 @@ def _load():
         "sfno_pointwise_conv_gelu_grad": (i32, [vp, vp, vp, vp, i32, i32, i32, i64, vp]),
         "sfno_pointwise_pack_weight_transposed": (i32, [vp, vp, i32, i32, vp]),
         "sfno_pointwise_pack_weight_both": (i32, [vp, vp, vp, i32, i32, vp]),
+        "sfno_pointwise_merge_weight": (i32, [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp]),
         "sfno_block_layout": (sz, [vp, i32, vp]),
         "sfno_block_workspace_bytes": (sz, [vp, i32]),
         "sfno_block_forward": (i32, [vp, i32, vp, vp, vp, sz, vp, sz, vp]),

@@ -151,18 +151,31 @@ def norm_mlp(x, scale, shift, w1, b1, w2, b2):
     return y
 
 
-def conv1x1_cat(x1, x2, weight, bias=None, act=None, out=None):
+def merged_weight(w, ws, scale, shift, bias, batch):
+    """The layer w (scale x1 + shift) + ws x2 + bias of each sample as a convolution for conv1x1_cat: packed weights bf16 [batch, n] and biases
+    float32 [batch, O]; w, ws float32 [O, K], scale, shift float32 [batch, K] (None: 1 and 0), bias [O] or None."""
+    O, K = w.shape
+    packed = torch.empty((batch, lib.sfno_pointwise_weight_elems(O, 2 * K)), dtype=torch.bfloat16, device=w.device)
+    shifted = torch.empty((batch, O), dtype=torch.float32, device=w.device)
+    bias = _vector(bias)
+    check(lib.sfno_pointwise_merge_weight(_ptr(w), _ptr(ws), _ptr(scale), _ptr(shift), _ptr(bias), _ptr(packed), _ptr(shifted), O, K, batch, _stream(w.device)),
+          "sfno_pointwise_merge_weight")
+    return packed, shifted
+
+
+def conv1x1_cat(x1, x2, weight, bias=None, act=None, out=None, packed=None):
     """act(conv1x1(cat([x1, x2], dim=1), weight) + bias) without building the concatenation  ->  bf16 [B, O, H, W];
-    weight [O, K1 + K2] (or [O, K1 + K2, 1, 1]); out: a contiguous bf16 tensor of the result's shape to write into."""
+    weight [O, K1 + K2] (or [O, K1 + K2, 1, 1]); out: a contiguous bf16 tensor of the result's shape to write into; packed: the weight's stream
+    where the caller has it (weight is then its shape)."""
     if not (supported(x1) and supported(x2)) or x1.shape[0] != x2.shape[0] or x1.shape[2:] != x2.shape[2:]:
         raise RuntimeError("conv1x1_cat takes two contiguous bfloat16 NCHW HIP tensors of one batch and grid size, H*W a multiple of 8")
     x1, x2 = _dense(x1), _dense(x2)
     B, K1, H, W = x1.shape
     K2 = x2.shape[1]
-    O = weight.shape[0]
-    if weight.reshape(O, -1).shape[1] != K1 + K2:
-        raise RuntimeError(f"conv1x1_cat: inputs have {K1} + {K2} channels, weight expects {weight.reshape(O, -1).shape[1]}")
-    pw = packed_weight(weight)
+    O, K = (weight.shape[0], weight.shape[1:].numel()) if packed is None else weight
+    if K != K1 + K2:
+        raise RuntimeError(f"conv1x1_cat: inputs have {K1} + {K2} channels, weight expects {K}")
+    pw = packed_weight(weight) if packed is None else packed
     if out is None:
         y = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x1.device)
     else:

@@ -503,21 +503,15 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
             if cached is None or cached[0] != stamp:
                 wd = conv_d.weight.detach().reshape(conv_d.weight.shape[0], -1).to(torch.bfloat16).float()
                 ws = blk.outer_skip.weight.detach().reshape(C, -1).to(torch.bfloat16).float()
-                cached = (stamp, wd, (wd @ ws).contiguous())
+                cached = (stamp, wd, (wd @ ws).float().contiguous())
                 self._merge_cache = cached
-            wd, wds = cached[1], cached[2]
-            if sc is None:
-                sc = torch.ones((B, C), dtype=torch.float32, device=m.device)
-                sh = torch.zeros_like(sc)
-            sc, sh = sc.clone(), sh.clone()          # ordinary tensors for the arithmetic below
-            # all samples at once: [W_d diag(scale_b) | W_d W_skip] and W_d shift_b (+ bias); only the left half depends on b
-            wcat = torch.cat([wd[None] * sc[:, None, :], wds[None].expand(B, -1, -1)], dim=2).contiguous()
-            bias = sh @ wd.t()
-            if conv_d.bias is not None:
-                bias = bias + conv_d.bias.detach().float()
-        y = torch.empty((B, wd.shape[0], m.shape[2], m.shape[3]), dtype=torch.bfloat16, device=m.device)
+        wd, wds = cached[1], cached[2]
+        # [W_d diag(scale_b) | W_d W_skip] and W_d shift_b + bias of every sample b
+        packed, bias = pw.merged_weight(wd, wds, sc, sh, conv_d.bias, B)
+        O = wd.shape[0]
+        y = torch.empty((B, O, m.shape[2], m.shape[3]), dtype=torch.bfloat16, device=m.device)
         for b in range(B):
-            pw.conv1x1_cat(m[b:b + 1], r[b:b + 1], wcat[b], bias[b], dec[0][1], out=y[b:b + 1])
+            pw.conv1x1_cat(m[b:b + 1], r[b:b + 1], (O, 2 * C), bias[b], dec[0][1], out=y[b:b + 1], packed=packed[b])
         return y, dec[1:]
 
     def _forward_fused(self, x, enc, dec):

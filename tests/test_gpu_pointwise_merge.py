@@ -1,0 +1,29 @@
+"""Weight and bias of the merged layer w (scale x1 + shift) + ws x2 + bias: the stream against packing the composed matrix, bit for bit, the bias against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("O,K,B", [(97, 1, 1), (98, 63, 3), (129, 65, 2), (104, 104, 1), (384, 384, 2), (3, 5, 300)])
+@pytest.mark.parametrize("norm,with_bias", [(True, True), (True, False), (False, True)])
+def test_merged_weight(lib_built, O, K, B, norm, with_bias):
+    from makani_amd import pointwise as pw
+
+    print(f"case merged weight O={O} K={K} B={B} norm={norm} bias={with_bias}", flush=True)
+    gen = torch.Generator().manual_seed(O * K + B)
+    w, ws = (torch.randn(O, K, generator=gen).cuda() for _ in range(2))
+    scale, shift = (torch.randn(B, K, generator=gen).cuda() if norm else None for _ in range(2))
+    bias = torch.randn(O, generator=gen).cuda() if with_bias else None
+    packed, shifted = pw.merged_weight(w, ws, scale, shift, bias, B)
+    torch.cuda.synchronize()
+    sh = torch.zeros(B, K, dtype=torch.float64) if shift is None else shift.cpu().double()
+    terms = sh[:, None, :] * w.cpu().double()
+    ref, size = terms.sum(-1), terms.abs().sum(-1)
+    if with_bias:
+        ref, size = ref + bias.cpu().double(), size + bias.cpu().double().abs()
+    # a chain of ceil(K / 64) products and sums, six foldings, the bias
+    assert bool(((shifted.cpu().double() - ref).abs() <= (-(-K // 64) + 7) * 2.0**-24 * size).all())
+    for b in range(B):
+        left = w if scale is None else w * scale[b]
+        assert torch.equal(packed[b], pw.packed_weight(torch.cat([left, ws], dim=1)))
