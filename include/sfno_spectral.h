@@ -286,6 +286,19 @@ int sfno_degree_norm(const float* spec, const float* weights, float* sums, float
 int sfno_degree_norm_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec,
                           int batch, int64_t channels, int lmax, int mmax, float alpha, int squared, void* stream);
 
+/* The coefficients of x - x2 and of x2 side by side, float32 [mmax][lmax][ld], ld = sfno_sht_analysis_pair_ld(p, rows), the second's rows from float ld / 2
+ * on: one Legendre stage for both (the relative form of GeometricH1Loss, makani/utils/losses.py:320-345).  ld is 0, and the call refused,
+ * where the plan or the size has no such path; `workspace` holds mmax * nlat * ld floats.  The norms of both, as sfno_degree_norm gives them for
+ * each (sums [2 batch][2]), and the gradient with respect to the coefficients of x - x2 alone, in their own layout. */
+int64_t sfno_sht_analysis_pair_ld(const sfno_sht_plan* p, int64_t rows);
+int sfno_sht_analysis_pair(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, int64_t rows, void* workspace,
+                           size_t workspace_bytes, void* stream);
+size_t sfno_degree_norm_pair_workspace_bytes(int batch, int64_t channels, int lmax);
+int sfno_degree_norm_pair(const float* spec, const float* weights, float* sums, float* norms, float* norms2, int batch, int64_t channels,
+                          int lmax, int mmax, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream);
+int sfno_degree_norm_pair_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec, int batch,
+                               int64_t channels, int lmax, int mmax, float alpha, int squared, void* stream);
+
 /* ---- "diagonal" operator ------------------------------------------------------------- */
 
 /* y[b,o,l,m] = sum_i x[b,i,l,m] w[i,o,l,m] (makani/models/common/contractions.py:121-127, operator_type

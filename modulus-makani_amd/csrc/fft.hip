@@ -391,10 +391,10 @@ static int pick_pairs(int n) {
     return 0;
 }
 
-int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2, const int* kept) {
-    if (mmax > p.n / 2 + 1 || ld % 4 != 0 || ld < 2 * rows) return SFNO_EINVAL;
-    if (fft_fast_supported(p.n)) return fft_fast_launch(false, p, xv, xm, rows, nlat, mmax, ld, x_dtype, s, nullptr, x2, kept);
-    if (x2 || kept) return SFNO_EUNSUPPORTED;
+int rfft_launch(const FftPlan& p, const void* xv, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2, const int* kept, int width) {
+    if (mmax > p.n / 2 + 1 || ld % 4 != 0 || ld < 2 * rows || width % 4 != 0 || (width && (width < 2 * rows || ld < 2 * width))) return SFNO_EINVAL;
+    if (fft_fast_supported(p.n)) return fft_fast_launch(false, p, xv, xm, rows, nlat, mmax, ld, x_dtype, s, nullptr, x2, kept, width);
+    if (x2 || kept || width) return SFNO_EUNSUPPORTED;
     if (x_dtype != SFNO_DTYPE_F32) return SFNO_EUNSUPPORTED;     // the generic kernels read float only
     const float* x = reinterpret_cast<const float*>(xv);
     switch (pick_pairs(p.n)) {

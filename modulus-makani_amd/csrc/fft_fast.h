@@ -8,7 +8,7 @@ namespace sfno {
 // all answer SFNO_EUNSUPPORTED for a length the part does not hold
 #define SFNO_FFT_PART_DECL(P)                                                                                                 \
     int fft_part_lon_##P(bool inverse, const FftPlan& p, const void* in, const void* in2, void* out, int64_t rows, int nlat, int mmax, int ld, \
-                         int grid_dtype, hipStream_t s, float2* lat_stats, const int* kept);                                                                   \
+                         int grid_dtype, hipStream_t s, float2* lat_stats, const int* kept, int width);                                                                   \
     int fft_part_lat_##P(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);   \
     int fft_part_rows_##P(bool inverse, const FftPlan& p, const float* in, float* out, int64_t rows, int nlat, int mmax, int cs, hipStream_t s); \
     int fft_part_cols_##P(bool inverse, const FftPlan& p, const float2* in, float2* out, int64_t rows, int mmax, int lmax, \
@@ -24,8 +24,8 @@ SFNO_FFT_PART_DECL(F);
 
 #define SFNO_FFT_LON_CASE(N_, A_, B_, C_)                                                                                    \
     case N_:                                                                                                                  \
-        return grid_dtype == SFNO_DTYPE_BF16 ? go_fast<N_, A_, B_, C_, true>(inverse, p, in, in2, out, rows, nlat, mmax, ld, lat_stats, kept, s) \
-                                             : go_fast<N_, A_, B_, C_, false>(inverse, p, in, in2, out, rows, nlat, mmax, ld, lat_stats, kept, s);
+        return grid_dtype == SFNO_DTYPE_BF16 ? go_fast<N_, A_, B_, C_, true>(inverse, p, in, in2, out, rows, nlat, mmax, ld, lat_stats, kept, width, s) \
+                                             : go_fast<N_, A_, B_, C_, false>(inverse, p, in, in2, out, rows, nlat, mmax, ld, lat_stats, kept, width, s);
 #define SFNO_FFT_LAT_CASE(N_, A_, B_, C_)                                                                                     \
     case N_:                                                                                                                  \
         if constexpr (N_ <= kLatMax) return go_lat<N_, A_, B_, C_>(inverse, p, in, out, mmax, lmax, ld, mscale, s);           \
@@ -40,7 +40,7 @@ SFNO_FFT_PART_DECL(F);
 #define SFNO_FFT_PART(P, LENGTHS)                                                                                             \
     namespace sfno {                                                                                                          \
     int fft_part_lon_##P(bool inverse, const FftPlan& p, const void* in, const void* in2, void* out, int64_t rows, int nlat, int mmax, int ld, \
-                        int grid_dtype, hipStream_t s, float2* lat_stats, const int* kept) {                                                                   \
+                        int grid_dtype, hipStream_t s, float2* lat_stats, const int* kept, int width) {                                                                   \
         switch (p.n) { LENGTHS(SFNO_FFT_LON_CASE) }                                                                           \
         return SFNO_EUNSUPPORTED;                                                                                             \
     }                                                                                                                         \

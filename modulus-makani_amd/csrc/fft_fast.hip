@@ -144,11 +144,11 @@ int fft_fast_plan_init(FftPlan& p) {
 }
 
 int fft_fast_launch(bool inverse, const FftPlan& p, const void* in, void* out, int64_t rows, int nlat, int mmax, int ld, int grid_dtype,
-                    hipStream_t s, float2* lat_stats, const void* in2, const int* kept) {
+                    hipStream_t s, float2* lat_stats, const void* in2, const int* kept, int width) {
     if (grid_dtype != SFNO_DTYPE_BF16 && grid_dtype != SFNO_DTYPE_F32) return SFNO_EUNSUPPORTED;
-    if ((lat_stats && !inverse) || (in2 && inverse)) return SFNO_EINVAL;
+    if ((lat_stats && !inverse) || (in2 && inverse) || (width && !in2)) return SFNO_EINVAL;
     for (auto part : {fft_part_lon_A, fft_part_lon_B, fft_part_lon_C, fft_part_lon_D, fft_part_lon_E, fft_part_lon_F}) {
-        const int rc = part(inverse, p, in, in2, out, rows, nlat, mmax, ld, grid_dtype, s, lat_stats, kept);
+        const int rc = part(inverse, p, in, in2, out, rows, nlat, mmax, ld, grid_dtype, s, lat_stats, kept, width);
         if (rc != SFNO_EUNSUPPORTED) return rc;
     }
     return SFNO_EUNSUPPORTED;

@@ -458,6 +458,10 @@ __device__ __forceinline__ int tile_orders(const int* kept, int lat, int mmax) {
 // registers are at their limit), their latency is the other workgroups' to hide: 73 x 721 x 1440 in 210 us (0.93 GB, 4.4 TB/s), where the
 // transform of a stored difference took 137 and the pass that stores it 183.
 //
+// both (with DIFF): the transform of x2 as well, its columns `width` floats behind those of x - x2.  Its tiles take turns with those of the difference on
+// one XCD, so that the rows of x2 are read twice at about the same time
+// (73 x 721 x 1440: 300 us for both, 187 and 118 one after the other).
+//
 // SHORT: the last batch of a latitude is not full (73 channels are 36.5 pairs in batches of 4).  A kernel of its own, for float32 fields: the comparisons cost
 // whole batches up to 2 % (721 x 1440: 73 channels 146 -> 145 us, inverse 154 -> 150; 9 channels 31.5 -> 28.8; 3 channels of 360 x 720 12.0 -> 9.9).
 //
@@ -465,14 +469,14 @@ __device__ __forceinline__ int tile_orders(const int* kept, int lat, int mmax) {
 template <int N, int R0, int R1, int R2, int S, int H, int FT, bool BF16, bool DIFF, bool SHORT = false>
 __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restrict__ tw0, const float2* __restrict__ tw1, const unsigned* __restrict__ post,
                                                           const void* __restrict__ x, const void* __restrict__ x2, float* __restrict__ xm, int64_t rows,
-                                                          int nlat, int mmax, const int* kept, int ld, int ngroups, float scale) {
+                                                          int nlat, int mmax, const int* kept, int ld, int width, int both, int ngroups, float scale) {
     using G = Geo<N, R0, R1, R2>;
     static_assert((S & (S - 1)) == 0 && FT % S == 0 && N % 4 == 0, "a power-of-two number of channel pairs shares the threads evenly");
     static_assert(H == 1 || H == 2, "one or two batches per tile");
     __shared__ __align__(16) float2 z[S * G::PITCH];
     __shared__ LdsTables<N, R0, R1, R2> tab;
     const int tid = threadIdx.x;
-    const TileWalk walk(nlat, ngroups);
+    const TileWalk walk(nlat, DIFF && both ? 2 * ngroups : ngroups);
     int t = walk.first();
     if (t >= walk.ntiles) return;
     lds_tables<N, R0, R1, R2, FT>(tab, tw0, tw1, post, tid);
@@ -486,9 +490,20 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
     const int pl = tid / TP, q0 = tid - pl * TP;
     typename Raw4<BF16>::type a[IT], b[IT];
     bool ha = false, hb = false;
+    // tile -> latitude, group of pairs, and whether it is one of x2 alone
+    auto locate = [&](int tile, int& lat, int& group, bool& plain) {
+        walk.locate(tile, lat, group);
+        plain = false;
+        if (DIFF && both) {
+            plain = group & 1;
+            group >>= 1;
+        }
+    };
     auto request = [&](int tile, int half) {
         int lat, group;
-        walk.locate(tile, lat, group);
+        bool plain;
+        locate(tile, lat, group, plain);
+        const void* src = DIFF && plain ? x2 : x;
         const int64_t r0 = 2 * (int64_t)((group * H + half) * S + pl);
         ha = r0 < rows;
         hb = r0 + 1 < rows;
@@ -498,15 +513,15 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
             // (a row can be shorter than one step of the TP threads: the fall-back address is the row's start, not the thread's)
             const bool in = (it + 1) * TP <= Q || q0 + it * TP < Q;
             const int off = in ? 4 * (q0 + it * TP) : 0;
-            a[it] = load_raw4<BF16>(x, ia + off);
-            b[it] = load_raw4<BF16>(x, ib + off);
+            a[it] = load_raw4<BF16>(src, ia + off);
+            b[it] = load_raw4<BF16>(src, ib + off);
         }
     };
     // the requested batch (of this tile and half) goes to LDS as complex sequences a + i b
-    auto fill = [&](int lat, int group, int half) {
+    auto fill = [&](int lat, int group, int half, bool plain) {
         float4* dst = reinterpret_cast<float4*>(z + pl * G::PITCH) + 2 * q0;
         typename Raw4<BF16>::type a2[DIFF ? IT : 1], b2[DIFF ? IT : 1];
-        if constexpr (DIFF) {
+        if (DIFF && !plain) {
             const int64_t r0 = 2 * (int64_t)((group * H + half) * S + pl);
             const int64_t ia = ((ha ? r0 : 0) * nlat + lat) * N, ib = ((hb ? r0 + 1 : 0) * nlat + lat) * N;
 #pragma unroll
@@ -526,7 +541,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
         for (int it = 0; it < IT; ++it) {
             if ((it + 1) * TP <= Q || q0 + it * TP < Q) {
                 float4 fa = widen4(a[it]), fb = widen4(b[it]);
-                if constexpr (DIFF) {
+                if (DIFF && !plain) {
                     const float4 ga = widen4(a2[it]), gb = widen4(b2[it]);
                     fa = make_float4(fa.x - ga.x, fa.y - ga.y, fa.z - ga.z, fa.w - ga.w);
                     fb = make_float4(fb.x - gb.x, fb.y - gb.y, fb.z - gb.z, fb.w - gb.w);
@@ -552,14 +567,15 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
     request(t, 0);
     for (;;) {
         int lat, group;
-        walk.locate(t, lat, group);
+        bool plain;
+        locate(t, lat, group, plain);
         const int tn = t + walk.step;
         const int tq = tn < walk.ntiles ? tn : t;       // the last tile requests itself again: always a request, never a branch around one
         const int pair = group * H * S + pp_;
         const int mleft = tile_orders(kept, lat, mmax) - mfirst;     // (of the orders from my first one on)
-        float* o = xm + ((int64_t)mfirst * nlat + lat) * ld + 4 * (int64_t)pair;
+        float* o = xm + ((int64_t)mfirst * nlat + lat) * ld + 4 * (int64_t)pair + (DIFF && plain ? width : 0);
         const int left = (int)((rows + 1) / 2) - group * H * S;      // pairs from here on; those that are not there are zeros in LDS and stay zeros
-        fill(lat, group, 0);
+        fill(lat, group, 0, plain);
         if (H == 2)
             request(t, 1);
         else
@@ -567,7 +583,7 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
         __syncthreads();
         passes_dif<N, R0, R1, R2, S, FT, SHORT>(z, tab.tw0, tab.tw1, tid, min(left, S));
         if constexpr (H == 1) {
-            if (pair < ld / 4) {
+            if (pair < width / 4) {
 #pragma unroll
                 for (int u = 0; u < NSW; ++u)
                     if (u * TP < mleft) *reinterpret_cast<float4*>(o + u * mstep) = split(mfirst + u * TP);
@@ -578,11 +594,11 @@ __global__ __launch_bounds__(FT, 4) void rfft_fast_kernel(const float2* __restri
             for (int u = 0; u < NSW; ++u)
                 if (u * TP < mleft) first[u] = split(mfirst + u * TP);
             __syncthreads();
-            fill(lat, group, 1);
+            fill(lat, group, 1, plain);
             request(tq, 0);
             __syncthreads();
             passes_dif<N, R0, R1, R2, S, FT, SHORT>(z, tab.tw0, tab.tw1, tid, min(left - S, S));
-            const bool va = pair < ld / 4, vb = pair + S < ld / 4;
+            const bool va = pair < width / 4, vb = pair + S < width / 4;
 #pragma unroll
             for (int u = 0; u < NSW; ++u) {
                 if (u * TP < mleft) {
@@ -1104,15 +1120,17 @@ __global__ __launch_bounds__(FT) void latfft_chirp_kernel(const float2* __restri
 
 template <int N, int R0, int R1, int R2, bool BF16>
 int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, void* out, int64_t rows, int nlat, int mmax, int ld, float2* lat_stats,
-            const int* kept, hipStream_t s) {
+            const int* kept, int width, hipStream_t s) {
     constexpr int S = (N >= 1024) ? 4 : 8;              // channel pairs in LDS at a time
     constexpr int H = 8 / S;                            // batches per tile: a tile owns 8 pairs = one 128-byte line per order
     constexpr int FT = (S * N >= 4096) ? 512 : 256;     // threads per workgroup
-    const int ngroups = (ld / 4 + S * H - 1) / (S * H);
+    const int both = width != 0;
+    if (!both) width = ld;
+    const int ngroups = (width / 4 + S * H - 1) / (S * H);
     // as many workgroups as stay resident (four wavefronts per SIMD: two workgroups of 512 threads or four of 256 per CU), the
     // same number on every XCD; fewer when an XCD has fewer tiles than that
     constexpr int WG_PER_CU = 1024 / FT;
-    const int64_t tiles_xcd = (int64_t)((nlat + 7) / 8) * ngroups;
+    const int64_t tiles_xcd = (int64_t)((nlat + 7) / 8) * ngroups * (both ? 2 : 1);
     const int per_xcd = (int)std::min<int64_t>(tiles_xcd, std::max(1, WG_PER_CU * p.n_cu / 8));
     dim3 grid((unsigned)(8 * per_xcd));
     const int64_t npairs = (rows + 1) / 2;
@@ -1121,7 +1139,7 @@ int go_fast(bool inverse, const FftPlan& p, const void* in, const void* in2, voi
         const bool full = BF16 || npairs % (S * H) == 0;
 #define RFFT_GO(DIFF_, SHORT_)                                                                                                                   \
     hipLaunchKernelGGL((rfft_fast_kernel<N, R0, R1, R2, S, H, FT, BF16, DIFF_, SHORT_>), grid, dim3(FT), 0, s, p.d_tw0, p.d_tw1, p.d_post, in, \
-                       in2, reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, ngroups, scale)
+                       in2, reinterpret_cast<float*>(out), rows, nlat, mmax, kept, ld, width, both, ngroups, scale)
         if (!in2) {
             if (full) RFFT_GO(false, false); else RFFT_GO(false, !BF16);
         } else if constexpr (!BF16) {

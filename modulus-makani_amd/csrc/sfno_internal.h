@@ -226,7 +226,7 @@ int fft_fast_plan_init(FftPlan& p);
 // kept (may be null: all of mmax): [nlat] orders that are exchanged with the Fourier buffer at each latitude, the first ones; at least one.  Forward leaves
 // the others as they are, inverse takes them for zero
 int fft_fast_launch(bool inverse, const FftPlan& p, const void* in, void* out, int64_t rows, int nlat, int mmax, int ld, int grid_dtype,
-                    hipStream_t s, float2* lat_stats = nullptr, const void* in2 = nullptr, const int* kept = nullptr);
+                    hipStream_t s, float2* lat_stats = nullptr, const void* in2 = nullptr, const int* kept = nullptr, int width = 0);
 // latitude FFT on the specialised passes; SFNO_EUNSUPPORTED for a length without them
 int latfft_fast_launch(bool inverse, const FftPlan& p, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
 // planar pair on the reference layout: real FFTs along the grid rows, x [rows][nlat][n] <-> y [rows][group][nlat][2^cs] complex (groups
@@ -241,9 +241,9 @@ int fft_plan_init(FftPlan& p, int n);
 int fft_chirp_plan_init(FftPlan& p);
 void fft_plan_free(FftPlan& p);
 // x [rows][nlat][nlon] -> xm [mmax][nlat][ld] (re,im of row r at 2r,2r+1), scaled by 2 pi / nlon
-// (x2 given: of x - x2, float32 fields and lengths with specialised kernels only)
+// (x2 given: of x - x2, float32 fields and lengths with specialised kernels only; width given too: of x - x2, and of x2 `width` floats further on)
 int rfft_launch(const FftPlan& p, const void* x, int x_dtype, float* xm, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, const void* x2 = nullptr,
-                const int* kept = nullptr);
+                const int* kept = nullptr, int width = 0);
 // xm [mmax][nlat][ld] -> x [rows][nlat][nlon]
 int irfft_launch(const FftPlan& p, const float* xm, void* x, int x_dtype, int64_t rows, int nlat, int mmax, int ld, hipStream_t s, float2* lat_stats = nullptr,
                  const int* kept = nullptr);
@@ -254,13 +254,14 @@ int latfft_launch(const FftPlan& p, bool inverse, const float* in, float* out, i
 // ---- per-degree power of spectral-layout coefficients and its gradient (degree_power.hip) ------------
 int degree_power_launch(const float* spec, float* power, int64_t rows, int lmax, int mmax, int ld, hipStream_t s);
 // sums over the channels and degrees of `channels` rows per example: sums[b] = (sum p, sum weights[l] p), norms[b] = alpha a + (1 - alpha) h of
-// them or of their square roots; partial: double2 [batch][degree_norm_segments] of workspace
+// them or of their square roots; partial: double2 [batch][degree_norm_segments] of workspace.  norms2 not null: of a second batch too, whose powers follow the
+// first's after `gap` values (sums and partial for both)
 int degree_norm_segments(int64_t channels, int lmax);
-int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, int batch, int64_t channels, int lmax,
-                       float alpha, int squared, hipStream_t s);
-// gradient of the above with respect to the coefficients
+int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, float* norms2, int64_t gap, int batch,
+                       int64_t channels, int lmax, float alpha, int squared, hipStream_t s);
+// gradient of the above with respect to the coefficients (rows of ld_in floats, the gradient's of ld)
 int degree_norm_grad_launch(const float* spec, const float* weights, const float2* sums, const float* gnorms, float* gspec, int batch, int64_t channels, int lmax,
-                            int mmax, int ld, float alpha, int squared, hipStream_t s);
+                            int mmax, int ld_in, int ld, float alpha, int squared, hipStream_t s);
 int degree_power_grad_launch(const float* spec, const float* gpower, float* gspec, int64_t rows, int lmax, int mmax, int ld, hipStream_t s);
 
 // ---- file-scope scratch array of sfno_sht_forward_static (static_scratch.hip) ----------------

@@ -9,7 +9,7 @@ import torch
 from torch import nn
 from torch.autograd.function import once_differentiable
 
-from ._lib import lib, check
+from ._lib import DTYPE_F32, lib, check
 from .sht import RealSHT, _ptr, _stream_ptr as _stream
 
 
@@ -64,6 +64,46 @@ class _DegreeNormFn(torch.autograd.Function):
         return gspec, None, None, None, None, None
 
 
+class _PairNormsFn(torch.autograd.Function):
+    """Norms [batch] of x - x2 and of x2, differentiable with respect to x: the analyses of both share one Legendre stage."""
+
+    @staticmethod
+    def forward(ctx, x, x2, weights, sht, ld, alpha, squared):
+        dev, batch = x.device, x.shape[0]
+        channels = x.numel() // (batch * sht.nlat * sht.nlon)
+        spec = torch.empty((sht.mmax, sht.lmax, ld), dtype=torch.float32, device=dev)
+        # the Fourier coefficients, and in their place the powers afterwards
+        need = lib.sfno_degree_norm_pair_workspace_bytes(batch, channels, sht.lmax)
+        nbytes = max(4 * sht.mmax * sht.nlat * ld, need)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        sums = torch.empty((2 * batch, 2), dtype=torch.float32, device=dev)
+        norms, norms2 = (torch.empty((batch,), dtype=torch.float32, device=dev) for _ in range(2))
+        s = _stream(dev)
+        check(lib.sfno_sht_analysis_pair(sht.plan(dev).handle, _ptr(x), _ptr(x2), _ptr(spec), batch * channels, _ptr(ws), nbytes, s), "sfno_sht_analysis_pair")
+        check(lib.sfno_degree_norm_pair(_ptr(spec), _ptr(weights), _ptr(sums), _ptr(norms), _ptr(norms2), batch, channels, sht.lmax, sht.mmax, alpha, squared,
+                                        _ptr(ws), nbytes, s), "sfno_degree_norm_pair")
+        ctx.save_for_backward(spec, weights, sums)
+        ctx.mark_non_differentiable(norms2)
+        ctx.sht, ctx.shape, ctx.cfg = sht, x.shape, (batch, channels, alpha, squared)
+        return norms, norms2
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g, _):
+        spec, weights, sums = ctx.saved_tensors
+        sht, (batch, channels, alpha, squared), s = ctx.sht, ctx.cfg, _stream(spec.device)
+        rows = batch * channels
+        g = g.float().contiguous()
+        gspec = torch.empty(sht.spectral_shape(rows), dtype=torch.float32, device=spec.device)
+        check(lib.sfno_degree_norm_pair_grad(_ptr(spec), _ptr(weights), _ptr(sums), _ptr(g), _ptr(gspec), batch, channels, sht.lmax, sht.mmax, alpha, squared, s),
+              "sfno_degree_norm_pair_grad")
+        gx = torch.empty(ctx.shape, dtype=torch.float32, device=spec.device)
+        plan = sht.plan(spec.device, adjoint=True)
+        ws, nbytes = sht.workspace(plan, rows, spec.device)
+        check(lib.sfno_sht_analysis_adjoint(plan.handle, _ptr(gspec), _ptr(gx), DTYPE_F32, rows, _ptr(ws), nbytes, s), "sfno_sht_analysis_adjoint")
+        return gx, None, None, None, None, None, None
+
+
 def degree_power(sht, x):
     """|c_l0|^2 + 2 sum_{m>0} |c_lm|^2 of sht(x) for every leading index: x [..., nlat, nlon] -> [..., lmax]."""
     lead = x.shape[:-2]
@@ -90,14 +130,28 @@ class GeometricH1Loss(nn.Module):
         h1_weights = torch.arange(self.sht.lmax).float()
         self.register_buffer("h1_weights", h1_weights * (h1_weights + 1))
 
+    def _direct(self, x):
+        """Whether the kernels form the norms of x directly: a batch of channels of fields, the weights as they were registered."""
+        sht, w = self.sht, self.h1_weights
+        return type(sht) is RealSHT and x.dim() >= 3 and x.numel() > 0 and x.is_cuda and isinstance(self.alpha, (int, float)) \
+            and w.shape == (sht.lmax,) and w.dtype == torch.float32 and w.device == x.device and w.is_contiguous() and not w.requires_grad
+
+    def _norm_pair(self, prd, tar):
+        """Norms of prd - tar and of tar: one pass of the transform over both where the target needs no gradient, else one after the other."""
+        if type(self)._norms is GeometricH1Loss._norms and isinstance(prd, torch.Tensor) and isinstance(tar, torch.Tensor) and self._direct(prd) \
+                and not (tar.requires_grad and torch.is_grad_enabled()) and self.sht.takes_diff(prd, tar):
+            sht = self.sht
+            ld = int(lib.sfno_sht_analysis_pair_ld(sht.plan(prd.device).handle, prd.numel() // (sht.nlat * sht.nlon)))
+            if ld:
+                return _PairNormsFn.apply(prd, tar, self.h1_weights, sht, ld, float(self.alpha), bool(self.squared))
+        return self._norms(prd, tar), self._norms(tar)
+
     def _norms(self, x, minus=None):
         """Norms of x, or of x - minus."""
         sht, w = self.sht, self.h1_weights
         if minus is not None and not (isinstance(x, torch.Tensor) and isinstance(minus, torch.Tensor)):
             x, minus = x - minus, None         # a number in place of one of the fields
-        # (a batch of channels of fields, the weights as they were registered: what the kernels form the norms of directly)
-        if type(sht) is RealSHT and x.dim() >= 3 and x.numel() > 0 and (minus is None or minus.shape == x.shape) and x.is_cuda and isinstance(self.alpha, (int, float)) \
-                and w.shape == (sht.lmax,) and w.dtype == torch.float32 and w.device == x.device and w.is_contiguous() and not w.requires_grad:
+        if self._direct(x) and (minus is None or minus.shape == x.shape):
             spec = sht.analysis(x) if minus is None else sht.analysis_diff(x, minus)
             rows = x.numel() // (sht.nlat * sht.nlon)
             return _DegreeNormFn.apply(spec, w, x.shape[0], rows // x.shape[0], float(self.alpha), bool(self.squared))
@@ -118,7 +172,8 @@ class GeometricH1Loss(nn.Module):
         return all_norms
 
     def rel(self, prd, tar, mask=None):
-        retval = self._norms(prd, tar) / self._norms(tar)
+        diff, norm = self._norm_pair(prd, tar)
+        retval = diff / norm
         if mask is not None:
             retval = retval * mask
         if self.reduction:

@@ -355,15 +355,17 @@ class RealSHT(_SHTBase):
             return _AnalysisFn.apply(x.contiguous(), self, _lib.DTYPE_BF16)
         return _AnalysisFn.apply(_as_fp32_rows(x, "grid"), self, _lib.DTYPE_F32)
 
-    def analysis_diff(self, x, x2):
-        """analysis(x - x2); float32 fields of one shape and layout without a pass for the difference."""
+    def takes_diff(self, x, x2):
+        """Whether the longitude transform reads x - x2 from the two fields: float32, of one shape and layout."""
         plain = type(x) in (torch.Tensor, torch.nn.Parameter) and type(x2) in (torch.Tensor, torch.nn.Parameter)
-        if not (plain and x.is_cuda and x.dtype == x2.dtype == torch.float32 and x.shape == x2.shape and x.device == x2.device and x.numel() > 0
+        return (plain and x.is_cuda and x.dtype == x2.dtype == torch.float32 and x.shape == x2.shape and x.device == x2.device and x.numel() > 0
                 and x.dim() >= 2 and tuple(x.shape[-2:]) == (self.nlat, self.nlon) and x.is_contiguous() and x2.is_contiguous()
                 and x.data_ptr() % 16 == 0 and x2.data_ptr() % 16 == 0 and not x.is_neg() and not x2.is_neg()
-                and lib.sfno_sht_io_dtype_supported(self.plan(x.device).handle, _lib.DTYPE_BF16)):
-            return self.analysis(x - x2)
-        return _AnalysisDiffFn.apply(x, x2, self)
+                and bool(lib.sfno_sht_io_dtype_supported(self.plan(x.device).handle, _lib.DTYPE_BF16)))
+
+    def analysis_diff(self, x, x2):
+        """analysis(x - x2); float32 fields of one shape and layout without a pass for the difference."""
+        return _AnalysisDiffFn.apply(x, x2, self) if self.takes_diff(x, x2) else self.analysis(x - x2)
 
     def _analysis(self, x, dt):
         plan = self.plan(x.device)
