@@ -501,7 +501,7 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
             cached = getattr(self, "_merge_cache", None)
             stamp = _stamp(conv_d.weight, blk.outer_skip.weight)
             if cached is None or cached[0] != stamp:
-                wd = conv_d.weight.detach().reshape(conv_d.weight.shape[0], -1).to(torch.bfloat16).float()
+                wd = conv_d.weight.detach().reshape(conv_d.weight.shape[0], -1).to(torch.bfloat16).float().contiguous()
                 ws = blk.outer_skip.weight.detach().reshape(C, -1).to(torch.bfloat16).float()
                 cached = (stamp, wd, (wd @ ws).float().contiguous())
                 self._merge_cache = cached

@@ -27,3 +27,27 @@ def test_merged_weight(lib_built, O, K, B, norm, with_bias):
     for b in range(B):
         left = w if scale is None else w * scale[b]
         assert torch.equal(packed[b], pw.packed_weight(torch.cat([left, ws], dim=1)))
+
+
+def test_transposed_decoder_weight(lib_built):
+    """A network whose decoder weight is a transpose in memory (tied to an encoder's, or taken over with assign=True) gives what its contiguous copy gives."""
+    import makani_amd as ma
+
+    print("case merged network, transposed decoder weight", flush=True)
+    torch.manual_seed(3)
+    net = ma.SphericalFourierNeuralOperatorNet(inp_shape=(48, 96), out_shape=(48, 96), inp_chans=5, out_chans=5, scale_factor=3, embed_dim=104, num_layers=3).cuda().eval()
+    x = torch.randn(2, 5, 48, 96, device="cuda")
+
+    def run():
+        with torch.inference_mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+            return net(x)
+
+    want = run()
+    assert net._merge_cache is not None
+    conv = net.decoder.fwd[0]
+    w = conv.weight.detach().reshape(104, 104)
+    conv.weight = torch.nn.Parameter(w.t().contiguous().t()[..., None, None])
+    assert not conv.weight.is_contiguous() and torch.equal(conv.weight.detach().reshape(104, 104), w)
+    assert torch.equal(run(), want)
+    net.merge_decoder = False
+    assert float((run().float() - want.float()).norm() / want.float().norm()) < 3e-2
