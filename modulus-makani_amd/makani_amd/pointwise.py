@@ -98,7 +98,7 @@ def _dense(x):
 
 
 def _vector(t):
-    """A parameter vector as the kernels read it: float32 and contiguous (None where there is none)."""
+    """A parameter as the kernels read it: float32 and contiguous (None where there is none)."""
     return t if t is None or (t.dtype == torch.float32 and t.is_contiguous()) else t.detach().float().contiguous()
 
 
@@ -153,11 +153,14 @@ def norm_mlp(x, scale, shift, w1, b1, w2, b2):
 
 def merged_weight(w, ws, scale, shift, bias, batch):
     """The layer w (scale x1 + shift) + ws x2 + bias of each sample as a convolution for conv1x1_cat: packed weights bf16 [batch, n] and biases
-    float32 [batch, O]; w, ws float32 [O, K], scale, shift float32 [batch, K] (None: 1 and 0), bias [O] or None."""
+    float32 [batch, O]; w, ws [O, K], scale, shift [batch, K] (both None: 1 and 0), bias [O] or None.  Strided operands are read as their values."""
     O, K = w.shape
+    if not w.is_cuda or ws.shape != w.shape or (scale is None) != (shift is None) or any(t is not None and t.device != w.device for t in (ws, scale, shift, bias)) \
+            or any(t is not None and t.shape != (batch, K) for t in (scale, shift)) or (bias is not None and bias.shape != (O,)):
+        raise RuntimeError(f"merged_weight: operands do not fit a weight {tuple(w.shape)} on {w.device} and {batch} samples")
     packed = torch.empty((batch, lib.sfno_pointwise_weight_elems(O, 2 * K)), dtype=torch.bfloat16, device=w.device)
     shifted = torch.empty((batch, O), dtype=torch.float32, device=w.device)
-    bias = _vector(bias)
+    w, ws, scale, shift, bias = (_vector(t) for t in (w, ws, scale, shift, bias))
     check(lib.sfno_pointwise_merge_weight(_ptr(w), _ptr(ws), _ptr(scale), _ptr(shift), _ptr(bias), _ptr(packed), _ptr(shifted), O, K, batch, _stream(w.device)),
           "sfno_pointwise_merge_weight")
     return packed, shifted
@@ -175,7 +178,12 @@ def conv1x1_cat(x1, x2, weight, bias=None, act=None, out=None, packed=None):
     O, K = (weight.shape[0], weight.shape[1:].numel()) if packed is None else weight
     if K != K1 + K2:
         raise RuntimeError(f"conv1x1_cat: inputs have {K1} + {K2} channels, weight expects {K}")
-    pw = packed_weight(weight) if packed is None else packed
+    if packed is None:
+        pw = packed_weight(weight)
+    elif packed.dtype != torch.bfloat16 or not packed.is_contiguous() or packed.device != x1.device or packed.numel() != lib.sfno_pointwise_weight_elems(O, K):
+        raise RuntimeError(f"conv1x1_cat: packed is not the stream of a weight [{O}, {K}]")
+    else:
+        pw = packed
     if out is None:
         y = torch.empty((B, O, H, W), dtype=torch.bfloat16, device=x1.device)
     else:

@@ -468,8 +468,8 @@ class SphericalFourierNeuralOperatorNet(nn.Module):
         blk = self.blocks[-1]
         if dec is None or not (isinstance(blk, FourierNeuralOperatorBlock) and blk._fusable() and getattr(blk, "fused_pointwise", True)):
             return False
-        wd = dec[0][0].weight
-        return wd.shape[0] > 96 and wd.shape[1] == blk.outer_skip.weight.shape[0]
+        wd, ws = dec[0][0].weight, blk.outer_skip.weight
+        return wd.shape[0] > 96 and wd.shape[1] == ws.shape[0] == ws.shape[1]
 
     def _tail_cat_ok(self, dec=None):
         dec = dec or _fused_chain(self.decoder.fwd)

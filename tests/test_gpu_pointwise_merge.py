@@ -51,3 +51,45 @@ def test_transposed_decoder_weight(lib_built):
     assert torch.equal(run(), want)
     net.merge_decoder = False
     assert float((run().float() - want.float()).norm() / want.float().norm()) < 3e-2
+
+
+def test_merged_operands(lib_built):
+    """Strided operands are read as their values; what does not fit is refused before a kernel reads it."""
+    from makani_amd import pointwise as pw
+
+    print("case merged operands", flush=True)
+    O, K, B = 104, 40, 3
+    gen = torch.Generator().manual_seed(9)
+    w, ws, scale, shift, bias = (torch.randn(*s, generator=gen).cuda() for s in ((O, K), (O, K), (B, K), (B, K), (O,)))
+
+    def strided(t):
+        return t.t().contiguous().t() if t.dim() == 2 else torch.stack([t, t], 1)[:, 0]
+
+    want = pw.merged_weight(w, ws, scale, shift, bias, B)
+    for i in range(5):
+        ops = [strided(t) if j == i else t for j, t in enumerate((w, ws, scale, shift, bias))]
+        assert not ops[i].is_contiguous()
+        assert all(torch.equal(a, b) for a, b in zip(pw.merged_weight(*ops, B), want))
+    assert all(torch.equal(a, b) for a, b in zip(pw.merged_weight(w.double(), ws, scale, shift, bias, B), want))
+    for bad in ((w.cpu(), ws.cpu(), None, None, None), (w, ws[:, :-1], scale, shift, bias), (w, ws[:-1], scale, shift, bias), (w, ws, scale[:, :-1], shift, bias),
+                (w, ws, scale, shift[:-1], bias), (w, ws, scale, None, bias), (w, ws, scale, shift, bias[:-1]), (w, ws, scale, shift, bias.cpu())):
+        with pytest.raises(RuntimeError):
+            pw.merged_weight(*bad, B)
+    x = torch.randn(1, K, 4, 8, generator=gen).bfloat16().cuda()
+    stream = want[0][0]
+    assert pw.conv1x1_cat(x, x, (O, 2 * K), packed=stream).shape == (1, O, 4, 8)
+    for bad in (stream[:-512], stream.float(), stream.cpu(), torch.stack([stream, stream], 1)[:, 0]):
+        with pytest.raises(RuntimeError):
+            pw.conv1x1_cat(x, x, (O, 2 * K), packed=bad)
+
+
+def test_skip_of_another_width_is_not_merged(lib_built):
+    """A last block whose skip convolution takes more channels than it gives keeps the layer-by-layer tail."""
+    import makani_amd as ma
+
+    print("case skip of another width", flush=True)
+    torch.manual_seed(4)
+    net = ma.SphericalFourierNeuralOperatorNet(inp_shape=(24, 48), out_shape=(24, 48), inp_chans=3, out_chans=3, scale_factor=1, embed_dim=104, num_layers=3).cuda().eval()
+    assert net._decoder_merge_ok()
+    net.blocks[-1].outer_skip = torch.nn.Conv2d(120, 104, 1, bias=False).cuda()
+    assert not net._decoder_merge_ok()
