@@ -286,18 +286,21 @@ int sfno_degree_norm(const float* spec, const float* weights, float* sums, float
 int sfno_degree_norm_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec,
                           int batch, int64_t channels, int lmax, int mmax, float alpha, int squared, void* stream);
 
-/* The coefficients of x - x2 and of x2 side by side, float32 [mmax][lmax][ld], ld = sfno_sht_analysis_pair_ld(p, rows), the second's rows from float ld / 2
- * on: one Legendre stage for both (the relative form of GeometricH1Loss, makani/utils/losses.py:320-345).  ld is 0, and the call refused,
- * where the plan or the size has no such path; `workspace` holds mmax * nlat * ld floats.  The norms of both, as sfno_degree_norm gives them for
- * each (sums [2 batch][2]), and the gradient with respect to the coefficients of x - x2 alone, in their own layout. */
+/* The same with respect to the field whose analysis spec is: the gradient of the coefficients, formed in the workspace (of
+ * sfno_sht_workspace_bytes), goes through the adjoint of the analysis (a plan with SFNO_DIR_FORWARD_ADJOINT); gx float32 [rows][nlat][nlon]. */
+int sfno_degree_norm_grad_field(const sfno_sht_plan* p, const float* spec, const float* weights, const float* sums, const float* gnorms, float* gx,
+                                int batch, int64_t channels, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream);
+
+/* The coefficients of x - x2 (spec) and of x2 (spec2), each as sfno_sht_analysis gives them: one Legendre stage for both (the relative form of
+ * GeometricH1Loss, makani/utils/losses.py:320-345).  `workspace` holds mmax * nlat * ld floats, ld = sfno_sht_analysis_pair_ld(p, rows): 0, and
+ * the call refused, where the plan or the size has no such path.  sfno_degree_norm_pair gives the norms of both, as sfno_degree_norm gives them for
+ * each (sums [2 batch][2], those of spec first: what the gradients above take). */
 int64_t sfno_sht_analysis_pair_ld(const sfno_sht_plan* p, int64_t rows);
-int sfno_sht_analysis_pair(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, int64_t rows, void* workspace,
-                           size_t workspace_bytes, void* stream);
+int sfno_sht_analysis_pair(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, float* spec2, int64_t rows,
+                           void* workspace, size_t workspace_bytes, void* stream);
 size_t sfno_degree_norm_pair_workspace_bytes(int batch, int64_t channels, int lmax);
-int sfno_degree_norm_pair(const float* spec, const float* weights, float* sums, float* norms, float* norms2, int batch, int64_t channels,
-                          int lmax, int mmax, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream);
-int sfno_degree_norm_pair_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec, int batch,
-                               int64_t channels, int lmax, int mmax, float alpha, int squared, void* stream);
+int sfno_degree_norm_pair(const float* spec, const float* spec2, const float* weights, float* sums, float* norms, float* norms2, int batch,
+                          int64_t channels, int lmax, int mmax, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- "diagonal" operator ------------------------------------------------------------- */
 

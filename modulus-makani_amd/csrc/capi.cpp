@@ -1,5 +1,6 @@
 // C ABI of libsfno_spectral: plan management and the enqueue-only compute entry points.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -158,7 +159,8 @@ PgemmArgs legendre_args(const sfno_sht_plan* p, const PgemmTable& t, const float
     a.lmax = p->lmax;
     a.nlat = p->nlat;
     a.mmax = p->mmax;
-    a.ld = (int)ld;
+    a.ld = a.ldo = (int)ld;
+    a.split = INT_MAX;
     a.items = t.items;
     a.chunks = t.chunks;
     a.longest = t.longest;
@@ -166,9 +168,6 @@ PgemmArgs legendre_args(const sfno_sht_plan* p, const PgemmTable& t, const float
 }
 
 bool rows_ok(int64_t rows) { return rows > 0 && sfno_spectral_ld(rows) < (int64_t)1 << 30; }
-
-// floats from the first to the second transform's columns where two share one spectral layout: whole 128-byte lines (one line for both up to 8 rows)
-int64_t pair_width(int64_t rows) { return rows <= 8 ? 16 : (2 * rows + 31) / 32 * 32; }
 
 // Planar plans (SFNO_GRID_PLANAR).  The longitude kernels are those of the spherical transforms,
 //   F: x -> s * sum_n x_n e^{-i m phi_n} (s = 2 pi / nlon)   and   C: the unnormalised complex-to-real transform,
@@ -416,22 +415,29 @@ extern "C" int sfno_sht_analysis_diff(const sfno_sht_plan* p, const float* x, co
     return analysis_launch(p, x, SFNO_DTYPE_F32, x2, w.xm, spec, rows, (hipStream_t)stream);
 }
 // Two fields through one Legendre stage: few channels leave that stage at the rate of its streams, which are read once instead of twice (2 channels of
-// 721 x 1440: 83 us each, 89 for both; relative H1 loss and gradient 355 -> 258 us), many gain the launches and the second reading of x2 (73 channels 1145 -> 1110).
+// 721 x 1440: 83 us each, 89 for both; relative H1 loss and gradient 416 -> 260 us), many gain the launches and the second reading of x2 (73 channels
+// 1221 -> 1086).  With one buffer of both kinds of coefficients, whose rows are whole lines, the 2 channels took 255, but a backward would keep both (665 instead of
+// 333 MB for 73 channels).
 extern "C" int64_t sfno_sht_analysis_pair_ld(const sfno_sht_plan* p, int64_t rows) {
     if (!p || !rows_ok(rows) || planar(p) || !(p->directions & SFNO_DIR_FORWARD) || !fft_fast_supported(p->nlon)) return 0;
     if (rows > 1 << 21) return 0;                            // (the grid of degree_power_kernel over both)
-    const int64_t ld = 2 * pair_width(rows);
+    const int64_t ld = 2 * sfno_spectral_ld(rows);           // (no wider than two buffers: whole 128-byte lines for each gained nothing)
     return ld * std::max(p->nlat, p->lmax) < (int64_t)1 << 30 ? ld : 0;          // (the Legendre kernels' 32-bit offsets)
 }
-extern "C" int sfno_sht_analysis_pair(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, int64_t rows, void* workspace,
+extern "C" int sfno_sht_analysis_pair(const sfno_sht_plan* p, const float* x, const float* x2, float* spec, float* spec2, int64_t rows, void* workspace,
                                       size_t workspace_bytes, void* stream) {
-    if (!p || !x || !x2 || !spec) return SFNO_EINVAL;
+    if (!p || !x || !x2 || !spec || !spec2) return SFNO_EINVAL;
     const int64_t ld = sfno_sht_analysis_pair_ld(p, rows);
     if (ld == 0) return SFNO_EUNSUPPORTED;
     if (!workspace || workspace_bytes < sizeof(float) * (size_t)p->mmax * p->nlat * ld) return SFNO_EWORKSPACE;
     float* xm = reinterpret_cast<float*>(workspace);
     const int rc = rfft_launch(p->fft, x, SFNO_DTYPE_F32, xm, rows, p->nlat, p->mmax, (int)ld, (hipStream_t)stream, x2, kept_orders(p, p->fwd), (int)(ld / 2));
-    return rc != SFNO_OK ? rc : legendre_fold_launch(true, p->format, legendre_args(p, p->fwd, xm, spec, ld), p->fwd.n_work, (hipStream_t)stream);
+    if (rc != SFNO_OK) return rc;
+    // (the two need not lie in one allocation: the coefficients of x - x2 outlive those of x2 where a gradient follows)
+    PgemmArgs a = legendre_args(p, p->fwd, xm, spec, ld);
+    a.Out2 = spec2;
+    a.ldo = a.split = (int)(ld / 2);
+    return legendre_fold_launch(true, p->format, a, p->fwd.n_work, (hipStream_t)stream);
 }
 extern "C" int sfno_sht_analysis(const sfno_sht_plan* p, const void* x, int x_dtype, float* spec, int64_t rows, void* workspace,
                                  size_t workspace_bytes, void* stream) {
@@ -736,7 +742,7 @@ extern "C" int sfno_dhconv(const sfno_dhconv_weights* w, const void* x, void* y,
 
 extern "C" int sfno_degree_power(const float* spec, float* power, int64_t rows, int lmax, int mmax, void* stream) {
     if (!spec || !power || !rows_ok(rows)) return SFNO_EINVAL;
-    return degree_power_launch(spec, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
+    return degree_power_launch(spec, nullptr, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
 }
 
 extern "C" size_t sfno_degree_norm_workspace_bytes(int batch, int64_t channels, int lmax) {
@@ -749,41 +755,44 @@ extern "C" int sfno_degree_norm(const float* spec, const float* weights, float* 
     if (!workspace || workspace_bytes < sfno_degree_norm_workspace_bytes(batch, channels, lmax)) return SFNO_EWORKSPACE;
     float* power = reinterpret_cast<float*>(workspace);
     const int64_t rows = batch * channels;
-    int rc = degree_power_launch(spec, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
+    int rc = degree_power_launch(spec, nullptr, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
     if (rc != SFNO_OK) return rc;
     double2* partial = reinterpret_cast<double2*>(reinterpret_cast<char*>(workspace) + align_up(sizeof(float) * (size_t)rows * lmax, 256));
-    return degree_norm_launch(power, weights, partial, reinterpret_cast<float2*>(sums), norms, nullptr, 0, batch, channels, lmax, alpha, squared, (hipStream_t)stream);
+    return degree_norm_launch(power, weights, partial, reinterpret_cast<float2*>(sums), norms, nullptr, batch, channels, lmax, alpha, squared, (hipStream_t)stream);
 }
 extern "C" int sfno_degree_norm_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec, int batch, int64_t channels,
                                      int lmax, int mmax, float alpha, int squared, void* stream) {
     if (!spec || !weights || !sums || !gnorms || !gspec || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
     return degree_norm_grad_launch(spec, weights, reinterpret_cast<const float2*>(sums), gnorms, gspec, batch, channels, lmax, mmax,
-                                   (int)sfno_spectral_ld(batch * channels), (int)sfno_spectral_ld(batch * channels), alpha, squared, (hipStream_t)stream);
+                                   (int)sfno_spectral_ld(batch * channels), alpha, squared, (hipStream_t)stream);
+}
+
+extern "C" int sfno_degree_norm_grad_field(const sfno_sht_plan* p, const float* spec, const float* weights, const float* sums, const float* gnorms, float* gx,
+                                           int batch, int64_t channels, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!p || !spec || !weights || !sums || !gnorms || !gx || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
+    if (!(p->directions & SFNO_DIR_FORWARD_ADJOINT)) return SFNO_EINVAL;
+    const Ws w = carve(p, batch * channels, workspace);
+    if (!workspace || workspace_bytes < w.bytes) return SFNO_EWORKSPACE;
+    const int rc = sfno_degree_norm_grad(spec, weights, sums, gnorms, w.spec, batch, channels, p->lmax, p->mmax, alpha, squared, stream);
+    return rc != SFNO_OK ? rc : analysis_adjoint_launch(p, w.spec, gx, SFNO_DTYPE_F32, w.xm, batch * channels, (hipStream_t)stream);
 }
 
 extern "C" size_t sfno_degree_norm_pair_workspace_bytes(int batch, int64_t channels, int lmax) {
     if (batch < 1 || batch > (1 << 30) || channels < 1 || lmax < 1 || !rows_ok(batch * channels)) return 0;
     const int64_t rows = batch * channels;
-    return align_up(sizeof(float) * (size_t)(pair_width(rows) / 2 + rows) * lmax, 256) + 2 * sizeof(double2) * (size_t)batch * degree_norm_segments(channels, lmax);
+    return align_up(2 * sizeof(float) * (size_t)rows * lmax, 256) + 2 * sizeof(double2) * (size_t)batch * degree_norm_segments(channels, lmax);
 }
-extern "C" int sfno_degree_norm_pair(const float* spec, const float* weights, float* sums, float* norms, float* norms2, int batch, int64_t channels, int lmax,
-                                     int mmax, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream) {
-    if (!spec || !weights || !sums || !norms || !norms2 || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
+extern "C" int sfno_degree_norm_pair(const float* spec, const float* spec2, const float* weights, float* sums, float* norms, float* norms2, int batch,
+                                     int64_t channels, int lmax, int mmax, float alpha, int squared, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!spec || !spec2 || !weights || !sums || !norms || !norms2 || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
     const size_t need = sfno_degree_norm_pair_workspace_bytes(batch, channels, lmax);
     if (!workspace || need == 0 || workspace_bytes < need) return SFNO_EWORKSPACE;
     float* power = reinterpret_cast<float*>(workspace);
-    const int64_t rows = batch * channels, width = pair_width(rows), all = width / 2 + rows;     // (with the slots between the two)
-    const int rc = degree_power_launch(spec, power, all, lmax, mmax, (int)(2 * width), (hipStream_t)stream);
+    const int64_t rows = batch * channels;
+    const int rc = degree_power_launch(spec, spec2, power, rows, lmax, mmax, (int)sfno_spectral_ld(rows), (hipStream_t)stream);
     if (rc != SFNO_OK) return rc;
-    double2* partial = reinterpret_cast<double2*>(reinterpret_cast<char*>(workspace) + align_up(sizeof(float) * (size_t)all * lmax, 256));
-    return degree_norm_launch(power, weights, partial, reinterpret_cast<float2*>(sums), norms, norms2, (width / 2 - rows) * lmax, batch, channels, lmax, alpha,
-                              squared, (hipStream_t)stream);
-}
-extern "C" int sfno_degree_norm_pair_grad(const float* spec, const float* weights, const float* sums, const float* gnorms, float* gspec, int batch,
-                                          int64_t channels, int lmax, int mmax, float alpha, int squared, void* stream) {
-    if (!spec || !weights || !sums || !gnorms || !gspec || batch < 1 || channels < 1 || !rows_ok(batch * channels)) return SFNO_EINVAL;
-    return degree_norm_grad_launch(spec, weights, reinterpret_cast<const float2*>(sums), gnorms, gspec, batch, channels, lmax, mmax,
-                                   (int)(2 * pair_width(batch * channels)), (int)sfno_spectral_ld(batch * channels), alpha, squared, (hipStream_t)stream);
+    double2* partial = reinterpret_cast<double2*>(reinterpret_cast<char*>(workspace) + align_up(2 * sizeof(float) * (size_t)rows * lmax, 256));
+    return degree_norm_launch(power, weights, partial, reinterpret_cast<float2*>(sums), norms, norms2, batch, channels, lmax, alpha, squared, (hipStream_t)stream);
 }
 extern "C" int sfno_degree_power_grad(const float* spec, const float* gpower, float* gspec, int64_t rows, int lmax, int mmax, void* stream) {
     if (!spec || !gpower || !gspec || !rows_ok(rows)) return SFNO_EINVAL;

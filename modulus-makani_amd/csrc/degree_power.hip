@@ -39,14 +39,15 @@ __device__ __forceinline__ DpThread dp_thread(int64_t pairs, int lmax, int mmax)
     return t;
 }
 
-// grid (lmax, ceil(rows / 2 / DP_NX)), block DP_THREADS
-__global__ __launch_bounds__(DP_THREADS) void degree_power_kernel(const float* __restrict__ spec, float* __restrict__ power, int64_t rows, int lmax,
-                                                                  int mmax, int ld) {
+// grid (lmax, ceil(rows / 2 / DP_NX), sets of rows), block DP_THREADS; the second set's powers follow the first's
+__global__ __launch_bounds__(DP_THREADS) void degree_power_kernel(const float* __restrict__ spec, const float* __restrict__ spec2, float* __restrict__ power,
+                                                                  int64_t rows, int lmax, int mmax, int ld) {
     __shared__ float2 part[DP_NY][DP_NX];
     const DpThread t = dp_thread((rows + 1) / 2, lmax, mmax);
     float2 acc = make_float2(0.f, 0.f);
+    if (blockIdx.z) power += rows * lmax;
     if (t.on) {
-        const float* c0 = spec + (int64_t)t.l * ld + 4 * t.pair;
+        const float* c0 = (blockIdx.z ? spec2 : spec) + (int64_t)t.l * ld + 4 * t.pair;
 #pragma unroll 4
         for (int m = t.ty; m <= t.mtop; m += t.ny) {
             const float4 c = *reinterpret_cast<const float4*>(c0 + (int64_t)m * lmax * ld);
@@ -89,26 +90,26 @@ struct NormGrad {
 };
 
 // gspec[m][l][2r..2r+1] = w_m * 2 * g(r, l) * c[r,l,m]  (w_0 = 1, w_m = 2 otherwise); padding columns zero
-// (spec's rows are ld_in floats, gspec's ld)  grid (lmax, ceil(ld / 4 / DP_NX)), block DP_THREADS
+// grid (lmax, ceil(ld / 4 / DP_NX)), block DP_THREADS
 template <class Grad>
 __global__ __launch_bounds__(DP_THREADS) void degree_power_grad_kernel(const float* __restrict__ spec, Grad gpower, float* __restrict__ gspec, int64_t rows,
-                                                                       int lmax, int mmax, int ld_in, int ld) {
+                                                                       int lmax, int mmax, int ld) {
     const DpThread t = dp_thread(ld / 4, lmax, mmax);
     if (!t.on) return;
     const int64_t r = 2 * t.pair;
     const bool has0 = r < rows, has1 = r + 1 < rows;
     const float g0 = has0 ? 2.f * gpower(r, t.l) : 0.f, g1 = has1 ? 2.f * gpower(r + 1, t.l) : 0.f;
-    const float* __restrict__ src = spec + (int64_t)t.l * ld_in + 4 * t.pair;
-    float* __restrict__ dst = gspec + (int64_t)t.l * ld + 4 * t.pair;
+    const int64_t at = (int64_t)t.l * ld + 4 * t.pair;
 #pragma unroll 4
     for (int m = t.ty; m <= t.mtop; m += t.ny) {
-        float4 c = *reinterpret_cast<const float4*>(src + (int64_t)m * lmax * ld_in);
+        const int64_t i = at + (int64_t)m * lmax * ld;
+        float4 c = *reinterpret_cast<const float4*>(spec + i);
         const float w = m == 0 ? 1.f : 2.f;
         c.x = has0 ? w * g0 * c.x : 0.f;           // (a padding column may hold anything)
         c.y = has0 ? w * g0 * c.y : 0.f;
         c.z = has1 ? w * g1 * c.z : 0.f;
         c.w = has1 ? w * g1 * c.w : 0.f;
-        *reinterpret_cast<float4*>(dst + (int64_t)m * lmax * ld) = c;
+        *reinterpret_cast<float4*>(gspec + i) = c;
     }
 }
 
@@ -122,7 +123,7 @@ __device__ __forceinline__ void norm_of(double a, double h, float alpha, int squ
     *norm = squared ? alpha * s.x + (1.f - alpha) * s.y : alpha * sqrtf(s.x) + (1.f - alpha) * sqrtf(s.y);
 }
 
-// norms of one batch, or of two whose powers lie `gap` values apart
+// norms of one batch, or of two
 struct NormOut {
     float *first, *second;
     int batch;
@@ -130,11 +131,11 @@ struct NormOut {
 };
 
 __global__ __launch_bounds__(DN_THREADS) void degree_norm_kernel(const float* __restrict__ power, const float* __restrict__ weights,
-                                                                 double2* __restrict__ partial, float2* __restrict__ sums, NormOut norms, int64_t gap, int64_t n,
+                                                                 double2* __restrict__ partial, float2* __restrict__ sums, NormOut norms, int64_t n,
                                                                  int lmax, float alpha, int squared) {
     const int b = blockIdx.x, nseg = gridDim.y;
     const int64_t from = n * blockIdx.y / nseg, to = n * (blockIdx.y + 1) / nseg;
-    const float* __restrict__ p = power + (int64_t)b * n + (b < norms.batch ? 0 : gap);
+    const float* __restrict__ p = power + (int64_t)b * n;
     double a = 0.0, h = 0.0;
     int l = (int)((from + threadIdx.x) % lmax);
     const int step = DN_THREADS % lmax;
@@ -183,10 +184,10 @@ __global__ __launch_bounds__(64) void degree_norm_finish_kernel(const double2* _
 }  // namespace
 
 // (sfno_spectral_ld makes ld a multiple of 4: whole 16-byte pieces)
-int degree_power_launch(const float* spec, float* power, int64_t rows, int lmax, int mmax, int ld, hipStream_t s) {
+int degree_power_launch(const float* spec, const float* spec2, float* power, int64_t rows, int lmax, int mmax, int ld, hipStream_t s) {
     const int64_t blocks = ((rows + 1) / 2 + DP_NX - 1) / DP_NX;
     if (rows < 1 || lmax < 1 || mmax < 1 || ld < 2 * rows || ld % 4 != 0 || blocks > 65535) return SFNO_EINVAL;
-    hipLaunchKernelGGL(degree_power_kernel, dim3(lmax, (unsigned)blocks), dim3(DP_THREADS), 0, s, spec, power, rows, lmax, mmax, ld);
+    hipLaunchKernelGGL(degree_power_kernel, dim3(lmax, (unsigned)blocks, spec2 ? 2 : 1), dim3(DP_THREADS), 0, s, spec, spec2, power, rows, lmax, mmax, ld);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
@@ -194,30 +195,30 @@ int degree_power_grad_launch(const float* spec, const float* gpower, float* gspe
     const int64_t blocks = (ld / 4 + DP_NX - 1) / DP_NX;
     if (rows < 1 || lmax < 1 || mmax < 1 || ld < 2 * rows || ld % 4 != 0 || blocks > 65535) return SFNO_EINVAL;
     hipLaunchKernelGGL(degree_power_grad_kernel<PowerGrad>, dim3(lmax, (unsigned)blocks), dim3(DP_THREADS), 0, s, spec, PowerGrad{gpower, lmax}, gspec, rows, lmax,
-                       mmax, ld, ld);
+                       mmax, ld);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
 // some 8 thousand values per workgroup; by an example's size alone, so that it gives the same norm alone and in a batch
 int degree_norm_segments(int64_t channels, int lmax) { return (int)std::max<int64_t>(1, std::min<int64_t>(channels * lmax / 8192, 64)); }
 
-int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, float* norms2, int64_t gap, int batch,
-                       int64_t channels, int lmax, float alpha, int squared, hipStream_t s) {
+int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, float* norms2, int batch, int64_t channels,
+                       int lmax, float alpha, int squared, hipStream_t s) {
     if (batch < 1 || channels < 1 || lmax < 1) return SFNO_EINVAL;
     const int nseg = degree_norm_segments(channels, lmax);
     const NormOut out{norms, norms2, batch};
     const unsigned n = norms2 ? 2u * batch : batch;
-    hipLaunchKernelGGL(degree_norm_kernel, dim3(n, nseg), dim3(DN_THREADS), 0, s, power, weights, partial, sums, out, gap, channels * lmax, lmax, alpha, squared);
+    hipLaunchKernelGGL(degree_norm_kernel, dim3(n, nseg), dim3(DN_THREADS), 0, s, power, weights, partial, sums, out, channels * lmax, lmax, alpha, squared);
     if (nseg > 1) hipLaunchKernelGGL(degree_norm_finish_kernel, dim3(n), dim3(64), 0, s, partial, sums, out, nseg, alpha, squared);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
 int degree_norm_grad_launch(const float* spec, const float* weights, const float2* sums, const float* gnorms, float* gspec, int batch, int64_t channels, int lmax,
-                            int mmax, int ld_in, int ld, float alpha, int squared, hipStream_t s) {
+                            int mmax, int ld, float alpha, int squared, hipStream_t s) {
     const int64_t rows = batch * channels, blocks = (ld / 4 + DP_NX - 1) / DP_NX;
-    if (batch < 1 || channels < 1 || lmax < 1 || mmax < 1 || ld < 2 * rows || ld % 4 != 0 || ld_in < ld || ld_in % 4 != 0 || blocks > 65535) return SFNO_EINVAL;
+    if (batch < 1 || channels < 1 || lmax < 1 || mmax < 1 || ld < 2 * rows || ld % 4 != 0 || blocks > 65535) return SFNO_EINVAL;
     hipLaunchKernelGGL(degree_power_grad_kernel<NormGrad>, dim3(lmax, (unsigned)blocks), dim3(DP_THREADS), 0, s, spec,
-                       NormGrad{weights, gnorms, sums, channels, alpha, squared}, gspec, rows, lmax, mmax, ld_in, ld);
+                       NormGrad{weights, gnorms, sums, channels, alpha, squared}, gspec, rows, lmax, mmax, ld);
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 

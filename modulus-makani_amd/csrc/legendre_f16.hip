@@ -397,13 +397,14 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
         }
     } else if (ANALYSIS) {
         if (!active) return;
-        float* out = a.Out + (int64_t)m * lmax * ld;
-        if (PG_ROWS * (rb + 1) <= nrows && n0 + TN <= ld) {
+        const int ldo = a.ldo, split = a.split;
+        const int second = n0 >= split ? split : 0;             // (a tile of columns may also have both, see the checks below)
+        if (PG_ROWS * (rb + 1) <= nrows && n0 + TN - second <= ldo && (second || n0 + TN <= split)) {
             // no row or column of my tile needs a check: one address per row, the tiles at constant offsets from it
-            float* o = out + (int64_t)(m + par + 2 * (PG_ROWS * rb + 4 * kg)) * ld + n0 + cl;
+            float* o = (second ? a.Out2 : a.Out) + (int64_t)m * lmax * ldo + (int64_t)(m + par + 2 * (PG_ROWS * rb + 4 * kg)) * ldo + (n0 - second) + cl;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                float* orow = o + (int64_t)(2 * (8 * (v >> 2) + (v & 3))) * ld;
+                float* orow = o + (int64_t)(2 * (8 * (v >> 2) + (v & 3))) * ldo;
 #pragma unroll
                 for (int t = 0; t < NT; ++t) orow[32 * t] = acc[t][v];
             }
@@ -411,11 +412,13 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
+            int n = n0 + 32 * t + cl;
+            float* out = (n >= split ? a.Out2 : a.Out) + (int64_t)m * lmax * ldo;
+            n -= n >= split ? split : 0;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int r = PG_ROWS * rb + 8 * (v >> 2) + 4 * kg + (v & 3);
-                const int n = n0 + 32 * t + cl;
-                if (r < nrows && n < ld) out[(int64_t)(m + par + 2 * r) * ld + n] = acc[t][v];
+                if (r < nrows && n < ldo) out[(int64_t)(m + par + 2 * r) * ldo + n] = acc[t][v];
             }
         }
     } else {

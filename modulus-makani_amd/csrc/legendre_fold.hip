@@ -262,14 +262,16 @@ __global__ __launch_bounds__(256, lf_occupancy(NT, MODE)) void legendre_fold_ker
     // D layout of the 32x32 MFMA: register v of lane j holds D[8*(v/4) + 4*(j/32) + v%4][j%32].
     if (ANALYSIS) {
         if (!active) return;
-        float* out = a.Out + (int64_t)m * lmax * ld;
+        const int ldo = a.ldo, split = a.split;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
+            int n = n0 + 32 * t + cl;
+            float* out = (n >= split ? a.Out2 : a.Out) + (int64_t)m * lmax * ldo;
+            n -= n >= split ? split : 0;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int r = PG_ROWS * rb + 8 * (v >> 2) + 4 * kh + (v & 3);
-                const int n = n0 + 32 * t + cl;
-                if (r < nrows && n < ld) out[(int64_t)(m + par + 2 * r) * ld + n] = acc[t][v];
+                if (r < nrows && n < ldo) out[(int64_t)(m + par + 2 * r) * ldo + n] = acc[t][v];
             }
         }
     } else {

@@ -51,6 +51,10 @@ struct PgemmArgs {
     const float* rinv;             // two-part fp16 format: row factors, [entry position - 2 mmax][32]
     int lmax, nlat, mmax;          // Legendre modes
     int ld;                        // channel leading dimension of Q and Out (Legendre modes)
+    // analysis: rows of Out have ldo <= ld floats.  Where two transforms share the columns, those from `split` on are the second one's and go to Out2, of
+    // rows like Out's (one transform: ldo = ld, no column reaches split)
+    float* Out2;
+    int ldo, split;
     int drop;                      // synthesis: rows of orders that do not matter there (PgemmTable::d_kept) are not written
     int64_t items, chunks;         // as in PgemmTable
     int longest;
@@ -252,16 +256,17 @@ int irfft_launch(const FftPlan& p, const float* xm, void* x, int x_dtype, int64_
 int latfft_launch(const FftPlan& p, bool inverse, const float* in, float* out, int mmax, int lmax, int ld, const float* mscale, hipStream_t s);
 
 // ---- per-degree power of spectral-layout coefficients and its gradient (degree_power.hip) ------------
-int degree_power_launch(const float* spec, float* power, int64_t rows, int lmax, int mmax, int ld, hipStream_t s);
+// spec2 not null: of a second set of rows too, behind the first one's powers
+int degree_power_launch(const float* spec, const float* spec2, float* power, int64_t rows, int lmax, int mmax, int ld, hipStream_t s);
 // sums over the channels and degrees of `channels` rows per example: sums[b] = (sum p, sum weights[l] p), norms[b] = alpha a + (1 - alpha) h of
 // them or of their square roots; partial: double2 [batch][degree_norm_segments] of workspace.  norms2 not null: of a second batch too, whose powers follow the
-// first's after `gap` values (sums and partial for both)
+// first's (sums and partial for both)
 int degree_norm_segments(int64_t channels, int lmax);
-int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, float* norms2, int64_t gap, int batch,
-                       int64_t channels, int lmax, float alpha, int squared, hipStream_t s);
-// gradient of the above with respect to the coefficients (rows of ld_in floats, the gradient's of ld)
+int degree_norm_launch(const float* power, const float* weights, double2* partial, float2* sums, float* norms, float* norms2, int batch, int64_t channels,
+                       int lmax, float alpha, int squared, hipStream_t s);
+// gradient of the above with respect to the coefficients
 int degree_norm_grad_launch(const float* spec, const float* weights, const float2* sums, const float* gnorms, float* gspec, int batch, int64_t channels, int lmax,
-                            int mmax, int ld_in, int ld, float alpha, int squared, hipStream_t s);
+                            int mmax, int ld, float alpha, int squared, hipStream_t s);
 int degree_power_grad_launch(const float* spec, const float* gpower, float* gspec, int64_t rows, int lmax, int mmax, int ld, hipStream_t s);
 
 // ---- file-scope scratch array of sfno_sht_forward_static (static_scratch.hip) ----------------

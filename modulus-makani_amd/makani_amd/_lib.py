@@ -94,10 +94,10 @@ def _load():
         "sfno_degree_norm_workspace_bytes": (sz, [i32, i64, i32]),
         "sfno_degree_norm": (i32, [vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp, sz, vp]),
         "sfno_sht_analysis_pair_ld": (i64, [vp, i64]),
-        "sfno_sht_analysis_pair": (i32, [vp, vp, vp, vp, i64, vp, sz, vp]),
+        "sfno_sht_analysis_pair": (i32, [vp, vp, vp, vp, vp, i64, vp, sz, vp]),
         "sfno_degree_norm_pair_workspace_bytes": (sz, [i32, i64, i32]),
-        "sfno_degree_norm_pair": (i32, [vp, vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp, sz, vp]),
-        "sfno_degree_norm_pair_grad": (i32, [vp, vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp]),
+        "sfno_degree_norm_pair": (i32, [vp, vp, vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp, sz, vp]),
+        "sfno_degree_norm_grad_field": (i32, [vp, vp, vp, vp, vp, vp, i32, i64, c.c_float, i32, vp, sz, vp]),
         "sfno_degree_norm_grad": (i32, [vp, vp, vp, vp, vp, i32, i64, i32, i32, c.c_float, i32, vp]),
         "sfno_diagonal_contract": (i32, [vp, vp, vp, i32, i32, i32, i64, i32, vp]),
         "sfno_diagonal_weight_grad": (i32, [vp, vp, vp, i32, i32, i32, i64, vp]),

@@ -9,7 +9,7 @@ import torch
 from torch import nn
 from torch.autograd.function import once_differentiable
 
-from ._lib import DTYPE_F32, lib, check
+from ._lib import lib, check
 from .sht import RealSHT, _ptr, _stream_ptr as _stream
 
 
@@ -71,7 +71,8 @@ class _PairNormsFn(torch.autograd.Function):
     def forward(ctx, x, x2, weights, sht, ld, alpha, squared):
         dev, batch = x.device, x.shape[0]
         channels = x.numel() // (batch * sht.nlat * sht.nlon)
-        spec = torch.empty((sht.mmax, sht.lmax, ld), dtype=torch.float32, device=dev)
+        # (two tensors: the backward keeps the first alone)
+        spec, spec2 = (torch.empty(sht.spectral_shape(batch * channels), dtype=torch.float32, device=dev) for _ in range(2))
         # the Fourier coefficients, and in their place the powers afterwards
         need = lib.sfno_degree_norm_pair_workspace_bytes(batch, channels, sht.lmax)
         nbytes = max(4 * sht.mmax * sht.nlat * ld, need)
@@ -79,9 +80,10 @@ class _PairNormsFn(torch.autograd.Function):
         sums = torch.empty((2 * batch, 2), dtype=torch.float32, device=dev)
         norms, norms2 = (torch.empty((batch,), dtype=torch.float32, device=dev) for _ in range(2))
         s = _stream(dev)
-        check(lib.sfno_sht_analysis_pair(sht.plan(dev).handle, _ptr(x), _ptr(x2), _ptr(spec), batch * channels, _ptr(ws), nbytes, s), "sfno_sht_analysis_pair")
-        check(lib.sfno_degree_norm_pair(_ptr(spec), _ptr(weights), _ptr(sums), _ptr(norms), _ptr(norms2), batch, channels, sht.lmax, sht.mmax, alpha, squared,
-                                        _ptr(ws), nbytes, s), "sfno_degree_norm_pair")
+        check(lib.sfno_sht_analysis_pair(sht.plan(dev).handle, _ptr(x), _ptr(x2), _ptr(spec), _ptr(spec2), batch * channels, _ptr(ws), nbytes, s),
+              "sfno_sht_analysis_pair")
+        check(lib.sfno_degree_norm_pair(_ptr(spec), _ptr(spec2), _ptr(weights), _ptr(sums), _ptr(norms), _ptr(norms2), batch, channels, sht.lmax, sht.mmax, alpha,
+                                        squared, _ptr(ws), nbytes, s), "sfno_degree_norm_pair")
         ctx.save_for_backward(spec, weights, sums)
         ctx.mark_non_differentiable(norms2)
         ctx.sht, ctx.shape, ctx.cfg = sht, x.shape, (batch, channels, alpha, squared)
@@ -91,16 +93,13 @@ class _PairNormsFn(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, g, _):
         spec, weights, sums = ctx.saved_tensors
-        sht, (batch, channels, alpha, squared), s = ctx.sht, ctx.cfg, _stream(spec.device)
-        rows = batch * channels
+        sht, (batch, channels, alpha, squared) = ctx.sht, ctx.cfg
         g = g.float().contiguous()
-        gspec = torch.empty(sht.spectral_shape(rows), dtype=torch.float32, device=spec.device)
-        check(lib.sfno_degree_norm_pair_grad(_ptr(spec), _ptr(weights), _ptr(sums), _ptr(g), _ptr(gspec), batch, channels, sht.lmax, sht.mmax, alpha, squared, s),
-              "sfno_degree_norm_pair_grad")
         gx = torch.empty(ctx.shape, dtype=torch.float32, device=spec.device)
         plan = sht.plan(spec.device, adjoint=True)
-        ws, nbytes = sht.workspace(plan, rows, spec.device)
-        check(lib.sfno_sht_analysis_adjoint(plan.handle, _ptr(gspec), _ptr(gx), DTYPE_F32, rows, _ptr(ws), nbytes, s), "sfno_sht_analysis_adjoint")
+        ws, nbytes = sht.workspace(plan, batch * channels, spec.device)
+        check(lib.sfno_degree_norm_grad_field(plan.handle, _ptr(spec), _ptr(weights), _ptr(sums), _ptr(g), _ptr(gx), batch, channels, alpha, squared, _ptr(ws), nbytes,
+                                              _stream(spec.device)), "sfno_degree_norm_grad_field")
         return gx, None, None, None, None, None, None
 
 
