@@ -99,10 +99,10 @@ __device__ __forceinline__ float gelu_grad(float x, float e) {
 __device__ __forceinline__ float gelu_grad(float x) { return gelu_grad(x, phi_neg(x)); }
 
 // Training applies both to numbers that were rounded to bf16.  From 2^-11 to the clamp at 6.5 these are 1728 magnitudes, and the convolutions in
-// front of and behind a GELU look phi_neg up in LDS: the same bits with 8 vector instructions a value where the GELU takes 18, and 17 where its derivative
-// takes 27.  The vector instructions of the epilogue find no matrix instruction to hide behind and bounded both kernels; now memory nearly does, as it does
-// the epilogue with an addend.  721 x 1440: derivative 384 -> 768 channels 1258 -> 1136 us, 384 -> 384 645 -> 588, 73 -> 384 425 -> 398; GELU 384 -> 768 1215 -> 1141,
-// 384 -> 384 606 -> 570, but 73 -> 384 446 -> 463 (at 240 x 480 43.8 -> 41.3).
+// front of and behind a GELU look phi_neg up in LDS: the same bits (but for arguments below 2^-120, whose half may round the other way) with 8 vector
+// instructions a value where the GELU takes 18, and 17 where its derivative takes 27.  The vector instructions of the epilogue find no matrix instruction to
+// hide behind and bounded both kernels; now memory nearly does, as it does the epilogue with an addend.  721 x 1440: derivative 384 -> 768 channels
+// 1258 -> 1136 us, 384 -> 384 645 -> 588, 73 -> 384 425 -> 398; GELU 384 -> 768 1215 -> 1141, 384 -> 384 606 -> 570.  See gelu_table_pays for the others.
 constexpr int GT_HI = 0x40d0, GT_N = 1728, GT_LO = GT_HI - GT_N + 1;             // 6.5 as bf16
 constexpr int GT_BYTES = 4 * GT_N;
 // phi_neg of a bf16 number's magnitude, of the nearest one in the table where it is smaller
@@ -117,7 +117,8 @@ __device__ __forceinline__ float gelu_from(float x, int magnitude, float entry) 
 
 // Epilogues: exact GELU on the output and / or "+ scale * addend + shift"; for training GELU_PRE (the output before the GELU is stored as
 // well, to a.Z, and activated as stored) and GELU_BWD (the output times the GELU's derivative at `addend`)
-enum { PW_PLAIN = 0, PW_GELU = 1, PW_ADD = 2, PW_GELU_PRE = 4, PW_GELU_BWD = 8 };
+// (GELU_PRE | FORMULA: without the table of the direct-to-LDS kernel)
+enum { PW_PLAIN = 0, PW_GELU = 1, PW_ADD = 2, PW_GELU_PRE = 4, PW_GELU_BWD = 8, PW_FORMULA = 16 };
 
 // NW = wavefronts per workgroup, side by side along the pixels, 64 pixels each: 8, or 2 where that leaves CUs idle
 template <int NW, int EPI>
@@ -400,7 +401,7 @@ template <int MT, int EPI>
 __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_kernel(PointwiseArgs a) {
     using DM = DmGeo<MT>;
     constexpr bool GELU = EPI & (PW_GELU | PW_GELU_PRE), AFF = EPI & PW_ADD, ADD = EPI & (PW_ADD | PW_GELU_BWD);
-    constexpr bool TAB = EPI & (PW_GELU_PRE | PW_GELU_BWD);
+    constexpr bool TAB = (EPI & (PW_GELU_PRE | PW_GELU_BWD)) && !(EPI & PW_FORMULA);
     static_assert(DM::WG_PER_CU * (DM::LDS + GT_BYTES) <= 160 * 1024, "resident workgroups");
     __shared__ __align__(16) unsigned char lds[DM::LDS + (TAB ? GT_BYTES : 0)];
     // tiles of this XCD, row block fastest: q -> (row block q % n_oblk, strip (q / n_oblk) * 8 + xcd); the workgroups of the
@@ -594,14 +595,17 @@ __global__ __launch_bounds__(512, 2 * DmGeo<MT>::WG_PER_CU) void pw_gemm_dma_ker
 #pragma unroll
                         for (int pp = 0; pp < 2; ++pp) {
                             z[pp] = bf16_pair(y[2 * pp], y[2 * pp + 1]);
-                            e[2 * pp] = gelu_look_up(lds + DM::LDS, z[pp] & 0x7fffu);
-                            e[2 * pp + 1] = gelu_look_up(lds + DM::LDS, z[pp] >> 16 & 0x7fffu);
+                            if constexpr (TAB) {
+                                e[2 * pp] = gelu_look_up(lds + DM::LDS, z[pp] & 0x7fffu);
+                                e[2 * pp + 1] = gelu_look_up(lds + DM::LDS, z[pp] >> 16 & 0x7fffu);
+                            }
                         }
                         *reinterpret_cast<u32x2*>(a.Z + lane_off + (int64_t)row_of(mt, v) * a.P) = z;
 #pragma unroll
                         for (int pp = 0; pp < 2; ++pp) {
-                            y[2 * pp] = gelu_from(__uint_as_float(z[pp] << 16), z[pp] & 0x7fffu, e[2 * pp]);
-                            y[2 * pp + 1] = gelu_from(__uint_as_float(z[pp] & 0xffff0000u), z[pp] >> 16 & 0x7fffu, e[2 * pp + 1]);
+                            const float u = __uint_as_float(z[pp] << 16), w = __uint_as_float(z[pp] & 0xffff0000u);
+                            y[2 * pp] = TAB ? gelu_from(u, z[pp] & 0x7fffu, e[2 * pp]) : gelu_train(u);
+                            y[2 * pp + 1] = TAB ? gelu_from(w, z[pp] >> 16 & 0x7fffu, e[2 * pp + 1]) : gelu_train(w);
                         }
                     } else if constexpr (GELU) {
 #pragma unroll
@@ -1124,11 +1128,32 @@ int pointwise_merge_launch(const float* w, const float* ws, const float* scale, 
     return hipGetLastError() == hipSuccess ? SFNO_OK : SFNO_EHIP;
 }
 
+// Whether the GELU of a training convolution takes Phi from the table (its derivative always does).  Not where the formula's instructions already hide behind the
+// stores, the faster epilogue is then up to 10 % the slower one: few chunks of 32 input channels and outputs far beyond the memory-side cache
+// (256 MB).  Rows that begin inside a 128-byte line are stored longer, so more chunks hide there; rows of the tile past the last channel and a second
+// block of rows cost instructions and no stores.  1200 shapes (16 to 768 channels, 2048 pixels to 721 x 1440), table against formula in us: 721 x 1440, 73 -> 384 channels
+// 461 / 444, 104 -> 384 472 / 440, 144 -> 384 475 / 457, 208 -> 384 478 / 494, 56 -> 448 513 / 467, 73 -> 448 471 / 495; 720 x 1440, 24 -> 512 422 / 417, 73 -> 384
+// 345 / 345, 73 -> 512 444 / 488; 361 x 720, 73 -> 384 139 / 141.  Of 150 shapes that take the formula it is 1.3 % faster on average, 3 % slower at worst; of the others
+// the table is 5 % faster on average and loses up to 5 % to it (more with less than 32 input channels).
+static bool gelu_table_pays(const PointwiseArgs& a, int mt) {
+    if (mt == 1 || 4 * (int64_t)a.B * a.O * a.P < (int64_t)512 << 20) return true;
+    const int chunks = (a.K + 31) / 32;
+    if (a.P % 64 == 0) return chunks > 1 || a.O < 256;
+    return chunks > 7.0 * a.O / (128 * mt * a.n_oblk) - (mt == 3 ? 1.6 : 2.6) - (a.n_oblk > 1 ? 1.0 : 0.0);
+}
+
 template <int MT>
 static void dma_go(const PointwiseArgs& a, int64_t blocks, int epi, hipStream_t s) {
     const dim3 grid((unsigned)std::min<int64_t>(blocks, std::max(8, DmGeo<MT>::WG_PER_CU * (device_cus() / 8 * 8))));
     switch (epi) {
-        case PW_GELU_PRE: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU_PRE>), grid, dim3(512), 0, s, a); break;
+        case PW_GELU_PRE:
+            if constexpr (MT > 1)
+                if (!gelu_table_pays(a, MT)) {
+                    hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU_PRE | PW_FORMULA>), grid, dim3(512), 0, s, a);
+                    break;
+                }
+            hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU_PRE>), grid, dim3(512), 0, s, a);
+            break;
         case PW_GELU_BWD: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU_BWD>), grid, dim3(512), 0, s, a); break;
         case PW_GELU | PW_ADD: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU | PW_ADD>), grid, dim3(512), 0, s, a); break;
         case PW_GELU: hipLaunchKernelGGL((pw_gemm_dma_kernel<MT, PW_GELU>), grid, dim3(512), 0, s, a); break;

@@ -39,3 +39,27 @@ def test_table_is_the_formula(lib_built, channels):
     assert torch.equal(torch.isnan(g0), torch.isnan(g1))
     ok = ~torch.isnan(g0)
     assert torch.equal(g0[ok].view(torch.int16), g1[ok].view(torch.int16))
+
+
+@pytest.mark.parametrize("K,O,P", [(24, 160, 840008), (64, 200, 671112), (73, 256, 524296), (40, 320, 420008), (24, 384, 349568)])
+def test_long_layers_take_the_formula(lib_built, K, O, P):
+    """Few input channels in front of outputs far beyond the caches: the formula in place of the table, the same activations as the shorter pieces give."""
+    from makani_amd import pointwise as pw
+    from makani_amd._lib import check, lib
+
+    print(f"case gelu formula {K} -> {O}, {P} pixels", flush=True)
+    assert 4 * O * P >= 512 << 20
+    gen = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(K, P, device="cuda", generator=gen).bfloat16()
+    w, bias = torch.randn(O, K, device="cuda", generator=gen) / K**0.5, torch.randn(O, device="cuda", generator=gen)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+
+    def conv(x):
+        y, z = (torch.empty(O, x.shape[1], dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        check(lib.sfno_pointwise_conv_gelu(ptr(x), ptr(pw.packed_weight(w)), ptr(bias), ptr(y), ptr(z), 1, K, O, x.shape[1], pw._stream(x.device)), "forward")
+        return y, z
+
+    y, z = conv(x)
+    for p in (0, P // 16 * 8, P - 4104):
+        ys, zs = conv(x[:, p:p + 4104].contiguous())
+        assert torch.equal(y[:, p:p + 4104], ys) and torch.equal(z[:, p:p + 4104], zs)
