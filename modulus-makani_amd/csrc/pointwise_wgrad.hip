@@ -128,13 +128,14 @@ static WgradShape wgrad_shape(int O, int K, int B, int64_t P) {
     // channels asks for half the rows, and the way to the first chunk and the stores of a short share are spread over twice the workgroups.
     // 1000 shapes (2 to 768 channels, 1024 to 1.5 million pixels), times against the larger tiles: 0.66 where a tile takes the place of one, 0.74 to 0.95
     // for three in place of two, for two in place of one 0.75 with shares of less than 24 chunks and up to 1.19 with longer ones (but 0.7 with at most 64
-    // output channels), for four 0.8 with less than 6 chunks and 1.2 with longer ones.  20 % faster on average, 10 % slower at worst.
+    // output channels), for four 0.65 to 0.85 with shares of four chunks while all workgroups are resident at once, 0.97 to 1.07 past that and 1.2 with longer
+    // shares.  20 % faster on average; of 1600 shapes two are more than 2 % slower (4 %: 250000 pixels and more, two in place of one).
     // 128 channels of 2 x 90 x 180 18.4 -> 12.6 us, 96 of 4 x 128 x 247 51 -> 36.
     const WgradShape small = wgrad_shape(O, K, B, P, WG_SMALL);
     const int n = small.n_ot * small.n_kt, n2 = square.n_ot * square.n_kt;
     const int64_t share = (square.chunks + square.splits - 1) / square.splits;
     const bool few = 2 * n <= 3 * n2;
-    if (best.kind == WG_SQUARE ? few || (n <= 2 * n2 && (share < 24 || O <= 64)) || (share < 6 && n2 <= 6) : few && share < 32) return small;
+    if (best.kind == WG_SQUARE ? few || (n <= 2 * n2 && (share < 24 || O <= 64)) || (share < 6 && n2 <= 6 && n * small.splits <= 2 * device_cus()) : few && share < 32) return small;
     return best;
 }
 

@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 # (batch, in, out, pixels): shares of 256 x 256 tiles hold max(4, chunks / 256) chunks of 64 pixels
 CASES = [(1, 127, 128, 8), (1, 128, 128, 64), (2, 128, 127, 264), (3, 129, 128, 1000), (1, 128, 129, 4096), (2, 255, 256, 3048), (1, 257, 128, 9000), (1, 384, 128, 9000),
-         (5, 256, 64, 2008), (1, 64, 8, 70000), (1, 200, 60, 420000), (1, 130, 100, 420000), (1, 60, 200, 300000), (1, 700, 130, 1200), (2, 40, 300, 504)]
+         (1, 200, 192, 32768), (1, 200, 192, 33800), (5, 256, 64, 2008), (1, 64, 8, 70000), (1, 200, 60, 420000), (1, 130, 100, 420000), (1, 60, 200, 300000), (1, 700, 130, 1200), (2, 40, 300, 504)]
 
 
 @pytest.mark.parametrize("B,K,O,P", CASES)
