@@ -289,10 +289,17 @@ int dhconv_wgrad_launch(const DhconvWgradArgs& a, hipStream_t s) {
     const int tile = narrow ? 32 : 64;
     const int ni = (a.I + tile - 1) / tile, no = (a.O + tile - 1) / tile;
     // Two units per group: as many queues as XCDs where there are few groups (384 x 384 channels, 45 degrees, eight samples 158 -> 107 us; 190 x 190 and 60
-    // degrees, two samples, 28 -> 22.5), more shares than 32 CUs can take at a time where there are many (36 tiles of 64 x 64 of a group; 240 degrees
-    // with 2 samples 425 -> 411, 241 with one 387 -> 353; 232 with one lose 2 %).  Small tiles whose queues are even keep one unit, whose tiles share all
-    // rows (120 degrees 75.5 against 77).
-    const int split = ni < 2 ? 1 : !narrow || 10 * fullest_queue(a, ni, no, 1) > 11 * fullest_queue(a, ni, no, 2) ? 2 : 1;
+    // degrees, two samples, 28 -> 22.5), more shares than an XCD's 32 CUs can take at a time where there are many (36 tiles of 64 x 64 of a group: 240 degrees
+    // with 2 samples 425 -> 411, 241 with one 387 -> 353).  One unit, whose tiles share all rows, where they find a place at once: large tiles of 250 shapes, time of
+    // two units against one 0.95 for 30 and more of them (the worst 1.03), 0.97 for 5 x 5 with several samples and 1.02 with one, 1.02 for 16 to 28 of them (up to
+    // 1.12: 367 -> 248 channels, 204 degrees) unless one XCD's queue is the longer by more than a fifteenth (0.79 to 1).  Small tiles, 770 shapes: 1.01 with less than twelve
+    // of them, where the queues are even 1.02 (120 degrees 75.5 against 77), else 0.91 on average, 0.54 at best; 68 lose more than 3 %, one sample of 40 to 64
+    // degrees up to 15, which no line drawn by queues, tiles and samples tells from those that gain 25.
+    int split = 1;
+    if (ni >= 2) {
+        const int64_t n = (int64_t)ni * no, one = fullest_queue(a, ni, no, 1), two = fullest_queue(a, ni, no, 2);
+        if (narrow ? n >= 12 && 10 * one > 11 * two : n >= 30 || (n >= 25 && ni >= 5 && no >= 5 && a.B > 1) || 14 * one > 15 * two) split = 2;
+    }
     const int64_t blocks = groups * ni * no;
     if (blocks > 0x7fffffffLL) return SFNO_EUNSUPPORTED;
     const dim3 grid((unsigned)blocks), block(64 * WG_DEG);
