@@ -395,12 +395,14 @@ static int analysis_with(const sfno_sht_plan* p, const PgemmTable& table, const 
 }
 
 int sfno::analysis_launch(const sfno_sht_plan* p, const void* x, int x_dtype, const float* x2, float* xm, float* spec, int64_t rows, hipStream_t s) {
+    if (!rows_ok(rows)) return SFNO_EINVAL;
     if (!planar(p)) return analysis_with(p, p->fwd, x, x_dtype, x2, xm, spec, rows, s);
     const int rc = rfft_launch(p->fft, x, x_dtype, xm, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), s, x2);
     return rc != SFNO_OK ? rc : planar_stage(p, MS_FWD, false, xm, spec, rows, s);
 }
 
 int sfno::synthesis_launch(const sfno_sht_plan* p, const float* spec, float* xm, void* x, int x_dtype, float2* lat_stats, int64_t rows, hipStream_t s) {
+    if (!rows_ok(rows)) return SFNO_EINVAL;
     if (!planar(p)) return synthesis_from(p, p->inv, spec, xm, x, x_dtype, lat_stats, rows, s);
     const int rc = planar_stage(p, MS_INV, true, spec, xm, rows, s);
     return rc != SFNO_OK ? rc : irfft_launch(p->fft, xm, x, x_dtype, rows, p->nlat, p->mmax, (int)sfno_spectral_ld(rows), s, lat_stats);
@@ -518,14 +520,14 @@ extern "C" int sfno_sht_inverse(const sfno_sht_plan* p, const void* coeffs, floa
 
 // spectral layout -> grid / grid -> spectral layout with the Fourier buffer passed in
 int sfno::analysis_adjoint_launch(const sfno_sht_plan* p, const float* gspec, void* gx, int x_dtype, float* xm, int64_t rows, hipStream_t s) {
-    if (!(p->directions & SFNO_DIR_FORWARD_ADJOINT)) return SFNO_EINVAL;
+    if (!(p->directions & SFNO_DIR_FORWARD_ADJOINT) || !rows_ok(rows)) return SFNO_EINVAL;
     if (!planar(p)) return synthesis_from(p, p->fwd_adj, gspec, xm, gx, x_dtype, nullptr, rows, s);
     const int rc = planar_stage(p, MS_FWD_ADJ, true, gspec, xm, rows, s);
     return rc != SFNO_OK ? rc : sfno_irfft(p, xm, gx, x_dtype, rows, s);
 }
 
 int sfno::synthesis_adjoint_launch(const sfno_sht_plan* p, const void* gx, int x_dtype, float* xm, float* gspec, int64_t rows, hipStream_t s) {
-    if (!(p->directions & SFNO_DIR_INVERSE_ADJOINT)) return SFNO_EINVAL;
+    if (!(p->directions & SFNO_DIR_INVERSE_ADJOINT) || !rows_ok(rows)) return SFNO_EINVAL;
     if (!planar(p)) return analysis_with(p, p->inv_adj, gx, x_dtype, nullptr, xm, gspec, rows, s);
     const int rc = sfno_rfft(p, gx, x_dtype, xm, rows, s);
     return rc != SFNO_OK ? rc : planar_stage(p, MS_INV_ADJ, false, xm, gspec, rows, s);

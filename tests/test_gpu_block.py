@@ -519,3 +519,23 @@ def test_validation_with_gradients_enabled_packs_no_adjoint(lib_built):
     for y in ys:
         y.float().sum().backward()
     assert used() == [True] * 4
+
+
+def test_batches_past_the_row_limit_are_refused(lib_built):
+    """A batch whose rows do not fit the spectral layout's 31-bit row length is refused before anything is launched."""
+    import ctypes
+
+    import makani_amd as ma
+    from makani_amd import block as nb
+    from makani_amd._lib import lib
+
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    with torch.no_grad():
+        c = nb._Call(blk, x, nb.block_params(blk))
+        huge = 1 << 62
+        for batch in ((1 << 25) + 1, 1 << 26, (1 << 31) - 1):        # from 2^29 rows on
+            c.b.batch = batch
+            assert lib.sfno_block_forward(ctypes.byref(c.b), 0, x.data_ptr(), x.data_ptr(), x.data_ptr(), huge, x.data_ptr(), huge, c.stream) == -1
+    torch.cuda.synchronize()
