@@ -28,9 +28,6 @@
 // FFT has an error of that second kind already (relative to the largest value of a latitude row).
 #include "sfno_internal.h"
 
-#include <algorithm>
-#include <cmath>
-
 namespace sfno {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -479,7 +476,7 @@ int legendre_f16_tiles(bool analysis, int64_t ncols, int64_t items, int64_t chun
         const double groups = (double)((ncols + 32 * nt - 1) / (32 * nt));
         const double one = longest * (alone[analysis][0] + alone[analysis][1] * nt) + alone[analysis][2] + alone[analysis][3] * nt;
         const double all = groups * ((double)chunks * per_chunk[analysis][nt - 1] + (double)items * per_item[analysis][nt - 1]) / cus;
-        const double t = std::pow(std::pow(one, 4) + std::pow(all, 4), 0.25);
+        const double one2 = one * one, all2 = all * all, t = one2 * one2 + all2 * all2;      // (the time's fourth power: 0.3 us of a launch less than with std::pow)
         if (nt == 1 || t < best_t) { best_t = t; best = nt; }
     }
     return best;
