@@ -33,9 +33,6 @@ namespace sfno {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef __fp16 fp16x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 typedef int i4 __attribute__((ext_vector_type(4)));
 
 constexpr int LH_TOP = 14;             // scaled magnitudes stay below 2^(TOP + 1)
@@ -44,14 +41,12 @@ constexpr int LH_SH = LH_TOP + 127;    // scaled = x * 2^(SH - E), E = biased ex
 constexpr int LH_EMIN = LH_SH - 127;   // smallest bound: its scale is the largest power of two of fp32 (columns below 2^-112 keep 25 bits above 2^-151)
 
 // resident workgroups per CU: set by the 16 NT accumulator registers and the staged rows held across the matrix phase
-constexpr int lh_occupancy(int nt, bool analysis) { return nt <= 4 ? 4 : 3; }
-
-__device__ __forceinline__ unsigned int lh_pk(float a, float b) { return __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(a, b)); }
+constexpr int lh_occupancy(int nt) { return nt <= 4 ? 4 : 3; }
 
 // COEFFS: the spectral side is the reference layout, complex [rows][lmax][mmax] (zeros above the diagonal included), and no layout pass
 // runs: an order's values lie 8 mmax bytes apart there, eight bytes at a time, so this is for small transforms only (legendre_coeffs_fit).
 template <int NT, bool ANALYSIS, bool COEFFS>
-__global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_kernel(PgemmArgs a) {
+__global__ __launch_bounds__(256, lh_occupancy(NT)) void legendre_f16_kernel(PgemmArgs a) {
     constexpr int TN = 32 * NT;            // columns per workgroup
     constexpr int QN = TN / 4;             // column quads
     // LDS image of one (buffer, panel, plane): column c = 4 j + cc lives in class cc at slot j; a slot is the column's 16 k
@@ -59,7 +54,7 @@ __global__ __launch_bounds__(256, lh_occupancy(NT, ANALYSIS)) void legendre_f16_
     // classes 2 and 3, so that the 16-byte fragment reads of 16 consecutive columns cover all banks
     constexpr int CS = QN * 32 + 128;
     constexpr int PLANE = 4 * CS;
-    constexpr int PLANES = 2 * 2 * 2 * PLANE < 18432 ? 18432 : 2 * 2 * 2 * PLANE;      // [buffer][panel][plane]; at least the 16 KiB of the parity exchange
+    constexpr int PLANES = 2 * 2 * 2 * PLANE < 18432 ? 18432 : 2 * 2 * 2 * PLANE;      // [buffer][panel][plane]; at least the four tiles of 32 x 36 floats of the parity exchange
     __shared__ __align__(16) unsigned char planes[PLANES];
     __shared__ __align__(16) int expo[2][2][TN];   // [buffer][panel][column]: exponent bound the chunk was cut with
 
