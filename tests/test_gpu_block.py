@@ -539,3 +539,103 @@ def test_batches_past_the_row_limit_are_refused(lib_built):
             c.b.batch = batch
             assert lib.sfno_block_forward(ctypes.byref(c.b), 0, x.data_ptr(), x.data_ptr(), x.data_ptr(), huge, x.data_ptr(), huge, c.stream) == -1
     torch.cuda.synchronize()
+
+
+class Rolled(nn.Module):
+    """(a factor would not do: the norms take those of the layers in front of them out again)"""
+
+    def forward(self, w):
+        return w.roll(1, 0)
+
+
+@pytest.mark.parametrize("where", ["filter.filter", "norm0", "norm1", "mlp.fwd.0", "mlp.fwd.3", "outer_skip"])
+def test_parametrised_members(lib_built, where):
+    """A parameter that its module computes is read as the module computes it, in training and in inference, native or not."""
+    import makani_amd as ma
+
+    print(f"case parametrised {where}", flush=True)
+    torch.manual_seed(8)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(2, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    gy = torch.randn_like(x)
+    m = blk.get_submodule(where)
+    nn.utils.parametrize.register_parametrization(m, "weight", Rolled())
+    rolled = passes(blk, x, gy, True)
+    ref = passes(blk, x.float(), gy.float(), False)
+    assert rel(rolled["y"], ref["y"]) < 1.5e-2
+    g = f"{where}.parametrizations.weight.original"
+    assert rel(rolled[g], ref[g]) < 1.5e-2
+    with torch.inference_mode(), torch.autocast("cuda", dtype=torch.bfloat16):
+        assert rel(blk.eval()(x), ref["y"]) < 1.5e-2
+    # (the test sees the order)
+    nn.utils.parametrize.remove_parametrizations(m, "weight", leave_parametrized=False)
+    assert rel(passes(blk.train(), x.float(), gy.float(), False)["y"], ref["y"]) > 3e-2
+
+
+def test_weight_norm_in_the_mlp(lib_built):
+    """weight_norm replaces the parameter by an attribute that a hook sets before each call."""
+    import warnings
+
+    import makani_amd as ma
+
+    torch.manual_seed(9)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(2, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    gy = torch.randn_like(x)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        nn.utils.weight_norm(blk.mlp.fwd[0])
+    with torch.no_grad():
+        blk.mlp.fwd[0].weight_g.mul_(3.0)
+    got, ref = passes(blk, x, gy, True), passes(blk, x.float(), gy.float(), False)
+    assert rel(got["y"], ref["y"]) < 1.5e-2 and rel(got["mlp.fwd.0.weight_g"], ref["mlp.fwd.0.weight_g"]) < 1.5e-2
+
+
+def test_hooks_on_single_members(lib_built):
+    """A hook on any one member is called in training: the block then runs its modules."""
+    import makani_amd as ma
+
+    torch.manual_seed(10)
+    sht, isht = ma.RealSHT(16, 32, grid="legendre-gauss"), ma.InverseRealSHT(16, 32, grid="legendre-gauss")
+    blk = make_block(sht, isht, 16, 2.0)
+    x = torch.randn(1, 16, 16, 32, device="cuda").to(torch.bfloat16)
+    gy = torch.randn_like(x)
+    names = ["filter", "filter.filter", "norm0", "act_layer0", "mlp", "mlp.fwd", *(f"mlp.fwd.{i}" for i in range(len(blk.mlp.fwd))), "norm1", "outer_skip"]
+    for name in names:
+        for register in ("register_forward_hook", "register_forward_pre_hook"):
+            seen = []
+            handle = getattr(blk.get_submodule(name), register)(lambda *a: seen.append(1))
+            passes(blk, x, gy, True)
+            handle.remove()
+            assert seen, (name, register)
+
+
+def test_members_of_wrapped_modules(lib_built):
+    """member() and has_member() find what attribute look-up finds: tables, class attributes, instance attributes and what a wrapper hands on."""
+    from makani_amd.block import has_member, member
+
+    class Wrapper(nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def __getattr__(self, name):
+            try:
+                return super().__getattr__(name)
+            except AttributeError:
+                return getattr(super().__getattr__("inner"), name)
+
+    conv = nn.Conv2d(3, 4, 1, bias=False)
+    conv.note = "here"
+    conv.register_buffer("table", torch.zeros(2))
+    for m in (conv, Wrapper(conv)):
+        for name in ("weight", "bias", "table", "note", "in_channels", "forward"):
+            assert has_member(m, name)
+            a, b = member(m, name), getattr(m, name)
+            assert a is b or a == b, name
+        assert not has_member(m, "absent")
+        with pytest.raises(AttributeError):
+            member(m, "absent")
+    assert member(Wrapper(conv), "inner") is conv

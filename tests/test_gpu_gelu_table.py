@@ -1,5 +1,6 @@
 """The training GELU and its derivative by table (convolutions of more than 96 output channels, one to three row tiles per wavefront) against the formulas that narrower
-convolutions evaluate, on every bf16 value: the same activations and derivatives, NaN at the same places."""
+convolutions evaluate: the derivative at every bf16 value, the activation at every finite one through the product and at infinities, NaN and every exponent through the bias, the same bits and
+NaN at the same places; and the layers that take the formula all the same."""
 import ctypes
 
 import pytest
@@ -39,6 +40,44 @@ def test_table_is_the_formula(lib_built, channels):
     assert torch.equal(torch.isnan(g0), torch.isnan(g1))
     ok = ~torch.isnan(g0)
     assert torch.equal(g0[ok].view(torch.int16), g1[ok].view(torch.int16))
+
+
+@pytest.mark.parametrize("channels", [97, 128, 200, 300, 384])
+def test_every_value_through_the_bias(lib_built, channels):
+    """Infinities and NaN reach the activation by the bias (in the product they would meet the other weights' zeros)."""
+    from makani_amd import pointwise as pw
+    from makani_amd._lib import check, lib
+
+    print(f"case gelu table, bias {channels}", flush=True)
+    x = torch.zeros(1, 8, 8, dtype=torch.bfloat16, device="cuda")
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+
+    def activations(O, values):
+        """of `values` [n], n a multiple of O: pixel 0 of O channels with these biases, call by call"""
+        w = pw.packed_weight(torch.zeros(O, 8, device="cuda"))
+        ys, zs = [], []
+        for b in values.split(O):
+            y, z = (torch.empty(O, 8, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+            check(lib.sfno_pointwise_conv_gelu(ptr(x), ptr(w), ptr(b), ptr(y), ptr(z), 1, 8, O, 8, pw._stream(x.device)), "forward")
+            ys.append(y[:, 0])
+            zs.append(z[:, 0])
+        return torch.cat(ys).cpu(), torch.cat(zs).cpu()
+
+    # every exponent of either sign with a few mantissas, infinities and NaN among them
+    bits = torch.arange(512, dtype=torch.int32)[:, None] * 128 + torch.tensor([0, 1, 37, 64, 127], dtype=torch.int32)
+    z = bits.flatten().to(torch.int16).view(torch.bfloat16)
+    n = -(-z.numel() // channels) * channels
+    values = torch.zeros(-(-n // 64) * 64)
+    values[:z.numel()] = z.float()
+    values = values.cuda()
+    (y0, z0), (y1, z1) = activations(64, values), activations(channels, values[:n])
+    y0, z0, y1, z1 = (t[:z.numel()] for t in (y0, z0, y1, z1))
+    assert bool(torch.isinf(z0).any() and torch.isnan(z0).any())
+    assert torch.equal(torch.isnan(z0), torch.isnan(z1)) and torch.equal(torch.isnan(y0), torch.isnan(y1))
+    ok = ~torch.isnan(z0)
+    assert torch.equal(z0[ok].view(torch.int16), z1[ok].view(torch.int16))
+    ok = ~torch.isnan(y0) & ~(z.abs() < 2.0**-120)
+    assert torch.equal(y0[ok].view(torch.int16), y1[ok].view(torch.int16))
 
 
 @pytest.mark.parametrize("K,O,P", [(24, 160, 840008), (64, 200, 671112), (73, 256, 524296), (40, 320, 420008), (24, 384, 349568)])
