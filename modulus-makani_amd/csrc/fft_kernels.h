@@ -455,12 +455,12 @@ __device__ __forceinline__ int tile_orders(const int* kept, int lat, int mmax) {
 // registers and stores both halves together, and the inverse kernel requests both halves together.
 //
 // DIFF: the transform of x - x2, formed as a batch is copied to LDS.  The rows of x2 are asked for there and not a tile ahead (the
-// registers are at their limit), their latency is the other workgroups' to hide: 73 x 721 x 1440 in 210 us (0.93 GB, 4.4 TB/s), where the
-// transform of a stored difference took 137 and the pass that stores it 183.
+// registers are at their limit), their latency is the other workgroups' to hide: 73 x 721 x 1440 in 186 us (0.93 GB, 5.0 TB/s), where the
+// transform of a stored difference takes 137 and the pass that stores it 183.
 //
 // both (with DIFF): the transform of x2 as well, its columns `width` floats behind those of x - x2.  Its tiles take turns with those of the difference on
 // one XCD, so that the rows of x2 are read twice at about the same time
-// (73 x 721 x 1440: 300 us for both, 187 and 118 one after the other).
+// (73 x 721 x 1440: 309 us for both, 186 and 137 one after the other).
 //
 // SHORT: the last batch of a latitude is not full (73 channels are 36.5 pairs in batches of 4).  A kernel of its own, for float32 fields: the comparisons cost
 // whole batches up to 2 % (721 x 1440: 73 channels 146 -> 145 us, inverse 154 -> 150; 9 channels 31.5 -> 28.8; 3 channels of 360 x 720 12.0 -> 9.9).
